@@ -196,8 +196,16 @@ struct CrFace {
   // per face)
   bool qpat = false;
   int nsup = 0;
+  std::vector<int> h_sup;          // d_sup on the host
+  unsigned long long support = 0;  // a new number for every support built
   crimson::DBuf<int> d_sup, d_qptr, d_qa, d_qk;
   crimson::DBuf<double> d_q;  // the functional's coefficients, per solve
+};
+
+// One entry of the coupled faces' merged supports: a node, the face (its place among
+// the coupled ones) and the node's place in that face's support.
+struct CrFaceEnt {
+  int node, f, s;
 };
 
 // memLS matrix handle.  The matrix of block size vdof (1..4) is held as
@@ -220,5 +228,21 @@ struct crimson_lhs {
   crimson::DBuf<double> d_Gt;     // [3][nnz] when !gt_is_d
   crimson::DBuf<float> d_Gt32;    // the same for an FP32 matrix
   std::vector<CrFace> face;
+  // the coupled faces' merged supports and their first entries per 256 nodes,
+  // for the faces whose supports fent_sig lists
+  std::vector<unsigned long long> fent_sig;
+  crimson::DBuf<CrFaceEnt> d_fent;
+  crimson::DBuf<int> d_ftptr;
+  // the Schur complement of the NS solver's CG on the graph's two-ring: 0 not
+  // looked at yet, 1 its pattern is here (schur_nnz entries, schur_row at most in
+  // a row; columns as offsets from the row in d_scol16 where they fit), 2 this
+  // graph keeps the two-pass operator
+  int schur = 0, schur_row = 0;
+  long long schur_nnz = 0;
+  int band = 0;  // largest |column - row| (with d_col16)
+  crimson::DBuf<int> d_sptr, d_scol;
+  crimson::DBuf<short> d_scol16;
+  crimson::DBuf<double> d_S;
+  crimson::DBuf<float> d_S32;
   hipEvent_t ev0 = nullptr, ev1 = nullptr;
 };

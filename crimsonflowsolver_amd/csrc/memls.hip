@@ -144,13 +144,18 @@ __global__ void __launch_bounds__(256) spmv_kernel(int nNo, const int *__restric
 // Z(0:3, j) = (Ps_j, W o t1_j) (the same operations, in the same order, as
 // the two separate products).
 constexpr int kNarrowLanes = 4;
+// Workgroups of a CG sweep at most (8 per CU): each writes one part of a dot,
+// and every workgroup of the next sweep sums all of them.
+constexpr int kCgGrid = 2048;
 
-// A coupled face of the Schur CG (ADDBCMUL's PRE, memLS.f90:1719-1735):
-// its nodes, valM, coefficient -res/(1 + res nS), and the face dot
-// S_f = valM_f . t1 restated as a functional of the G product's operand,
-// S_f = sum_j q_j Ps_j over the support sup (the columns of the face nodes'
-// rows), q_j = sum over the pairs (a, k) of column j of
-// valM(i, a) W_u(i, glob(a)) G_i(k), i < min(dof, 3).
+// A coupled face of the Schur CG (ADDBCMUL's PRE, memLS.f90:1719-1735).  PRE
+// adds coef_f S_f valM_f to t1 = G P with S_f = valM_f . t1; with Gt = -G^T
+// (DEPART) that is the symmetric rank-one term c_f q_f q_f^T on the
+// Schur operator, q_f = W_p o (G^T (W_u o valM_f)) on the columns of the
+// face nodes' rows (sup): q_j = W_p(j) sum over the pairs (a, k) of column j
+// of valM(i, a) W_u(i, glob(a)) G_i(k), i < min(dof, 3).  So S_f = q_f . P is
+// formed from the direction, the denominator P . SP gains c_f S_f^2 and the
+// residual update alpha c_f S_f q_f: the operator's kernels see no face.
 struct FaceDev {
   const int *glob;
   const double *valM;
@@ -162,16 +167,19 @@ struct FaceDev {
   const double *q;
   int nsup;
 };
-// Workgroups per face computing S_f's partial sums beside the G product.
+// Workgroups per face computing S_f's partial sums beside the direction update.
 constexpr int kFaceDotBlocks = 4;
-
-// The Schur operator's vectors pre-multiplied by their column scaling, so
-// that its two row kernels gather no W: Ps = W_p o P (written by the CG's
-// direction update, scale_p_kernel for the first direction); the G product
-// writes t1 = W_u o (G Ps) and, per node i, Z(0:3, i) = (Ps_i, W_u o t1_i):
-// the Schur pass gathers both of its operands of a column as one 4-wide
-// entry (two 16-byte loads in FP64, one in FP32).  Same products in the
-// same order as the unscaled kernels.
+// The faces' supports merged for the residual update: the entries (node,
+// face, place in the face's support) sorted by node, then face; tptr[t] is
+// the first entry of nodes 256 t and above.
+using FaceEnt = CrFaceEnt;
+struct FaceList {
+  int nfc;               // coupled faces
+  const FaceDev *fd;
+  const FaceEnt *ent;
+  const int *tptr;       // (N / 256 rounded up) + 1 entries
+  double *part;          // kFaceDotBlocks partial sums of S_f per face
+};
 
 // Wave-level sum (64 lanes) then across the 4 waves of a 256-thread group.
 template <class T>
@@ -208,8 +216,12 @@ __device__ inline T block_sum_all(T v, T *sh) {
 // product is not added), so the accumulation order is the plain loop's.
 constexpr int kNarrowUnroll = 4;
 
-// `done` (may be null): the CG's converged flag; the remaining iterations of
-// a batch launched after convergence return at once.
+// The Schur operator as two passes, for a matrix whose complement is not
+// formed (schur_pattern): on Ps = W_p o P the G product writes
+// Z(0:3, i) = (Ps_i, W_u o (W_u o G Ps)_i), and the second pass
+// gathers both of its operands of a column as one 4-wide entry (two 16-byte
+// loads in FP64, one in FP32): SP_i = W_i (sum_j L_ij Ps_j - Gt_ij . Z(1:3, j)) + fix_i P_i.
+// `done`: the CG's converged flag; launches after it return at once.
 template <class T>
 __global__ void scale_p_kernel(int n, const T *__restrict__ W, int wdof, int off, const T *__restrict__ x,
                                T *__restrict__ y, const double *__restrict__ done) {
@@ -217,49 +229,13 @@ __global__ void scale_p_kernel(int n, const T *__restrict__ W, int wdof, int off
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i < n) y[i] = W[off + (size_t)wdof * i] * x[i];
 }
-// The first nfc * kFaceDotBlocks workgroups form the coupled faces' dots
-// from Ps (fpart[f * kFaceDotBlocks + b]: the b-th workgroup's share, entries
-// s = b * 256 + t + 1024 u), so that no launch between the two row kernels
-// waits for t1; the rest form t1.
 template <class T, class IX, int U = kNarrowUnroll>
 __global__ void __launch_bounds__(256) g_product_kernel(int nNo, const int *__restrict__ rowptr,
                                                         const IX *__restrict__ col, MatView<T> G,
-                                                        const T *__restrict__ Ps, T *__restrict__ t1,
-                                                        T *__restrict__ t1s, int nfc,
-                                                        const FaceDev *__restrict__ fd,
-                                                        double *__restrict__ fpart,
+                                                        const T *__restrict__ Ps, T *__restrict__ Z,
                                                         const double *__restrict__ done) {
   if (done && *done != 0.0) return;
-  const unsigned nx = (unsigned)nfc * kFaceDotBlocks;
-  if (blockIdx.x < nx) {
-    __shared__ double sh[4];
-    const int f = blockIdx.x / kFaceDotBlocks, b = blockIdx.x % kFaceDotBlocks;
-    const int *sup = fd[f].sup;
-    const double *q = fd[f].q;
-    const int ns = fd[f].nsup;
-    constexpr int kStride = 256 * kFaceDotBlocks;
-    double s = 0.0;
-    for (int s0 = b * 256 + threadIdx.x; s0 < ns; s0 += kStride * 4) {
-      int j[4];
-      double qv[4];
-#pragma unroll
-      for (int u = 0; u < 4; ++u) {
-        const int e = min(s0 + kStride * u, ns - 1);
-        j[u] = sup[e];
-        qv[u] = q[e];
-      }
-      T pv[4];
-#pragma unroll
-      for (int u = 0; u < 4; ++u) pv[u] = Ps[j[u]];
-#pragma unroll
-      for (int u = 0; u < 4; ++u)
-        if (s0 + kStride * u < ns) s += qv[u] * (double)pv[u];
-    }
-    s = block_sum(s, sh);
-    if (threadIdx.x == 0) fpart[blockIdx.x] = s;
-    return;
-  }
-  const int gid = crimson::xcd_block(kRowXcdChunk, blockIdx.x - nx, gridDim.x - nx) * blockDim.x + threadIdx.x;
+  const int gid = crimson::xcd_block(kRowXcdChunk) * blockDim.x + threadIdx.x;
   const int row = gid / kNarrowLanes;
   const int lane = threadIdx.x % kNarrowLanes;
   T acc[3] = {T(0), T(0), T(0)};
@@ -301,20 +277,16 @@ __global__ void __launch_bounds__(256) g_product_kernel(int nNo, const int *__re
 #pragma unroll
     for (int r = 0; r < 3; ++r) {
       const T w = G.W[G.r0 + r + (size_t)G.wdof * row];
-      T v = w * acc[r];
-      v *= T(1);
-      t1[r + (size_t)3 * row] = v;
-      z[1 + r] = w * v;
+      z[1 + r] = w * (w * acc[r]);
     }
-    store4(t1s + (size_t)4 * row, z);
+    store4(Z + (size_t)4 * row, z);
   }
 }
 template <class T, class IX, int U = kNarrowUnroll>
 __global__ void __launch_bounds__(256) schur_kernel(int nNo, const int *__restrict__ rowptr,
                                                     const IX *__restrict__ col, MatView<T> Lv, MatView<T> Gv,
-                                                    const T *__restrict__ P, const T *__restrict__ Ps,
-                                                    const T *__restrict__ t1s, T *__restrict__ SP,
-                                                    const double *__restrict__ done) {
+                                                    const T *__restrict__ P, const T *__restrict__ Z,
+                                                    T *__restrict__ SP, const double *__restrict__ done) {
   if (done && *done != 0.0) return;
   const int gid = crimson::xcd_block(kRowXcdChunk) * blockDim.x + threadIdx.x;
   const int row = gid / kNarrowLanes;
@@ -340,7 +312,7 @@ __global__ void __launch_bounds__(256) schur_kernel(int nNo, const int *__restri
         b1[u] = d1[kc[u]];
         b2[u] = d2[kc[u]];
         T z[4];
-        load4(t1s + (size_t)4 * j[u], z);  // (Ps_j, W_u o t1_j)
+        load4(Z + (size_t)4 * j[u], z);
         ps[u] = z[0];
         x0[u] = z[1];
         x1[u] = z[2];
@@ -364,12 +336,238 @@ __global__ void __launch_bounds__(256) schur_kernel(int nNo, const int *__restri
   if (row < nNo && lane == 0) {
     T v = Lv.W[Lv.r0 + (size_t)Lv.wdof * row] * aL;
     if (Lv.fix) v += Lv.fix[Lv.r0 + (size_t)Lv.wdof * row] * P[row];
-    v *= T(1);
     const T t2 = Gv.W[Gv.r0 + (size_t)Gv.wdof * row] * aG;
-    SP[row] = v + T(-1) * t2;
+    SP[row] = v - t2;
   }
 }
 
+// ----- the Schur complement formed explicitly -----
+// S = W_p (L - Gt W_u^2 G) W_p + fix on the graph's two-ring (a node's
+// neighbours' neighbours), one row kernel per CG iteration instead of the
+// two passes above.
+// What it saves: on the Kuhn meshes a row has 65 entries of S (10 bytes each
+// with the 2-byte column) against 14.7 blocks of seven planes read in two
+// passes (60 bytes each), and one launch less; the vector P is gathered
+// directly (the scaling is in S).
+// The pattern is a property of the graph: built once per handle on the
+// device, one wave per row, the union of the neighbours' rows in an LDS hash
+// set.  A row with more than kSchurRow entries (or an S of more bytes than
+// the passes read: schur_pattern) keeps the two passes.
+constexpr int kSchurRow = 320;   // entries of a row of S at most: 16 rows' staging fits 64 KB of LDS
+constexpr int kSchurHash = 512;  // LDS hash slots per row, a power of two above kSchurRow
+// Orders LDS accesses of the lanes of one wavefront.
+__device__ inline void wave_lds_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+// FILL false: cnt[row] = the row's entries (kSchurRow + 1 when it has more);
+// FILL true: the row's columns, ascending, at scol[sptr[row]] (as offsets
+// from the row when OX is short).
+template <class IX, class OX, bool FILL>
+__global__ void __launch_bounds__(256) schur_pattern_kernel(int nNo, const int *__restrict__ rowptr,
+                                                            const IX *__restrict__ col, int *__restrict__ cnt,
+                                                            const int *__restrict__ sptr, OX *__restrict__ scol) {
+  __shared__ int key_all[4][kSchurHash];
+  __shared__ int list_all[FILL ? 4 : 1][kSchurRow];
+  __shared__ int num_all[4];
+  const int w = threadIdx.x / 64, lane = threadIdx.x % 64;
+  const int row = blockIdx.x * 4 + w;
+  if (row >= nNo) return;  // whole waves: nothing below synchronises the workgroup
+  int *key = key_all[w];
+  int *num = num_all + w;
+  for (int t = lane; t < kSchurHash; t += 64) key[t] = -1;
+  if (lane == 0) *num = 0;
+  wave_lds_sync();
+  bool over = false;
+  for (int k = rowptr[row]; k < rowptr[row + 1]; ++k) {
+    const int j = col_at(col, k, row);
+    const int m1 = rowptr[j + 1];
+    for (int m = rowptr[j] + lane; m < m1; m += 64) {
+      const int c = col_at(col, m, j);
+      unsigned h = ((unsigned)c * 2654435761u) >> 23;
+      for (int t = 0; t < kSchurHash; ++t, h = (h + 1) & (kSchurHash - 1)) {  // ends when the table is full
+        const int old = atomicCAS(&key[h], -1, c);
+        if (old == -1) atomicAdd(num, 1);
+        if (old == -1 || old == c) break;
+      }
+    }
+    wave_lds_sync();
+    if (*(volatile int *)num > kSchurRow) {
+      over = true;
+      break;
+    }
+  }
+  if (!FILL) {
+    if (lane == 0) cnt[row] = over ? kSchurRow + 1 : *num;
+    return;
+  }
+  // the keys compacted, then each written at its rank
+  int *list = list_all[FILL ? w : 0];
+  int n = 0;
+  for (int t = lane; t < kSchurHash; t += 64) {
+    const bool has = key[t] >= 0;
+    const unsigned long long mask = __ballot(has);
+    const int at = n + __popcll(mask & ((1ull << lane) - 1ull));
+    if (has && at < kSchurRow) list[at] = key[t];
+    n += __popcll(mask);
+  }
+  wave_lds_sync();
+  const int s0 = sptr[row];
+  n = min(n, sptr[row + 1] - s0);
+  for (int t = lane; t < n; t += 64) {
+    const int c = list[t];
+    int rank = 0;
+    for (int u = 0; u < n; ++u) rank += list[u] < c;
+    scol[s0 + rank] = (OX)(sizeof(OX) == 2 ? c - row : c);
+  }
+}
+// The values of S, 16 lanes per row: the row's accumulators and columns in
+// LDS; for each neighbour j the lanes take the entries of row j of G (all of
+// different columns, so no two lanes add to one accumulator), in row order;
+// sums in FP64.
+// Dynamic LDS: 16 rows x maxn (double, int).
+template <class T, class IX, class OX>
+__global__ void __launch_bounds__(256) schur_values_kernel(int nNo, const int *__restrict__ rowptr,
+                                                           const IX *__restrict__ col, MatView<T> Lv, MatView<T> Gtv,
+                                                           MatView<T> Gv, const int *__restrict__ sptr,
+                                                           const OX *__restrict__ scol, T *__restrict__ S, int maxn) {
+  extern __shared__ double dyn[];
+  const int g = threadIdx.x / 16, lane = threadIdx.x % 16;
+  double *acc = dyn + (size_t)g * maxn;
+  int *sc = reinterpret_cast<int *>(dyn + (size_t)16 * maxn) + (size_t)g * maxn;
+  const int row = crimson::xcd_block(kRowXcdChunk) * 16 + g;
+  const bool live = row < nNo;
+  const int s0 = live ? sptr[row] : 0, n = live ? sptr[row + 1] - s0 : 0;
+  for (int t = lane; t < n; t += 16) {
+    sc[t] = col_at(scol, s0 + t, row);
+    acc[t] = 0.0;
+  }
+  wave_lds_sync();
+  auto find = [&](int c) {  // c is in the row
+    int lo = 0, hi = n - 1;
+    while (lo < hi) {
+      const int mid = (lo + hi) >> 1;
+      if (sc[mid] < c)
+        lo = mid + 1;
+      else
+        hi = mid;
+    }
+    return lo;
+  };
+  const T *lp = Lv.base + (size_t)Lv.plane[0] * Lv.nnz;
+  const T *b0 = Gtv.base + (size_t)Gtv.plane[0] * Gtv.nnz, *b1 = Gtv.base + (size_t)Gtv.plane[1] * Gtv.nnz,
+          *b2 = Gtv.base + (size_t)Gtv.plane[2] * Gtv.nnz;
+  const T *g0 = Gv.base + (size_t)Gv.plane[0] * Gv.nnz, *g1 = Gv.base + (size_t)Gv.plane[4] * Gv.nnz,
+          *g2 = Gv.base + (size_t)Gv.plane[8] * Gv.nnz;
+  const int k0 = live ? rowptr[row] : 0, k1 = live ? rowptr[row + 1] : 0;
+  for (int kb = k0; kb < k1; kb += 16) {
+    const int k = kb + lane;
+    int m0 = 0, m1 = 0, j = 0;
+    double d0 = 0.0, d1 = 0.0, d2 = 0.0;
+    if (k < k1) {
+      j = col_at(col, k, row);
+      m0 = rowptr[j];
+      m1 = rowptr[j + 1];
+      const T *w = Gv.W + Gv.r0 + (size_t)Gv.wdof * j;
+      d0 = (double)b0[k] * ((double)w[0] * (double)w[0]);
+      d1 = (double)b1[k] * ((double)w[1] * (double)w[1]);
+      d2 = (double)b2[k] * ((double)w[2] * (double)w[2]);
+      acc[find(j)] += (double)lp[k];
+    }
+    wave_lds_sync();
+    const int cnt = min(16, k1 - kb);
+    for (int t = 0; t < cnt; ++t) {
+      const int a0 = __shfl(m0, t, 16), a1 = __shfl(m1, t, 16), jj = __shfl(j, t, 16);
+      const double e0 = __shfl(d0, t, 16), e1 = __shfl(d1, t, 16), e2 = __shfl(d2, t, 16);
+      for (int m = a0 + lane; m < a1; m += 16) {
+        const double v = e0 * (double)g0[m] + e1 * (double)g1[m] + e2 * (double)g2[m];
+        acc[find(col_at(col, m, jj))] -= v;
+      }
+      wave_lds_sync();
+    }
+  }
+  if (!live) return;
+  const double wr = (double)Lv.W[Lv.r0 + (size_t)Lv.wdof * row];
+  const double fx = Lv.fix ? (double)Lv.fix[Lv.r0 + (size_t)Lv.wdof * row] : 0.0;
+  for (int t = lane; t < n; t += 16) {
+    const int c = sc[t];
+    double v = wr * acc[t] * (double)Lv.W[Lv.c0 + (size_t)Lv.wdof * c];
+    if (c == row) v += fx;
+    S[s0 + t] = (T)v;
+  }
+}
+// SP = S P and the workgroup's part of P . SP, 16 lanes per row.  At most
+// kCgGrid workgroups walk the row tiles, so that the residual update sums at
+// most that many parts; the next tile's row pointers are loaded during a tile.
+// Bound by the read of S: 65 entries per row and 458,000 rows (297 MB) take 74 us,
+// 4.0 TB/s of a copy's 4.65; the two passes it replaces took 92 us.  A lane loads kSUnroll
+// entries at once, so that the Kuhn meshes' rows (65 at most) are one turn: 98 us
+// with four, 90 with 8 lanes of eight, 99 with 32 lanes of two, 95 with a wave
+// per run of four rows summed through LDS; unbounded grid 67 us, but then a dot
+// kernel of its own follows.
+constexpr int kSLanes = 16, kSUnroll = 5;
+template <class T, class OX>
+__global__ void __launch_bounds__(256) s_product_kernel(int nNo, int ntile, const int *__restrict__ sptr,
+                                                        const OX *__restrict__ scol, const T *__restrict__ S,
+                                                        const T *__restrict__ P, T *__restrict__ SP,
+                                                        double *__restrict__ dpart, const double *__restrict__ done) {
+  __shared__ double sh[4];
+  const double stop = *done;
+  const int lane = threadIdx.x % kSLanes;
+  auto row_of = [&](int vb) {
+    return (int)crimson::xcd_block(kRowXcdChunk, vb, ntile) * (256 / kSLanes) + (int)threadIdx.x / kSLanes;
+  };
+  int rown = row_of(blockIdx.x), kbn = sptr[min(rown, nNo)], ken = sptr[min(rown + 1, nNo)];
+  if (stop != 0.0) return;
+  double den = 0.0;
+  for (int vb = blockIdx.x; vb < ntile; vb += gridDim.x) {
+    const int row = rown, kb = kbn, ke = ken;  // rows past the last one: kb = ke
+    const int vn = vb + gridDim.x;
+    if (vn < ntile) {
+      rown = row_of(vn);
+      kbn = sptr[min(rown, nNo)];
+      ken = sptr[min(rown + 1, nNo)];
+    }
+    T acc = T(0);
+    for (int k = kb + lane; k < ke; k += kSLanes * kSUnroll) {
+      T v[kSUnroll], x[kSUnroll];
+      int j[kSUnroll];
+#pragma unroll
+      for (int u = 0; u < kSUnroll; ++u) {
+        const int kc = min(k + kSLanes * u, ke - 1);
+        j[u] = col_at(scol, kc, row);
+        v[u] = S[kc];
+      }
+#pragma unroll
+      for (int u = 0; u < kSUnroll; ++u) x[u] = P[j[u]];
+#pragma unroll
+      for (int u = 0; u < kSUnroll; ++u)
+        if (k + kSLanes * u < ke) acc += v[u] * x[u];
+    }
+#pragma unroll
+    for (int off = kSLanes / 2; off > 0; off >>= 1) acc += __shfl_xor(acc, off, kSLanes);
+    if (row < nNo && lane == 0) {
+      SP[row] = acc;
+      den += (double)P[row] * (double)acc;
+    }
+  }
+  den = block_sum(den, sh);
+  if (threadIdx.x == 0) dpart[blockIdx.x] = den;
+}
+// The sum of n <= kCgGrid parts, in every thread, always in the same order: every
+// thread's parts are loaded together (one wait instead of eight).
+__device__ inline double sum_parts(const double *__restrict__ part, int n, double more, double *sh) {
+  double v[kCgGrid / 256];
+#pragma unroll
+  for (int u = 0; u < kCgGrid / 256; ++u) {
+    const int b = threadIdx.x + 256 * u;
+    v[u] = b < n ? part[b] : 0.0;
+  }
+#pragma unroll
+  for (int u = 0; u < kCgGrid / 256; ++u) more += v[u];
+  return block_sum_all(more, sh);
+}
 
 // partial[blk][j] = sum over this block's chunk of U_j . v for j < m, and
 // partial[blk][m] = v . v when self != 0.  U_j = U0 + j * ustride.  Vectors
@@ -581,32 +779,7 @@ __global__ void face_axpy_kernel(int n, int xdof, int fdof, const int *__restric
   const double s = (coefp ? *coefp : coef) * *S;
   for (int i = 0; i < nc; ++i) Y[i + (size_t)xdof * glob[a]] += (T)(valM[i + (size_t)fdof * a] * s);
 }
-// A coupled face on the device, with its PRE coefficient -res/(1 + res nS)
-// (memLS.f90:1096-1118 with BCPRE's nS).
-// ADDBCMUL's PRE on the Schur CG's G product t1 (3, N): face by face
-// t1 += coef_f S_f valM_f, with Z(1:3) = W_u o t1 rewritten at the same nodes
-// (one launch per face, since faces may share nodes).  S_f, every face's dot
-// of the unmodified t1, is the sum of its kFaceDotBlocks partials from the G
-// product (summed here in a fixed order).
-template <class T>
-__global__ void __launch_bounds__(256) face_pre_apply_kernel(FaceDev F, const double *__restrict__ part,
-                                                             T *__restrict__ t1, T *__restrict__ t1s,
-                                                             const T *__restrict__ W, int wdof,
-                                                             const double *__restrict__ done) {
-  if (done && *done != 0.0) return;
-  const int a = blockIdx.x * blockDim.x + threadIdx.x;
-  if (a >= F.nNo) return;
-  const int nc = F.dof < 3 ? F.dof : 3;
-  double S = 0.0;
-#pragma unroll
-  for (int b = 0; b < kFaceDotBlocks; ++b) S += part[b];
-  const double sc = (F.coefp ? *F.coefp : F.coef) * S;
-  const size_t g = F.glob[a];
-  for (int i = 0; i < nc; ++i) t1[i + 3 * g] += (T)(F.valM[i + (size_t)F.dof * a] * sc);
-#pragma unroll
-  for (int c = 0; c < 3; ++c) t1s[1 + c + 4 * g] = W[c + (size_t)wdof * g] * t1[c + 3 * g];
-}
-// The same three face operations for every coupled face in one launch, when
+// The same two face operations for every coupled face in one launch, when
 // the faces share no node (then the faces' updates commute): one
 // 1024-thread workgroup per face for the dots (face_dot_kernel's order), and
 // a grid row per face for the updates.  Per face the arithmetic is the
@@ -643,32 +816,11 @@ __global__ void face_axpy_multi_kernel(const FaceDev *__restrict__ fd, int xdof,
   const double s = (pre ? (F.coefp ? *F.coefp : F.coef) : F.res) * S[blockIdx.y];
   for (int i = 0; i < nc; ++i) Y[i + (size_t)xdof * F.glob[a]] += (T)(F.valM[i + (size_t)F.dof * a] * s);
 }
-template <class T>
-__global__ void __launch_bounds__(256) face_pre_apply_multi_kernel(const FaceDev *__restrict__ fd,
-                                                                   const double *__restrict__ part,
-                                                                   T *__restrict__ t1, T *__restrict__ t1s,
-                                                                   const T *__restrict__ W, int wdof,
-                                                                   const double *__restrict__ done) {
-  if (done && *done != 0.0) return;
-  const FaceDev F = fd[blockIdx.y];
-  const int a = blockIdx.x * blockDim.x + threadIdx.x;
-  if (a >= F.nNo) return;
-  const int nc = F.dof < 3 ? F.dof : 3;
-  const double *pf = part + (size_t)kFaceDotBlocks * blockIdx.y;
-  double Sv = 0.0;
-#pragma unroll
-  for (int b = 0; b < kFaceDotBlocks; ++b) Sv += pf[b];
-  const double sc = (F.coefp ? *F.coefp : F.coef) * Sv;
-  const size_t g = F.glob[a];
-  for (int i = 0; i < nc; ++i) t1[i + 3 * g] += (T)(F.valM[i + (size_t)F.dof * a] * sc);
-#pragma unroll
-  for (int c = 0; c < 3; ++c) t1s[1 + c + 4 * g] = W[c + (size_t)wdof * g] * t1[c + 3 * g];
-}
 // The face functional's coefficients q (FaceDev), one thread per support
 // column, its pairs in their stored order, in FP64.
 template <class T>
-__global__ void face_q_kernel(int nsup, const int *__restrict__ qptr, const int *__restrict__ qa,
-                              const int *__restrict__ qk, const int *__restrict__ glob,
+__global__ void face_q_kernel(int nsup, const int *__restrict__ sup, const int *__restrict__ qptr,
+                              const int *__restrict__ qa, const int *__restrict__ qk, const int *__restrict__ glob,
                               const double *__restrict__ valM, int dof, MatView<T> G, double *__restrict__ q) {
   const int s = blockIdx.x * blockDim.x + threadIdx.x;
   if (s >= nsup) return;
@@ -681,7 +833,7 @@ __global__ void face_q_kernel(int nsup, const int *__restrict__ qptr, const int 
       v += valM[i + (size_t)dof * a] * (double)G.W[G.r0 + i + (size_t)G.wdof * g] *
            (double)G.base[(size_t)G.plane[4 * i] * G.nnz + k];
   }
-  q[s] = v;
+  q[s] = v * (double)G.W[G.c0 + (size_t)G.wdof * sup[s]];
 }
 // DGKS decision: gate = ||w'||^2 < 0.5 ||w||^2
 __global__ void dgks_kernel(const double *__restrict__ n0, const double *__restrict__ n1, int *__restrict__ gate,
@@ -713,7 +865,19 @@ __global__ void gt_kernel(size_t nnz, const T *__restrict__ V, const int *__rest
 }
 
 // ----- CG (device-resident iterations with a convergence flag) -----
-// scal layout: 0 err, 1 errO, 2 eps2, 3 den, 4 (unused), 5 done, 6 itr, 7 mItr, 8 suc
+// Three launches per iteration on the Schur complement: SP = S P with the
+// parts of P . SP (s_product_kernel), the residual update with the parts of
+// R . R, and the direction update, which also advances the state.  Every
+// workgroup sums the parts it needs itself, in one fixed order, so that no
+// one-workgroup launch stands between two sweeps; before, the product, the
+// face term, the dot, the update, the error and the direction took seven
+// launches (28.3 us of kernels per iteration at 36,000 nodes, 120 us at
+// 458,000).
+// The state is kept twice (kCgState doubles each): iteration k reads copy k & 1 and
+// the direction update writes the other, so that no workgroup reads what
+// another is writing.
+// State: 0 err, 1 errO, 2 eps2, 3 alpha, 5 done, 6 itr, 7 mItr, 8 suc.
+constexpr int kCgState = 16;
 // Top-of-iteration test of CGRAD (memLS.f90:413-427): stop at mItr or when
 // err < eps^2; otherwise errO = err and count the iteration.
 __device__ inline void check_next(double *scal) {
@@ -730,66 +894,208 @@ __device__ inline void check_next(double *scal) {
   scal[1] = scal[0];  // errO = err
   scal[6] += 1.0;
 }
-__global__ void cg_check_kernel(double *__restrict__ scal) { check_next(scal); }
-// X += alpha P ; R -= alpha SP ; partial of R.R.  den = P . SP is summed
-// from its nblk workgroup partials by every workgroup (reduce_kernel's
-// order, so the same bits in each), which saves a launch per iteration.
-template <class T>
-__global__ void __launch_bounds__(256) cg_update_kernel(size_t L, const double *__restrict__ scal,
-                                                        const T *__restrict__ dpart, int nblk,
-                                                        T *__restrict__ X, T *__restrict__ R,
-                                                        const T *__restrict__ P, const T *__restrict__ SP,
-                                                        T *__restrict__ partial) {
-  if (scal[5] != 0.0) return;
-  __shared__ T sh[4];
-  T d = T(0);
-  for (int b = threadIdx.x; b < nblk; b += 256) d += dpart[b];
-  const T den = block_sum_all(d, sh);
-  const T alpha = (T)(scal[1] / (double)den);  // errO / den (CGRAD's alpha)
-  const size_t base = (size_t)blockIdx.x * kChunk;
-  T s = T(0);
+__device__ inline double face_coef(const FaceDev &F) { return F.coefp ? *F.coefp : F.coef; }
+__device__ inline double face_sum(const FaceList &fl, int f) {
+  double S = 0.0;
 #pragma unroll
-  for (int t = 0; t < kChunk / 256; ++t) {
-    const size_t e = base + threadIdx.x + 256 * t;
-    if (e < L) {
-      X[e] = X[e] + alpha * P[e];
-      const T r = R[e] - alpha * SP[e];
-      R[e] = r;
-      s += r * r;
+  for (int b = 0; b < kFaceDotBlocks; ++b) S += fl.part[f * kFaceDotBlocks + b];
+  return S;
+}
+// Workgroup b of a face's kFaceDotBlocks: its share of q_f . P, entries
+// b * 256 + t + 1024 u; p_at(j) gives the direction at column j.
+template <class P>
+__device__ inline void face_part(const FaceList &fl, int wg, double *sh, P p_at) {
+  const int f = wg / kFaceDotBlocks, b = wg % kFaceDotBlocks;
+  const int *sup = fl.fd[f].sup;
+  const double *q = fl.fd[f].q;
+  const int ns = fl.fd[f].nsup;
+  double s = 0.0;
+  constexpr int kStep = 256 * kFaceDotBlocks;
+  for (int e0 = b * 256 + threadIdx.x; e0 < ns; e0 += 4 * kStep) {  // four entries' loads together
+    int j[4];
+    double qv[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const int e = min(e0 + kStep * u, ns - 1);
+      j[u] = sup[e];
+      qv[u] = e0 + kStep * u < ns ? q[e] : 0.0;
+    }
+#pragma unroll
+    for (int u = 0; u < 4; ++u) s += qv[u] * (double)p_at(j[u]);
+  }
+  s = block_sum(s, sh);
+  if (threadIdx.x == 0) fl.part[wg] = s;
+}
+// The first direction P = R (and Ps = W_p o P for the two-pass operator), X = 0 in
+// place of the right-hand side, which moves to Rv.
+template <class T>
+__global__ void __launch_bounds__(256) cg_begin_vec_kernel(size_t L, T *__restrict__ X, T *__restrict__ Rv,
+                                                           T *__restrict__ P, const T *__restrict__ W, int wdof,
+                                                           int off, T *__restrict__ Ps,
+                                                           const double *__restrict__ skip) {
+  if (skip && *skip != 0.0) return;
+  const size_t e = (size_t)blockIdx.x * 256 + threadIdx.x;
+  if (e >= L) return;
+  const T r = X[e];
+  Rv[e] = r;
+  P[e] = r;
+  if (Ps) Ps[e] = W[off + (size_t)wdof * e] * r;
+  X[e] = T(0);
+}
+// the faces' dots with the first direction
+template <class T>
+__global__ void __launch_bounds__(256) cg_begin_face_kernel(FaceList fl, const T *__restrict__ P,
+                                                            const double *__restrict__ skip) {
+  if (skip && *skip != 0.0) return;
+  __shared__ double sh[4];
+  face_part(fl, blockIdx.x, sh, [&](int j) { return P[j]; });
+}
+// parts of P . SP for an operator that does not form them
+template <class T>
+__global__ void __launch_bounds__(256) cg_den_kernel(size_t L, const T *__restrict__ P, const T *__restrict__ SP,
+                                                     double *__restrict__ dpart, const double *__restrict__ done) {
+  if (*done != 0.0) return;
+  __shared__ double sh[4];
+  double s = 0.0;
+  for (size_t e = (size_t)blockIdx.x * 256 + threadIdx.x; e < L; e += (size_t)gridDim.x * 256)
+    s += (double)P[e] * (double)SP[e];
+  s = block_sum(s, sh);
+  if (threadIdx.x == 0) dpart[blockIdx.x] = s;
+}
+// R -= alpha SP (with the faces' rank-one terms), alpha = errO / (P . SP);
+// the workgroup's part of R . R.  E entries per thread and turn (cg_grid).
+template <class T, int E>
+__global__ void __launch_bounds__(256) cg_r_kernel(size_t L, double *__restrict__ scal,
+                                                   const double *__restrict__ dpart, int nd, FaceList fl,
+                                                   T *__restrict__ R, const T *__restrict__ SP,
+                                                   double *__restrict__ rpart) {
+  __shared__ double sh[4];
+  __shared__ T corr[E * 256];
+  const double stop = scal[5], errO = scal[1];
+  T r[E], sp[E];
+  auto load = [&](size_t base) {
+#pragma unroll
+    for (int t = 0; t < E; ++t) {
+      const size_t e = base + threadIdx.x + 256 * t;
+      r[t] = e < L ? R[e] : T(0);
+      sp[t] = e < L ? SP[e] : T(0);
+    }
+  };
+  const int nt = (int)((L + 255) / 256);
+  int e0 = 0, e1 = 0;  // the faces' entries of the turn's nodes
+  auto range = [&](size_t base) {
+    if (fl.nfc == 0) return;
+    const int t0 = (int)(base / 256);
+    e0 = fl.tptr[t0];
+    e1 = fl.tptr[min(t0 + E, nt)];
+  };
+  size_t base = (size_t)blockIdx.x * (E * 256);
+  load(base);  // all in flight while the parts are summed
+  range(base);
+  double d = 0.0;
+  for (int f = threadIdx.x; f < fl.nfc; f += 256) {
+    const double S = face_sum(fl, f);
+    d += face_coef(fl.fd[f]) * S * S;
+  }
+  if (stop != 0.0) return;
+  const double den = sum_parts(dpart, nd, d, sh);
+  const double a = errO / den;  // CGRAD's alpha
+  if (blockIdx.x == 0 && threadIdx.x == 0) scal[3] = a;
+  const T alpha = (T)a;
+  double s = 0.0;
+  while (base < L) {
+    if (e1 > e0) {  // the same for the whole workgroup
+#pragma unroll
+      for (int t = 0; t < E; ++t) corr[threadIdx.x + 256 * t] = T(0);
+      __syncthreads();
+      for (int e = e0 + threadIdx.x; e < e1; e += 256) {
+        const int node = fl.ent[e].node;
+        if (e > e0 && fl.ent[e - 1].node == node) continue;  // the node's first entry sums them all
+        double v = 0.0;
+        for (int x = e; x < e1 && fl.ent[x].node == node; ++x) {
+          const FaceDev &F = fl.fd[fl.ent[x].f];
+          v += face_coef(F) * face_sum(fl, fl.ent[x].f) * F.q[fl.ent[x].s];
+        }
+        corr[node - (int)base] = (T)v;
+      }
+      __syncthreads();
+#pragma unroll
+      for (int t = 0; t < E; ++t) sp[t] += corr[threadIdx.x + 256 * t];
+      __syncthreads();
+    }
+#pragma unroll
+    for (int t = 0; t < E; ++t) {
+      const size_t e = base + threadIdx.x + 256 * t;
+      if (e < L) {
+        const T v = r[t] - alpha * sp[t];
+        R[e] = v;
+        s += (double)v * (double)v;
+      }
+    }
+    base += (size_t)gridDim.x * (E * 256);
+    if (base < L) {
+      load(base);
+      range(base);
     }
   }
   s = block_sum(s, sh);
-  if (threadIdx.x == 0) partial[blockIdx.x] = s;
+  if (threadIdx.x == 0) rpart[blockIdx.x] = s;
 }
-// err = NORMS(R)**2 from the per-workgroup partials of R.R (fixed order);
-// then beta = err/errO for the direction update, and the convergence test
-// of the next iteration (cg_check_kernel's, with the same err).
-template <class T>
-__global__ void __launch_bounds__(256) cg_err_kernel(int nblk, const T *__restrict__ partial,
-                                                     double *__restrict__ scal) {
-  if (scal[5] != 0.0) return;
-  __shared__ T sh[4];
-  T s = T(0);
-  for (int b = threadIdx.x; b < nblk; b += 256) s += partial[b];
-  s = block_sum(s, sh);
-  if (threadIdx.x == 0) {
-    const double n = sqrt((double)s);
-    scal[0] = n * n;
-    scal[4] = scal[0] / scal[1];
-    check_next(scal);
+// err = R . R from the parts, beta = err / errO; X += alpha P, the next
+// direction Pn = R + beta P (with its scaled copy Ps, and in the first
+// workgroups the faces' dots with it), and the next iteration's state.
+template <class T, int E>
+__global__ void __launch_bounds__(256) cg_p_kernel(size_t L, const double *__restrict__ scal,
+                                                   double *__restrict__ next, const double *__restrict__ rpart, int nr,
+                                                   FaceList fl, T *__restrict__ X, const T *__restrict__ R,
+                                                   const T *__restrict__ P, T *__restrict__ Pn,
+                                                   const T *__restrict__ W, int wdof, int off, T *__restrict__ Ps) {
+  const int nf = fl.nfc * kFaceDotBlocks, blk = (int)blockIdx.x - nf;
+  __shared__ double sh[4];
+  const double stop = scal[5], errO = scal[1], al = scal[3];
+  T r[E], p[E], x[E];
+  auto load = [&](size_t base) {
+#pragma unroll
+    for (int t = 0; t < E; ++t) {
+      const size_t e = base + threadIdx.x + 256 * t;
+      r[t] = e < L ? R[e] : T(0);
+      p[t] = e < L ? P[e] : T(0);
+      x[t] = e < L ? X[e] : T(0);
+    }
+  };
+  size_t base = (size_t)max(blk, 0) * (E * 256);
+  if (blk >= 0) load(base);  // in flight while the parts are summed
+  if (stop != 0.0) {
+    if (blockIdx.x == 0 && threadIdx.x < kCgState) next[threadIdx.x] = scal[threadIdx.x];
+    return;
   }
-}
-// P = R + beta P, and optionally Ps = W(off + wdof i) P (the operator's
-// scaled copy of the new direction)
-template <class T>
-__global__ void cg_p_kernel(size_t L, const double *__restrict__ scal, const T *__restrict__ R, T *__restrict__ P,
-                            const T *__restrict__ W, int wdof, int off, T *__restrict__ Ps) {
-  if (scal[5] != 0.0) return;
-  const size_t e = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (e >= L) return;
-  const T p = R[e] + (T)scal[4] * P[e];
-  P[e] = p;
-  if (Ps) Ps[e] = W[off + (size_t)wdof * e] * p;
+  const double n = sqrt(sum_parts(rpart, nr, 0.0, sh));  // NORMS(R)
+  const double err = n * n;
+  const T alpha = (T)al, beta = (T)(err / errO);
+  if (blockIdx.x == 0 && threadIdx.x == 0) {
+    double st[kCgState];
+    for (int k = 0; k < kCgState; ++k) st[k] = scal[k];
+    st[0] = err;
+    check_next(st);
+    for (int k = 0; k < kCgState; ++k) next[k] = st[k];
+  }
+  if (blk < 0) {
+    face_part(fl, blockIdx.x, sh, [&](int j) { return R[j] + beta * P[j]; });
+    return;
+  }
+  while (base < L) {
+#pragma unroll
+    for (int t = 0; t < E; ++t) {
+      const size_t e = base + threadIdx.x + 256 * t;
+      if (e >= L) continue;
+      X[e] = x[t] + alpha * p[t];
+      const T v = r[t] + beta * p[t];
+      Pn[e] = v;
+      if (Ps) Ps[e] = W[off + (size_t)wdof * e] * v;
+    }
+    base += (size_t)(gridDim.x - nf) * (E * 256);
+    if (base < L) load(base);
+  }
 }
 }  // namespace
 
@@ -821,6 +1127,7 @@ struct Ctx {
   crimson::DBuf<double> dsc, hcol;
   crimson::DBuf<double> fsum;  // one face dot per face (ADDBCMUL)
   crimson::DBuf<double> fpart;  // the Schur CG's face dot partials (kFaceDotBlocks per coupled face)
+  crimson::DBuf<double> cgst;   // the CG's state, twice
   crimson::DBuf<FaceDev> fdev;  // coupled faces with their PRE coefficients (Schur CG)
   std::vector<FaceDev> hfdev;
   crimson::DBuf<int> gate;
@@ -851,6 +1158,10 @@ struct Ctx {
     return CRIMSON_OK;
   }
 
+  FaceList face_list() const {
+    return FaceList{(int)hfdev.size(), fdev.p, lhs->d_fent.p, lhs->d_ftptr.p, fpart.p};
+  }
+
   int init(crimson_lhs *l, int d) {
     lhs = l;
     s = l->stream;
@@ -860,7 +1171,8 @@ struct Ctx {
     nblk_max = (int)((L + kChunk - 1) / kChunk);
     CR_TRY(W.alloc(L));
     CR_TRY(fix.alloc(L));
-    CR_TRY(partial.alloc((size_t)nblk_max * 256));
+    CR_TRY(partial.alloc(std::max<size_t>((size_t)nblk_max * 256, 2 * kCgGrid)));
+    CR_TRY(cgst.alloc(2 * kCgState));
     CR_TRY(dsc.alloc(64));
     CR_TRY(hcol.alloc(4 * 256));
     CR_TRY(fsum.alloc(std::max<size_t>(1, l->face.size())));
@@ -1124,57 +1436,103 @@ int gmres_dev(Ctx<T> &c, const MatView<T> &A, int nd, SubLs &ls, const T *R, T *
   return CRIMSON_OK;
 }
 
-// The operator's column-scaled copy of the CG direction, Ps(i) = W(off +
-// wdof i) P(i), kept up to date by the direction update (Ps null: none).
+// What a CG's operator needs beside its direction: the coupled faces' rank-one
+// terms, and the scaled copy Ps(i) = W(off + wdof i) P(i) kept by the
+// direction update (Ps null: none).
 template <class T>
-struct Prescale {
+struct CgAux {
+  FaceList fl{0, nullptr, nullptr, nullptr, nullptr};
   const T *W = nullptr;
   int wdof = 0, off = 0;
   T *Ps = nullptr;
 };
+// Entries per thread and workgroups of the CG's vector sweeps.
+struct CgGrid {
+  int entries, blocks;
+};
+inline CgGrid cg_grid(size_t L) {
+  const int E = L > (size_t)256 * kCgGrid / 2 ? 4 : 1;
+  return CgGrid{E, (int)std::min<size_t>((L + (size_t)256 * E - 1) / ((size_t)256 * E), kCgGrid)};
+}
+// The iterations' vector work: iteration `it` after its operator left SP and nd
+// parts of P . SP.  P and Pn swap roles every iteration.
+template <class T>
+int cg_sweeps(Ctx<T> &c, size_t L, int it, int nd, const CgAux<T> &ax, T *X, T *R, const T *P, T *Pn, const T *SP) {
+  double *scal = c.cgst.p + (it & 1) * kCgState, *next = c.cgst.p + ((it + 1) & 1) * kCgState;
+  double *dpart = c.partial.p, *rpart = c.partial.p + kCgGrid;
+  const CgGrid g = cg_grid(L);
+  const int gp = g.blocks + ax.fl.nfc * kFaceDotBlocks;
+  if (g.entries == 1) {
+    cg_r_kernel<T, 1><<<g.blocks, 256, 0, c.s>>>(L, scal, dpart, nd, ax.fl, R, SP, rpart);
+    cg_p_kernel<T, 1><<<gp, 256, 0, c.s>>>(L, scal, next, rpart, g.blocks, ax.fl, X, R, P, Pn, ax.W, ax.wdof, ax.off,
+                                           ax.Ps);
+  } else {
+    cg_r_kernel<T, 4><<<g.blocks, 256, 0, c.s>>>(L, scal, dpart, nd, ax.fl, R, SP, rpart);
+    cg_p_kernel<T, 4><<<gp, 256, 0, c.s>>>(L, scal, next, rpart, g.blocks, ax.fl, X, R, P, Pn, ax.W, ax.wdof, ax.off,
+                                           ax.Ps);
+  }
+  CR_HIP(hipGetLastError());
+  return CRIMSON_OK;
+}
+// R = P = X, X = 0, and the faces' dots with the first direction.
+template <class T>
+int cg_begin_vec(Ctx<T> &c, size_t L, const CgAux<T> &ax, T *X, T *R, T *P, const double *skip) {
+  cg_begin_vec_kernel<T><<<crimson::grid_for(L, 256), 256, 0, c.s>>>(L, X, R, P, ax.W, ax.wdof, ax.off, ax.Ps, skip);
+  if (ax.fl.nfc > 0) cg_begin_face_kernel<T><<<ax.fl.nfc * kFaceDotBlocks, 256, 0, c.s>>>(ax.fl, P, skip);
+  CR_HIP(hipGetLastError());
+  return CRIMSON_OK;
+}
+
+// Parts of P . SP of an operator that leaves none.
+template <class T>
+int cg_den(Ctx<T> &c, size_t L, const T *P, const T *SP, const double *done, int &nd) {
+  nd = (int)std::min<size_t>((L + 255) / 256, kCgGrid);
+  cg_den_kernel<T><<<nd, 256, 0, c.s>>>(L, P, SP, c.partial.p, done);
+  CR_HIP(hipGetLastError());
+  return CRIMSON_OK;
+}
 
 // Generic CG driver on device vectors (memLS CGRAD / CGRADV / CGRADS).
-// op(P, SP) computes SP for the iteration; R is overwritten with X.
+// op(P, SP, done, nd) computes SP and nd parts of P . SP; X holds the right-hand
+// side in and the solution out.
 template <class T, class Op>
-int cg_dev(Ctx<T> &c, size_t L, SubLs &ls, T *R, Op op, T *X, T *P, T *SP, bool schur,
-           Prescale<T> ps = Prescale<T>()) {
+int cg_dev(Ctx<T> &c, size_t L, SubLs &ls, T *X, Op op, T *R, T *P, T *P2, T *SP, bool schur,
+           const CgAux<T> &ax = CgAux<T>()) {
   const double t0 = now_s();
-  double *scal = c.dsc.p;  // 0 err 1 errO 2 eps2 3 den 4 beta 5 done 6 itr 7 mItr 8 suc
   ls.suc = 0;
   int rc = CRIMSON_OK;
-  const double errO0 = host_norm(c, L, R, &rc);
+  const double errO0 = host_norm(c, L, X, &rc);
   if (rc) return rc;
   ls.iNorm = errO0;
   double eps = std::max(ls.absTol, ls.relTol * errO0);
   eps = eps * eps;
-  double hs[9] = {errO0 * errO0, errO0 * errO0, eps, 0, 0, 0, 0, (double)ls.mItr, 0};
-  CR_HIP(hipMemcpyAsync(scal, hs, sizeof(hs), hipMemcpyHostToDevice, c.s));
-  CR_HIP(hipMemsetAsync(X, 0, L * sizeof(T), c.s));
-  CR_HIP(hipMemcpyAsync(P, R, L * sizeof(T), hipMemcpyDeviceToDevice, c.s));
-  if (ps.Ps)
-    scale_p_kernel<T><<<crimson::grid_for(L, 256), 256, 0, c.s>>>((int)L, ps.W, ps.wdof, ps.off, P, ps.Ps, nullptr);
-  const int nblk = (int)((L + kChunk - 1) / kChunk);
-  const int batch = 8;
+  double hs[kCgState] = {errO0 * errO0, errO0 * errO0, eps, 0, 0, 0, 0, (double)ls.mItr, 0};
+  // the first iteration's test (check_next)
+  if (hs[6] >= hs[7]) {
+    hs[5] = 1.0;
+  } else if (hs[0] < hs[2]) {
+    hs[5] = hs[8] = 1.0;
+  } else {
+    hs[6] = 1.0;
+  }
+  CR_HIP(hipMemcpyAsync(c.cgst.p, hs, sizeof(hs), hipMemcpyHostToDevice, c.s));
+  CR_TRY(cg_begin_vec(c, L, ax, X, R, P, nullptr));
+  constexpr int batch = 8;  // even: a batch ends on the state's first copy
   double back[9];
   CR_TRY(c.readback_slots());
+  T *Pk = P, *Pn = P2;
   // a batch of iterations, then the flags' copy into read-back slot `slot`
   auto enqueue_batch = [&](int slot) -> int {
     for (int b = 0; b < batch; ++b) {
-      CR_TRY(op(P, SP, scal));
-      // den = P . SP
-      T *pt = reinterpret_cast<T *>(c.partial.p);
-      mdot_kernel<T, T><<<nblk, 256, 0, c.s>>>(L, SP, P, 0, 1, 0, pt, 1, nullptr, nullptr);
-      cg_update_kernel<T><<<nblk, 256, 0, c.s>>>(L, scal, pt, nblk, X, R, P, SP, pt + nblk);
-      cg_err_kernel<T><<<1, 256, 0, c.s>>>(nblk, pt + nblk, scal);
-      cg_p_kernel<T><<<crimson::grid_for(L, 256), 256, 0, c.s>>>(L, scal, R, P, ps.W, ps.wdof, ps.off, ps.Ps);
+      int nd = 0;
+      CR_TRY(op(Pk, SP, c.cgst.p + (b & 1) * kCgState + 5, nd));
+      CR_TRY(cg_sweeps(c, L, b, nd, ax, X, R, Pk, Pn, SP));
+      std::swap(Pk, Pn);
     }
-    CR_HIP(hipGetLastError());
-    CR_HIP(hipMemcpyAsync(c.hback + 16 * slot, scal, sizeof(back), hipMemcpyDeviceToHost, c.s));
+    CR_HIP(hipMemcpyAsync(c.hback + 16 * slot, c.cgst.p, sizeof(back), hipMemcpyDeviceToHost, c.s));
     CR_HIP(hipEventRecord(c.evb[slot], c.s));
     return CRIMSON_OK;
   };
-  // the first iteration's test; cg_err_kernel makes each later one
-  cg_check_kernel<<<1, 1, 0, c.s>>>(scal);
   CR_TRY(enqueue_batch(0));
   for (int k = 0;; ++k) {
     // the next batch is queued before this one's flags are read, so that the
@@ -1187,7 +1545,6 @@ int cg_dev(Ctx<T> &c, size_t L, SubLs &ls, T *R, Op op, T *X, T *P, T *SP, bool 
     if (back[5] != 0.0) break;
   }
   // the flag is raised at the top of the iteration after the last one
-  CR_HIP(hipMemcpyAsync(R, X, L * sizeof(T), hipMemcpyDeviceToDevice, c.s));
   const double err = back[0], errO = back[1];
   ls.suc = back[8] != 0.0;
   ls.fNorm = std::sqrt(err);
@@ -1199,6 +1556,143 @@ int cg_dev(Ctx<T> &c, size_t L, SubLs &ls, T *R, Op op, T *X, T *P, T *SP, bool 
     ls.itr = done_itr;
   ls.callD = now_s() - t0 + (schur ? ls.callD : 0.0);
   return CRIMSON_OK;
+}
+
+// ----- the Schur operator: formed (schur_pattern) or in two passes -----
+inline crimson::DBuf<double> &schur_buf(crimson_lhs *l, double) { return l->d_S; }
+inline crimson::DBuf<float> &schur_buf(crimson_lhs *l, float) { return l->d_S32; }
+
+// An allocation that may fail without failing the solve: the error state is
+// cleared and the caller takes the path that needs no such buffer.
+template <class B>
+bool try_alloc(B &b, size_t n) {
+  if (b.alloc(n) == CRIMSON_OK) return true;
+  (void)hipGetLastError();
+  return false;
+}
+
+// The pattern of S, once per handle: schur = 1 when it is there, 2 when this
+// graph keeps the two passes.  S is formed when its rows fit the value kernel's staging
+// (kSchurRow) and it has at most kSchurFill entries per block: the two passes
+// read 60 bytes per block (32 in FP32), S 10 (6) per entry plus the vector
+// work of one more launch.
+constexpr int kSchurFill = 6;
+template <class IX, class OX>
+int schur_pattern_fill(crimson_lhs *l, const IX *col, crimson::DBuf<OX> &scol, long long n) {
+  if (!try_alloc(scol, (size_t)n)) {
+    l->schur = 2;
+    return CRIMSON_OK;
+  }
+  schur_pattern_kernel<IX, OX, true><<<crimson::grid_for(l->nNo, 4), 256, 0, l->stream>>>(l->nNo, l->d_rowptr.p, col,
+                                                                                         nullptr, l->d_sptr.p, scol.p);
+  CR_HIP(hipGetLastError());
+  CR_HIP(hipStreamSynchronize(l->stream));
+  l->schur = 1;
+  return CRIMSON_OK;
+}
+int schur_pattern(crimson_lhs *l) {
+  if (l->schur) return CRIMSON_OK;
+  const int N = l->nNo;
+  crimson::DBuf<int> cnt;
+  if (!try_alloc(cnt, (size_t)N) || !try_alloc(l->d_sptr, (size_t)N + 1)) {
+    l->schur = 2;
+    return CRIMSON_OK;
+  }
+  const unsigned G = crimson::grid_for(N, 4);
+  if (l->d_col16.p)
+    schur_pattern_kernel<short, int, false><<<G, 256, 0, l->stream>>>(N, l->d_rowptr.p, l->d_col16.p, cnt.p, nullptr,
+                                                                      nullptr);
+  else
+    schur_pattern_kernel<int, int, false><<<G, 256, 0, l->stream>>>(N, l->d_rowptr.p, l->d_col.p, cnt.p, nullptr,
+                                                                    nullptr);
+  CR_HIP(hipGetLastError());
+  std::vector<int> ptr((size_t)N + 1);
+  CR_HIP(hipMemcpyAsync(ptr.data() + 1, cnt.p, (size_t)N * sizeof(int), hipMemcpyDeviceToHost, l->stream));
+  CR_HIP(hipStreamSynchronize(l->stream));
+  long long n = 0;
+  int most = 0;
+  ptr[0] = 0;
+  for (int i = 1; i <= N; ++i) {
+    most = std::max(most, ptr[i]);
+    n += ptr[i];
+    ptr[i] = (int)n;
+    if (most > kSchurRow || n > (long long)kSchurFill * l->nnz || n > 0x7fffff00LL) {
+      l->schur = 2;
+      l->d_sptr.release();
+      return CRIMSON_OK;
+    }
+  }
+  l->schur_row = most;
+  l->schur_nnz = n;
+  CR_TRY(l->d_sptr.upload(ptr.data(), ptr.size(), l->stream));
+  if (l->d_col16.p) {
+    if (2 * l->band <= 32767) return schur_pattern_fill(l, l->d_col16.p, l->d_scol16, n);
+    return schur_pattern_fill(l, l->d_col16.p, l->d_scol, n);
+  }
+  return schur_pattern_fill(l, l->d_col.p, l->d_scol, n);
+}
+
+template <class T>
+struct SchurOp {
+  bool formed = false;
+  MatView<T> L, Gt, G;
+  T *Z = nullptr, *Ps = nullptr;  // two passes: Z(4, N) and the scaled direction
+};
+// S's pattern and storage (before a capture); formed = false when the two
+// passes are taken.
+template <class T>
+int schur_ready(crimson_lhs *l, SchurOp<T> &o) {
+  CR_TRY(schur_pattern(l));
+  o.formed = l->schur == 1 && try_alloc(schur_buf(l, T(0)), (size_t)l->schur_nnz);
+  return CRIMSON_OK;
+}
+// S's values from the matrix and the scaling of this solve.
+template <class T>
+int schur_form(Ctx<T> &c, const SchurOp<T> &o) {
+  if (!o.formed) return CRIMSON_OK;
+  crimson_lhs *l = c.lhs;
+  const unsigned G = crimson::grid_for(l->nNo, 16);
+  const size_t sh = (size_t)16 * l->schur_row * (sizeof(double) + sizeof(int));
+  T *S = schur_buf(l, T(0)).p;
+#define CR_SV(IX_, CP_, OX_, SP_)                                                                                  \
+  schur_values_kernel<T, IX_, OX_><<<G, 256, sh, c.s>>>(l->nNo, l->d_rowptr.p, CP_, o.L, o.Gt, o.G, l->d_sptr.p, SP_, \
+                                                        S, l->schur_row)
+  if (l->d_scol16.p)
+    CR_SV(short, l->d_col16.p, short, l->d_scol16.p);
+  else if (l->d_col16.p)
+    CR_SV(short, l->d_col16.p, int, l->d_scol.p);
+  else
+    CR_SV(int, l->d_col.p, int, l->d_scol.p);
+#undef CR_SV
+  CR_HIP(hipGetLastError());
+  return CRIMSON_OK;
+}
+// SP = S P and the parts of P . SP; the faces' terms join in the CG's sweeps.
+template <class T>
+int schur_apply(Ctx<T> &c, const SchurOp<T> &o, const T *P, T *SP, const double *done, int &nd) {
+  crimson_lhs *l = c.lhs;
+  const int N = l->nNo;
+  double *dpart = c.partial.p;
+  if (o.formed) {
+    const int ntile = (int)crimson::grid_for((size_t)N, 256 / kSLanes);
+    nd = std::min(ntile, kCgGrid);
+    const T *S = schur_buf(l, T(0)).p;
+    if (l->d_scol16.p)
+      s_product_kernel<T, short><<<nd, 256, 0, c.s>>>(N, ntile, l->d_sptr.p, l->d_scol16.p, S, P, SP, dpart, done);
+    else
+      s_product_kernel<T, int><<<nd, 256, 0, c.s>>>(N, ntile, l->d_sptr.p, l->d_scol.p, S, P, SP, dpart, done);
+    CR_HIP(hipGetLastError());
+    return CRIMSON_OK;
+  }
+  const unsigned gr = crimson::grid_for((size_t)N * kNarrowLanes, 256);
+  if (l->d_col16.p) {
+    g_product_kernel<T, short><<<gr, 256, 0, c.s>>>(N, l->d_rowptr.p, l->d_col16.p, o.G, o.Ps, o.Z, done);
+    schur_kernel<T, short><<<gr, 256, 0, c.s>>>(N, l->d_rowptr.p, l->d_col16.p, o.L, o.Gt, P, o.Z, SP, done);
+  } else {
+    g_product_kernel<T, int><<<gr, 256, 0, c.s>>>(N, l->d_rowptr.p, l->d_col.p, o.G, o.Ps, o.Z, done);
+    schur_kernel<T, int><<<gr, 256, 0, c.s>>>(N, l->d_rowptr.p, l->d_col.p, o.L, o.Gt, P, o.Z, SP, done);
+  }
+  return cg_den(c, (size_t)N, P, SP, done, nd);
 }
 
 // NSSOLVER (memLS.f90:1460-1759) on device; Ri (4,N) device in/out
@@ -1225,6 +1719,8 @@ int face_support(crimson_lhs *l, CrFace &fa) {
   }
   ptr.push_back((int)t.size());
   fa.nsup = (int)sup.size();
+  fa.h_sup = sup;
+  fa.support = crimson::next_alloc_serial();
   if (fa.nsup > 0) {
     CR_TRY(fa.d_sup.upload(sup.data(), sup.size(), l->stream));
     CR_TRY(fa.d_qptr.upload(ptr.data(), ptr.size(), l->stream));
@@ -1234,6 +1730,54 @@ int face_support(crimson_lhs *l, CrFace &fa) {
     CR_HIP(hipStreamSynchronize(l->stream));
   }
   fa.qpat = true;
+  return CRIMSON_OK;
+}
+
+// The coupled faces (c.hfdev, in face order) on the device, and their merged
+// supports (FaceList), which the handle keeps while the same faces are coupled.
+template <class T>
+int face_list(Ctx<T> &c) {
+  crimson_lhs *l = c.lhs;
+  const size_t nfc = c.hfdev.size();
+  if (nfc == 0) return CRIMSON_OK;
+  CR_TRY(c.fdev.alloc(nfc));
+  CR_HIP(hipMemcpyAsync(c.fdev.p, c.hfdev.data(), nfc * sizeof(FaceDev), hipMemcpyHostToDevice, c.s));
+  std::vector<unsigned long long> sig;
+  for (const auto &fa : l->face)
+    if (fa.coupled) sig.push_back(fa.support);
+  if (sig != l->fent_sig || !l->d_ftptr.p) {
+    std::vector<FaceEnt> ent;
+    int f = 0;
+    for (const auto &fa : l->face) {
+      if (!fa.coupled) continue;
+      for (size_t k = 0; k < fa.h_sup.size(); ++k) ent.push_back(FaceEnt{fa.h_sup[k], f, (int)k});
+      ++f;
+    }
+    std::sort(ent.begin(), ent.end(),
+              [](const FaceEnt &a, const FaceEnt &b) { return a.node != b.node ? a.node < b.node : a.f < b.f; });
+    std::vector<int> ptr((size_t)(l->nNo + 255) / 256 + 1);
+    size_t e = 0;
+    for (size_t t = 0; t < ptr.size(); ++t) {
+      while (e < ent.size() && ent[e].node < (long long)t * 256) ++e;
+      ptr[t] = (int)e;
+    }
+    ptr.back() = (int)ent.size();
+    CR_TRY(l->d_fent.upload(ent.data(), ent.size(), c.s));
+    CR_TRY(l->d_ftptr.upload(ptr.data(), ptr.size(), c.s));
+    CR_HIP(hipStreamSynchronize(c.s));
+    l->fent_sig = sig;
+  }
+  CR_HIP(hipStreamSynchronize(c.s));
+  return CRIMSON_OK;
+}
+// The faces' functionals q for this solve's matrix and scaling.
+template <class T>
+int face_functionals(Ctx<T> &c, const MatView<T> &G) {
+  for (auto &fa : c.lhs->face)
+    if (fa.coupled && fa.nsup > 0)
+      face_q_kernel<T><<<crimson::grid_for(fa.nsup, 256), 256, 0, c.s>>>(
+          fa.nsup, fa.d_sup.p, fa.d_qptr.p, fa.d_qa.p, fa.d_qk.p, fa.d_glob.p, fa.d_valM.p, fa.dof, G, fa.d_q.p);
+  CR_HIP(hipGetLastError());
   return CRIMSON_OK;
 }
 
@@ -1316,48 +1860,30 @@ int nssolver_dev(Ctx<T> &c, crimson_ls *ls, T *Ri) {
   for (auto &fa : l->face) {
     if (!fa.coupled) continue;
     CR_TRY(face_support(l, fa));
-    if (fa.nsup > 0) {
-      face_q_kernel<T><<<crimson::grid_for(fa.nsup, 256), 256, 0, c.s>>>(
-          fa.nsup, fa.d_qptr.p, fa.d_qa.p, fa.d_qk.p, fa.d_glob.p, fa.d_valM.p, fa.dof, mG, fa.d_q.p);
-      CR_HIP(hipGetLastError());
-    }
     c.hfdev.push_back(FaceDev{fa.d_glob.p, fa.d_valM.p, -fa.res / (1.0 + fa.res * fa.nS), nullptr, fa.res, fa.nNo, fa.dof,
                               fa.d_sup.p, fa.d_q.p, fa.nsup});
   }
-  const int nfc = (int)c.hfdev.size();
-  if (nfc > 0) {
-    CR_TRY(c.fdev.alloc(c.hfdev.size()));
-    CR_HIP(hipMemcpyAsync(c.fdev.p, c.hfdev.data(), c.hfdev.size() * sizeof(FaceDev), hipMemcpyHostToDevice, c.s));
-    CR_HIP(hipStreamSynchronize(c.s));
+  CR_TRY(face_list(c));
+  CR_TRY(face_functionals(c, mG));
+  SchurOp<T> so;
+  so.L = mL;
+  so.Gt = Gt;
+  so.G = mG;
+  so.Z = ws.tmp.p;
+  CR_TRY(schur_ready(l, so));
+  CR_TRY(schur_form(c, so));
+  CgAux<T> ax;
+  ax.fl = c.face_list();
+  if (!so.formed) {
+    ax.W = c.W.p;
+    ax.wdof = 4;
+    ax.off = mG.c0;
+    ax.Ps = so.Ps = t2.p;
   }
-  // Schur operator of CGRAD: SP = L P - Gt (G P + PRE), on P and its
-  // scaled copy Ps = W_p o P in t2 (kept by the CG's direction update)
-  auto schur_op = [&](const T *Pv, T *SPv, const double *scal) -> int {
-    const double *done = scal + 5;
-    const unsigned gr = crimson::grid_for((size_t)N * kNarrowLanes, 256);
-    if (l->d_col16.p)
-      g_product_kernel<T, short><<<gr + nfc * kFaceDotBlocks, 256, 0, c.s>>>(
-          N, l->d_rowptr.p, l->d_col16.p, mG, t2.p, t1.p, ws.tmp.p, nfc, c.fdev.p, c.fpart.p, done);
-    else
-      g_product_kernel<T, int><<<gr + nfc * kFaceDotBlocks, 256, 0, c.s>>>(
-          N, l->d_rowptr.p, l->d_col.p, mG, t2.p, t1.p, ws.tmp.p, nfc, c.fdev.p, c.fpart.p, done);
-    for (int f = 0; f < nfc; ++f)
-      if (c.hfdev[f].nNo > 0)
-        face_pre_apply_kernel<T><<<crimson::grid_for(c.hfdev[f].nNo, 256), 256, 0, c.s>>>(
-          c.hfdev[f], c.fpart.p + f * kFaceDotBlocks, t1.p, ws.tmp.p, c.W.p, 4, done);
-    if (l->d_col16.p)
-      schur_kernel<T, short><<<gr, 256, 0, c.s>>>(N, l->d_rowptr.p, l->d_col16.p, mL, Gt, Pv, t2.p, ws.tmp.p, SPv,
-                                                  done);
-    else
-      schur_kernel<T, int><<<gr, 256, 0, c.s>>>(N, l->d_rowptr.p, l->d_col.p, mL, Gt, Pv, t2.p, ws.tmp.p, SPv, done);
-    CR_HIP(hipGetLastError());
-    return CRIMSON_OK;
+  // Schur operator of CGRAD: SP = L P - Gt (G P + PRE)
+  auto schur_op = [&](const T *Pv, T *SPv, const double *done, int &nd) -> int {
+    return schur_apply(c, so, Pv, SPv, done, nd);
   };
-  Prescale<T> pre_p;
-  pre_p.W = c.W.p;
-  pre_p.wdof = 4;
-  pre_p.off = mG.c0;
-  pre_p.Ps = t2.p;
   std::vector<double> A((size_t)nB * nB, 0.0), Bv(nB, 0.0), xB(nB, 0.0);
   std::vector<double> dots(2 * nB + 4);
   int i, iBB = 0;
@@ -1370,7 +1896,7 @@ int nssolver_dev(Ctx<T> &c, crimson_ls *ls, T *Ri) {
     T *MPb = MP.p + (size_t)N * (iB - 1), *MPbb = MP.p + (size_t)N * (iBB - 1);
     CR_TRY(gmres_dev(c, mK, 3, ls->GM, Rm.p, Ui, ws, true));
     CR_TRY(spmv(c, mD, 1, 3, Ui, Pi, -1.0, Rc.p, 1.0));  // P = Rc - D U
-    CR_TRY(cg_dev(c, (size_t)N, ls->CG, Pi, schur_op, t3.p, t4.p, MPb, true, pre_p));
+    CR_TRY(cg_dev(c, (size_t)N, ls->CG, Pi, schur_op, t3.p, t4.p, t1.p, MPb, true, ax));
     CR_TRY(spmv(c, mG, 3, 1, Pi, MUb));
     CR_TRY(axpby(c, mn, 1.0, Rm.p, 0.0, MUbb));
     CR_TRY(axpby(c, mn, -1.0, MUb, 1.0, MUbb));  // MU(iBB) = Rm - MU(iB)
@@ -1573,12 +2099,16 @@ int solve_impl(crimson_lhs *l, crimson_ls *ls, int dof, double *d_Ri, const int 
     }
   } else if (ls->LS_type == CRIMSON_LS_CG) {
     const MatView<T> A = view<T>(c, V, dof, 0, 0, dof, dof, c.W.p, c.fix.p, dof);
-    crimson::DBuf<T> X, P, SP;
+    crimson::DBuf<T> X, P, P2, SP;
     CR_TRY(X.alloc(L));
     CR_TRY(P.alloc(L));
+    CR_TRY(P2.alloc(L));
     CR_TRY(SP.alloc(L));
-    auto op = [&](const T *Pv, T *SPv, const double *) -> int { return spmv<T>(c, A, dof, dof, Pv, SPv); };
-    rc = cg_dev<T>(c, L, ls->RI, R, op, X.p, P.p, SP.p, false);
+    auto op = [&](const T *Pv, T *SPv, const double *done, int &nd) -> int {
+      CR_TRY(spmv<T>(c, A, dof, dof, Pv, SPv, 1.0, static_cast<const T *>(nullptr), 0.0, done));
+      return cg_den(c, L, Pv, SPv, done, nd);
+    };
+    rc = cg_dev<T>(c, L, ls->RI, R, op, X.p, P.p, P2.p, SP.p, false);
   } else {
     crimson::set_error("LS_type %d not defined", ls->LS_type);
     return CRIMSON_EARG;
@@ -1844,6 +2374,7 @@ __global__ void cg_begin_kernel(double *__restrict__ scal, double *__restrict__ 
   scal[3] = scal[4] = scal[5] = scal[6] = 0.0;
   scal[7] = (double)mItr;
   scal[8] = 0.0;
+  check_next(scal);  // the first iteration's test
 }
 __global__ void cg_end_kernel(const double *__restrict__ scal, double *__restrict__ g) {
   if (g[G_RI_SKIP] != 0.0) return;
@@ -1952,6 +2483,7 @@ struct NsGraphWork {
   int sD = 0, nB = 0, mRI = 0, mGM = 0, mCG = 0;
   double riAbs = 0, riRel = 0, gmAbs = 0, gmRel = 0, cgAbs = 0, cgRel = 0;
   bool disjoint = false;  // the coupled faces share no node: one launch for all of them
+  bool formed = false;    // the Schur complement is formed (schur_ready)
   int maxfn = 0;          // the largest coupled face
   crimson::DBuf<double> msum;  // the faces' dots of the batched ADDBCMUL
   struct SegCapture *cap = nullptr;  // the capture in progress, cut between the solve's phases
@@ -2034,27 +2566,19 @@ int gmres_graph(NsGraphWork<T> &w, const MatView<T> &A, int nd, const T *R, T *X
 // CGRAD on the Schur operator (cg_dev with schur = true) device-driven:
 // mItr iteration bodies, each launch returning at once after the flag.
 template <class T, class Op>
-int cg_graph(NsGraphWork<T> &w, size_t L, T *R, Op op, T *X, T *P, T *SP, Prescale<T> ps) {
+int cg_graph(NsGraphWork<T> &w, size_t L, T *X, Op op, T *R, T *P, T *P2, T *SP, const CgAux<T> &ax) {
   Ctx<T> &c = w.c;
-  double *g = w.gst.p, *scal = c.dsc.p;
-  const unsigned GL = crimson::grid_for(L, 256);
-  CR_TRY(mdot<T>(c, L, R, nullptr, 0, 0, true, c.dsc.p + 41, nullptr, true, g + G_RI_SKIP));
+  double *g = w.gst.p, *scal = c.cgst.p;
+  CR_TRY(mdot<T>(c, L, X, nullptr, 0, 0, true, c.dsc.p + 41, nullptr, true, g + G_RI_SKIP));
   cg_begin_kernel<<<1, 1, 0, c.s>>>(scal, g, c.dsc.p + 41, w.cgAbs, w.cgRel, w.mCG);
-  gfill_kernel<T><<<GL, 256, 0, c.s>>>(L, X, scal + 5);
-  gcopy_kernel<T><<<GL, 256, 0, c.s>>>(L, R, P, scal + 5, nullptr);
-  if (ps.Ps) scale_p_kernel<T><<<GL, 256, 0, c.s>>>((int)L, ps.W, ps.wdof, ps.off, P, ps.Ps, scal + 5);
-  const int nblk = (int)((L + kChunk - 1) / kChunk);
-  cg_check_kernel<<<1, 1, 0, c.s>>>(scal);
+  CR_TRY(cg_begin_vec(c, L, ax, X, R, P, g + G_RI_SKIP));
   for (int it = 0; it < w.mCG; ++it) {
-    CR_TRY(op(P, SP, scal));
-    T *pt = reinterpret_cast<T *>(c.partial.p);
-    mdot_kernel<T, T><<<nblk, 256, 0, c.s>>>(L, SP, P, 0, 1, 0, pt, 1, nullptr, scal + 5);
-    cg_update_kernel<T><<<nblk, 256, 0, c.s>>>(L, scal, pt, nblk, X, R, P, SP, pt + nblk);
-    cg_err_kernel<T><<<1, 256, 0, c.s>>>(nblk, pt + nblk, scal);
-    cg_p_kernel<T><<<GL, 256, 0, c.s>>>(L, scal, R, P, ps.W, ps.wdof, ps.off, ps.Ps);
+    int nd = 0;
+    CR_TRY(op(P, SP, c.cgst.p + (it & 1) * kCgState + 5, nd));
+    CR_TRY(cg_sweeps(c, L, it, nd, ax, X, R, P, P2, SP));
+    std::swap(P, P2);
   }
-  gcopy_kernel<T><<<GL, 256, 0, c.s>>>(L, X, R, g + G_RI_SKIP, nullptr);
-  cg_end_kernel<<<1, 1, 0, c.s>>>(scal, g);
+  cg_end_kernel<<<1, 1, 0, c.s>>>(c.cgst.p + (w.mCG & 1) * kCgState, g);
   CR_HIP(hipGetLastError());
   return CRIMSON_OK;
 }
@@ -2099,42 +2623,27 @@ int nssolver_graph(NsGraphWork<T> &w, T *Ri) {
     CrFace &fa = l->face[f];
     if (!fa.coupled) continue;
     face_pre_coef_kernel<<<1, 1, 0, c.s>>>(fa.nNo, fa.dof, nsd, fa.d_valM.p, fa.res, w.fcoef.p + f);
-    if (fa.nsup > 0)
-      face_q_kernel<T><<<crimson::grid_for(fa.nsup, 256), 256, 0, c.s>>>(
-          fa.nsup, fa.d_qptr.p, fa.d_qa.p, fa.d_qk.p, fa.d_glob.p, fa.d_valM.p, fa.dof, mG, fa.d_q.p);
   }
   CR_HIP(hipGetLastError());
-  const int nfc = (int)c.hfdev.size();
-  T *t1 = w.t1.p, *t2 = w.t2.p, *tmp = w.gmTmp.p;
-  auto schur_op = [&](const T *Pv, T *SPv, const double *scal) -> int {
-    const double *done = scal + 5;
-    const unsigned gr = crimson::grid_for((size_t)N * kNarrowLanes, 256);
-    if (l->d_col16.p)
-      g_product_kernel<T, short><<<gr + nfc * kFaceDotBlocks, 256, 0, c.s>>>(
-          N, l->d_rowptr.p, l->d_col16.p, mG, t2, t1, tmp, nfc, c.fdev.p, c.fpart.p, done);
-    else
-      g_product_kernel<T, int><<<gr + nfc * kFaceDotBlocks, 256, 0, c.s>>>(
-          N, l->d_rowptr.p, l->d_col.p, mG, t2, t1, tmp, nfc, c.fdev.p, c.fpart.p, done);
-    if (w.disjoint && nfc > 1)
-      face_pre_apply_multi_kernel<T><<<dim3(crimson::grid_for(std::max(1, w.maxfn), 256), nfc), 256, 0, c.s>>>(
-          c.fdev.p, c.fpart.p, t1, tmp, c.W.p, 4, done);
-    else
-      for (int f = 0; f < nfc; ++f)
-        if (c.hfdev[f].nNo > 0)
-          face_pre_apply_kernel<T><<<crimson::grid_for(c.hfdev[f].nNo, 256), 256, 0, c.s>>>(
-              c.hfdev[f], c.fpart.p + f * kFaceDotBlocks, t1, tmp, c.W.p, 4, done);
-    if (l->d_col16.p)
-      schur_kernel<T, short><<<gr, 256, 0, c.s>>>(N, l->d_rowptr.p, l->d_col16.p, mL, Gt, Pv, t2, tmp, SPv, done);
-    else
-      schur_kernel<T, int><<<gr, 256, 0, c.s>>>(N, l->d_rowptr.p, l->d_col.p, mL, Gt, Pv, t2, tmp, SPv, done);
-    CR_HIP(hipGetLastError());
-    return CRIMSON_OK;
+  CR_TRY(face_functionals(c, mG));
+  SchurOp<T> so;
+  so.formed = w.formed;
+  so.L = mL;
+  so.Gt = Gt;
+  so.G = mG;
+  so.Z = w.gmTmp.p;
+  CR_TRY(schur_form(c, so));
+  CgAux<T> ax;
+  ax.fl = c.face_list();
+  if (!so.formed) {
+    ax.W = c.W.p;
+    ax.wdof = 4;
+    ax.off = mG.c0;
+    ax.Ps = so.Ps = w.t2.p;
+  }
+  auto schur_op = [&](const T *Pv, T *SPv, const double *done, int &nd) -> int {
+    return schur_apply(c, so, Pv, SPv, done, nd);
   };
-  Prescale<T> pre_p;
-  pre_p.W = c.W.p;
-  pre_p.wdof = 4;
-  pre_p.off = mG.c0;
-  pre_p.Ps = t2;
   const int nB = w.nB;
   for (int i = 1; i <= w.mRI; ++i) {
     const int iB = 2 * i - 1, iBB = 2 * i;
@@ -2145,7 +2654,7 @@ int nssolver_graph(NsGraphWork<T> &w, T *Ri) {
     CR_TRY(gmres_graph(w, mK, 3, w.Rm.p, Ui));
     CR_TRY(w.cut());
     CR_TRY(spmv(c, mD, 1, 3, Ui, Pi, -1.0, w.Rc.p, 1.0, ri));  // P = Rc - D U
-    CR_TRY(cg_graph(w, (size_t)N, Pi, schur_op, w.t3.p, w.t4.p, MPb, pre_p));
+    CR_TRY(cg_graph(w, (size_t)N, Pi, schur_op, w.t3.p, w.t4.p, w.t1.p, MPb, ax));
     CR_TRY(w.cut());
     CR_TRY(spmv(c, mG, 3, 1, Pi, MUb, 1.0, static_cast<const T *>(nullptr), 0.0, ri));
     gaxpby_kernel<T><<<Gmn, 256, 0, c.s>>>(mn, T(1), w.Rm.p, T(0), MUbb, ri);
@@ -2281,9 +2790,11 @@ int ns_graph_setup(NsGraphWork<T> &w, crimson_lhs *l, crimson_ls *ls, const int 
     c.hfdev.push_back(FaceDev{fa.d_glob.p, fa.d_valM.p, 0.0, w.fcoef.p + f, fa.res, fa.nNo, fa.dof, fa.d_sup.p,
                               fa.d_q.p, fa.nsup});
   }
-  if (!c.hfdev.empty()) {
-    CR_TRY(c.fdev.alloc(c.hfdev.size()));
-    CR_HIP(hipMemcpyAsync(c.fdev.p, c.hfdev.data(), c.hfdev.size() * sizeof(FaceDev), hipMemcpyHostToDevice, s));
+  CR_TRY(face_list(c));
+  {
+    SchurOp<T> so;
+    CR_TRY(schur_ready(l, so));
+    w.formed = so.formed;
   }
   CR_TRY(w.msum.alloc(std::max<size_t>(1, c.hfdev.size())));
   {
@@ -2574,6 +3085,7 @@ extern "C" int crimson_lhs_create(int gnNo, int nNo, int nnz, const int *gNodes,
           fits = false;
           break;
         }
+        l->band = std::max(l->band, std::abs(d));
         c16[k] = (short)d;
       }
     if (fits && (rc = l->d_col16.upload(c16.data(), nnz, l->stream))) return fail(rc);
