@@ -8,6 +8,7 @@
 #include <cstdarg>
 #include <cstdio>
 #include <cstdint>
+#include <memory>
 #include <string>
 #include <vector>
 
@@ -41,6 +42,10 @@ inline unsigned long long next_alloc_serial() {
   static std::atomic<unsigned long long> counter{0};
   return ++counter;
 }
+
+// Frees the solver workspaces that matrix handles keep for their next solve
+// (memls.hip); false when there was none.  Called when an allocation fails.
+bool release_idle_work();
 
 // Owning device allocation.
 template <class T>
@@ -80,6 +85,10 @@ struct DBuf {
     release();
     if (count == 0) return CRIMSON_OK;
     hipError_t e = hipMalloc((void **)&p, count * sizeof(T));
+    if (e == hipErrorOutOfMemory && release_idle_work()) {
+      (void)hipGetLastError();
+      e = hipMalloc((void **)&p, count * sizeof(T));
+    }
     if (e != hipSuccess) {
       p = nullptr;
       set_error("hipMalloc of %zu bytes failed: %s", count * sizeof(T), hipGetErrorString(e));
@@ -202,6 +211,14 @@ struct CrFace {
   crimson::DBuf<double> d_q;  // the functional's coefficients, per solve
 };
 
+namespace crimson {
+// A solve's workspaces, as a matrix handle keeps them (memls.hip).
+struct SolveWorkBase {
+  virtual ~SolveWorkBase() = default;
+  virtual size_t bytes() const = 0;
+};
+}  // namespace crimson
+
 // One entry of the coupled faces' merged supports: a node, the face (its place among
 // the coupled ones) and the node's place in that face's support.
 struct CrFaceEnt {
@@ -244,5 +261,7 @@ struct crimson_lhs {
   crimson::DBuf<short> d_scol16;
   crimson::DBuf<double> d_S;
   crimson::DBuf<float> d_S32;
+  // the workspaces of the last plain solve in FP64 and in FP32 (work_take, work_keep)
+  std::unique_ptr<crimson::SolveWorkBase> work[2];
   hipEvent_t ev0 = nullptr, ev1 = nullptr;
 };

@@ -11,16 +11,17 @@
 //    where fix marks the diagonal entries memLS forces to 1 (zero diagonal,
 //    Dirichlet-masked DOF; memLS.f90:1815-1820,1923-1929).  This saves the two
 //    read+write sweeps over Val per solve.
-//  * Dots and norms are two-stage deterministic reductions (per-workgroup
-//    partials in a fixed order, then one workgroup per result).
+//  * Dots and norms are two-stage deterministic reductions: parts per
+//    workgroup in a fixed order, summed by whichever kernel needs the result.
 //  * GMRES orthogonalises with classical Gram-Schmidt and a DGKS second pass
 //    (taken when ||w'|| < ||w||/sqrt 2), computing all i projections of a
 //    step in one sweep.  memLS uses modified Gram-Schmidt (memLS.f90:743-746);
 //    both produce the same Krylov space, and solutions agree to the solver
-//    tolerance.  Givens rotations, the convergence test and the triangular
-//    solve run on the host in FP64 exactly as memLS.f90:750-775.
-//  * CG iterations run device-resident with a device-side convergence flag;
-//    the host enqueues them in batches and reads the flag between batches.
+//    tolerance.
+//  * Every decision of a solve (Givens rotations, convergence tests, CGRAD's
+//    iteration count, NSSOLVER's least squares) is taken on the device.  A
+//    captured solve enqueues every possible iteration; a plain one runs the
+//    same launches, polls the flags from pinned memory and stops enqueueing.
 
 #include <hip/hip_runtime.h>
 
@@ -30,6 +31,8 @@
 #include <cmath>
 #include <cstring>
 #include <functional>
+#include <memory>
+#include <mutex>
 #include <vector>
 
 #include "common.hpp"
@@ -148,6 +151,18 @@ constexpr int kNarrowLanes = 4;
 // and every workgroup of the next sweep sums all of them.
 constexpr int kCgGrid = 2048;
 
+// What a deciding kernel tells the host of a solve that is not captured: its
+// place in the solve's sequence and whether the loop it belongs to is over,
+// as one word of pinned memory that the host polls, so that no copy or event
+// stands between two steps.  p is null in a captured solve.
+struct HostFlag {
+  unsigned long long *p;
+  unsigned long long seq;
+  __device__ void tell(bool stop) const {
+    if (p) __hip_atomic_store(p, seq << 1 | (stop ? 1u : 0u), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+  }
+};
+
 // A coupled face of the Schur CG (ADDBCMUL's PRE, memLS.f90:1719-1735).  PRE
 // adds coef_f S_f valM_f to t1 = G P with S_f = valM_f . t1; with Gt = -G^T
 // (DEPART) that is the symmetric rank-one term c_f q_f q_f^T on the
@@ -159,8 +174,7 @@ constexpr int kCgGrid = 2048;
 struct FaceDev {
   const int *glob;
   const double *valM;
-  double coef;
-  const double *coefp;  // the coefficient on the device (device-driven solves), or null: coef
+  const double *coefp;  // c_f = -res / (1 + res nS) (BCPRE)
   double res;           // the face's coupling coefficient (ADDBCMUL without PRE)
   int nNo, dof;
   const int *sup;
@@ -569,111 +583,294 @@ __device__ inline double sum_parts(const double *__restrict__ part, int n, doubl
   return block_sum_all(more, sh);
 }
 
-// partial[blk][j] = sum over this block's chunk of U_j . v for j < m, and
-// partial[blk][m] = v . v when self != 0.  U_j = U0 + j * ustride.  Vectors
-// of type T, products and sums in Acc.
-template <class T, class Acc>
-__global__ void __launch_bounds__(256) mdot_kernel(size_t L, const T *__restrict__ v, const T *__restrict__ U0,
-                                                   size_t ustride, int m, int self, Acc *__restrict__ partial,
-                                                   int pstride, const int *__restrict__ gate,
-                                                   const double *__restrict__ skip) {
-  if ((gate && *gate == 0) || (skip && *skip != 0.0)) return;
-  __shared__ Acc sh[4];
-  const size_t base = (size_t)blockIdx.x * kChunk;
-  Acc vv[kChunk / 256];
+// ----- dots and the Arnoldi step -----
+// v (1024 threads) summed over the workgroup, in every thread, always in the
+// same order.
+constexpr int kDotThreads = 1024, kDotGrid = 256, kDotGroup = 8;
+__device__ inline double wave_sum(double v) {
 #pragma unroll
-  for (int t = 0; t < kChunk / 256; ++t) {
-    const size_t e = base + threadIdx.x + 256 * t;
-    vv[t] = e < L ? (Acc)v[e] : Acc(0);
-  }
-  Acc *out = partial + (size_t)blockIdx.x * pstride;
-  for (int j = 0; j < m; ++j) {
-    const T *u = U0 + ustride * j;
-    Acc s = Acc(0);
-#pragma unroll
-    for (int t = 0; t < kChunk / 256; ++t) {
-      const size_t e = base + threadIdx.x + 256 * t;
-      if (e < L) s += (Acc)u[e] * vv[t];
-    }
-    s = block_sum(s, sh);
-    if (threadIdx.x == 0) out[j] = s;
-  }
-  if (self) {
-    Acc s = Acc(0);
-#pragma unroll
-    for (int t = 0; t < kChunk / 256; ++t) s += vv[t] * vv[t];
-    s = block_sum(s, sh);
-    if (threadIdx.x == 0) out[m] = s;
-  }
+  for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
+  return v;
 }
-
-// out[j] = sum_blk partial[blk][j], j < m, one workgroup per j, fixed order
-// (summed in T, stored as double for the host-side FP64 scalars).
-template <class T>
-__global__ void __launch_bounds__(256) reduce_kernel(int nblk, const T *__restrict__ partial, int pstride,
-                                                     double *__restrict__ out, const int *__restrict__ gate,
-                                                     const double *__restrict__ skip) {
-  __shared__ T sh[4];
-  const int j = blockIdx.x;
-  if (skip && *skip != 0.0) return;
-  if (gate && *gate == 0) {
-    if (threadIdx.x == 0) out[j] = 0.0;
-    return;
-  }
-  T s = T(0);
-  for (int b = threadIdx.x; b < nblk; b += 256) s += partial[(size_t)b * pstride + j];
-  s = block_sum(s, sh);
-  if (threadIdx.x == 0) out[j] = (double)s;
-}
-
-// y -= sum_j coef[j] U_j (coef on the device), then the block's partial of
-// y . y into partial[blk * pstride].
-template <class T>
-__global__ void __launch_bounds__(256) msub_norm_kernel(size_t L, T *__restrict__ y, const T *__restrict__ U0,
-                                                        size_t ustride, int m, const double *__restrict__ coef,
-                                                        T *__restrict__ partial, int pstride,
-                                                        const int *__restrict__ gate,
-                                                        const double *__restrict__ skip) {
-  if ((gate && *gate == 0) || (skip && *skip != 0.0)) return;
-  __shared__ T sh[4];
-  __shared__ T cs[256];
-  for (int j = threadIdx.x; j < m && j < 256; j += 256) cs[j] = (T)coef[j];
+__device__ inline double block_sum_1024(double v, double *sh) {
+  v = wave_sum(v);
+  if ((threadIdx.x & 63) == 0) sh[threadIdx.x / 64] = v;
   __syncthreads();
-  const size_t base = (size_t)blockIdx.x * kChunk;
-  T s = T(0);
+  double t = threadIdx.x % 64 < 16 ? sh[threadIdx.x % 64] : 0.0;
 #pragma unroll
-  for (int t = 0; t < kChunk / 256; ++t) {
-    const size_t e = base + threadIdx.x + 256 * t;
-    if (e < L) {
-      T w = y[e];
-      for (int j = 0; j < m; ++j) w -= cs[j] * U0[ustride * j + e];
-      y[e] = w;
-      s += w * w;
-    }
+  for (int off = 8; off > 0; off >>= 1) t += __shfl_xor(t, off, 16);
+  t = __shfl(t, 0, 64);
+  __syncthreads();
+  return t;
+}
+// Parts of the dots of v with U_j = U0 + j ustride, j < m, and of v with itself
+// as the m-th when self: part[j * gridDim.x + blockIdx.x], summed by the kernel
+// that needs them.  At most kDotGrid workgroups of 16 waves walk the entries;
+// a grid row takes kDotGroup vectors.  (All vectors in one grid row, one after the
+// other with two barriers each, took 43 us for 50 vectors of 20,000 entries.)
+template <class T>
+__device__ inline void dots_body(size_t L, const T *__restrict__ v, const T *__restrict__ U0, size_t ustride, int m,
+                                 int self, double *__restrict__ part, double (*sh)[kDotGroup]) {
+  const int j0 = blockIdx.y * kDotGroup, nb = gridDim.x;
+  const int n = min(kDotGroup, m + self - j0);
+  double acc[kDotGroup];
+#pragma unroll
+  for (int q = 0; q < kDotGroup; ++q) acc[q] = 0.0;
+  for (size_t e = (size_t)blockIdx.x * kDotThreads + threadIdx.x; e < L; e += (size_t)nb * kDotThreads) {
+    const double x = (double)v[e];
+    T u[kDotGroup];
+#pragma unroll
+    for (int q = 0; q < kDotGroup; ++q) u[q] = j0 + q < m ? U0[ustride * (j0 + q) + e] : v[e];
+#pragma unroll
+    for (int q = 0; q < kDotGroup; ++q) acc[q] += (double)u[q] * x;
   }
-  s = block_sum(s, sh);
-  if (threadIdx.x == 0) partial[(size_t)blockIdx.x * pstride] = s;
+#pragma unroll
+  for (int q = 0; q < kDotGroup; ++q)
+    if (q < n) acc[q] = wave_sum(acc[q]);  // n is the workgroup's
+  if ((threadIdx.x & 63) == 0)
+#pragma unroll
+    for (int q = 0; q < kDotGroup; ++q) sh[threadIdx.x / 64][q] = acc[q];
+  __syncthreads();
+  if ((int)threadIdx.x < n) {
+    double t = 0.0;
+    for (int w = 0; w < kDotThreads / 64; ++w) t += sh[w][threadIdx.x];
+    part[(size_t)(j0 + threadIdx.x) * nb + blockIdx.x] = t;
+  }
+}
+template <class T>
+__global__ void __launch_bounds__(kDotThreads) dots_kernel(size_t L, const T *__restrict__ v,
+                                                           const T *__restrict__ U0, size_t ustride, int m, int self,
+                                                           double *__restrict__ part,
+                                                           const double *__restrict__ skip) {
+  if (skip && *skip != 0.0) return;
+  __shared__ double sh[kDotThreads / 64][kDotGroup];
+  dots_body(L, v, U0, ustride, m, self, part, sh);
+}
+// The sum of n <= kDotGrid parts by one wave, in every lane.
+__device__ inline double wave_parts(const double *__restrict__ part, int n) {
+  const int lane = threadIdx.x % 64;
+  double v[kDotGrid / 64];
+#pragma unroll
+  for (int u = 0; u < kDotGrid / 64; ++u) v[u] = lane + 64 * u < n ? part[lane + 64 * u] : 0.0;
+  double t = 0.0;
+#pragma unroll
+  for (int u = 0; u < kDotGrid / 64; ++u) t += v[u];
+  return wave_sum(t);
 }
 
-// y += sum_j coef[j] U_j, coef on the device.
+// One Arnoldi step (classical Gram-Schmidt with one DGKS pass) in six
+// launches without a host decision:
+//   arnoldi_spmv   u = scale w (the new basis vector) and y = A u
+//   face_apply     the coupled faces' terms on y (when there are any)
+//   dots           y against the basis, and y . y
+//   arnoldi_sub    y -= U h, W o y for the next product, parts of y . y
+//   dots, sub      the second pass, where ||y'||^2 < ||y||^2 / 2 (every workgroup
+//                  takes that decision itself from the same parts)
+//   gm_givens      the Hessenberg column, rotations, test and 1 / ||y||
+// scale is 1 / ||w||; U_j is stored normalised.  The product gathers W o w, one
+// aligned entry of 2 or 4 components per column, in place of W and w.
+template <int NC>
+struct ArnoldiPad {
+  static constexpr int n = NC == 3 ? 4 : NC;  // components of a gathered entry
+};
+template <int NC, class T>
+__device__ inline void load_entry(const T *__restrict__ p, T (&x)[NC]) {
+  if constexpr (NC >= 3) {
+    T z[4];
+    load4(p, z);
+#pragma unroll
+    for (int c = 0; c < NC; ++c) x[c] = z[c];
+  } else {
+#pragma unroll
+    for (int c = 0; c < NC; ++c) x[c] = p[c];
+  }
+}
+template <int NC, class T, class IX>
+__global__ void __launch_bounds__(256) arnoldi_spmv_kernel(int nNo, const int *__restrict__ rowptr,
+                                                           const IX *__restrict__ col, MatView<T> A,
+                                                           const T *__restrict__ w, const T *__restrict__ ws,
+                                                           const double *__restrict__ scale, T *__restrict__ u,
+                                                           T *__restrict__ y, const double *__restrict__ skip) {
+  constexpr int LANES = NC >= 3 ? kRowLanes : kNarrowLanes, PAD = ArnoldiPad<NC>::n;
+  const double stop = *skip;
+  const int gid = crimson::xcd_block(kRowXcdChunk) * blockDim.x + threadIdx.x;
+  const int row = gid / LANES, lane = threadIdx.x % LANES;
+  const int kb = rowptr[min(row, nNo)], ke = rowptr[min(row + 1, nNo)];
+  if (stop != 0.0) return;
+  T acc[NC];
+#pragma unroll
+  for (int r = 0; r < NC; ++r) acc[r] = T(0);
+  for (int k = kb + lane; k < ke; k += LANES) {
+    T a[NC * NC], x[NC];
+    const int j = col_at(col, k, row);
+#pragma unroll
+    for (int r = 0; r < NC; ++r)
+#pragma unroll
+      for (int c = 0; c < NC; ++c) a[r * NC + c] = A.base[(size_t)A.plane[r * 4 + c] * A.nnz + k];
+    load_entry<NC>(ws + (size_t)PAD * j, x);
+#pragma unroll
+    for (int r = 0; r < NC; ++r)
+#pragma unroll
+      for (int c = 0; c < NC; ++c) acc[r] += a[r * NC + c] * x[c];
+  }
+#pragma unroll
+  for (int off = LANES / 2; off > 0; off >>= 1)
+#pragma unroll
+    for (int r = 0; r < NC; ++r) acc[r] += __shfl_xor(acc[r], off, LANES);
+  if (row < nNo && lane == 0) {
+    const T s = (T)*scale;
+#pragma unroll
+    for (int r = 0; r < NC; ++r) {
+      const size_t e = r + (size_t)NC * row, f = A.r0 + r + (size_t)A.wdof * row;
+      const T ur = s * w[e];
+      u[e] = ur;
+      y[e] = A.W[f] * (s * acc[r]) + A.fix[f] * ur;
+    }
+  }
+}
+// whether the second pass is taken: parts n1[0, nb) of ||y'||^2 against n0 =
+// ||y||^2; the same answer in every thread of every workgroup
+__device__ inline bool dgks_pass(const double *__restrict__ n0, const double *__restrict__ n1, int nb, double *sh) {
+  const double s = block_sum_1024((int)threadIdx.x < nb ? n1[threadIdx.x] : 0.0, sh);
+  return s < 0.5 * *n0;
+}
 template <class T>
-__global__ void maxpy_kernel(size_t L, T *__restrict__ y, const T *__restrict__ U0, size_t ustride, int m,
-                             const double *__restrict__ coef, double sign) {
+__global__ void __launch_bounds__(kDotThreads) dots2_kernel(size_t L, const T *__restrict__ v,
+                                                            const T *__restrict__ U0, size_t ustride, int m,
+                                                            double *__restrict__ part,
+                                                            const double *__restrict__ n0,
+                                                            const double *__restrict__ n1, int nb,
+                                                            const double *__restrict__ skip) {
+  if (*skip != 0.0) return;
+  __shared__ double sh[kDotThreads / 64][kDotGroup];
+  if (!dgks_pass(n0, n1, nb, &sh[0][0])) return;
+  dots_body(L, v, U0, ustride, m, 0, part, sh);
+}
+// h = the dots' sums (np parts each; self: the m-th is ||y||^2), y -= U h and
+// its scaled copy, parts of y . y.  JS threads share an entry's sum over the
+// basis: one for long vectors, four for short ones, which leave a
+// thread alone with a chain of m loads.  n1 (the second pass): taken or left
+// as dgks_pass says.
+constexpr int kSubGrid = 1024;
+template <class T, int JS>
+__global__ void __launch_bounds__(kDotThreads) arnoldi_sub_kernel(
+    size_t L, int nc, int pad, const T *__restrict__ W, int wdof, int w0, T *__restrict__ y, T *__restrict__ ys,
+    const T *__restrict__ U0, size_t ustride, int m, int self, const double *__restrict__ part, int np,
+    double *__restrict__ h, double *__restrict__ npart, const double *__restrict__ n0, const double *__restrict__ n1,
+    const double *__restrict__ skip) {
+  if (*skip != 0.0) return;
+  constexpr int kE = kDotThreads / JS;  // entries a turn
+  __shared__ double sh[16];
+  __shared__ T cs[256];
+  __shared__ T comb[JS > 1 ? kDotThreads : 1];
+  if (n1 && !dgks_pass(n0, n1, gridDim.x, sh)) return;
+  for (int j = threadIdx.x / 64; j < m + self; j += kDotThreads / 64) {
+    const double t = wave_parts(part + (size_t)j * np, np);
+    if (threadIdx.x % 64 == 0) {
+      if (j < m) cs[j] = (T)t;
+      if (blockIdx.x == 0) h[j] = t;
+    }
+  }
+  __syncthreads();
+  const int js = threadIdx.x / kE;
+  double s = 0.0;
+  for (size_t b = (size_t)blockIdx.x * kE; b < L; b += (size_t)gridDim.x * kE) {
+    const size_t e = b + threadIdx.x % kE;
+    T t = T(0);
+    if (e < L) {
+      int j = js;
+      for (; j + 7 * JS < m; j += 8 * JS) {
+        T u[8];
+#pragma unroll
+        for (int q = 0; q < 8; ++q) u[q] = U0[ustride * (j + q * JS) + e];
+#pragma unroll
+        for (int q = 0; q < 8; ++q) t += cs[j + q * JS] * u[q];
+      }
+      for (; j < m; j += JS) t += cs[j] * U0[ustride * j + e];
+    }
+    if (JS > 1) {
+      __syncthreads();  // the previous turn's sums are read
+      comb[threadIdx.x] = t;
+      __syncthreads();
+      if (js == 0)
+#pragma unroll
+        for (int q = 1; q < JS; ++q) t += comb[threadIdx.x + q * kE];
+    }
+    if (js == 0 && e < L) {
+      const T v = y[e] - t;
+      y[e] = v;
+      const size_t i = e / nc, c = e % nc;
+      ys[pad * i + c] = W[w0 + c + wdof * i] * v;
+      s += (double)v * (double)v;
+    }
+  }
+  s = block_sum_1024(s, sh);
+  if (threadIdx.x == 0) npart[blockIdx.x] = s;
+}
+// The cycle's first vector: w (already R or R - A X with the faces' PRE), its
+// scaled copy and parts of w . w.
+template <class T>
+__global__ void __launch_bounds__(kDotThreads) arnoldi_first_kernel(size_t L, int nc, int pad,
+                                                                    const T *__restrict__ W, int wdof, int w0,
+                                                                    const T *__restrict__ w, T *__restrict__ ws,
+                                                                    double *__restrict__ npart,
+                                                                    const double *__restrict__ skip) {
+  if (*skip != 0.0) return;
+  __shared__ double sh[16];
+  double s = 0.0;
+  for (size_t e = (size_t)blockIdx.x * kDotThreads + threadIdx.x; e < L; e += (size_t)gridDim.x * kDotThreads) {
+    const T v = w[e];
+    const size_t i = e / nc, c = e % nc;
+    ws[pad * i + c] = W[w0 + c + wdof * i] * v;
+    s += (double)v * (double)v;
+  }
+  s = block_sum_1024(s, sh);
+  if (threadIdx.x == 0) npart[blockIdx.x] = s;
+}
+
+// ----- plain vector sweeps (skip: return at once when *skip is set; may be null) -----
+template <class T>
+__global__ void fill_kernel(size_t L, T *__restrict__ x, const double *__restrict__ skip) {
+  if (skip && *skip != 0.0) return;
+  const size_t e = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (e < L) x[e] = T(0);
+}
+template <class T>
+__global__ void copy_kernel(size_t L, const T *__restrict__ src, T *__restrict__ dst,
+                            const double *__restrict__ skip) {
+  if (skip && *skip != 0.0) return;
+  const size_t e = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (e < L) dst[e] = src[e];
+}
+// z = x - y
+template <class T>
+__global__ void diff_kernel(size_t L, const T *__restrict__ x, const T *__restrict__ y, T *__restrict__ z,
+                            const double *__restrict__ skip) {
+  if (skip && *skip != 0.0) return;
+  const size_t e = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (e < L) z[e] = x[e] - y[e];
+}
+// y = x + sign sum_j coef[j] U_j, j < m (*m_dev when given); x may be y
+template <class T>
+__global__ void combine_kernel(size_t L, const T *__restrict__ x, T *__restrict__ y, const T *__restrict__ U0,
+                               size_t ustride, int m, const double *__restrict__ m_dev,
+                               const double *__restrict__ coef, double sign, const double *__restrict__ skip) {
+  if (skip && *skip != 0.0) return;
   const size_t e = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (e >= L) return;
-  T w = y[e];
-  for (int j = 0; j < m; ++j) w += (T)(sign * coef[j]) * U0[ustride * j + e];
+  if (m_dev) m = (int)*m_dev;
+  T w = x[e];
+  int j = 0;
+  for (; j + 8 <= m; j += 8) {
+    T u[8];
+#pragma unroll
+    for (int q = 0; q < 8; ++q) u[q] = U0[ustride * (j + q) + e];
+#pragma unroll
+    for (int q = 0; q < 8; ++q) w += (T)(sign * coef[j + q]) * u[q];
+  }
+  for (; j < m; ++j) w += (T)(sign * coef[j]) * U0[ustride * j + e];
   y[e] = w;
 }
-
-// y = a x + b y
-template <class T>
-__global__ void axpby_kernel(size_t L, T a, const T *__restrict__ x, T b, T *__restrict__ y) {
-  const size_t e = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (e >= L) return;
-  y[e] = a * x[e] + (b == T(0) ? T(0) : b * y[e]);
-}
-
 // y = x * w elementwise (types may differ: the FP64 right-hand side in and
 // the solution out of an FP32 solve)
 template <class TX, class TW, class TY>
@@ -682,19 +879,44 @@ __global__ void mul_kernel(size_t L, const TX *__restrict__ x, const TW *__restr
   if (e >= L) return;
   y[e] = (TY)(x[e] * w[e]);
 }
-
-// Strided component extraction/insert between (dof,N) and (n,N) vectors.
+// The NS solver's vectors hold the velocity (3, N) and behind it the
+// pressure (N).  W o Ri (4, N) in that layout, into both r0 and r.
 template <class T>
-__global__ void extract_kernel(int N, int dof, int c0, int nc, const T *__restrict__ src, T *__restrict__ dst) {
+__global__ void ns_split_kernel(int N, const double *__restrict__ Ri, const T *__restrict__ W, T *__restrict__ r0,
+                                T *__restrict__ r) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= N) return;
-  for (int c = 0; c < nc; ++c) dst[c + (size_t)nc * i] = src[c0 + c + (size_t)dof * i];
+#pragma unroll
+  for (int c = 0; c < 4; ++c) {
+    const size_t s = c + (size_t)4 * i, d = c < 3 ? c + (size_t)3 * i : (size_t)3 * N + i;
+    const T v = (T)(Ri[s] * W[s]);
+    r0[d] = v;
+    r[d] = v;
+  }
 }
+// The solution: velocity sum_k cu[k] U_k, pressure sum_k cp[k] P_k (U_k and P_k
+// behind each other in X_k), times W, into Ri (4, N).
 template <class T>
-__global__ void insert_kernel(int N, int dof, int c0, int nc, const T *__restrict__ src, T *__restrict__ dst) {
+__global__ void ns_join_kernel(int N, const T *__restrict__ X0, const double *__restrict__ cnt,
+                               const double *__restrict__ cu, const double *__restrict__ cp, const T *__restrict__ W,
+                               double *__restrict__ Ri, const double *__restrict__ skip) {
+  if (*skip != 0.0) return;
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= N) return;
-  for (int c = 0; c < nc; ++c) dst[c0 + c + (size_t)dof * i] = src[c + (size_t)nc * i];
+  const int n = (int)*cnt;
+  const size_t st = (size_t)4 * N;
+  T v[4] = {T(0), T(0), T(0), T(0)};
+  for (int k = 0; k < n; ++k) {
+    const T a = (T)cu[k], b = (T)cp[k];
+#pragma unroll
+    for (int c = 0; c < 3; ++c) v[c] += a * X0[st * k + 3 * (size_t)i + c];
+    v[3] += b * X0[st * k + (size_t)3 * N + i];
+  }
+#pragma unroll
+  for (int c = 0; c < 4; ++c) {
+    const size_t s = c + (size_t)4 * i;
+    Ri[s] = (double)(v[c] * W[s]);
+  }
 }
 
 // PRECOND part 1: W from the diagonal, fix for zero diagonals.
@@ -744,77 +966,57 @@ __global__ void face_valm_kernel(int n, int dof, int fdof, const int *__restrict
   for (int i = 0; i < nc; ++i)
     valM[i + (size_t)fdof * a] = val[i + (size_t)fdof * a] * (double)W[i + (size_t)dof * glob[a]];
 }
-// S = sum_a sum_i valM(i,a) X(i, glob(a)) in one 1024-thread workgroup
-// (faces are small): per-wave sums, then the 16 wave sums in a fixed order.
+// ADDBCMUL (memLS.f90:206-268) on the coupled faces: with ADD, Y += res_f (v_f .
+// X) v_f; with PRE, then Y += coef_f (v_f . Y) v_f, every dot taken before any
+// update of its kind (memLS's copy unCondU).  One 1024-thread workgroup per
+// face when no two share a node (then they do not see each other's
+// updates), one for all of them otherwise (each face in turn between
+// barriers).  Replaces a dot and an update launch per face and kind.
+constexpr int kFaceAdd = 1, kFacePre = 2;
 template <class T>
-__global__ void __launch_bounds__(1024) face_dot_kernel(int n, int xdof, int fdof, const int *__restrict__ glob,
-                                                        const double *__restrict__ valM, const T *__restrict__ X,
-                                                        double *__restrict__ out, const double *__restrict__ skip) {
+__global__ void __launch_bounds__(1024) face_apply_kernel(const FaceDev *__restrict__ fd, int nfc, int what, int xdof,
+                                                          const T *__restrict__ X, T *__restrict__ Y,
+                                                          double *__restrict__ sum, const double *__restrict__ skip) {
   if (skip && *skip != 0.0) return;
   __shared__ double sh[16];
-  const int nc = fdof < xdof ? fdof : xdof;
-  double s = 0.0;
-  for (int a = threadIdx.x; a < n; a += 1024)
-    for (int i = 0; i < nc; ++i) s += valM[i + (size_t)fdof * a] * (double)X[i + (size_t)xdof * glob[a]];
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) s += __shfl_xor(s, off, 64);
-  if ((threadIdx.x & 63) == 0) sh[threadIdx.x / 64] = s;
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    double t = 0.0;
-    for (int w = 0; w < 16; ++w) t += sh[w];
-    *out = t;
+  const int f0 = gridDim.x > 1 ? blockIdx.x : 0, f1 = gridDim.x > 1 ? f0 + 1 : nfc;
+  auto dot = [&](const FaceDev &F, const T *x) {
+    const int nc = F.dof < xdof ? F.dof : xdof;
+    double s = 0.0;
+    for (int a = threadIdx.x; a < F.nNo; a += 1024)
+      for (int i = 0; i < nc; ++i) s += F.valM[i + (size_t)F.dof * a] * (double)x[i + (size_t)xdof * F.glob[a]];
+    return block_sum_1024(s, sh);
+  };
+  auto add = [&](const FaceDev &F, double c) {
+    const int nc = F.dof < xdof ? F.dof : xdof;
+    for (int a = threadIdx.x; a < F.nNo; a += 1024)
+      for (int i = 0; i < nc; ++i) Y[i + (size_t)xdof * F.glob[a]] += (T)(F.valM[i + (size_t)F.dof * a] * c);
+  };
+  for (int kind = kFaceAdd; kind <= kFacePre; kind <<= 1) {
+    if (!(what & kind)) continue;
+    for (int f = f0; f < f1; ++f) {
+      const double d = dot(fd[f], kind == kFaceAdd ? X : Y);
+      if (threadIdx.x == 0) sum[f] = d;
+    }
+    __syncthreads();
+    for (int f = f0; f < f1; ++f) {
+      add(fd[f], (kind == kFaceAdd ? fd[f].res : *fd[f].coefp) * sum[f]);
+      __syncthreads();
+    }
   }
 }
-// Y(i, glob(a)) += valM(i,a) * coef * S (coef from *coefp when given)
-template <class T>
-__global__ void face_axpy_kernel(int n, int xdof, int fdof, const int *__restrict__ glob,
-                                 const double *__restrict__ valM, const double *__restrict__ S, double coef,
-                                 T *__restrict__ Y, const double *__restrict__ coefp,
-                                 const double *__restrict__ skip) {
-  if (skip && *skip != 0.0) return;
-  const int a = blockIdx.x * blockDim.x + threadIdx.x;
-  if (a >= n) return;
-  const int nc = fdof < xdof ? fdof : xdof;
-  const double s = (coefp ? *coefp : coef) * *S;
-  for (int i = 0; i < nc; ++i) Y[i + (size_t)xdof * glob[a]] += (T)(valM[i + (size_t)fdof * a] * s);
-}
-// The same two face operations for every coupled face in one launch, when
-// the faces share no node (then the faces' updates commute): one
-// 1024-thread workgroup per face for the dots (face_dot_kernel's order), and
-// a grid row per face for the updates.  Per face the arithmetic is the
-// single-face kernels'.
-template <class T>
-__global__ void __launch_bounds__(1024) face_dot_multi_kernel(const FaceDev *__restrict__ fd, int xdof,
-                                                              const T *__restrict__ X, double *__restrict__ out,
-                                                              const double *__restrict__ skip) {
-  if (skip && *skip != 0.0) return;
+// BCPRE's nS of the coupled faces (memLS.f90:1683-1716: ||valM||^2 over nsd
+// components) and their PRE coefficients -res / (1 + res nS), a workgroup each
+__global__ void __launch_bounds__(1024) face_coef_kernel(const FaceDev *__restrict__ fd, int nsd,
+                                                         double *__restrict__ coef) {
   __shared__ double sh[16];
   const FaceDev F = fd[blockIdx.x];
-  const int nc = F.dof < xdof ? F.dof : xdof;
+  const int nc = F.dof < nsd ? F.dof : nsd;
   double s = 0.0;
   for (int a = threadIdx.x; a < F.nNo; a += 1024)
-    for (int i = 0; i < nc; ++i) s += F.valM[i + (size_t)F.dof * a] * (double)X[i + (size_t)xdof * F.glob[a]];
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) s += __shfl_xor(s, off, 64);
-  if ((threadIdx.x & 63) == 0) sh[threadIdx.x / 64] = s;
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    double t = 0.0;
-    for (int w = 0; w < 16; ++w) t += sh[w];
-    out[blockIdx.x] = t;
-  }
-}
-template <class T>
-__global__ void face_axpy_multi_kernel(const FaceDev *__restrict__ fd, int xdof, const double *__restrict__ S,
-                                       int pre, T *__restrict__ Y, const double *__restrict__ skip) {
-  if (skip && *skip != 0.0) return;
-  const FaceDev F = fd[blockIdx.y];
-  const int a = blockIdx.x * blockDim.x + threadIdx.x;
-  if (a >= F.nNo) return;
-  const int nc = F.dof < xdof ? F.dof : xdof;
-  const double s = (pre ? (F.coefp ? *F.coefp : F.coef) : F.res) * S[blockIdx.y];
-  for (int i = 0; i < nc; ++i) Y[i + (size_t)xdof * F.glob[a]] += (T)(F.valM[i + (size_t)F.dof * a] * s);
+    for (int i = 0; i < nc; ++i) s += F.valM[i + (size_t)F.dof * a] * F.valM[i + (size_t)F.dof * a];
+  s = block_sum_1024(s, sh);
+  if (threadIdx.x == 0) coef[blockIdx.x] = -F.res / (1.0 + F.res * s);
 }
 // The face functional's coefficients q (FaceDev), one thread per support
 // column, its pairs in their stored order, in FP64.
@@ -834,12 +1036,6 @@ __global__ void face_q_kernel(int nsup, const int *__restrict__ sup, const int *
            (double)G.base[(size_t)G.plane[4 * i] * G.nnz + k];
   }
   q[s] = v * (double)G.W[G.c0 + (size_t)G.wdof * sup[s]];
-}
-// DGKS decision: gate = ||w'||^2 < 0.5 ||w||^2
-__global__ void dgks_kernel(const double *__restrict__ n0, const double *__restrict__ n1, int *__restrict__ gate,
-                            const double *__restrict__ skip) {
-  if (skip && *skip != 0.0) return;
-  *gate = (*n1 < 0.5 * *n0) ? 1 : 0;
 }
 // AoS (vdof*vdof, nnz) -> planes, and Gt = -mG^T via the transpose map
 template <class TS, class TD>
@@ -894,7 +1090,7 @@ __device__ inline void check_next(double *scal) {
   scal[1] = scal[0];  // errO = err
   scal[6] += 1.0;
 }
-__device__ inline double face_coef(const FaceDev &F) { return F.coefp ? *F.coefp : F.coef; }
+__device__ inline double face_coef(const FaceDev &F) { return *F.coefp; }
 __device__ inline double face_sum(const FaceList &fl, int f) {
   double S = 0.0;
 #pragma unroll
@@ -1049,7 +1245,8 @@ __global__ void __launch_bounds__(256) cg_p_kernel(size_t L, const double *__res
                                                    double *__restrict__ next, const double *__restrict__ rpart, int nr,
                                                    FaceList fl, T *__restrict__ X, const T *__restrict__ R,
                                                    const T *__restrict__ P, T *__restrict__ Pn,
-                                                   const T *__restrict__ W, int wdof, int off, T *__restrict__ Ps) {
+                                                   const T *__restrict__ W, int wdof, int off, T *__restrict__ Ps,
+                                                   HostFlag hf) {
   const int nf = fl.nfc * kFaceDotBlocks, blk = (int)blockIdx.x - nf;
   __shared__ double sh[4];
   const double stop = scal[5], errO = scal[1], al = scal[3];
@@ -1067,6 +1264,7 @@ __global__ void __launch_bounds__(256) cg_p_kernel(size_t L, const double *__res
   if (blk >= 0) load(base);  // in flight while the parts are summed
   if (stop != 0.0) {
     if (blockIdx.x == 0 && threadIdx.x < kCgState) next[threadIdx.x] = scal[threadIdx.x];
+    if (blockIdx.x == 0 && threadIdx.x == 0) hf.tell(true);
     return;
   }
   const double n = sqrt(sum_parts(rpart, nr, 0.0, sh));  // NORMS(R)
@@ -1078,6 +1276,7 @@ __global__ void __launch_bounds__(256) cg_p_kernel(size_t L, const double *__res
     st[0] = err;
     check_next(st);
     for (int k = 0; k < kCgState; ++k) next[k] = st[k];
+    hf.tell(st[5] != 0.0);
   }
   if (blk < 0) {
     face_part(fl, blockIdx.x, sh, [&](int j) { return R[j] + beta * P[j]; });
@@ -1099,6 +1298,50 @@ __global__ void __launch_bounds__(256) cg_p_kernel(size_t L, const double *__res
 }
 }  // namespace
 
+// The solver workspaces that handles keep, process-wide: every handle that holds
+// one, under one lock.
+namespace crimson {
+namespace {
+std::mutex g_work_lock;
+std::vector<crimson_lhs *> g_work_lhs;
+size_t g_work_bytes = 0;
+std::unique_ptr<SolveWorkBase> work_drop(crimson_lhs *l, int k) {  // under the lock
+  std::unique_ptr<SolveWorkBase> w = std::move(l->work[k]);
+  if (w) g_work_bytes -= w->bytes();
+  if (!l->work[0] && !l->work[1])
+    g_work_lhs.erase(std::remove(g_work_lhs.begin(), g_work_lhs.end(), l), g_work_lhs.end());
+  return w;
+}
+std::unique_ptr<SolveWorkBase> work_take(crimson_lhs *l, bool fp32) {
+  std::lock_guard<std::mutex> hold(g_work_lock);
+  return work_drop(l, fp32 ? 1 : 0);
+}
+void work_keep(crimson_lhs *l, bool fp32, std::unique_ptr<SolveWorkBase> w, size_t most) {
+  std::lock_guard<std::mutex> hold(g_work_lock);
+  std::unique_ptr<SolveWorkBase> old = work_drop(l, fp32 ? 1 : 0);
+  if (g_work_bytes + w->bytes() > most) return;
+  g_work_bytes += w->bytes();
+  l->work[fp32 ? 1 : 0] = std::move(w);
+  if (std::find(g_work_lhs.begin(), g_work_lhs.end(), l) == g_work_lhs.end()) g_work_lhs.push_back(l);
+}
+void work_forget(crimson_lhs *l) {
+  std::lock_guard<std::mutex> hold(g_work_lock);
+  (void)work_drop(l, 0);
+  (void)work_drop(l, 1);
+}
+}  // namespace
+bool release_idle_work() {
+  std::lock_guard<std::mutex> hold(g_work_lock);
+  const bool any = !g_work_lhs.empty();
+  while (!g_work_lhs.empty()) {
+    crimson_lhs *l = g_work_lhs.back();
+    (void)work_drop(l, 0);
+    (void)work_drop(l, 1);
+  }
+  return any;
+}
+}  // namespace crimson
+
 struct crimson_ls {
   SubLs GM, CG, RI;
   int LS_type = 0, Resm = 0, Resc = 0;
@@ -1116,71 +1359,39 @@ inline const float *planes(const crimson_lhs *l, float) { return l->d_V32.p; }
 inline crimson::DBuf<double> &gt_buf(crimson_lhs *l, double) { return l->d_Gt; }
 inline crimson::DBuf<float> &gt_buf(crimson_lhs *l, float) { return l->d_Gt32; }
 
-// Per-solve context: device workspaces sized for this lhs and dof.
+// What every kernel of a solve shares: the handle, the stream, PRECOND's
+// scaling, the reduction scratch and the coupled faces.
 template <class T>
 struct Ctx {
-  crimson_lhs *lhs;
-  hipStream_t s;
-  int N, dof;
+  crimson_lhs *lhs = nullptr;
+  hipStream_t s = nullptr;
+  int N = 0, dof = 0;
   crimson::DBuf<T> W, fix;
-  crimson::DBuf<double> partial;  // per-workgroup partial sums (viewed as T for FP32 accumulation)
-  crimson::DBuf<double> dsc, hcol;
-  crimson::DBuf<double> fsum;  // one face dot per face (ADDBCMUL)
-  crimson::DBuf<double> fpart;  // the Schur CG's face dot partials (kFaceDotBlocks per coupled face)
-  crimson::DBuf<double> cgst;   // the CG's state, twice
-  crimson::DBuf<FaceDev> fdev;  // coupled faces with their PRE coefficients (Schur CG)
-  std::vector<FaceDev> hfdev;
-  crimson::DBuf<int> gate;
-  std::vector<double> hbuf;
-  bool coupled = false;
-  int nblk_max = 0;
-  // the CG's flag read-back: two pinned slots and their events
-  double *hback = nullptr;
-  hipEvent_t evb[2] = {nullptr, nullptr};
+  crimson::DBuf<double> part;    // dot parts: kDotGrid per dot, 2 * kCgGrid in the CG
+  crimson::DBuf<double> cgst;    // the CG's state, twice
+  crimson::DBuf<FaceDev> fdev;   // the coupled faces, in face order
+  crimson::DBuf<double> fcoef;   // their PRE coefficients
+  crimson::DBuf<double> fsum;    // one dot per coupled face (face_apply_kernel)
+  crimson::DBuf<double> fpart;   // the Schur CG's face dot parts (kFaceDotBlocks per face)
+  std::vector<FaceDev> hfdev;    // fdev on the host
+  bool disjoint = true;          // no two coupled faces share a node
+  int nfc() const { return (int)hfdev.size(); }
+  FaceList face_list() const { return FaceList{nfc(), fdev.p, lhs->d_fent.p, lhs->d_ftptr.p, fpart.p}; }
 
-  Ctx() = default;
-  Ctx(const Ctx &) = delete;
-  Ctx &operator=(const Ctx &) = delete;
-  ~Ctx() {
-    if (hback || evb[0] || evb[1]) (void)hipStreamSynchronize(s);  // a read-back may still be in flight
-    if (hback) (void)hipHostFree(hback);
-    for (hipEvent_t e : evb)
-      if (e) (void)hipEventDestroy(e);
-  }
-  int readback_slots() {
-    if (!hback && hipHostMalloc((void **)&hback, 2 * 16 * sizeof(double)) != hipSuccess) {
-      hback = nullptr;
-      crimson::set_error("hipHostMalloc of the CG read-back slots failed");
-      return CRIMSON_ENOMEM;
-    }
-    for (hipEvent_t &e : evb)
-      if (!e) CR_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
-    return CRIMSON_OK;
-  }
-
-  FaceList face_list() const {
-    return FaceList{(int)hfdev.size(), fdev.p, lhs->d_fent.p, lhs->d_ftptr.p, fpart.p};
-  }
-
-  int init(crimson_lhs *l, int d) {
+  int init(crimson_lhs *l, int d, hipStream_t st) {
     lhs = l;
-    s = l->stream;
+    s = st;
     N = l->nNo;
     dof = d;
     const size_t L = (size_t)dof * N;
-    nblk_max = (int)((L + kChunk - 1) / kChunk);
     CR_TRY(W.alloc(L));
     CR_TRY(fix.alloc(L));
-    CR_TRY(partial.alloc(std::max<size_t>((size_t)nblk_max * 256, 2 * kCgGrid)));
+    CR_TRY(part.alloc((size_t)kDotGrid * 3 * 264));
     CR_TRY(cgst.alloc(2 * kCgState));
-    CR_TRY(dsc.alloc(64));
-    CR_TRY(hcol.alloc(4 * 256));
-    CR_TRY(fsum.alloc(std::max<size_t>(1, l->face.size())));
-    CR_TRY(fpart.alloc(std::max<size_t>(1, l->face.size()) * kFaceDotBlocks));
-    CR_TRY(gate.alloc(4));
     return CRIMSON_OK;
   }
 };
+static_assert(kDotGrid * 3 * 264 >= 2 * kCgGrid, "the CG's parts fit the dots'");
 
 template <class T>
 MatView<T> view(const Ctx<T> &c, const T *base, int vdof, int r0, int c0, int nr, int nc, const T *W, const T *fix,
@@ -1240,202 +1451,6 @@ int spmv(Ctx<T> &c, const MatView<T> &A, int nr, int nc, const T *x, T *y, doubl
   return CRIMSON_OK;
 }
 
-// dots of v with U_j (j < m) [+ v.v] -> dst on device (m [+1] values).
-// Accumulation in T, or in FP64 when acc64 (the NS least-squares system and
-// the norms that set the stopping tests of an FP32 solve).
-template <class T>
-int mdot(Ctx<T> &c, size_t L, const T *v, const T *U0, size_t ustride, int m, bool self, double *dst,
-         const int *gate = nullptr, bool acc64 = false, const double *skip = nullptr) {
-  const int nblk = (int)((L + kChunk - 1) / kChunk);
-  const int pst = m + (self ? 1 : 0);
-  if (pst > 256) {
-    crimson::set_error("more than 255 simultaneous projections");
-    return CRIMSON_EUNSUPPORTED;
-  }
-  if (acc64 || sizeof(T) == sizeof(double)) {
-    mdot_kernel<T, double><<<nblk, 256, 0, c.s>>>(L, v, U0, ustride, m, self ? 1 : 0, c.partial.p, pst, gate,
-                                                   skip);
-    reduce_kernel<double><<<pst, 256, 0, c.s>>>(nblk, c.partial.p, pst, dst, gate, skip);
-  } else {
-    T *pt = reinterpret_cast<T *>(c.partial.p);
-    mdot_kernel<T, T><<<nblk, 256, 0, c.s>>>(L, v, U0, ustride, m, self ? 1 : 0, pt, pst, gate, skip);
-    reduce_kernel<T><<<pst, 256, 0, c.s>>>(nblk, pt, pst, dst, gate, skip);
-  }
-  CR_HIP(hipGetLastError());
-  return CRIMSON_OK;
-}
-
-template <class T>
-int axpby(Ctx<T> &c, size_t L, double a, const T *x, double b, T *y) {
-  axpby_kernel<T><<<crimson::grid_for(L, 256), 256, 0, c.s>>>(L, (T)a, x, (T)b, y);
-  CR_HIP(hipGetLastError());
-  return CRIMSON_OK;
-}
-
-template <class T>
-int sync_read(Ctx<T> &c, const double *d, double *h, size_t n) {
-  CR_HIP(hipMemcpyAsync(h, d, n * sizeof(double), hipMemcpyDeviceToHost, c.s));
-  CR_HIP(hipStreamSynchronize(c.s));
-  return CRIMSON_OK;
-}
-
-template <class T>
-double host_norm(Ctx<T> &c, size_t L, const T *v, int *rc) {
-  *rc = mdot<T>(c, L, v, nullptr, 0, 0, true, c.dsc.p + 40, nullptr, true);
-  if (*rc) return 0.0;
-  double h = 0;
-  *rc = sync_read(c, c.dsc.p + 40, &h, 1);
-  return std::sqrt(h);
-}
-
-// ADDBCMUL (memLS.f90:206-268) over all coupled faces, X (xdof, N) -> Y.
-// X may be Y: every face's dot product is taken (stream order) before any
-// face's update is applied, which is what memLS's copy unCondU provides.
-// skip (device, may be null): the device-driven solve's flag that makes
-// these launches return at once; fcoef (device, may be null): every face's
-// PRE coefficient computed on the device (indexed like lhs->face).
-template <class T>
-int addbcmul(Ctx<T> &c, bool pre, int xdof, const T *X, T *Y, const double *skip = nullptr,
-             const double *fcoef = nullptr) {
-  if (!c.coupled) return CRIMSON_OK;
-  auto &faces = c.lhs->face;
-  // all face dots first (PRE reads the unmodified vector, as unCondU does)
-  for (size_t f = 0; f < faces.size(); ++f) {
-    const CrFace &fa = faces[f];
-    if (!fa.coupled) continue;
-    face_dot_kernel<<<1, 1024, 0, c.s>>>(fa.nNo, xdof, fa.dof, fa.d_glob.p, fa.d_valM.p, X, c.fsum.p + f,
-                                         skip);
-  }
-  for (size_t f = 0; f < faces.size(); ++f) {
-    const CrFace &fa = faces[f];
-    if (!fa.coupled) continue;
-    if (fa.nNo == 0) continue;
-    const double coef = pre ? -fa.res / (1.0 + fa.res * fa.nS) : fa.res;
-    face_axpy_kernel<<<crimson::grid_for(fa.nNo, 256), 256, 0, c.s>>>(
-        fa.nNo, xdof, fa.dof, fa.d_glob.p, fa.d_valM.p, c.fsum.p + f, coef, Y, (pre && fcoef) ? fcoef + f : nullptr,
-        skip);
-  }
-  CR_HIP(hipGetLastError());
-  return CRIMSON_OK;
-}
-
-// GMRES (memLS.f90:681-788) for the operator x -> A x + ADD(x), left
-// preconditioned by PRE when faces are coupled; R, X are (nd, N) device.
-template <class T>
-struct Workspace {
-  crimson::DBuf<T> U;  // (sD+1) vectors
-  crimson::DBuf<T> tmp;
-};
-
-template <class T>
-int gmres_dev(Ctx<T> &c, const MatView<T> &A, int nd, SubLs &ls, const T *R, T *X, Workspace<T> &ws, bool pre_ok,
-              bool count_first = false) {
-  const size_t L = (size_t)nd * c.N;
-  const int sD = ls.sD;
-  CR_TRY(ws.U.alloc(L * (sD + 1)));
-  T *U = ws.U.p;
-  std::vector<double> h((size_t)(sD + 1) * sD, 0.0), y(sD), cs(sD), sn(sD), err(sD + 1);
-  auto H = [&](int i, int j) -> double & { return h[(size_t)i + (size_t)(sD + 1) * j]; };
-  const double t0 = now_s();
-  ls.suc = 0;
-  CR_HIP(hipMemsetAsync(X, 0, L * sizeof(T), c.s));
-  double eps = 0.0;
-  int rc = CRIMSON_OK;
-  std::vector<double> hc(2 * (sD + 2) + 4);
-  for (int l = 1; l <= ls.mItr; ++l) {
-    if (l == 1) {
-      // X = 0 here, so R - A X is R (GMRESV still counts the product)
-      if (count_first) ls.itr = ls.itr + 1;
-      CR_HIP(hipMemcpyAsync(U, R, L * sizeof(T), hipMemcpyDeviceToDevice, c.s));
-    } else {
-      ls.itr = ls.itr + 1;
-      CR_TRY(spmv(c, A, nd, nd, X, U));
-      CR_TRY(addbcmul(c, false, nd, X, U));
-      CR_TRY(axpby(c, L, 1.0, R, -1.0, U));
-    }
-    if (c.coupled && pre_ok) CR_TRY(addbcmul(c, true, nd, U, U));
-    err[0] = host_norm(c, L, U, &rc);
-    if (rc) return rc;
-    if (l == 1) {
-      eps = err[0];
-      if (eps <= ls.absTol) {
-        ls.callD = 0.0;
-        ls.dB = 0.0;
-        return CRIMSON_OK;
-      }
-      ls.iNorm = eps;
-      ls.fNorm = eps;
-      eps = std::max(ls.absTol, ls.relTol * eps);
-    }
-    ls.dB = ls.fNorm;
-    CR_TRY(axpby(c, L, 1.0 / err[0], U, 0.0, U));
-    int i;
-    for (i = 1; i <= sD; ++i) {
-      ls.itr = ls.itr + 1;
-      T *ui = U + L * (size_t)i;
-      const T *uprev = U + L * (size_t)(i - 1);
-      CR_TRY(spmv(c, A, nd, nd, uprev, ui));
-      CR_TRY(addbcmul(c, false, nd, uprev, ui));
-      if (c.coupled && pre_ok) CR_TRY(addbcmul(c, true, nd, ui, ui));
-      // CGS pass 1: h1 = U^T w, n0 = w.w ; w -= U h1 ; n1 = w.w
-      double *h1 = c.hcol.p, *h2 = c.hcol.p + 256, *nrm = c.hcol.p + 512;
-      const int nblk = (int)((L + kChunk - 1) / kChunk);
-      CR_TRY(mdot(c, L, ui, U, L, i, true, h1));  // h1[i] = n0
-      T *pt = reinterpret_cast<T *>(c.partial.p);
-      msub_norm_kernel<T><<<nblk, 256, 0, c.s>>>(L, ui, U, L, i, h1, pt, 1, nullptr, nullptr);
-      reduce_kernel<T><<<1, 256, 0, c.s>>>(nblk, pt, 1, nrm + 1, nullptr, nullptr);
-      dgks_kernel<<<1, 1, 0, c.s>>>(h1 + i, nrm + 1, c.gate.p, nullptr);
-      // DGKS pass 2 (gated)
-      CR_TRY(mdot(c, L, ui, U, L, i, false, h2, c.gate.p));
-      msub_norm_kernel<T><<<nblk, 256, 0, c.s>>>(L, ui, U, L, i, h2, pt, 1, c.gate.p, nullptr);
-      reduce_kernel<T><<<1, 256, 0, c.s>>>(nblk, pt, 1, nrm + 2, c.gate.p, nullptr);
-      CR_HIP(hipGetLastError());
-      // read h1[0..i], h2[0..i-1], n1, n2, gate
-      CR_HIP(hipMemcpyAsync(hc.data(), h1, (i + 1) * sizeof(double), hipMemcpyDeviceToHost, c.s));
-      CR_HIP(hipMemcpyAsync(hc.data() + (sD + 2), h2, i * sizeof(double), hipMemcpyDeviceToHost, c.s));
-      double nn[3];
-      CR_HIP(hipMemcpyAsync(nn, nrm, 3 * sizeof(double), hipMemcpyDeviceToHost, c.s));
-      int gate = 0;
-      CR_HIP(hipMemcpyAsync(&gate, c.gate.p, sizeof(int), hipMemcpyDeviceToHost, c.s));
-      CR_HIP(hipStreamSynchronize(c.s));
-      for (int j = 1; j <= i; ++j) H(j - 1, i - 1) = hc[j - 1] + (gate ? hc[(sD + 2) + j - 1] : 0.0);
-      H(i, i - 1) = std::sqrt(gate ? nn[2] : nn[1]);
-      CR_TRY(axpby(c, L, 1.0 / H(i, i - 1), ui, 0.0, ui));
-      for (int j = 1; j <= i - 1; ++j) {
-        const double tmp = cs[j - 1] * H(j - 1, i - 1) + sn[j - 1] * H(j, i - 1);
-        H(j, i - 1) = -sn[j - 1] * H(j - 1, i - 1) + cs[j - 1] * H(j, i - 1);
-        H(j - 1, i - 1) = tmp;
-      }
-      const double tmp = std::sqrt(H(i - 1, i - 1) * H(i - 1, i - 1) + H(i, i - 1) * H(i, i - 1));
-      cs[i - 1] = H(i - 1, i - 1) / tmp;
-      sn[i - 1] = H(i, i - 1) / tmp;
-      H(i - 1, i - 1) = tmp;
-      H(i, i - 1) = 0.0;
-      err[i] = -sn[i - 1] * err[i - 1];
-      err[i - 1] = cs[i - 1] * err[i - 1];
-      if (std::fabs(err[i]) < eps) {
-        ls.suc = 1;
-        break;
-      }
-    }
-    if (i > sD) i = sD;
-    for (int j = 0; j < i; ++j) y[j] = err[j];
-    for (int j = i; j >= 1; --j) {
-      for (int k = j + 1; k <= i; ++k) y[j - 1] = y[j - 1] - H(j - 1, k - 1) * y[k - 1];
-      y[j - 1] = y[j - 1] / H(j - 1, j - 1);
-    }
-    CR_HIP(hipMemcpyAsync(c.hcol.p + 768, y.data(), i * sizeof(double), hipMemcpyHostToDevice, c.s));
-    maxpy_kernel<T><<<crimson::grid_for(L, 256), 256, 0, c.s>>>(L, X, U, L, i, c.hcol.p + 768, 1.0);
-    CR_HIP(hipGetLastError());
-    CR_HIP(hipStreamSynchronize(c.s));  // y is a host buffer read by the copy above
-    ls.fNorm = std::fabs(err[i]);
-    if (ls.suc) break;
-  }
-  ls.callD = now_s() - t0 + ls.callD;
-  ls.dB = 10.0 * std::log(ls.fNorm / ls.dB);
-  return CRIMSON_OK;
-}
-
 // What a CG's operator needs beside its direction: the coupled faces' rank-one
 // terms, and the scaled copy Ps(i) = W(off + wdof i) P(i) kept by the
 // direction update (Ps null: none).
@@ -1457,19 +1472,20 @@ inline CgGrid cg_grid(size_t L) {
 // The iterations' vector work: iteration `it` after its operator left SP and nd
 // parts of P . SP.  P and Pn swap roles every iteration.
 template <class T>
-int cg_sweeps(Ctx<T> &c, size_t L, int it, int nd, const CgAux<T> &ax, T *X, T *R, const T *P, T *Pn, const T *SP) {
+int cg_sweeps(Ctx<T> &c, size_t L, int it, int nd, const CgAux<T> &ax, T *X, T *R, const T *P, T *Pn, const T *SP,
+              HostFlag hf) {
   double *scal = c.cgst.p + (it & 1) * kCgState, *next = c.cgst.p + ((it + 1) & 1) * kCgState;
-  double *dpart = c.partial.p, *rpart = c.partial.p + kCgGrid;
+  double *dpart = c.part.p, *rpart = c.part.p + kCgGrid;
   const CgGrid g = cg_grid(L);
   const int gp = g.blocks + ax.fl.nfc * kFaceDotBlocks;
   if (g.entries == 1) {
     cg_r_kernel<T, 1><<<g.blocks, 256, 0, c.s>>>(L, scal, dpart, nd, ax.fl, R, SP, rpart);
     cg_p_kernel<T, 1><<<gp, 256, 0, c.s>>>(L, scal, next, rpart, g.blocks, ax.fl, X, R, P, Pn, ax.W, ax.wdof, ax.off,
-                                           ax.Ps);
+                                           ax.Ps, hf);
   } else {
     cg_r_kernel<T, 4><<<g.blocks, 256, 0, c.s>>>(L, scal, dpart, nd, ax.fl, R, SP, rpart);
     cg_p_kernel<T, 4><<<gp, 256, 0, c.s>>>(L, scal, next, rpart, g.blocks, ax.fl, X, R, P, Pn, ax.W, ax.wdof, ax.off,
-                                           ax.Ps);
+                                           ax.Ps, hf);
   }
   CR_HIP(hipGetLastError());
   return CRIMSON_OK;
@@ -1487,74 +1503,8 @@ int cg_begin_vec(Ctx<T> &c, size_t L, const CgAux<T> &ax, T *X, T *R, T *P, cons
 template <class T>
 int cg_den(Ctx<T> &c, size_t L, const T *P, const T *SP, const double *done, int &nd) {
   nd = (int)std::min<size_t>((L + 255) / 256, kCgGrid);
-  cg_den_kernel<T><<<nd, 256, 0, c.s>>>(L, P, SP, c.partial.p, done);
+  cg_den_kernel<T><<<nd, 256, 0, c.s>>>(L, P, SP, c.part.p, done);
   CR_HIP(hipGetLastError());
-  return CRIMSON_OK;
-}
-
-// Generic CG driver on device vectors (memLS CGRAD / CGRADV / CGRADS).
-// op(P, SP, done, nd) computes SP and nd parts of P . SP; X holds the right-hand
-// side in and the solution out.
-template <class T, class Op>
-int cg_dev(Ctx<T> &c, size_t L, SubLs &ls, T *X, Op op, T *R, T *P, T *P2, T *SP, bool schur,
-           const CgAux<T> &ax = CgAux<T>()) {
-  const double t0 = now_s();
-  ls.suc = 0;
-  int rc = CRIMSON_OK;
-  const double errO0 = host_norm(c, L, X, &rc);
-  if (rc) return rc;
-  ls.iNorm = errO0;
-  double eps = std::max(ls.absTol, ls.relTol * errO0);
-  eps = eps * eps;
-  double hs[kCgState] = {errO0 * errO0, errO0 * errO0, eps, 0, 0, 0, 0, (double)ls.mItr, 0};
-  // the first iteration's test (check_next)
-  if (hs[6] >= hs[7]) {
-    hs[5] = 1.0;
-  } else if (hs[0] < hs[2]) {
-    hs[5] = hs[8] = 1.0;
-  } else {
-    hs[6] = 1.0;
-  }
-  CR_HIP(hipMemcpyAsync(c.cgst.p, hs, sizeof(hs), hipMemcpyHostToDevice, c.s));
-  CR_TRY(cg_begin_vec(c, L, ax, X, R, P, nullptr));
-  constexpr int batch = 8;  // even: a batch ends on the state's first copy
-  double back[9];
-  CR_TRY(c.readback_slots());
-  T *Pk = P, *Pn = P2;
-  // a batch of iterations, then the flags' copy into read-back slot `slot`
-  auto enqueue_batch = [&](int slot) -> int {
-    for (int b = 0; b < batch; ++b) {
-      int nd = 0;
-      CR_TRY(op(Pk, SP, c.cgst.p + (b & 1) * kCgState + 5, nd));
-      CR_TRY(cg_sweeps(c, L, b, nd, ax, X, R, Pk, Pn, SP));
-      std::swap(Pk, Pn);
-    }
-    CR_HIP(hipMemcpyAsync(c.hback + 16 * slot, c.cgst.p, sizeof(back), hipMemcpyDeviceToHost, c.s));
-    CR_HIP(hipEventRecord(c.evb[slot], c.s));
-    return CRIMSON_OK;
-  };
-  CR_TRY(enqueue_batch(0));
-  for (int k = 0;; ++k) {
-    // the next batch is queued before this one's flags are read, so that the
-    // GPU does not idle while the host waits and launches; once the flag is
-    // raised every kernel that changes the state returns at once, so the
-    // extra batch leaves the state as this one did
-    CR_TRY(enqueue_batch((k + 1) & 1));
-    CR_HIP(hipEventSynchronize(c.evb[k & 1]));
-    std::memcpy(back, c.hback + 16 * (k & 1), sizeof(back));
-    if (back[5] != 0.0) break;
-  }
-  // the flag is raised at the top of the iteration after the last one
-  const double err = back[0], errO = back[1];
-  ls.suc = back[8] != 0.0;
-  ls.fNorm = std::sqrt(err);
-  ls.dB = 5.0 * std::log(err / errO);
-  const int done_itr = (int)back[6];
-  if (schur)
-    ls.itr = ls.itr + done_itr;  // CGRAD accumulates (memLS.f90:428)
-  else
-    ls.itr = done_itr;
-  ls.callD = now_s() - t0 + (schur ? ls.callD : 0.0);
   return CRIMSON_OK;
 }
 
@@ -1672,7 +1622,7 @@ template <class T>
 int schur_apply(Ctx<T> &c, const SchurOp<T> &o, const T *P, T *SP, const double *done, int &nd) {
   crimson_lhs *l = c.lhs;
   const int N = l->nNo;
-  double *dpart = c.partial.p;
+  double *dpart = c.part.p;
   if (o.formed) {
     const int ntile = (int)crimson::grid_for((size_t)N, 256 / kSLanes);
     nd = std::min(ntile, kCgGrid);
@@ -1695,8 +1645,6 @@ int schur_apply(Ctx<T> &c, const SchurOp<T> &o, const T *P, T *SP, const double 
   return cg_den(c, (size_t)N, P, SP, done, nd);
 }
 
-// NSSOLVER (memLS.f90:1460-1759) on device; Ri (4,N) device in/out
-// (preconditioned RHS in, preconditioned solution out).
 // The support of a coupled face's dot functional (FaceDev): the columns of
 // the face nodes' rows, each with its (face node, CSR entry) pairs, from the
 // host copy of the pattern; built once per face (the pattern is fixed).
@@ -1733,41 +1681,36 @@ int face_support(crimson_lhs *l, CrFace &fa) {
   return CRIMSON_OK;
 }
 
-// The coupled faces (c.hfdev, in face order) on the device, and their merged
-// supports (FaceList), which the handle keeps while the same faces are coupled.
+// The merged supports of the coupled faces (FaceList), which the handle keeps
+// while the same faces are coupled.
 template <class T>
 int face_list(Ctx<T> &c) {
   crimson_lhs *l = c.lhs;
-  const size_t nfc = c.hfdev.size();
-  if (nfc == 0) return CRIMSON_OK;
-  CR_TRY(c.fdev.alloc(nfc));
-  CR_HIP(hipMemcpyAsync(c.fdev.p, c.hfdev.data(), nfc * sizeof(FaceDev), hipMemcpyHostToDevice, c.s));
+  if (c.nfc() == 0) return CRIMSON_OK;
   std::vector<unsigned long long> sig;
   for (const auto &fa : l->face)
     if (fa.coupled) sig.push_back(fa.support);
-  if (sig != l->fent_sig || !l->d_ftptr.p) {
-    std::vector<FaceEnt> ent;
-    int f = 0;
-    for (const auto &fa : l->face) {
-      if (!fa.coupled) continue;
-      for (size_t k = 0; k < fa.h_sup.size(); ++k) ent.push_back(FaceEnt{fa.h_sup[k], f, (int)k});
-      ++f;
-    }
-    std::sort(ent.begin(), ent.end(),
-              [](const FaceEnt &a, const FaceEnt &b) { return a.node != b.node ? a.node < b.node : a.f < b.f; });
-    std::vector<int> ptr((size_t)(l->nNo + 255) / 256 + 1);
-    size_t e = 0;
-    for (size_t t = 0; t < ptr.size(); ++t) {
-      while (e < ent.size() && ent[e].node < (long long)t * 256) ++e;
-      ptr[t] = (int)e;
-    }
-    ptr.back() = (int)ent.size();
-    CR_TRY(l->d_fent.upload(ent.data(), ent.size(), c.s));
-    CR_TRY(l->d_ftptr.upload(ptr.data(), ptr.size(), c.s));
-    CR_HIP(hipStreamSynchronize(c.s));
-    l->fent_sig = sig;
+  if (sig == l->fent_sig && l->d_ftptr.p) return CRIMSON_OK;
+  std::vector<FaceEnt> ent;
+  int f = 0;
+  for (const auto &fa : l->face) {
+    if (!fa.coupled) continue;
+    for (size_t k = 0; k < fa.h_sup.size(); ++k) ent.push_back(FaceEnt{fa.h_sup[k], f, (int)k});
+    ++f;
   }
+  std::sort(ent.begin(), ent.end(),
+            [](const FaceEnt &a, const FaceEnt &b) { return a.node != b.node ? a.node < b.node : a.f < b.f; });
+  std::vector<int> ptr((size_t)(l->nNo + 255) / 256 + 1);
+  size_t e = 0;
+  for (size_t t = 0; t < ptr.size(); ++t) {
+    while (e < ent.size() && ent[e].node < (long long)t * 256) ++e;
+    ptr[t] = (int)e;
+  }
+  ptr.back() = (int)ent.size();
+  CR_TRY(l->d_fent.upload(ent.data(), ent.size(), c.s));
+  CR_TRY(l->d_ftptr.upload(ptr.data(), ptr.size(), c.s));
   CR_HIP(hipStreamSynchronize(c.s));
+  l->fent_sig = sig;
   return CRIMSON_OK;
 }
 // The faces' functionals q for this solve's matrix and scaling.
@@ -1781,372 +1724,6 @@ int face_functionals(Ctx<T> &c, const MatView<T> &G) {
   return CRIMSON_OK;
 }
 
-template <class T>
-int nssolver_dev(Ctx<T> &c, crimson_ls *ls, T *Ri) {
-  crimson_lhs *l = c.lhs;
-  const int N = c.N, nsd = 3;
-  const size_t mn = (size_t)nsd * N;
-  int iB = ls->RI.mItr;
-  const int nB = 2 * iB;
-  crimson::DBuf<T> Rm, Rc, Rmi, Rci, U, P, MU, MP, t1, t2, t3, t4;
-  crimson::DBuf<double> dxB;
-  CR_TRY(Rm.alloc(mn));
-  CR_TRY(Rc.alloc(N));
-  CR_TRY(Rmi.alloc(mn));
-  CR_TRY(Rci.alloc(N));
-  CR_TRY(U.alloc(mn * iB));
-  CR_TRY(P.alloc((size_t)N * iB));
-  CR_TRY(MU.alloc(mn * nB));
-  CR_TRY(MP.alloc((size_t)N * nB));
-  CR_TRY(t1.alloc(mn));
-  CR_TRY(t2.alloc(N));
-  CR_TRY(t3.alloc(N));
-  CR_TRY(t4.alloc(N));
-  CR_TRY(dxB.alloc(nB));
-  Workspace<T> ws;
-  CR_TRY(ws.tmp.alloc(std::max(mn, (size_t)4 * N)));  // GMRES scratch; the Schur CG's Z(4, N)
-  const unsigned gN = crimson::grid_for(N, 256);
-  extract_kernel<<<gN, 256, 0, c.s>>>(N, 4, 0, 3, Ri, Rmi.p);
-  extract_kernel<<<gN, 256, 0, c.s>>>(N, 4, 3, 1, Ri, Rci.p);
-  CR_HIP(hipMemcpyAsync(Rm.p, Rmi.p, mn * sizeof(T), hipMemcpyDeviceToDevice, c.s));
-  CR_HIP(hipMemcpyAsync(Rc.p, Rci.p, N * sizeof(T), hipMemcpyDeviceToDevice, c.s));
-  int rc = CRIMSON_OK;
-  const double a1 = host_norm(c, mn, Rm.p, &rc);
-  if (rc) return rc;
-  const double a2 = host_norm(c, N, Rc.p, &rc);
-  if (rc) return rc;
-  double eps = std::sqrt(a1 * a1 + a2 * a2);
-  ls->RI.iNorm = eps;
-  ls->RI.fNorm = eps;
-  ls->CG.callD = 0.0;
-  ls->GM.callD = 0.0;
-  ls->CG.itr = 0;
-  ls->GM.itr = 0;
-  ls->RI.suc = 0;
-  const double t0 = now_s();
-  eps = std::max(ls->RI.absTol, ls->RI.relTol * eps);
-  // DEPART: views on the 4x4 planes (memLS.f90:1612-1679); Gt = -mG^T
-  const T *V = planes(l, T(0));
-  const MatView<T> mK = view<T>(c, V, 4, 0, 0, 3, 3, c.W.p, c.fix.p, 4);
-  const MatView<T> mG = view<T>(c, V, 4, 0, 3, 3, 1, c.W.p, nullptr, 4);
-  const MatView<T> mD = view<T>(c, V, 4, 3, 0, 1, 3, c.W.p, nullptr, 4);
-  const MatView<T> mL = view<T>(c, V, 4, 3, 3, 1, 1, c.W.p, c.fix.p, 4);
-  MatView<T> Gt = mD;
-  if (!l->gt_is_d) {
-    crimson::DBuf<T> &gtb = gt_buf(l, T(0));
-    CR_TRY(gtb.alloc((size_t)3 * l->nnz));
-    gt_kernel<T><<<crimson::grid_for(l->nnz, 256), 256, 0, c.s>>>(l->nnz, V, l->d_tr.p, gtb.p);
-    CR_HIP(hipGetLastError());
-    Gt = view<T>(c, gtb.p, 1, 0, 0, 1, 3, c.W.p, nullptr, 4);
-    Gt.plane[0] = 0;
-    Gt.plane[1] = 1;
-    Gt.plane[2] = 2;
-    Gt.r0 = 3;
-    Gt.c0 = 0;
-  }
-  // BCPRE (memLS.f90:1683-1716): nS = ||valM||^2 over nsd components
-  for (auto &fa : l->face) {
-    if (!fa.coupled) continue;
-    std::vector<double> vm((size_t)fa.dof * fa.nNo);
-    CR_HIP(hipMemcpyAsync(vm.data(), fa.d_valM.p, vm.size() * sizeof(double), hipMemcpyDeviceToHost, c.s));
-    CR_HIP(hipStreamSynchronize(c.s));
-    fa.nS = 0.0;
-    const int nc = std::min(fa.dof, nsd);
-    for (int a = 0; a < fa.nNo; ++a)
-      for (int i = 0; i < nc; ++i) fa.nS = fa.nS + vm[i + (size_t)fa.dof * a] * vm[i + (size_t)fa.dof * a];
-  }
-  // the coupled faces with their PRE coefficients and dot functionals
-  c.hfdev.clear();
-  for (auto &fa : l->face) {
-    if (!fa.coupled) continue;
-    CR_TRY(face_support(l, fa));
-    c.hfdev.push_back(FaceDev{fa.d_glob.p, fa.d_valM.p, -fa.res / (1.0 + fa.res * fa.nS), nullptr, fa.res, fa.nNo, fa.dof,
-                              fa.d_sup.p, fa.d_q.p, fa.nsup});
-  }
-  CR_TRY(face_list(c));
-  CR_TRY(face_functionals(c, mG));
-  SchurOp<T> so;
-  so.L = mL;
-  so.Gt = Gt;
-  so.G = mG;
-  so.Z = ws.tmp.p;
-  CR_TRY(schur_ready(l, so));
-  CR_TRY(schur_form(c, so));
-  CgAux<T> ax;
-  ax.fl = c.face_list();
-  if (!so.formed) {
-    ax.W = c.W.p;
-    ax.wdof = 4;
-    ax.off = mG.c0;
-    ax.Ps = so.Ps = t2.p;
-  }
-  // Schur operator of CGRAD: SP = L P - Gt (G P + PRE)
-  auto schur_op = [&](const T *Pv, T *SPv, const double *done, int &nd) -> int {
-    return schur_apply(c, so, Pv, SPv, done, nd);
-  };
-  std::vector<double> A((size_t)nB * nB, 0.0), Bv(nB, 0.0), xB(nB, 0.0);
-  std::vector<double> dots(2 * nB + 4);
-  int i, iBB = 0;
-  for (i = 1; i <= ls->RI.mItr; ++i) {
-    iB = 2 * i - 1;
-    iBB = 2 * i;
-    ls->RI.dB = ls->RI.fNorm;
-    T *Ui = U.p + mn * (i - 1), *Pi = P.p + (size_t)N * (i - 1);
-    T *MUb = MU.p + mn * (iB - 1), *MUbb = MU.p + mn * (iBB - 1);
-    T *MPb = MP.p + (size_t)N * (iB - 1), *MPbb = MP.p + (size_t)N * (iBB - 1);
-    CR_TRY(gmres_dev(c, mK, 3, ls->GM, Rm.p, Ui, ws, true));
-    CR_TRY(spmv(c, mD, 1, 3, Ui, Pi, -1.0, Rc.p, 1.0));  // P = Rc - D U
-    CR_TRY(cg_dev(c, (size_t)N, ls->CG, Pi, schur_op, t3.p, t4.p, t1.p, MPb, true, ax));
-    CR_TRY(spmv(c, mG, 3, 1, Pi, MUb));
-    CR_TRY(axpby(c, mn, 1.0, Rm.p, 0.0, MUbb));
-    CR_TRY(axpby(c, mn, -1.0, MUb, 1.0, MUbb));  // MU(iBB) = Rm - MU(iB)
-    CR_TRY(gmres_dev(c, mK, 3, ls->GM, MUbb, Ui, ws, true));
-    CR_TRY(spmv(c, mK, 3, 3, Ui, MUbb));
-    CR_TRY(addbcmul(c, false, 3, Ui, MUbb));
-    CR_TRY(spmv(c, mL, 1, 1, Pi, MPb));
-    CR_TRY(spmv(c, mD, 1, 3, Ui, MPbb));
-    // Gram matrix rows iB, iBB: dots with all previous columns and the RHS
-    for (int k = iB; k <= iBB; ++k) {
-      const T *MUk = MU.p + mn * (k - 1), *MPk = MP.p + (size_t)N * (k - 1);
-      // MU_j . MU_k for j < k, then MU_k.MU_k ; plus MU_k . Rmi
-      CR_TRY(mdot<T>(c, mn, MUk, MU.p, mn, k - 1, true, c.hcol.p, nullptr, true));
-      CR_TRY(mdot<T>(c, mn, MUk, Rmi.p, 0, 1, false, c.hcol.p + 256, nullptr, true));
-      CR_TRY(mdot<T>(c, N, MPk, MP.p, N, k - 1, true, c.hcol.p + 512, nullptr, true));
-      CR_TRY(mdot<T>(c, N, MPk, Rci.p, 0, 1, false, c.hcol.p + 768, nullptr, true));
-      std::vector<double> h1(k + 1), h2(k + 1), r1(1), r2(1);
-      CR_HIP(hipMemcpyAsync(h1.data(), c.hcol.p, (k) * sizeof(double), hipMemcpyDeviceToHost, c.s));
-      CR_HIP(hipMemcpyAsync(r1.data(), c.hcol.p + 256, sizeof(double), hipMemcpyDeviceToHost, c.s));
-      CR_HIP(hipMemcpyAsync(h2.data(), c.hcol.p + 512, (k) * sizeof(double), hipMemcpyDeviceToHost, c.s));
-      CR_HIP(hipMemcpyAsync(r2.data(), c.hcol.p + 768, sizeof(double), hipMemcpyDeviceToHost, c.s));
-      CR_HIP(hipStreamSynchronize(c.s));
-      for (int j = 1; j <= k - 1; ++j) {
-        A[(j - 1) + (size_t)nB * (k - 1)] = h1[j - 1] + h2[j - 1];
-        A[(k - 1) + (size_t)nB * (j - 1)] = A[(j - 1) + (size_t)nB * (k - 1)];
-      }
-      const double n1 = std::sqrt(h1[k - 1]), n2 = std::sqrt(h2[k - 1]);
-      A[(k - 1) + (size_t)nB * (k - 1)] = n1 * n1 + n2 * n2;
-      Bv[k - 1] = r1[0] + r2[0];
-    }
-    for (int k = 0; k < iBB; ++k) xB[k] = Bv[k];
-    // GE (memLS.f90:607-677)
-    {
-      const int Nn = iBB;
-      if (Nn == 2) {
-        const double a11 = A[0], a21 = A[1], a12 = A[(size_t)nB], a22 = A[(size_t)nB + 1];
-        const double pivot = a11 * a22 - a21 * a12;
-        const double saveEl = (xB[0] * a22 - xB[1] * a12) / pivot;
-        xB[1] = (xB[1] * a11 - xB[0] * a21) / pivot;
-        xB[0] = saveEl;
-      } else {
-        std::vector<double> Cm((size_t)Nn * (Nn + 1));
-        auto CC = [&](int r, int cc) -> double & { return Cm[r + (size_t)Nn * cc]; };
-        for (int cc = 0; cc < Nn; ++cc)
-          for (int r = 0; r < Nn; ++r) CC(r, cc) = A[r + (size_t)nB * cc];
-        for (int r = 0; r < Nn; ++r) CC(r, Nn) = xB[r];
-        for (int m = 0; m < Nn - 1; ++m) {
-          int ipv = m;
-          double pivot = std::fabs(CC(m, m));
-          for (int r = m + 1; r < Nn; ++r)
-            if (std::fabs(CC(r, m)) > pivot) {
-              ipv = r;
-              pivot = std::fabs(CC(r, m));
-            }
-          if (pivot < 2.0 * 2.220446049250313e-16) {
-            crimson::set_error("memLS GE: singular matrix");
-            return CRIMSON_ESINGULAR;
-          }
-          if (ipv != m)
-            for (int cc = m; cc <= Nn; ++cc) std::swap(CC(m, cc), CC(ipv, cc));
-          for (int r = m + 1; r < Nn; ++r) {
-            const double sv = CC(r, m) / CC(m, m);
-            CC(r, m) = 0.0;
-            for (int cc = m + 1; cc <= Nn; ++cc) CC(r, cc) = CC(r, cc) - sv * CC(m, cc);
-          }
-        }
-        for (int j = Nn - 1; j >= 0; --j) {
-          for (int r = j + 1; r < Nn; ++r) CC(j, Nn) = CC(j, Nn) - CC(j, r) * CC(r, Nn);
-          CC(j, Nn) = CC(j, Nn) / CC(j, j);
-        }
-        for (int r = 0; r < Nn; ++r) xB[r] = CC(r, Nn);
-      }
-    }
-    double sxb = 0.0;
-    for (int k = 0; k < iBB; ++k) sxb = sxb + xB[k] * Bv[k];
-    ls->RI.fNorm = std::sqrt(ls->RI.iNorm * ls->RI.iNorm - sxb);
-    if (ls->RI.fNorm < eps) {
-      ls->RI.suc = 1;
-      break;
-    }
-    CR_HIP(hipMemcpyAsync(dxB.p, xB.data(), iBB * sizeof(double), hipMemcpyHostToDevice, c.s));
-    CR_TRY(axpby(c, mn, 1.0, Rmi.p, 0.0, Rm.p));
-    CR_TRY(axpby(c, N, 1.0, Rci.p, 0.0, Rc.p));
-    maxpy_kernel<<<crimson::grid_for(mn, 256), 256, 0, c.s>>>(mn, Rm.p, MU.p, mn, iBB, dxB.p, -1.0);
-    maxpy_kernel<<<crimson::grid_for(N, 256), 256, 0, c.s>>>(N, Rc.p, MP.p, N, iBB, dxB.p, -1.0);
-    CR_HIP(hipGetLastError());
-    CR_HIP(hipStreamSynchronize(c.s));
-  }
-  if (i > ls->RI.mItr) {
-    ls->RI.itr = ls->RI.mItr;
-  } else {
-    ls->RI.itr = i;
-    CR_HIP(hipMemcpyAsync(dxB.p, xB.data(), iBB * sizeof(double), hipMemcpyHostToDevice, c.s));
-    CR_TRY(axpby(c, N, 1.0, Rci.p, 0.0, Rc.p));
-    maxpy_kernel<<<crimson::grid_for(N, 256), 256, 0, c.s>>>(N, Rc.p, MP.p, N, iBB, dxB.p, -1.0);
-    CR_HIP(hipGetLastError());
-  }
-  {
-    const double rcn = host_norm(c, N, Rc.p, &rc) / ls->RI.fNorm;
-    if (rc) return rc;
-    ls->Resc = (int)std::lround(100.0 * rcn * rcn);
-    ls->Resm = 100 - ls->Resc;
-  }
-  // solution: Rmi = sum xB(2i) U_i, Rci = sum xB(2i-1) P_i
-  {
-    const int nit = ls->RI.itr;
-    std::vector<double> cu(nit), cp(nit);
-    for (int k = 1; k <= nit; ++k) {
-      cu[k - 1] = xB[2 * k - 1];
-      cp[k - 1] = xB[2 * k - 2];
-    }
-    CR_HIP(hipMemcpyAsync(c.hcol.p, cu.data(), nit * sizeof(double), hipMemcpyHostToDevice, c.s));
-    CR_HIP(hipMemcpyAsync(c.hcol.p + 256, cp.data(), nit * sizeof(double), hipMemcpyHostToDevice, c.s));
-    CR_HIP(hipMemsetAsync(Rmi.p, 0, mn * sizeof(T), c.s));
-    CR_HIP(hipMemsetAsync(Rci.p, 0, N * sizeof(T), c.s));
-    maxpy_kernel<<<crimson::grid_for(mn, 256), 256, 0, c.s>>>(mn, Rmi.p, U.p, mn, nit, c.hcol.p, 1.0);
-    maxpy_kernel<<<crimson::grid_for(N, 256), 256, 0, c.s>>>(N, Rci.p, P.p, N, nit, c.hcol.p + 256, 1.0);
-    insert_kernel<<<gN, 256, 0, c.s>>>(N, 4, 0, 3, Rmi.p, Ri);
-    insert_kernel<<<gN, 256, 0, c.s>>>(N, 4, 3, 1, Rci.p, Ri);
-    CR_HIP(hipGetLastError());
-    CR_HIP(hipStreamSynchronize(c.s));
-  }
-  ls->RI.callD = now_s() - t0;
-  ls->RI.dB = 10.0 * std::log(ls->RI.fNorm / ls->RI.dB);
-  return CRIMSON_OK;
-}
-
-// One memLS_SOLVE in arithmetic type T.  d_Ri is the FP64 (dof,N) right-hand
-// side in and solution out; for T = float the solve runs on an FP32 copy.
-template <class T>
-int solve_impl(crimson_lhs *l, crimson_ls *ls, int dof, double *d_Ri, const int *incL, const double *res) {
-  Ctx<T> c;
-  CR_TRY(c.init(l, dof));
-  // face flags (memLS.f90:1965-1986)
-  for (int f = 0; f < l->nFaces; ++f) {
-    CrFace &fa = l->face[f];
-    fa.inc = true;
-    if (incL && incL[f] == 0) fa.inc = false;
-    fa.coupled = false;
-    if (!fa.inc || !fa.created) continue;
-    if (fa.bGrp == CRIMSON_BC_NEU && res && res[f] != 0.0) {
-      fa.res = res[f];
-      fa.coupled = true;
-      c.coupled = true;
-    }
-  }
-  const int N = l->nNo;
-  const size_t L = (size_t)dof * N;
-  const unsigned gN = crimson::grid_for(N, 256);
-  const T *V = planes(l, T(0));
-  // PRECOND (memLS.f90:1763-1943) as the W/fix vectors
-  precond_diag_kernel<T><<<gN, 256, 0, c.s>>>(N, dof, l->vdof, V, l->nnz, l->d_diag.p, c.W.p, c.fix.p);
-  for (auto &fa : l->face)
-    if (fa.created && fa.inc && fa.bGrp == CRIMSON_BC_DIR && fa.nNo > 0)
-      precond_face_kernel<T><<<crimson::grid_for(fa.nNo, 256), 256, 0, c.s>>>(fa.nNo, dof, fa.dof, fa.d_glob.p,
-                                                                              fa.d_val.p, c.W.p);
-  precond_fix_kernel<T><<<gN, 256, 0, c.s>>>(N, dof, l->vdof, V, l->nnz, l->d_diag.p, c.W.p, c.fix.p);
-  for (auto &fa : l->face)
-    if (fa.coupled && fa.nNo > 0) {
-      CR_TRY(fa.d_valM.alloc((size_t)fa.dof * fa.nNo));
-      face_valm_kernel<T><<<crimson::grid_for(fa.nNo, 256), 256, 0, c.s>>>(fa.nNo, dof, fa.dof, fa.d_glob.p,
-                                                                            fa.d_val.p, c.W.p, fa.d_valM.p);
-    }
-  // R = W R (into the working vector of type T)
-  crimson::DBuf<T> Rw;
-  T *R = nullptr;
-  if (sizeof(T) == sizeof(double)) {
-    R = reinterpret_cast<T *>(d_Ri);
-  } else {
-    CR_TRY(Rw.alloc(L));
-    R = Rw.p;
-  }
-  mul_kernel<double, T, T><<<crimson::grid_for(L, 256), 256, 0, c.s>>>(L, d_Ri, c.W.p, R);
-  CR_HIP(hipGetLastError());
-  int rc = CRIMSON_OK;
-  if (ls->LS_type == CRIMSON_LS_NS) {
-    rc = nssolver_dev<T>(c, ls, R);
-  } else if (ls->LS_type == CRIMSON_LS_GMRES) {
-    // GMRESV (memLS.f90:792-883): no PRE application, restart from X
-    Workspace<T> ws;
-    CR_TRY(ws.tmp.alloc(L));
-    crimson::DBuf<T> X;
-    CR_TRY(X.alloc(L));
-    const MatView<T> A = view<T>(c, V, dof, 0, 0, dof, dof, c.W.p, c.fix.p, dof);
-    ls->RI.itr = 0;
-    const double nr = host_norm(c, L, R, &rc);
-    if (rc) return rc;
-    if (nr <= ls->RI.absTol) {
-      ls->RI.iNorm = nr;
-      ls->RI.fNorm = nr;
-      ls->RI.suc = 0;
-      ls->RI.callD = 0.0;
-      ls->RI.dB = 0.0;
-      CR_HIP(hipMemsetAsync(R, 0, L * sizeof(T), c.s));
-    } else {
-      // GMRESV counts the residual product of every cycle (memLS.f90:827-829)
-      rc = gmres_dev<T>(c, A, dof, ls->RI, R, X.p, ws, false, true);
-      if (rc) return rc;
-      CR_HIP(hipMemcpyAsync(R, X.p, L * sizeof(T), hipMemcpyDeviceToDevice, c.s));
-    }
-  } else if (ls->LS_type == CRIMSON_LS_CG) {
-    const MatView<T> A = view<T>(c, V, dof, 0, 0, dof, dof, c.W.p, c.fix.p, dof);
-    crimson::DBuf<T> X, P, P2, SP;
-    CR_TRY(X.alloc(L));
-    CR_TRY(P.alloc(L));
-    CR_TRY(P2.alloc(L));
-    CR_TRY(SP.alloc(L));
-    auto op = [&](const T *Pv, T *SPv, const double *done, int &nd) -> int {
-      CR_TRY(spmv<T>(c, A, dof, dof, Pv, SPv, 1.0, static_cast<const T *>(nullptr), 0.0, done));
-      return cg_den(c, L, Pv, SPv, done, nd);
-    };
-    rc = cg_dev<T>(c, L, ls->RI, R, op, X.p, P.p, P2.p, SP.p, false);
-  } else {
-    crimson::set_error("LS_type %d not defined", ls->LS_type);
-    return CRIMSON_EARG;
-  }
-  if (rc) return rc;
-  mul_kernel<T, T, double><<<crimson::grid_for(L, 256), 256, 0, c.s>>>(L, R, c.W.p, d_Ri);  // R = R W
-  CR_HIP(hipGetLastError());
-  CR_HIP(hipStreamSynchronize(c.s));
-  return CRIMSON_OK;
-}
-
-int solve_dev(crimson_lhs *l, crimson_ls *ls, int dof, double *d_Ri, const int *incL, const double *res) {
-  if (l->vdof != dof || !(l->prec == 32 ? (const void *)l->d_V32.p : (const void *)l->d_V.p)) {
-    crimson::set_error("lhs holds no matrix of block size %d (stored: %d)", dof, l->vdof);
-    return CRIMSON_ESTATE;
-  }
-  if (ls->LS_type == CRIMSON_LS_NS && dof != 4) {
-    crimson::set_error("LS_TYPE_NS needs dof = 4 (got %d)", dof);
-    return CRIMSON_EUNSUPPORTED;
-  }
-  if (l->prec == 32) return solve_impl<float>(l, ls, dof, d_Ri, incL, res);
-  return solve_impl<double>(l, ls, dof, d_Ri, incL, res);
-}
-
-
-// ---------------------------------------------------------------------------
-// Device-driven NSSOLVER: the same kernels and the same arithmetic as
-// nssolver_dev, with every host decision of the solve (GMRES's Givens
-// rotations, back substitution and convergence test, CGRAD's iteration
-// count, NSSOLVER's least-squares Gram system, its pivoted GE and stopping
-// test, BCPRE's nS and the PRE coefficients) moved into one-thread kernels,
-// so that the whole solve is one fixed launch sequence that a HIP graph can
-// hold.  Every possible iteration is enqueued (GMRES: mItr cycles of sD
-// Arnoldi steps; CGRAD: mItr iterations; NSSOLVER: mItr outer iterations);
-// the launches past convergence see their flag and return at once.  The
-// scalar kernels keep the host's operation order with FMA contraction off,
-// so the solve gives the host-driven solve's bits.
-//
 // gst (double, device): the state of the solve and of its last GMRES and
 // CG calls, then the GMRES Hessenberg system, the Gram system and the
 // solution coefficients.
@@ -2181,60 +1758,26 @@ enum GstIdx : int {
   G_CG_ERRO,
   G_RC_N2 = 30,
   G_NS_CNT,
+  G_GM_E0,  // the first residual norm of the GMRES call
   G_ARR = 64
 };
 
-template <class T>
-__global__ void gfill_kernel(size_t L, T *__restrict__ x, const double *__restrict__ skip) {
-  if (skip && *skip != 0.0) return;
-  const size_t e = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (e < L) x[e] = T(0);
-}
-// dst = src when *skip is 0 (skip may be null) and *runif is not 0 (runif may be null)
-template <class T>
-__global__ void gcopy_kernel(size_t L, const T *__restrict__ src, T *__restrict__ dst,
-                             const double *__restrict__ skip, const double *__restrict__ runif) {
-  if ((skip && *skip != 0.0) || (runif && *runif == 0.0)) return;
-  const size_t e = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (e < L) dst[e] = src[e];
-}
-// x = (T)(*s) x, as axpby(s, x, 0, x)
-template <class T>
-__global__ void gscale_kernel(size_t L, T *__restrict__ x, const double *__restrict__ s,
-                              const double *__restrict__ skip) {
-  if (skip && *skip != 0.0) return;
-  const size_t e = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (e < L) x[e] = (T)(*s) * x[e];
-}
-template <class T>
-__global__ void gaxpby_kernel(size_t L, T a, const T *__restrict__ x, T b, T *__restrict__ y,
-                              const double *__restrict__ skip) {
-  if (skip && *skip != 0.0) return;
-  const size_t e = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (e >= L) return;
-  y[e] = a * x[e] + (b == T(0) ? T(0) : b * y[e]);
-}
-// maxpy_kernel with the count m_host, or *m_dev when given
-template <class T>
-__global__ void gmaxpy_kernel(size_t L, T *__restrict__ y, const T *__restrict__ U0, size_t ustride, int m_host,
-                              const double *__restrict__ m_dev, const double *__restrict__ coef, double sign,
-                              const double *__restrict__ skip, const double *__restrict__ runif) {
-  if ((skip && *skip != 0.0) || (runif && *runif == 0.0)) return;
-  const size_t e = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (e >= L) return;
-  const int m = m_dev ? (int)*m_dev : m_host;
-  T w = y[e];
-  for (int j = 0; j < m; ++j) w += (T)(sign * coef[j]) * U0[ustride * j + e];
-  y[e] = w;
-}
-
 __device__ inline double dmax(double a, double b) { return a < b ? b : a; }  // std::max's choice
 
-__global__ void ns_begin_kernel(double *__restrict__ g, const double *__restrict__ n2a,
-                                const double *__restrict__ n2b, double absTol, double relTol) {
+// The deciding kernels: one workgroup of kDotThreads, which sums the dots'
+// parts; thread 0 decides, in the order of operations of the host form of
+// memLS (FMA contraction off).
+__device__ inline double sum_dots(const double *__restrict__ part, int n, double *sh) {
+  double v = 0.0;
+  for (int k = threadIdx.x; k < n; k += kDotThreads) v += part[k];
+  return block_sum_1024(v, sh);
+}
+__global__ void __launch_bounds__(kDotThreads) ns_begin_kernel(double *__restrict__ g, const double *__restrict__ part,
+                                                               int nb, double absTol, double relTol) {
 #pragma clang fp contract(off)
-  const double a1 = sqrt(*n2a), a2 = sqrt(*n2b);
-  const double eps = sqrt(a1 * a1 + a2 * a2);
+  __shared__ double sh[16];
+  const double eps = sqrt(sum_dots(part, nb, sh));
+  if (threadIdx.x != 0) return;
   g[G_RI_INORM] = eps;
   g[G_RI_FNORM] = eps;
   g[G_RI_EPS] = dmax(absTol, relTol * eps);
@@ -2246,42 +1789,33 @@ __global__ void ns_begin_kernel(double *__restrict__ g, const double *__restrict
   g[G_CG_ITR] = 0.0;
   g[G_GM_LASTF] = g[G_GM_LASTD] = 0.0;
 }
-// BCPRE's nS of a coupled face (memLS.f90:1683-1716, summed in the host's
-// order) and its PRE coefficient -res / (1 + res nS)
-__global__ void face_pre_coef_kernel(int nNo, int fdof, int nsd, const double *__restrict__ valM, double res,
-                                     double *__restrict__ coef) {
-#pragma clang fp contract(off)
-  double nS = 0.0;
-  const int nc = fdof < nsd ? fdof : nsd;
-  for (int a = 0; a < nNo; ++a)
-    for (int i = 0; i < nc; ++i) nS = nS + valM[i + (size_t)fdof * a] * valM[i + (size_t)fdof * a];
-  *coef = -res / (1.0 + res * nS);
-}
-__global__ void gm_begin_kernel(double *__restrict__ g) {
-  if (g[G_RI_SKIP] != 0.0) {
+// skip (may be null): the outer loop is over, the call does nothing
+__global__ void gm_begin_kernel(double *__restrict__ g, const double *__restrict__ skip) {
+  g[G_GM_RAN] = 0.0;
+  g[G_GM_ARN] = 1.0;
+  if (skip && *skip != 0.0) {
     g[G_GM_CYC] = 1.0;
-    g[G_GM_ARN] = 1.0;
-    g[G_GM_RAN] = 0.0;
     return;
   }
   g[G_GM_CYC] = 0.0;
-  g[G_GM_ARN] = 1.0;
   g[G_GM_SUC] = 0.0;
-  g[G_GM_RAN] = 0.0;
   g[G_GM_EARLY] = 0.0;
 }
-__global__ void gm_count_kernel(double *__restrict__ g) {
-  if (g[G_GM_CYC] != 0.0) return;
-  g[G_GM_ITR] = g[G_GM_ITR] + 1.0;
-}
-__global__ void gm_cycle_kernel(double *__restrict__ g, int l, double absTol, double relTol,
-                                const double *__restrict__ n2, double *__restrict__ err) {
+// the norm of a cycle's first vector (parts npart[0, nb)), the first cycle's
+// targets; count: this cycle's residual took a product
+__global__ void __launch_bounds__(kDotThreads) gm_cycle_kernel(double *__restrict__ g, int l, int count,
+                                                               double absTol, double relTol,
+                                                               const double *__restrict__ npart, int nb,
+                                                               double *__restrict__ err) {
 #pragma clang fp contract(off)
   if (g[G_GM_CYC] != 0.0) return;
-  const double e0 = sqrt(*n2);
+  __shared__ double sh[16];
+  const double e0 = sqrt(sum_dots(npart, nb, sh));
+  if (threadIdx.x != 0) return;
   err[0] = e0;
   if (l == 1) {
     const double eps = e0;
+    g[G_GM_E0] = e0;
     if (eps <= absTol) {
       g[G_GM_EARLY] = 1.0;
       g[G_GM_CYC] = 1.0;
@@ -2292,80 +1826,120 @@ __global__ void gm_cycle_kernel(double *__restrict__ g, int l, double absTol, do
     g[G_GM_FNORM] = eps;
     g[G_GM_EPS] = dmax(absTol, relTol * eps);
   }
+  if (count) g[G_GM_ITR] = g[G_GM_ITR] + 1.0;
   g[G_GM_DBPRE] = g[G_GM_FNORM];
   g[G_GM_SCALE] = 1.0 / e0;
   g[G_GM_ARN] = 0.0;
   g[G_GM_RAN] = 1.0;
   g[G_GM_I] = 0.0;
 }
-// Arnoldi step i's Hessenberg column, rotations and test (gmres_dev's host
-// part); H (sD+1, sD) column-major
-__global__ void gm_givens_kernel(double *__restrict__ g, int i, int sD, const double *__restrict__ h1,
-                                 const double *__restrict__ h2, const double *__restrict__ nrm,
-                                 const int *__restrict__ gate, double *__restrict__ H, double *__restrict__ cs,
-                                 double *__restrict__ sn, double *__restrict__ err) {
+// Arnoldi step i's Hessenberg column, rotations and test; H (sD+1, sD)
+// column-major.  The column and the rotations pass through LDS, where the
+// chain of rotations takes an LDS read a step instead of a memory round trip.
+__global__ void __launch_bounds__(kDotThreads) gm_givens_kernel(double *__restrict__ g, int i, int sD,
+                                                                const double *__restrict__ h1,
+                                                                const double *__restrict__ h2,
+                                                                const double *__restrict__ n1,
+                                                                const double *__restrict__ n2, int nb,
+                                                                double *__restrict__ H, double *__restrict__ cs,
+                                                                double *__restrict__ sn, double *__restrict__ err,
+                                                                HostFlag hf) {
 #pragma clang fp contract(off)
-  if (g[G_GM_ARN] != 0.0) return;
-  g[G_GM_ITR] = g[G_GM_ITR] + 1.0;
-  const int ld = sD + 1;
-  const bool gt = *gate != 0;
-  for (int j = 1; j <= i; ++j) H[(j - 1) + (size_t)ld * (i - 1)] = h1[j - 1] + (gt ? h2[j - 1] : 0.0);
-  H[i + (size_t)ld * (i - 1)] = sqrt(gt ? nrm[2] : nrm[1]);
-  g[G_GM_SCALE] = 1.0 / H[i + (size_t)ld * (i - 1)];
-  for (int j = 1; j <= i - 1; ++j) {
-    const double a = H[(j - 1) + (size_t)ld * (i - 1)], b = H[j + (size_t)ld * (i - 1)];
-    const double tmp = cs[j - 1] * a + sn[j - 1] * b;
-    H[j + (size_t)ld * (i - 1)] = -sn[j - 1] * a + cs[j - 1] * b;
-    H[(j - 1) + (size_t)ld * (i - 1)] = tmp;
+  if (g[G_GM_ARN] != 0.0) {
+    if (threadIdx.x == 0) hf.tell(true);
+    return;
   }
-  const double a = H[(i - 1) + (size_t)ld * (i - 1)], b = H[i + (size_t)ld * (i - 1)];
-  const double tmp = sqrt(a * a + b * b);
-  cs[i - 1] = a / tmp;
-  sn[i - 1] = b / tmp;
-  H[(i - 1) + (size_t)ld * (i - 1)] = tmp;
-  H[i + (size_t)ld * (i - 1)] = 0.0;
-  err[i] = -sn[i - 1] * err[i - 1];
-  err[i - 1] = cs[i - 1] * err[i - 1];
-  g[G_GM_I] = (double)i;
-  if (fabs(err[i]) < g[G_GM_EPS]) {
-    g[G_GM_SUC] = 1.0;
-    g[G_GM_ARN] = 1.0;
+  __shared__ double sh[16], hc[256], c[256], s[256];
+  const int t = threadIdx.x, ld = sD + 1;
+  const double a1 = t < nb ? n1[t] : 0.0, a2 = t < nb ? n2[t] : 0.0;
+  const double s1 = block_sum_1024(a1, sh);
+  const bool gt = s1 < 0.5 * h1[i];  // dgks_pass's decision
+  const double s2 = block_sum_1024(a2, sh);
+  if (t < i) {
+    hc[t] = h1[t] + (gt ? h2[t] : 0.0);
+    if (t < i - 1) {
+      c[t] = cs[t];
+      s[t] = sn[t];
+    }
   }
+  __syncthreads();
+  if (t == 0) {
+    const double hl = sqrt(gt ? s2 : s1);
+    g[G_GM_ITR] = g[G_GM_ITR] + 1.0;
+    g[G_GM_SCALE] = 1.0 / hl;
+    double a = hc[0];
+    for (int j = 1; j <= i - 1; ++j) {
+      const double b = hc[j];
+      hc[j - 1] = c[j - 1] * a + s[j - 1] * b;
+      a = -s[j - 1] * a + c[j - 1] * b;
+    }
+    const double tmp = sqrt(a * a + hl * hl);
+    const double ci = a / tmp, si = hl / tmp;
+    cs[i - 1] = ci;
+    sn[i - 1] = si;
+    hc[i - 1] = tmp;
+    const double e = err[i - 1];
+    err[i] = -si * e;
+    err[i - 1] = ci * e;
+    g[G_GM_I] = (double)i;
+    const bool done = fabs(-si * e) < g[G_GM_EPS];
+    if (done) {
+      g[G_GM_SUC] = 1.0;
+      g[G_GM_ARN] = 1.0;
+    }
+    hf.tell(done);
+  }
+  __syncthreads();
+  if (t < i) H[t + (size_t)ld * (i - 1)] = hc[t];
 }
-// the cycle's back substitution (gmres_dev's host part)
-__global__ void gm_solve_kernel(double *__restrict__ g, int sD, const double *__restrict__ H,
-                                const double *__restrict__ err, double *__restrict__ y) {
+// the cycle's back substitution, one thread per unknown, a column at a time
+// (its read is in flight during the column before)
+__global__ void __launch_bounds__(256) gm_solve_kernel(double *__restrict__ g, int sD, const double *__restrict__ H,
+                                                       const double *__restrict__ err, double *__restrict__ y) {
 #pragma clang fp contract(off)
   if (g[G_GM_CYC] != 0.0) return;
-  const int ld = sD + 1;
+  __shared__ double yj[2];
+  const int ld = sD + 1, t = threadIdx.x;
   const int i = (int)g[G_GM_I];
-  for (int j = 0; j < i; ++j) y[j] = err[j];
-  for (int j = i; j >= 1; --j) {
-    for (int k = j + 1; k <= i; ++k) y[j - 1] = y[j - 1] - H[(j - 1) + (size_t)ld * (k - 1)] * y[k - 1];
-    y[j - 1] = y[j - 1] / H[(j - 1) + (size_t)ld * (j - 1)];
+  double v = t < i ? err[t] : 0.0;
+  double h = i > 0 && t < i ? H[t + (size_t)ld * (i - 1)] : 0.0;
+  for (int j = i - 1; j >= 0; --j) {
+    const double hn = j > 0 && t < j ? H[t + (size_t)ld * (j - 1)] : 0.0;
+    if (t == j) {
+      v = v / h;
+      yj[j & 1] = v;
+    }
+    __syncthreads();
+    if (t < j) v = v - h * yj[j & 1];
+    h = hn;
   }
-  g[G_GM_APPLY] = (double)i;
-  g[G_GM_FNORM] = fabs(err[i]);
+  if (t < i) y[t] = v;
+  if (t == 0) {
+    g[G_GM_APPLY] = (double)i;
+    g[G_GM_FNORM] = fabs(err[i]);
+  }
 }
 __global__ void gm_endcycle_kernel(double *__restrict__ g) {
   if (g[G_GM_CYC] != 0.0) return;
   if (g[G_GM_SUC] != 0.0) g[G_GM_CYC] = 1.0;
   g[G_GM_ARN] = 1.0;
-}
-__global__ void gm_finish_kernel(double *__restrict__ g) {
-  if (g[G_RI_SKIP] != 0.0 || g[G_GM_RAN] == 0.0) return;
   g[G_GM_LASTF] = g[G_GM_FNORM];
   g[G_GM_LASTD] = g[G_GM_DBPRE];
 }
-__global__ void cg_begin_kernel(double *__restrict__ scal, double *__restrict__ g, const double *__restrict__ n2,
-                                double absTol, double relTol, int mItr) {
+// skip and g may be null (a plain CG solve)
+__global__ void __launch_bounds__(kDotThreads) cg_begin_kernel(double *__restrict__ scal, double *__restrict__ g,
+                                                               const double *__restrict__ skip,
+                                                               const double *__restrict__ part, int nb, double absTol,
+                                                               double relTol, int mItr) {
 #pragma clang fp contract(off)
-  if (g[G_RI_SKIP] != 0.0) {
-    scal[5] = 1.0;
+  if (skip && *skip != 0.0) {
+    if (threadIdx.x == 0) scal[5] = 1.0;
     return;
   }
-  const double e = sqrt(*n2);
-  g[G_CG_INORM] = e;
+  __shared__ double sh[16];
+  const double e = sqrt(sum_dots(part, nb, sh));
+  if (threadIdx.x != 0) return;
+  if (g) g[G_CG_INORM] = e;
   double eps = dmax(absTol, relTol * e);
   eps = eps * eps;
   scal[0] = e * e;
@@ -2374,91 +1948,145 @@ __global__ void cg_begin_kernel(double *__restrict__ scal, double *__restrict__ 
   scal[3] = scal[4] = scal[5] = scal[6] = 0.0;
   scal[7] = (double)mItr;
   scal[8] = 0.0;
+  scal[9] = e;
   check_next(scal);  // the first iteration's test
 }
-__global__ void cg_end_kernel(const double *__restrict__ scal, double *__restrict__ g) {
-  if (g[G_RI_SKIP] != 0.0) return;
+__global__ void cg_end_kernel(const double *__restrict__ scal, double *__restrict__ g,
+                              const double *__restrict__ skip) {
+  if (*skip != 0.0) return;
   g[G_CG_ITR] = g[G_CG_ITR] + (double)(int)scal[6];
   g[G_CG_SUC] = scal[8];
   g[G_CG_ERR] = scal[0];
   g[G_CG_ERRO] = scal[1];
 }
+// NSSOLVER iteration i's dots in one launch, grid z: MX(iB) against MX(1..iB),
+// MX(iBB) against MX(1..iBB), and the right-hand side against the two
+// (L = 4 N: velocity and pressure parts together).
+template <class T>
+__global__ void __launch_bounds__(kDotThreads) ns_dots_kernel(size_t L, const T *__restrict__ MX,
+                                                              const T *__restrict__ r0, int iB,
+                                                              double *__restrict__ part, size_t pz,
+                                                              const double *__restrict__ skip) {
+  if (*skip != 0.0) return;
+  __shared__ double sh[kDotThreads / 64][kDotGroup];
+  const int z = blockIdx.z;
+  const T *b = MX + L * (size_t)(iB - 1);
+  const int m = z == 0 ? iB : z == 1 ? iB + 1 : 2;
+  if ((int)blockIdx.y * kDotGroup >= m) return;
+  dots_body(L, z == 0 ? b : z == 1 ? b + L : r0, z == 2 ? b : MX, L, m, 0, part + pz * z, sh);
+}
 // NSSOLVER iteration i's Gram rows iB = 2i-1, iBB = 2i from their dots
-// (dk: for each of the two, h1 at 0, r1 at 256, h2 at 512, r2 at 768),
-// then GE (memLS.f90:607-677) and the stopping test; A (nB, nB), C the GE
-// scratch (Nn, Nn+1)
-__global__ void ns_gram_kernel(double *__restrict__ g, int i, int nB, const double *__restrict__ dk,
-                               double *__restrict__ A, double *__restrict__ Bv, double *__restrict__ xB,
-                               double *__restrict__ C) {
+// (ns_dots_kernel's parts), then GE (memLS.f90:607-677) and the stopping test;
+// A (nB, nB), C the GE scratch (Nn, Nn+1) when it does not fit the workgroup's.
+// Pivot search and back substitution by thread 0, the eliminations by all.
+constexpr int kGeLds = 48;
+__global__ void __launch_bounds__(kDotThreads) ns_gram_kernel(double *__restrict__ g, int i, int nB,
+                                                              const double *__restrict__ part, size_t pz, int nb,
+                                                              double *__restrict__ A, double *__restrict__ Bv,
+                                                              double *__restrict__ xB, double *__restrict__ Cg,
+                                                              HostFlag hf) {
 #pragma clang fp contract(off)
-  if (g[G_RI_SKIP] != 0.0) return;
-  const int iB = 2 * i - 1, iBB = 2 * i;
-  g[G_RI_DBPRE] = g[G_RI_FNORM];
-  for (int k = iB; k <= iBB; ++k) {
-    const double *d = dk + (size_t)1024 * (k - iB);
-    const double *h1 = d, *r1 = d + 256, *h2 = d + 512, *r2 = d + 768;
-    for (int j = 1; j <= k - 1; ++j) {
-      A[(j - 1) + (size_t)nB * (k - 1)] = h1[j - 1] + h2[j - 1];
-      A[(k - 1) + (size_t)nB * (j - 1)] = A[(j - 1) + (size_t)nB * (k - 1)];
-    }
-    const double n1 = sqrt(h1[k - 1]), n2 = sqrt(h2[k - 1]);
-    A[(k - 1) + (size_t)nB * (k - 1)] = n1 * n1 + n2 * n2;
-    Bv[k - 1] = r1[0] + r2[0];
+  if (g[G_RI_SKIP] != 0.0) {
+    if (threadIdx.x == 0) hf.tell(true);
+    return;
   }
-  for (int k = 0; k < iBB; ++k) xB[k] = Bv[k];
-  const int Nn = iBB;
+  __shared__ double Cl[kGeLds * (kGeLds + 1)];
+  __shared__ int piv, bad;
+  const int iB = 2 * i - 1, iBB = 2 * i, Nn = iBB, t = threadIdx.x;
+  for (int d = t / 64; d < iB + iBB + 2; d += kDotThreads / 64) {
+    const int z = d < iB ? 0 : d < iB + iBB ? 1 : 2;
+    const int j = z == 0 ? d : z == 1 ? d - iB : d - iB - iBB;
+    const double v = wave_parts(part + pz * z + (size_t)j * nb, nb);
+    if (t % 64 == 0) {
+      if (z == 2) {
+        Bv[iB - 1 + j] = v;
+      } else {
+        const int k = z == 0 ? iB - 1 : iBB - 1;
+        A[j + (size_t)nB * k] = v;
+        A[k + (size_t)nB * j] = v;
+      }
+    }
+  }
+  if (t == 0) {
+    g[G_RI_DBPRE] = g[G_RI_FNORM];
+    bad = 0;
+  }
+  __syncthreads();
   if (Nn == 2) {
-    const double a11 = A[0], a21 = A[1], a12 = A[nB], a22 = A[nB + 1];
-    const double pivot = a11 * a22 - a21 * a12;
-    const double saveEl = (xB[0] * a22 - xB[1] * a12) / pivot;
-    xB[1] = (xB[1] * a11 - xB[0] * a21) / pivot;
-    xB[0] = saveEl;
+    if (t == 0) {
+      const double a11 = A[0], a21 = A[1], a12 = A[nB], a22 = A[nB + 1], b0 = Bv[0], b1 = Bv[1];
+      const double pivot = a11 * a22 - a21 * a12;
+      xB[0] = (b0 * a22 - b1 * a12) / pivot;
+      xB[1] = (b1 * a11 - b0 * a21) / pivot;
+    }
   } else {
+    double *C = Nn <= kGeLds ? Cl : Cg;
 #define CC(r, cc) C[(r) + (size_t)Nn * (cc)]
-    for (int cc = 0; cc < Nn; ++cc)
-      for (int r = 0; r < Nn; ++r) CC(r, cc) = A[r + (size_t)nB * cc];
-    for (int r = 0; r < Nn; ++r) CC(r, Nn) = xB[r];
+    for (int e = t; e < Nn * (Nn + 1); e += kDotThreads) {
+      const int r = e % Nn, cc = e / Nn;
+      C[e] = cc < Nn ? A[r + (size_t)nB * cc] : Bv[r];
+    }
+    __syncthreads();
     for (int m = 0; m < Nn - 1; ++m) {
-      int ipv = m;
-      double pivot = fabs(CC(m, m));
-      for (int r = m + 1; r < Nn; ++r)
-        if (fabs(CC(r, m)) > pivot) {
-          ipv = r;
-          pivot = fabs(CC(r, m));
-        }
-      if (pivot < 2.0 * 2.220446049250313e-16) {
-        g[G_ERR] = 1.0;
-        g[G_RI_SKIP] = 1.0;
-        return;
+      if (t == 0) {
+        int ipv = m;
+        double pivot = fabs(CC(m, m));
+        for (int r = m + 1; r < Nn; ++r)
+          if (fabs(CC(r, m)) > pivot) {
+            ipv = r;
+            pivot = fabs(CC(r, m));
+          }
+        piv = ipv;
+        if (pivot < 2.0 * 2.220446049250313e-16) bad = 1;
       }
+      __syncthreads();
+      if (bad) break;
+      const int ipv = piv;
       if (ipv != m)
-        for (int cc = m; cc <= Nn; ++cc) {
-          const double t = CC(m, cc);
+        for (int cc = m + t; cc <= Nn; cc += kDotThreads) {
+          const double v = CC(m, cc);
           CC(m, cc) = CC(ipv, cc);
-          CC(ipv, cc) = t;
+          CC(ipv, cc) = v;
         }
-      for (int r = m + 1; r < Nn; ++r) {
+      __syncthreads();
+      const int nr = Nn - 1 - m, ncol = Nn - m;  // rows below m, columns past m
+      for (int e = t; e < nr * ncol; e += kDotThreads) {
+        const int r = m + 1 + e % nr, cc = m + 1 + e / nr;
         const double sv = CC(r, m) / CC(m, m);
-        CC(r, m) = 0.0;
-        for (int cc = m + 1; cc <= Nn; ++cc) CC(r, cc) = CC(r, cc) - sv * CC(m, cc);
+        CC(r, cc) = CC(r, cc) - sv * CC(m, cc);
+      }
+      __syncthreads();
+    }
+    if (t == 0 && !bad) {
+      for (int j = Nn - 1; j >= 0; --j) {
+        double v = CC(j, Nn);
+        for (int r = j + 1; r < Nn; ++r) v = v - CC(j, r) * CC(r, Nn);
+        v = v / CC(j, j);
+        CC(j, Nn) = v;
+        xB[j] = v;
       }
     }
-    for (int j = Nn - 1; j >= 0; --j) {
-      for (int r = j + 1; r < Nn; ++r) CC(j, Nn) = CC(j, Nn) - CC(j, r) * CC(r, Nn);
-      CC(j, Nn) = CC(j, Nn) / CC(j, j);
-    }
-    for (int r = 0; r < Nn; ++r) xB[r] = CC(r, Nn);
 #undef CC
+  }
+  if (t != 0) return;
+  if (bad) {
+    g[G_ERR] = 1.0;
+    g[G_RI_SKIP] = 1.0;
+    hf.tell(true);
+    return;
   }
   double sxb = 0.0;
   for (int k = 0; k < iBB; ++k) sxb = sxb + xB[k] * Bv[k];
   const double iN = g[G_RI_INORM];
-  g[G_RI_FNORM] = sqrt(iN * iN - sxb);
-  if (g[G_RI_FNORM] < g[G_RI_EPS]) {
+  const double fN = sqrt(iN * iN - sxb);
+  g[G_RI_FNORM] = fN;
+  const bool done = fN < g[G_RI_EPS];
+  if (done) {
     g[G_RI_SUC] = 1.0;
     g[G_RI_ITR] = (double)i;
     g[G_RI_SKIP] = 1.0;
   }
+  hf.tell(done);
 }
 // after the outer loop: the iteration count, and the solution's
 // coefficients cu(k) = xB(2k), cp(k) = xB(2k-1) (1-based)
@@ -2473,134 +2101,257 @@ __global__ void ns_final_kernel(double *__restrict__ g, int mItr, const double *
     cp[k - 1] = xB[2 * k - 2];
   }
 }
+__global__ void __launch_bounds__(kDotThreads) ns_rc_kernel(double *__restrict__ g, const double *__restrict__ part,
+                                                            int nb) {
+  if (g[G_ERR] != 0.0) return;
+  __shared__ double sh[16];
+  const double s = sum_dots(part, nb, sh);
+  if (threadIdx.x == 0) g[G_RC_N2] = s;
+}
 
-// Device workspaces of one device-driven solve (allocated before capture).
+struct SegCapture;
+int seg_cut(SegCapture *cap);
+// The workspaces of a solve and its progress.  A captured solve owns one and enqueues
+// every possible iteration (GMRES: mItr cycles of sD Arnoldi steps; CGRAD: mItr
+// iterations; NSSOLVER: mItr outer iterations), whose launches past
+// convergence see their flag and return at once.  A plain solve runs the same launch sequence,
+// polls the flags a step behind (HostFlag) and stops enqueueing; its workspace
+// stays with the matrix handle for the next solve (take_work).
 template <class T>
-struct NsGraphWork {
+struct SolveWork : crimson::SolveWorkBase {
   Ctx<T> c;
-  crimson::DBuf<T> Rm, Rc, Rmi, Rci, U, P, MU, MP, t1, t2, t3, t4, Rw, gmU, gmTmp;
-  crimson::DBuf<double> gst, fcoef, dots;
+  crimson::DBuf<T> r0, r, X, MX;          // NS: (3,N)|(N) vectors; X: U_i|P_i, MX: their images
+  crimson::DBuf<T> t3, t4, t5, ps, z;     // CG: R, the two directions; two-pass operator: Ps, Z
+  crimson::DBuf<T> wa, wb, ws, gmU;       // GMRES: the two working vectors, W o w, the basis
+  crimson::DBuf<double> gst, npart, h;    // state and small systems; norm parts (2 kSubGrid); h1, h2
   int sD = 0, nB = 0, mRI = 0, mGM = 0, mCG = 0;
   double riAbs = 0, riRel = 0, gmAbs = 0, gmRel = 0, cgAbs = 0, cgRel = 0;
-  bool disjoint = false;  // the coupled faces share no node: one launch for all of them
   bool formed = false;    // the Schur complement is formed (schur_ready)
-  int maxfn = 0;          // the largest coupled face
-  crimson::DBuf<double> msum;  // the faces' dots of the batched ADDBCMUL
-  struct SegCapture *cap = nullptr;  // the capture in progress, cut between the solve's phases
-  int cut();
+  SegCapture *cap = nullptr;  // the capture in progress, cut between the solve's phases
   size_t oH = 0, ocs = 0, osn = 0, oerr = 0, oy = 0, oA = 0, oBv = 0, oxB = 0, oC = 0, ocu = 0, ocp = 0;
-  double *G(size_t off) { return gst.p + off; }
-};
+  // a plain solve's flag word (pinned) and the number of its last teller
+  bool polled = false;
+  unsigned long long *word = nullptr, seq = 0;
+  double tGM = 0.0, tCG = 0.0;  // its time in the momentum solves and in the CG (callD)
 
-// ADDBCMUL of the device-driven solve: the batched face kernels when the
-// coupled faces are disjoint, addbcmul's per-face launches otherwise.
+  ~SolveWork() override {
+    if (word) (void)hipHostFree(word);
+  }
+  size_t bytes() const override {
+    return sizeof(T) * (c.W.n + c.fix.n + r0.n + r.n + X.n + MX.n + t3.n + t4.n + t5.n + ps.n + z.n + wa.n + wb.n +
+                        ws.n + gmU.n) +
+           sizeof(double) * (c.part.n + gst.n + npart.n + h.n);
+  }
+  double *G(size_t off) { return gst.p + off; }
+  int cut();
+  int poll_ready() {
+    polled = true;
+    if (word) return CRIMSON_OK;
+    if (hipHostMalloc((void **)&word, 64) != hipSuccess) {
+      word = nullptr;
+      (void)hipGetLastError();
+      crimson::set_error("hipHostMalloc of the solve's flag word failed");
+      return CRIMSON_ENOMEM;
+    }
+    *(volatile unsigned long long *)word = 0;
+    return CRIMSON_OK;
+  }
+  HostFlag flag() { return polled ? HostFlag{word, ++seq} : HostFlag{nullptr, 0}; }
+  // Waits for teller `k` (or a later one); *stop: whether its loop is over.  Ends also when the
+  // stream has failed, or is idle without the teller having told.
+  int wait(unsigned long long k, bool *stop) {
+    const volatile unsigned long long *w = word;
+    for (unsigned n = 1;; ++n) {
+      const unsigned long long v = *w;
+      if (v >> 1 >= k) {
+        *stop = v & 1;
+        return CRIMSON_OK;
+      }
+      if (n % 4096 == 0) {
+        const hipError_t e = hipStreamQuery(c.s);
+        if (e == hipErrorNotReady) continue;
+        if (e == hipSuccess && *w >> 1 >= k) continue;
+        crimson::set_error("memLS: the solve's stream ended before its step reported: %s", hipGetErrorString(e));
+        return CRIMSON_EHIP;
+      }
+    }
+  }
+};
 template <class T>
-int addbcmul_graph(NsGraphWork<T> &w, bool pre, int xdof, const T *X, T *Y, const double *skip) {
-  Ctx<T> &c = w.c;
-  if (!c.coupled) return CRIMSON_OK;
-  const int nfc = (int)c.hfdev.size();
-  if (!w.disjoint || nfc < 2) return addbcmul(c, pre, xdof, X, Y, skip, pre ? w.fcoef.p : nullptr);
-  face_dot_multi_kernel<T><<<nfc, 1024, 0, c.s>>>(c.fdev.p, xdof, X, w.msum.p, skip);
-  face_axpy_multi_kernel<T><<<dim3(crimson::grid_for(std::max(1, w.maxfn), 256), nfc), 256, 0, c.s>>>(
-      c.fdev.p, xdof, w.msum.p, pre ? 1 : 0, Y, skip);
+int SolveWork<T>::cut() {
+  return seg_cut(cap);
+}
+
+inline int dot_blocks(size_t L) { return (int)std::min<size_t>((L + kDotThreads - 1) / kDotThreads, kDotGrid); }
+template <class T>
+int dots(Ctx<T> &c, size_t L, const T *v, const T *U0, size_t ustride, int m, bool self, double *part,
+         const double *skip) {
+  dots_kernel<T><<<dim3(dot_blocks(L), (m + (self ? 1 : 0) + kDotGroup - 1) / kDotGroup), kDotThreads, 0, c.s>>>(
+      L, v, U0, ustride, m, self ? 1 : 0, part, skip);
+  CR_HIP(hipGetLastError());
+  return CRIMSON_OK;
+}
+template <class T>
+int face_apply(Ctx<T> &c, int what, int xdof, const T *X, T *Y, const double *skip) {
+  if (c.nfc() == 0) return CRIMSON_OK;
+  face_apply_kernel<T><<<c.disjoint ? c.nfc() : 1, 1024, 0, c.s>>>(c.fdev.p, c.nfc(), what, xdof, X, Y, c.fsum.p,
+                                                                  skip);
   CR_HIP(hipGetLastError());
   return CRIMSON_OK;
 }
 
-// GMRES (gmres_dev) device-driven, on the operator x -> A x + ADD(x) with
-// PRE (the NS solver's momentum solves: pre_ok, GMRESV's first-product
-// count not kept)
+// Grid of the Arnoldi sweeps over L entries: four threads per entry while
+// that fills the card no more than once (measured at 60 vectors of 20,000 entries: 10
+// -> 6 us), one beyond.
+struct SubGrid {
+  int js, blocks;
+};
+inline SubGrid sub_grid(size_t L) {
+  const int js = L <= (size_t)256 * kSubGrid ? 4 : 1;
+  const size_t e = kDotThreads / js;
+  return SubGrid{js, (int)std::min<size_t>((L + e - 1) / e, kSubGrid)};
+}
+template <class T, class IX>
+void arnoldi_spmv_ix(Ctx<T> &c, const MatView<T> &A, int nd, const IX *col, const T *w, const T *ws,
+                     const double *scale, T *u, T *y, const double *skip) {
+  const int *rp = c.lhs->d_rowptr.p;
+  const unsigned G = crimson::grid_for((size_t)c.N * kRowLanes, 256),
+                 Gn = crimson::grid_for((size_t)c.N * kNarrowLanes, 256);
+  switch (nd) {
+    case 1: arnoldi_spmv_kernel<1, T, IX><<<Gn, 256, 0, c.s>>>(c.N, rp, col, A, w, ws, scale, u, y, skip); break;
+    case 2: arnoldi_spmv_kernel<2, T, IX><<<Gn, 256, 0, c.s>>>(c.N, rp, col, A, w, ws, scale, u, y, skip); break;
+    case 3: arnoldi_spmv_kernel<3, T, IX><<<G, 256, 0, c.s>>>(c.N, rp, col, A, w, ws, scale, u, y, skip); break;
+    default: arnoldi_spmv_kernel<4, T, IX><<<G, 256, 0, c.s>>>(c.N, rp, col, A, w, ws, scale, u, y, skip); break;
+  }
+}
 template <class T>
-int gmres_graph(NsGraphWork<T> &w, const MatView<T> &A, int nd, const T *R, T *X) {
+void arnoldi_sub(Ctx<T> &c, const SubGrid &sg, size_t L, int nd, const MatView<T> &A, T *y, T *ys, const T *U, int m,
+                 bool self, int np, double *h, double *npart, const double *n0, const double *n1,
+                 const double *skip) {
+  const int pad = nd == 3 ? 4 : nd;
+  if (sg.js == 4)
+    arnoldi_sub_kernel<T, 4><<<sg.blocks, kDotThreads, 0, c.s>>>(L, nd, pad, A.W, A.wdof, A.c0, y, ys, U, L, m,
+                                                                 self ? 1 : 0, c.part.p, np, h, npart, n0, n1, skip);
+  else
+    arnoldi_sub_kernel<T, 1><<<sg.blocks, kDotThreads, 0, c.s>>>(L, nd, pad, A.W, A.wdof, A.c0, y, ys, U, L, m,
+                                                                 self ? 1 : 0, c.part.p, np, h, npart, n0, n1, skip);
+}
+
+// GMRES (memLS.f90:681-788) for the operator x -> A x + ADD(x), left
+// preconditioned by PRE (pre: the NS solver's momentum solves; GMRESV takes
+// none, and counts the first residual too, :827-829); R, X are (nd, N).  Classical Gram-Schmidt with
+// a DGKS second pass where memLS orthogonalises one vector after the other
+// (:743-746): the same Krylov space, solutions equal to the solver tolerance.
+struct GmParams {
+  int mItr, sD;
+  double absTol, relTol;
+  bool pre, count_first;
+};
+template <class T>
+int gmres_run(SolveWork<T> &w, const MatView<T> &A, int nd, const T *R, T *X, const GmParams &p, const double *skip) {
   Ctx<T> &c = w.c;
   const size_t L = (size_t)nd * c.N;
-  const int sD = w.sD;
-  double *g = w.gst.p;
-  const double *cyc = g + G_GM_CYC, *arn = g + G_GM_ARN, *ri = g + G_RI_SKIP;
-  T *U = w.gmU.p;
+  const int pad = nd == 3 ? 4 : nd;
+  double *g = w.gst.p, *h1 = w.h.p, *h2 = w.h.p + 256, *n1 = w.npart.p, *n2 = w.npart.p + kSubGrid;
+  const double *cyc = g + G_GM_CYC, *arn = g + G_GM_ARN;
+  T *U = w.gmU.p, *v = w.wa.p, *y = w.wb.p;
   const unsigned GL = crimson::grid_for(L, 256);
-  gm_begin_kernel<<<1, 1, 0, c.s>>>(g);
-  gfill_kernel<T><<<GL, 256, 0, c.s>>>(L, X, ri);
-  const int nblk = (int)((L + kChunk - 1) / kChunk);
-  double *h1 = c.hcol.p, *h2 = c.hcol.p + 256, *nrm = c.hcol.p + 512;
-  T *pt = reinterpret_cast<T *>(c.partial.p);
-  for (int l = 1; l <= w.mGM; ++l) {
+  const SubGrid sg = sub_grid(L);
+  const int nb0 = (int)std::min<size_t>((L + kDotThreads - 1) / kDotThreads, kSubGrid), np = dot_blocks(L);
+  gm_begin_kernel<<<1, 1, 0, c.s>>>(g, skip);
+  fill_kernel<T><<<GL, 256, 0, c.s>>>(L, X, skip);
+  for (int l = 1; l <= p.mItr; ++l) {
     if (l == 1) {
-      gcopy_kernel<T><<<GL, 256, 0, c.s>>>(L, R, U, cyc, nullptr);
+      copy_kernel<T><<<GL, 256, 0, c.s>>>(L, R, v, cyc);  // X = 0: R - A X is R
     } else {
-      gm_count_kernel<<<1, 1, 0, c.s>>>(g);
-      CR_TRY(spmv(c, A, nd, nd, X, U, 1.0, static_cast<const T *>(nullptr), 0.0, cyc));
-      CR_TRY(addbcmul_graph(w, false, nd, X, U, cyc));
-      gaxpby_kernel<T><<<GL, 256, 0, c.s>>>(L, T(1), R, T(-1), U, cyc);
+      CR_TRY(spmv(c, A, nd, nd, X, v, 1.0, static_cast<const T *>(nullptr), 0.0, cyc));
+      CR_TRY(face_apply(c, kFaceAdd, nd, X, v, cyc));
+      diff_kernel<T><<<GL, 256, 0, c.s>>>(L, R, v, v, cyc);
     }
-    CR_TRY(addbcmul_graph(w, true, nd, U, U, cyc));
-    CR_TRY(mdot<T>(c, L, U, nullptr, 0, 0, true, c.dsc.p + 40, nullptr, true, cyc));
-    gm_cycle_kernel<<<1, 1, 0, c.s>>>(g, l, w.gmAbs, w.gmRel, c.dsc.p + 40, w.G(w.oerr));
-    gscale_kernel<T><<<GL, 256, 0, c.s>>>(L, U, g + G_GM_SCALE, cyc);
-    for (int i = 1; i <= sD; ++i) {
-      T *ui = U + L * (size_t)i;
-      const T *uprev = U + L * (size_t)(i - 1);
-      CR_TRY(spmv(c, A, nd, nd, uprev, ui, 1.0, static_cast<const T *>(nullptr), 0.0, arn));
-      CR_TRY(addbcmul_graph(w, false, nd, uprev, ui, arn));
-      CR_TRY(addbcmul_graph(w, true, nd, ui, ui, arn));
-      CR_TRY(mdot(c, L, ui, U, L, i, true, h1, nullptr, false, arn));
-      msub_norm_kernel<T><<<nblk, 256, 0, c.s>>>(L, ui, U, L, i, h1, pt, 1, nullptr, arn);
-      reduce_kernel<T><<<1, 256, 0, c.s>>>(nblk, pt, 1, nrm + 1, nullptr, arn);
-      dgks_kernel<<<1, 1, 0, c.s>>>(h1 + i, nrm + 1, c.gate.p, arn);
-      CR_TRY(mdot(c, L, ui, U, L, i, false, h2, c.gate.p, false, arn));
-      msub_norm_kernel<T><<<nblk, 256, 0, c.s>>>(L, ui, U, L, i, h2, pt, 1, c.gate.p, arn);
-      reduce_kernel<T><<<1, 256, 0, c.s>>>(nblk, pt, 1, nrm + 2, c.gate.p, arn);
-      gm_givens_kernel<<<1, 1, 0, c.s>>>(g, i, sD, h1, h2, nrm, c.gate.p, w.G(w.oH), w.G(w.ocs), w.G(w.osn),
-                                         w.G(w.oerr));
-      gscale_kernel<T><<<GL, 256, 0, c.s>>>(L, ui, g + G_GM_SCALE, arn);
+    if (p.pre) CR_TRY(face_apply(c, kFacePre, nd, v, v, cyc));
+    arnoldi_first_kernel<T><<<nb0, kDotThreads, 0, c.s>>>(L, nd, pad, A.W, A.wdof, A.c0, v, w.ws.p, n1, cyc);
+    gm_cycle_kernel<<<1, kDotThreads, 0, c.s>>>(g, l, l > 1 || p.count_first, p.absTol, p.relTol, n1, nb0,
+                                                w.G(w.oerr));
+    bool stop = false;
+    for (int i = 1; i <= p.sD; ++i) {
+      T *u = U + L * (size_t)(i - 1);
+      if (c.lhs->d_col16.p)
+        arnoldi_spmv_ix(c, A, nd, c.lhs->d_col16.p, v, w.ws.p, g + G_GM_SCALE, u, y, arn);
+      else
+        arnoldi_spmv_ix(c, A, nd, c.lhs->d_col.p, v, w.ws.p, g + G_GM_SCALE, u, y, arn);
+      CR_TRY(face_apply(c, kFaceAdd | (p.pre ? kFacePre : 0), nd, u, y, arn));
+      CR_TRY(dots(c, L, y, U, L, i, true, c.part.p, arn));
+      arnoldi_sub(c, sg, L, nd, A, y, w.ws.p, U, i, true, np, h1, n1, static_cast<const double *>(nullptr),
+                  static_cast<const double *>(nullptr), arn);
+      dots2_kernel<T><<<dim3(np, (i + kDotGroup - 1) / kDotGroup), kDotThreads, 0, c.s>>>(
+          L, y, U, L, i, c.part.p, h1 + i, n1, sg.blocks, arn);
+      arnoldi_sub(c, sg, L, nd, A, y, w.ws.p, U, i, false, np, h2, n2, h1 + i, n1, arn);
+      gm_givens_kernel<<<1, kDotThreads, 0, c.s>>>(g, i, p.sD, h1, h2, n1, n2, sg.blocks, w.G(w.oH), w.G(w.ocs),
+                                                   w.G(w.osn), w.G(w.oerr), w.flag());
+      CR_HIP(hipGetLastError());
+      std::swap(v, y);
+      // a plain solve looks at the step before while this one runs
+      if (w.polled && i > 1) CR_TRY(w.wait(w.seq - 1, &stop));
+      if (stop) break;
     }
-    gm_solve_kernel<<<1, 1, 0, c.s>>>(g, sD, w.G(w.oH), w.G(w.oerr), w.G(w.oy));
-    gmaxpy_kernel<T><<<GL, 256, 0, c.s>>>(L, X, U, L, 0, g + G_GM_APPLY, w.G(w.oy), 1.0, cyc, nullptr);
+    gm_solve_kernel<<<1, 256, 0, c.s>>>(g, p.sD, w.G(w.oH), w.G(w.oerr), w.G(w.oy));
+    combine_kernel<T><<<GL, 256, 0, c.s>>>(L, X, X, U, L, 0, g + G_GM_APPLY, w.G(w.oy), 1.0, cyc);
     gm_endcycle_kernel<<<1, 1, 0, c.s>>>(g);
+    CR_HIP(hipGetLastError());
+    if (w.polled) {
+      if (!stop) CR_TRY(w.wait(w.seq, &stop));
+      if (stop) break;
+    }
   }
-  gm_finish_kernel<<<1, 1, 0, c.s>>>(g);
-  CR_HIP(hipGetLastError());
   return CRIMSON_OK;
 }
 
-// CGRAD on the Schur operator (cg_dev with schur = true) device-driven:
-// mItr iteration bodies, each launch returning at once after the flag.
+// CGRAD / CGRADV / CGRADS (memLS.f90:367-430): op(P, SP, done, nd) computes SP and
+// nd parts of P . SP; X holds the right-hand side in and the solution out.
+// *state: the state's copy that holds the end.
+constexpr int kCgLag = 4;  // iterations a plain solve runs ahead of the flag it has read
 template <class T, class Op>
-int cg_graph(NsGraphWork<T> &w, size_t L, T *X, Op op, T *R, T *P, T *P2, T *SP, const CgAux<T> &ax) {
+int cg_run(SolveWork<T> &w, size_t L, T *X, Op op, T *R, T *P, T *P2, T *SP, const CgAux<T> &ax, double absTol,
+           double relTol, int mItr, double *g, const double *skip, double **state) {
   Ctx<T> &c = w.c;
-  double *g = w.gst.p, *scal = c.cgst.p;
-  CR_TRY(mdot<T>(c, L, X, nullptr, 0, 0, true, c.dsc.p + 41, nullptr, true, g + G_RI_SKIP));
-  cg_begin_kernel<<<1, 1, 0, c.s>>>(scal, g, c.dsc.p + 41, w.cgAbs, w.cgRel, w.mCG);
-  CR_TRY(cg_begin_vec(c, L, ax, X, R, P, g + G_RI_SKIP));
-  for (int it = 0; it < w.mCG; ++it) {
+  CR_TRY(dots(c, L, X, static_cast<const T *>(nullptr), 0, 0, true, c.part.p, skip));
+  cg_begin_kernel<<<1, kDotThreads, 0, c.s>>>(c.cgst.p, g, skip, c.part.p, dot_blocks(L), absTol, relTol, mItr);
+  CR_TRY(cg_begin_vec(c, L, ax, X, R, P, skip));
+  const unsigned long long s0 = w.seq;
+  int it = 0;
+  // the flag is raised at the top of the iteration after the last one, so a
+  // plain solve runs past mItr by its lag at most
+  for (; w.polled || it < mItr; ++it) {
     int nd = 0;
     CR_TRY(op(P, SP, c.cgst.p + (it & 1) * kCgState + 5, nd));
-    CR_TRY(cg_sweeps(c, L, it, nd, ax, X, R, P, P2, SP));
+    CR_TRY(cg_sweeps(c, L, it, nd, ax, X, R, P, P2, SP, w.flag()));
     std::swap(P, P2);
+    bool stop = false;
+    if (w.polled && it >= kCgLag) CR_TRY(w.wait(s0 + 1 + it - kCgLag, &stop));
+    if (stop) {
+      ++it;
+      break;
+    }
   }
-  cg_end_kernel<<<1, 1, 0, c.s>>>(c.cgst.p + (w.mCG & 1) * kCgState, g);
-  CR_HIP(hipGetLastError());
+  *state = c.cgst.p + (it & 1) * kCgState;
   return CRIMSON_OK;
 }
 
-// NSSOLVER (nssolver_dev) device-driven on Ri (4, N): the whole solve is
-// enqueued on w.c.s with no host synchronisation.
+// NSSOLVER (memLS.f90:1460-1759) on d_Ri (4, N), PRECOND's W applied on the
+// way in and out.
 template <class T>
-int nssolver_graph(NsGraphWork<T> &w, T *Ri) {
+int ns_run(SolveWork<T> &w, double *d_Ri) {
   Ctx<T> &c = w.c;
   crimson_lhs *l = c.lhs;
-  const int N = c.N, nsd = 3;
-  const size_t mn = (size_t)nsd * N;
+  const int N = c.N;
+  const size_t mn = (size_t)3 * N, st = (size_t)4 * N;
   double *g = w.gst.p;
   const double *ri = g + G_RI_SKIP;
-  const unsigned gN = crimson::grid_for(N, 256), Gmn = crimson::grid_for(mn, 256);
-  extract_kernel<<<gN, 256, 0, c.s>>>(N, 4, 0, 3, Ri, w.Rmi.p);
-  extract_kernel<<<gN, 256, 0, c.s>>>(N, 4, 3, 1, Ri, w.Rci.p);
-  gcopy_kernel<T><<<Gmn, 256, 0, c.s>>>(mn, w.Rmi.p, w.Rm.p, nullptr, nullptr);
-  gcopy_kernel<T><<<gN, 256, 0, c.s>>>(N, w.Rci.p, w.Rc.p, nullptr, nullptr);
-  CR_TRY(mdot<T>(c, mn, w.Rm.p, nullptr, 0, 0, true, c.dsc.p + 42, nullptr, true));
-  CR_TRY(mdot<T>(c, N, w.Rc.p, nullptr, 0, 0, true, c.dsc.p + 43, nullptr, true));
-  ns_begin_kernel<<<1, 1, 0, c.s>>>(g, c.dsc.p + 42, c.dsc.p + 43, w.riAbs, w.riRel);
+  const unsigned gN = crimson::grid_for(N, 256), Gmn = crimson::grid_for(mn, 256), Gst = crimson::grid_for(st, 256);
+  ns_split_kernel<T><<<gN, 256, 0, c.s>>>(N, d_Ri, c.W.p, w.r0.p, w.r.p);
+  CR_TRY(dots(c, st, w.r0.p, static_cast<const T *>(nullptr), 0, 0, true, c.part.p, nullptr));
+  ns_begin_kernel<<<1, kDotThreads, 0, c.s>>>(g, c.part.p, dot_blocks(st), w.riAbs, w.riRel);
+  // DEPART: views on the 4x4 planes (memLS.f90:1612-1679); Gt = -mG^T
   const T *V = planes(l, T(0));
   const MatView<T> mK = view<T>(c, V, 4, 0, 0, 3, 3, c.W.p, c.fix.p, 4);
   const MatView<T> mG = view<T>(c, V, 4, 0, 3, 3, 1, c.W.p, nullptr, 4);
@@ -2617,21 +2368,15 @@ int nssolver_graph(NsGraphWork<T> &w, T *Ri) {
     Gt.r0 = 3;
     Gt.c0 = 0;
   }
-  // BCPRE and the faces' PRE coefficients on the device; the face
-  // functionals (c.hfdev / c.fdev: set up once by ns_graph_setup)
-  for (size_t f = 0; f < l->face.size(); ++f) {
-    CrFace &fa = l->face[f];
-    if (!fa.coupled) continue;
-    face_pre_coef_kernel<<<1, 1, 0, c.s>>>(fa.nNo, fa.dof, nsd, fa.d_valM.p, fa.res, w.fcoef.p + f);
-  }
-  CR_HIP(hipGetLastError());
+  // BCPRE (memLS.f90:1683-1716) and the faces' functionals
+  if (c.nfc() > 0) face_coef_kernel<<<c.nfc(), 1024, 0, c.s>>>(c.fdev.p, 3, c.fcoef.p);
   CR_TRY(face_functionals(c, mG));
   SchurOp<T> so;
   so.formed = w.formed;
   so.L = mL;
   so.Gt = Gt;
   so.G = mG;
-  so.Z = w.gmTmp.p;
+  so.Z = w.z.p;
   CR_TRY(schur_form(c, so));
   CgAux<T> ax;
   ax.fl = c.face_list();
@@ -2639,77 +2384,74 @@ int nssolver_graph(NsGraphWork<T> &w, T *Ri) {
     ax.W = c.W.p;
     ax.wdof = 4;
     ax.off = mG.c0;
-    ax.Ps = so.Ps = w.t2.p;
+    ax.Ps = so.Ps = w.ps.p;
   }
+  // Schur operator of CGRAD: SP = L P - Gt (G P + PRE)
   auto schur_op = [&](const T *Pv, T *SPv, const double *done, int &nd) -> int {
     return schur_apply(c, so, Pv, SPv, done, nd);
   };
-  const int nB = w.nB;
+  const GmParams gm{w.mGM, w.sD, w.gmAbs, w.gmRel, true, false};
+  const int nb = dot_blocks(st);
+  const size_t pz = (size_t)kDotGrid * 264;
   for (int i = 1; i <= w.mRI; ++i) {
     const int iB = 2 * i - 1, iBB = 2 * i;
-    T *Ui = w.U.p + mn * (i - 1), *Pi = w.P.p + (size_t)N * (i - 1);
-    T *MUb = w.MU.p + mn * (iB - 1), *MUbb = w.MU.p + mn * (iBB - 1);
-    T *MPb = w.MP.p + (size_t)N * (iB - 1), *MPbb = w.MP.p + (size_t)N * (iBB - 1);
+    T *Ui = w.X.p + st * (i - 1), *Pi = Ui + mn;
+    T *MUb = w.MX.p + st * (iB - 1), *MPb = MUb + mn, *MUbb = MUb + st, *MPbb = MUbb + mn;
     CR_TRY(w.cut());
-    CR_TRY(gmres_graph(w, mK, 3, w.Rm.p, Ui));
+    double t0 = now_s();
+    CR_TRY(gmres_run(w, mK, 3, w.r.p, Ui, gm, ri));
+    double t1 = now_s();
+    w.tGM += t1 - t0;
     CR_TRY(w.cut());
-    CR_TRY(spmv(c, mD, 1, 3, Ui, Pi, -1.0, w.Rc.p, 1.0, ri));  // P = Rc - D U
-    CR_TRY(cg_graph(w, (size_t)N, Pi, schur_op, w.t3.p, w.t4.p, w.t1.p, MPb, ax));
+    CR_TRY(spmv(c, mD, 1, 3, Ui, Pi, -1.0, w.r.p + mn, 1.0, ri));  // P = Rc - D U
+    double *state = nullptr;
+    CR_TRY(cg_run(w, (size_t)N, Pi, schur_op, w.t3.p, w.t4.p, w.t5.p, MPb, ax, w.cgAbs, w.cgRel, w.mCG, g, ri,
+                  &state));
+    cg_end_kernel<<<1, 1, 0, c.s>>>(state, g, ri);
+    t0 = now_s();
+    w.tCG += t0 - t1;
     CR_TRY(w.cut());
     CR_TRY(spmv(c, mG, 3, 1, Pi, MUb, 1.0, static_cast<const T *>(nullptr), 0.0, ri));
-    gaxpby_kernel<T><<<Gmn, 256, 0, c.s>>>(mn, T(1), w.Rm.p, T(0), MUbb, ri);
-    gaxpby_kernel<T><<<Gmn, 256, 0, c.s>>>(mn, T(-1), MUb, T(1), MUbb, ri);  // MU(iBB) = Rm - MU(iB)
-    CR_TRY(gmres_graph(w, mK, 3, MUbb, Ui));
+    diff_kernel<T><<<Gmn, 256, 0, c.s>>>(mn, w.r.p, MUb, MUbb, ri);  // MU(iBB) = Rm - MU(iB)
+    CR_TRY(gmres_run(w, mK, 3, MUbb, Ui, gm, ri));
+    w.tGM += now_s() - t0;
     CR_TRY(w.cut());
     CR_TRY(spmv(c, mK, 3, 3, Ui, MUbb, 1.0, static_cast<const T *>(nullptr), 0.0, ri));
-    CR_TRY(addbcmul_graph(w, false, 3, Ui, MUbb, ri));
+    CR_TRY(face_apply(c, kFaceAdd, 3, Ui, MUbb, ri));
     CR_TRY(spmv(c, mL, 1, 1, Pi, MPb, 1.0, static_cast<const T *>(nullptr), 0.0, ri));
     CR_TRY(spmv(c, mD, 1, 3, Ui, MPbb, 1.0, static_cast<const T *>(nullptr), 0.0, ri));
-    for (int k = iB; k <= iBB; ++k) {
-      const T *MUk = w.MU.p + mn * (k - 1), *MPk = w.MP.p + (size_t)N * (k - 1);
-      double *d = w.dots.p + (size_t)1024 * (k - iB);
-      CR_TRY(mdot<T>(c, mn, MUk, w.MU.p, mn, k - 1, true, d, nullptr, true, ri));
-      CR_TRY(mdot<T>(c, mn, MUk, w.Rmi.p, 0, 1, false, d + 256, nullptr, true, ri));
-      CR_TRY(mdot<T>(c, N, MPk, w.MP.p, N, k - 1, true, d + 512, nullptr, true, ri));
-      CR_TRY(mdot<T>(c, N, MPk, w.Rci.p, 0, 1, false, d + 768, nullptr, true, ri));
+    ns_dots_kernel<T><<<dim3(nb, (iBB + kDotGroup - 1) / kDotGroup, 3), kDotThreads, 0, c.s>>>(
+        st, w.MX.p, w.r0.p, iB, c.part.p, pz, ri);
+    ns_gram_kernel<<<1, kDotThreads, 0, c.s>>>(g, i, w.nB, c.part.p, pz, nb, w.G(w.oA), w.G(w.oBv), w.G(w.oxB),
+                                               w.G(w.oC), w.flag());
+    CR_HIP(hipGetLastError());
+    if (w.polled) {
+      bool stop = false;
+      CR_TRY(w.wait(w.seq, &stop));
+      if (stop) break;
     }
-    ns_gram_kernel<<<1, 1, 0, c.s>>>(g, i, nB, w.dots.p, w.G(w.oA), w.G(w.oBv), w.G(w.oxB), w.G(w.oC));
-    gcopy_kernel<T><<<Gmn, 256, 0, c.s>>>(mn, w.Rmi.p, w.Rm.p, ri, nullptr);
-    gcopy_kernel<T><<<gN, 256, 0, c.s>>>(N, w.Rci.p, w.Rc.p, ri, nullptr);
-    gmaxpy_kernel<T><<<Gmn, 256, 0, c.s>>>(mn, w.Rm.p, w.MU.p, mn, iBB, nullptr, w.G(w.oxB), -1.0, ri, nullptr);
-    gmaxpy_kernel<T><<<gN, 256, 0, c.s>>>(N, w.Rc.p, w.MP.p, N, iBB, nullptr, w.G(w.oxB), -1.0, ri, nullptr);
+    combine_kernel<T><<<Gst, 256, 0, c.s>>>(st, w.r0.p, w.r.p, w.MX.p, st, iBB, nullptr, w.G(w.oxB), -1.0, ri);
   }
   ns_final_kernel<<<1, 1, 0, c.s>>>(g, w.mRI, w.G(w.oxB), w.G(w.ocu), w.G(w.ocp));
-  const double *err = g + G_ERR, *suc = g + G_RI_SUC;
-  gcopy_kernel<T><<<gN, 256, 0, c.s>>>(N, w.Rci.p, w.Rc.p, err, suc);
-  gmaxpy_kernel<T><<<gN, 256, 0, c.s>>>(N, w.Rc.p, w.MP.p, N, 0, g + G_NS_CNT, w.G(w.oxB), -1.0, err, suc);
-  CR_TRY(mdot<T>(c, N, w.Rc.p, nullptr, 0, 0, true, g + G_RC_N2, nullptr, true, err));
-  // solution: Rmi = sum cu(k) U_k, Rci = sum cp(k) P_k
-  gfill_kernel<T><<<Gmn, 256, 0, c.s>>>(mn, w.Rmi.p, err);
-  gfill_kernel<T><<<gN, 256, 0, c.s>>>(N, w.Rci.p, err);
-  gmaxpy_kernel<T><<<Gmn, 256, 0, c.s>>>(mn, w.Rmi.p, w.U.p, mn, 0, g + G_RI_ITR, w.G(w.ocu), 1.0, err, nullptr);
-  gmaxpy_kernel<T><<<gN, 256, 0, c.s>>>(N, w.Rci.p, w.P.p, N, 0, g + G_RI_ITR, w.G(w.ocp), 1.0, err, nullptr);
-  insert_kernel<<<gN, 256, 0, c.s>>>(N, 4, 0, 3, w.Rmi.p, Ri);
-  insert_kernel<<<gN, 256, 0, c.s>>>(N, 4, 3, 1, w.Rci.p, Ri);
+  // the remaining pressure residual's share (Resc)
+  const double *err = g + G_ERR;
+  combine_kernel<T><<<gN, 256, 0, c.s>>>(N, w.r0.p + mn, w.r.p + mn, w.MX.p + mn, st, 0, g + G_NS_CNT, w.G(w.oxB),
+                                         -1.0, err);
+  CR_TRY(dots(c, N, w.r.p + mn, static_cast<const T *>(nullptr), 0, 0, true, c.part.p, err));
+  ns_rc_kernel<<<1, kDotThreads, 0, c.s>>>(g, c.part.p, dot_blocks(N));
+  ns_join_kernel<T><<<gN, 256, 0, c.s>>>(N, w.X.p, g + G_RI_ITR, w.G(w.ocu), w.G(w.ocp), c.W.p, d_Ri, err);
   CR_HIP(hipGetLastError());
   return CRIMSON_OK;
 }
 
-// The device-driven solve's workspaces and face set-up for lhs and ls
-// (allocations, face supports and their uploads: all before any capture).
-// res: memLS's face coefficients (res[f] != 0 couples Neumann face f), incL
-// as in memLS_SOLVE.
+// The coupled faces of this solve (memLS.f90:1965-1986; res[f] != 0 couples Neumann face
+// f) on the device.
 template <class T>
-int ns_graph_setup(NsGraphWork<T> &w, crimson_lhs *l, crimson_ls *ls, const int *incL, const double *res,
-                   hipStream_t s) {
-  if (ls->LS_type != CRIMSON_LS_NS) {
-    crimson::set_error("the device-driven solve is the NS solver's (LS_TYPE_NS)");
-    return CRIMSON_EUNSUPPORTED;
-  }
-  Ctx<T> &c = w.c;
-  CR_TRY(c.init(l, 4));
-  c.s = s;
-  c.coupled = false;
+int face_setup(Ctx<T> &c, const int *incL, const double *res, bool ns) {
+  crimson_lhs *l = c.lhs;
+  std::vector<FaceDev> fd;
+  std::vector<int> nodes;
+  int n = 0;
   for (int f = 0; f < l->nFaces; ++f) {
     CrFace &fa = l->face[f];
     fa.inc = !(incL && incL[f] == 0);
@@ -2718,15 +2460,58 @@ int ns_graph_setup(NsGraphWork<T> &w, crimson_lhs *l, crimson_ls *ls, const int 
     if (fa.bGrp == CRIMSON_BC_NEU && res && res[f] != 0.0) {
       fa.res = res[f];
       fa.coupled = true;
-      c.coupled = true;
+      ++n;
     }
   }
-  const int N = l->nNo;
-  const size_t mn = (size_t)3 * N;
+  CR_TRY(c.fcoef.alloc(std::max(1, n)));
+  CR_TRY(c.fsum.alloc(std::max(1, n)));
+  CR_TRY(c.fpart.alloc((size_t)std::max(1, n) * kFaceDotBlocks));
+  for (auto &fa : l->face) {
+    if (!fa.coupled) continue;
+    CR_TRY(fa.d_valM.alloc((size_t)fa.dof * fa.nNo));
+    if (ns) CR_TRY(face_support(l, fa));
+    FaceDev d{};
+    d.glob = fa.d_glob.p;
+    d.valM = fa.d_valM.p;
+    d.coefp = c.fcoef.p + fd.size();
+    d.res = fa.res;
+    d.nNo = fa.nNo;
+    d.dof = fa.dof;
+    d.sup = ns ? fa.d_sup.p : nullptr;
+    d.q = ns ? fa.d_q.p : nullptr;
+    d.nsup = ns ? fa.nsup : 0;
+    fd.push_back(d);
+    nodes.insert(nodes.end(), fa.glob.begin(), fa.glob.end());
+  }
+  std::sort(nodes.begin(), nodes.end());
+  c.disjoint = std::adjacent_find(nodes.begin(), nodes.end()) == nodes.end();
+  const bool same = fd.size() == c.hfdev.size() && c.fdev.p &&
+                    std::equal(fd.begin(), fd.end(), c.hfdev.begin(), [](const FaceDev &a, const FaceDev &b) {
+                      return a.glob == b.glob && a.valM == b.valM && a.coefp == b.coefp && a.res == b.res &&
+                             a.nNo == b.nNo && a.dof == b.dof && a.sup == b.sup && a.q == b.q && a.nsup == b.nsup;
+                    });
+  c.hfdev = fd;
+  if (!same && !fd.empty()) {
+    CR_TRY(c.fdev.upload(c.hfdev.data(), fd.size(), c.s));
+    CR_HIP(hipStreamSynchronize(c.s));
+  }
+  if (ns) CR_TRY(face_list(c));
+  return CRIMSON_OK;
+}
+
+// Workspaces and face set-up of one solve (allocations and uploads: all
+// before any capture).
+template <class T>
+int work_setup(SolveWork<T> &w, crimson_lhs *l, crimson_ls *ls, int dof, const int *incL, const double *res,
+               hipStream_t s) {
+  Ctx<T> &c = w.c;
+  CR_TRY(c.init(l, dof, s));
+  const bool ns = ls->LS_type == CRIMSON_LS_NS;
+  const size_t N = l->nNo, st = (size_t)dof * N;
   w.mRI = ls->RI.mItr;
   w.mGM = ls->GM.mItr;
   w.mCG = ls->CG.mItr;
-  w.sD = ls->GM.sD;
+  w.sD = ns ? ls->GM.sD : ls->RI.sD;
   w.nB = 2 * w.mRI;
   w.riAbs = ls->RI.absTol;
   w.riRel = ls->RI.relTol;
@@ -2734,95 +2519,66 @@ int ns_graph_setup(NsGraphWork<T> &w, crimson_lhs *l, crimson_ls *ls, const int 
   w.gmRel = ls->GM.relTol;
   w.cgAbs = ls->CG.absTol;
   w.cgRel = ls->CG.relTol;
-  if (w.mRI < 1 || w.mGM < 1 || w.mCG < 1 || w.sD < 1 || w.nB > 255 || w.sD > 255) {
-    crimson::set_error("device-driven NS solve: iteration limits out of range (RI %d, GM %d x %d, CG %d)", w.mRI,
-                       w.mGM, w.sD, w.mCG);
-    return CRIMSON_EARG;
-  }
-  CR_TRY(w.Rm.alloc(mn));
-  CR_TRY(w.Rc.alloc(N));
-  CR_TRY(w.Rmi.alloc(mn));
-  CR_TRY(w.Rci.alloc(N));
-  CR_TRY(w.U.alloc(mn * w.mRI));
-  CR_TRY(w.P.alloc((size_t)N * w.mRI));
-  CR_TRY(w.MU.alloc(mn * w.nB));
-  CR_TRY(w.MP.alloc((size_t)N * w.nB));
-  CR_TRY(w.t1.alloc(mn));
-  CR_TRY(w.t2.alloc(N));
-  CR_TRY(w.t3.alloc(N));
-  CR_TRY(w.t4.alloc(N));
-  CR_TRY(w.gmTmp.alloc(std::max(mn, (size_t)4 * N)));  // GMRES scratch; the Schur CG's Z(4, N)
-  CR_TRY(w.gmU.alloc(mn * (w.sD + 1)));
-  if (sizeof(T) != sizeof(double)) CR_TRY(w.Rw.alloc((size_t)4 * N));
+  CR_TRY(w.r0.alloc(st));
+  CR_TRY(w.npart.alloc(2 * kSubGrid));
+  CR_TRY(w.h.alloc(512));
   size_t o = G_ARR;
-  w.oH = o;
-  o += (size_t)(w.sD + 1) * w.sD;
-  w.ocs = o;
-  o += w.sD;
-  w.osn = o;
-  o += w.sD;
-  w.oerr = o;
-  o += w.sD + 1;
-  w.oy = o;
-  o += w.sD;
-  w.oA = o;
-  o += (size_t)w.nB * w.nB;
-  w.oBv = o;
-  o += w.nB;
-  w.oxB = o;
-  o += w.nB;
-  w.oC = o;
-  o += (size_t)w.nB * (w.nB + 1);
-  w.ocu = o;
-  o += w.mRI;
-  w.ocp = o;
-  o += w.mRI;
-  CR_TRY(w.gst.alloc(o));
-  CR_TRY(w.fcoef.alloc(std::max<size_t>(1, l->face.size())));
-  CR_TRY(w.dots.alloc(2048));
-  if (!l->gt_is_d) CR_TRY(gt_buf(l, T(0)).alloc((size_t)3 * l->nnz));
-  c.hfdev.clear();
-  for (size_t f = 0; f < l->face.size(); ++f) {
-    CrFace &fa = l->face[f];
-    if (!fa.coupled) continue;
-    CR_TRY(fa.d_valM.alloc((size_t)fa.dof * fa.nNo));
-    CR_TRY(face_support(l, fa));
-    c.hfdev.push_back(FaceDev{fa.d_glob.p, fa.d_valM.p, 0.0, w.fcoef.p + f, fa.res, fa.nNo, fa.dof, fa.d_sup.p,
-                              fa.d_q.p, fa.nsup});
+  auto place = [&](size_t &at, size_t n) {
+    at = o;
+    o += n;
+  };
+  if (ls->LS_type != CRIMSON_LS_CG) {
+    place(w.oH, (size_t)(w.sD + 1) * w.sD);
+    place(w.ocs, w.sD);
+    place(w.osn, w.sD);
+    place(w.oerr, w.sD + 1);
+    place(w.oy, w.sD);
+    const size_t nd = ns ? 3 : dof;
+    CR_TRY(w.wa.alloc(nd * N));
+    CR_TRY(w.wb.alloc(nd * N));
+    CR_TRY(w.ws.alloc((nd == 3 ? 4 : nd) * N));
+    CR_TRY(w.gmU.alloc(nd * N * w.sD));
   }
-  CR_TRY(face_list(c));
-  {
+  if (ns) {
+    place(w.oA, (size_t)w.nB * w.nB);
+    place(w.oBv, w.nB);
+    place(w.oxB, w.nB);
+    place(w.oC, (size_t)w.nB * (w.nB + 1));
+    place(w.ocu, w.mRI);
+    place(w.ocp, w.mRI);
+    CR_TRY(w.r.alloc(st));
+    CR_TRY(w.X.alloc(st * w.mRI));
+    CR_TRY(w.MX.alloc(st * w.nB));
+    if (!l->gt_is_d) CR_TRY(gt_buf(l, T(0)).alloc((size_t)3 * l->nnz));
     SchurOp<T> so;
     CR_TRY(schur_ready(l, so));
     w.formed = so.formed;
-  }
-  CR_TRY(w.msum.alloc(std::max<size_t>(1, c.hfdev.size())));
-  {
-    std::vector<char> seen(N, 0);
-    w.disjoint = true;
-    w.maxfn = 0;
-    for (auto &fa : l->face) {
-      if (!fa.coupled) continue;
-      w.maxfn = std::max(w.maxfn, fa.nNo);
-      for (int a = 0; a < fa.nNo; ++a) {
-        if (seen[fa.glob[a]]) w.disjoint = false;
-        seen[fa.glob[a]] = 1;
-      }
+    if (!w.formed) {
+      CR_TRY(w.ps.alloc(N));
+      CR_TRY(w.z.alloc((size_t)4 * N));
     }
+  } else {
+    CR_TRY(w.X.alloc(st));
   }
+  if (ls->LS_type != CRIMSON_LS_GMRES) {
+    const size_t n = ns ? N : st;
+    CR_TRY(w.t3.alloc(n));
+    CR_TRY(w.t4.alloc(n));
+    CR_TRY(w.t5.alloc(n));
+  }
+  const unsigned long long before = w.gst.serial;
+  CR_TRY(w.gst.alloc(o));
+  if (w.gst.serial != before) CR_HIP(hipMemsetAsync(w.gst.p, 0, o * sizeof(double), s));
+  CR_TRY(face_setup(c, incL, res, ns));
   CR_HIP(hipStreamSynchronize(s));
   return CRIMSON_OK;
 }
 
-// One memLS NS solve (solve_impl) enqueued device-driven on w.c.s: PRECOND,
-// R = W R, the solve, R W; d_Ri the FP64 (4, N) right-hand side in and
-// solution out.  No synchronisation, no allocation.
+// PRECOND (memLS.f90:1763-1943) as the W/fix vectors.
 template <class T>
-int ns_graph_enqueue(NsGraphWork<T> &w, double *d_Ri) {
-  Ctx<T> &c = w.c;
+int precond(Ctx<T> &c) {
   crimson_lhs *l = c.lhs;
-  const int N = l->nNo, dof = 4;
-  const size_t L = (size_t)dof * N;
+  const int N = c.N, dof = c.dof;
   const unsigned gN = crimson::grid_for(N, 256);
   const T *V = planes(l, T(0));
   precond_diag_kernel<T><<<gN, 256, 0, c.s>>>(N, dof, l->vdof, V, l->nnz, l->d_diag.p, c.W.p, c.fix.p);
@@ -2835,11 +2591,6 @@ int ns_graph_enqueue(NsGraphWork<T> &w, double *d_Ri) {
     if (fa.coupled && fa.nNo > 0)
       face_valm_kernel<T><<<crimson::grid_for(fa.nNo, 256), 256, 0, c.s>>>(fa.nNo, dof, fa.dof, fa.d_glob.p,
                                                                             fa.d_val.p, c.W.p, fa.d_valM.p);
-  T *R = sizeof(T) == sizeof(double) ? reinterpret_cast<T *>(d_Ri) : w.Rw.p;
-  mul_kernel<double, T, T><<<crimson::grid_for(L, 256), 256, 0, c.s>>>(L, d_Ri, c.W.p, R);
-  CR_HIP(hipGetLastError());
-  CR_TRY(nssolver_graph<T>(w, R));
-  mul_kernel<T, T, double><<<crimson::grid_for(L, 256), 256, 0, c.s>>>(L, R, c.W.p, d_Ri);  // R = R W
   CR_HIP(hipGetLastError());
   return CRIMSON_OK;
 }
@@ -2847,7 +2598,7 @@ int ns_graph_enqueue(NsGraphWork<T> &w, double *d_Ri) {
 // The solve's statistics from a copy of the first G_ARR entries of gst
 // into ls's fields (as nssolver_dev leaves them); CRIMSON_ESINGULAR when GE
 // met a singular pivot.
-int ns_graph_stats(const double *h, crimson_ls *ls) {
+int ns_stats(const double *h, crimson_ls *ls) {
   if (h[G_ERR] != 0.0) {
     crimson::set_error("memLS GE: singular matrix");
     return CRIMSON_ESINGULAR;
@@ -2876,6 +2627,156 @@ int ns_graph_stats(const double *h, crimson_ls *ls) {
   return CRIMSON_OK;
 }
 
+// GMRESV (memLS.f90:792-883) and CGRADV/CGRADS on the whole system: W R in
+// r0, the solution in X, out as W X.
+template <class T>
+int gmresv(SolveWork<T> &w, crimson_ls *ls) {
+  Ctx<T> &c = w.c;
+  const int dof = c.dof;
+  const MatView<T> A = view<T>(c, planes(c.lhs, T(0)), dof, 0, 0, dof, dof, c.W.p, c.fix.p, dof);
+  double *g = w.gst.p;
+  CR_HIP(hipMemsetAsync(g + G_GM_ITR, 0, sizeof(double), c.s));
+  CR_TRY(gmres_run(w, A, dof, w.r0.p, w.X.p, GmParams{ls->RI.mItr, w.sD, ls->RI.absTol, ls->RI.relTol, false, true},
+                   nullptr));
+  double h[G_ARR];
+  CR_HIP(hipMemcpyAsync(h, g, sizeof(h), hipMemcpyDeviceToHost, c.s));
+  CR_HIP(hipStreamSynchronize(c.s));
+  SubLs &r = ls->RI;
+  r.suc = h[G_GM_EARLY] == 0.0 && h[G_GM_SUC] != 0.0;
+  r.itr = h[G_GM_EARLY] != 0.0 ? 0 : (int)h[G_GM_ITR];
+  if (h[G_GM_EARLY] != 0.0) {
+    r.iNorm = r.fNorm = h[G_GM_E0];
+    r.callD = r.dB = 0.0;
+    return CRIMSON_OK;
+  }
+  r.iNorm = h[G_GM_INORM];
+  r.fNorm = h[G_GM_FNORM];
+  r.dB = 10.0 * std::log(h[G_GM_FNORM] / h[G_GM_DBPRE]);
+  return CRIMSON_OK;
+}
+template <class T>
+int cgradv(SolveWork<T> &w, crimson_ls *ls) {
+  Ctx<T> &c = w.c;
+  const int dof = c.dof;
+  const size_t L = (size_t)dof * c.N;
+  const MatView<T> A = view<T>(c, planes(c.lhs, T(0)), dof, 0, 0, dof, dof, c.W.p, c.fix.p, dof);
+  copy_kernel<T><<<crimson::grid_for(L, 256), 256, 0, c.s>>>(L, w.r0.p, w.X.p, nullptr);
+  auto op = [&](const T *Pv, T *SPv, const double *done, int &nd) -> int {
+    CR_TRY(spmv<T>(c, A, dof, dof, Pv, SPv, 1.0, static_cast<const T *>(nullptr), 0.0, done));
+    return cg_den(c, L, Pv, SPv, done, nd);
+  };
+  double *state = nullptr;
+  SubLs &r = ls->RI;
+  CR_TRY(cg_run(w, L, w.X.p, op, w.t3.p, w.t4.p, w.t5.p, w.r0.p, CgAux<T>(), r.absTol, r.relTol, r.mItr,
+                static_cast<double *>(nullptr), static_cast<const double *>(nullptr), &state));
+  double h[kCgState];
+  CR_HIP(hipMemcpyAsync(h, state, sizeof(h), hipMemcpyDeviceToHost, c.s));
+  CR_HIP(hipStreamSynchronize(c.s));
+  r.iNorm = h[9];
+  r.suc = h[8] != 0.0;
+  r.fNorm = std::sqrt(h[0]);
+  r.dB = 5.0 * std::log(h[0] / h[1]);
+  r.itr = (int)h[6];
+  return CRIMSON_OK;
+}
+
+// The workspace of a plain solve stays with the matrix handle: allocating and
+// freeing it took 5 to 7 ms a solve, a third of the reference case's.  Kept
+// while the process keeps at most kKeepBytes of them (a larger one is freed after its
+// solve, where the solve is long); a solve takes it out, so that a second
+// solve of the handle at the same time has one of its own; given back with the
+// handle, or when an allocation fails (release_idle_work).
+constexpr size_t kKeepBytes = (size_t)8 << 30;
+template <class T>
+std::unique_ptr<SolveWork<T>> take_work(crimson_lhs *l) {
+  std::unique_ptr<crimson::SolveWorkBase> w = crimson::work_take(l, sizeof(T) == 4);
+  if (w) return std::unique_ptr<SolveWork<T>>(static_cast<SolveWork<T> *>(w.release()));
+  return std::make_unique<SolveWork<T>>();
+}
+
+// One memLS_SOLVE in arithmetic type T.  d_Ri is the FP64 (dof,N) right-hand
+// side in and solution out; for T = float the solve runs on an FP32 copy.
+template <class T>
+int solve_run(SolveWork<T> &w, crimson_lhs *l, crimson_ls *ls, int dof, double *d_Ri, const int *incL,
+              const double *res) {
+  Ctx<T> &c = w.c;
+  const double t0 = now_s();
+  CR_TRY(work_setup(w, l, ls, dof, incL, res, l->stream));
+  CR_TRY(w.poll_ready());
+  w.tGM = w.tCG = 0.0;
+  CR_TRY(precond(c));
+  if (ls->LS_type == CRIMSON_LS_NS) {
+    CR_TRY(ns_run(w, d_Ri));
+    double h[G_ARR];
+    CR_HIP(hipMemcpyAsync(h, w.gst.p, sizeof(h), hipMemcpyDeviceToHost, c.s));
+    CR_HIP(hipStreamSynchronize(c.s));
+    CR_TRY(ns_stats(h, ls));
+    ls->RI.callD = now_s() - t0;
+    ls->GM.callD = w.tGM;
+    ls->CG.callD = w.tCG;
+    return CRIMSON_OK;
+  }
+  const size_t L = (size_t)dof * c.N;
+  mul_kernel<double, T, T><<<crimson::grid_for(L, 256), 256, 0, c.s>>>(L, d_Ri, c.W.p, w.r0.p);
+  CR_HIP(hipGetLastError());
+  if (ls->LS_type == CRIMSON_LS_GMRES)
+    CR_TRY(gmresv(w, ls));
+  else
+    CR_TRY(cgradv(w, ls));
+  if (ls->LS_type == CRIMSON_LS_CG || ls->RI.itr > 0) ls->RI.callD = now_s() - t0;
+  mul_kernel<T, T, double><<<crimson::grid_for(L, 256), 256, 0, c.s>>>(L, w.X.p, c.W.p, d_Ri);
+  CR_HIP(hipGetLastError());
+  CR_HIP(hipStreamSynchronize(c.s));
+  return CRIMSON_OK;
+}
+template <class T>
+int solve_impl(crimson_lhs *l, crimson_ls *ls, int dof, double *d_Ri, const int *incL, const double *res) {
+  std::unique_ptr<SolveWork<T>> w = take_work<T>(l);
+  const int rc = solve_run(*w, l, ls, dof, d_Ri, incL, res);
+  if (rc) {
+    (void)hipStreamSynchronize(l->stream);  // nothing of the workspace is in use when it goes
+    return rc;
+  }
+  crimson::work_keep(l, sizeof(T) == 4, std::move(w), kKeepBytes);
+  return CRIMSON_OK;
+}
+
+int solve_dev(crimson_lhs *l, crimson_ls *ls, int dof, double *d_Ri, const int *incL, const double *res) {
+  if (l->vdof != dof || !(l->prec == 32 ? (const void *)l->d_V32.p : (const void *)l->d_V.p)) {
+    crimson::set_error("lhs holds no matrix of block size %d (stored: %d)", dof, l->vdof);
+    return CRIMSON_ESTATE;
+  }
+  if (ls->LS_type == CRIMSON_LS_NS && dof != 4) {
+    crimson::set_error("LS_TYPE_NS needs dof = 4 (got %d)", dof);
+    return CRIMSON_EUNSUPPORTED;
+  }
+  if (l->prec == 32) return solve_impl<float>(l, ls, dof, d_Ri, incL, res);
+  return solve_impl<double>(l, ls, dof, d_Ri, incL, res);
+}
+
+// The device-driven solve of a capture: the limits it can enqueue, then its
+// set-up (all allocations and uploads) and its launches.
+template <class T>
+int ns_graph_setup(SolveWork<T> &w, crimson_lhs *l, crimson_ls *ls, const int *incL, const double *res,
+                   hipStream_t s) {
+  if (ls->LS_type != CRIMSON_LS_NS) {
+    crimson::set_error("the device-driven solve is the NS solver's (LS_TYPE_NS)");
+    return CRIMSON_EUNSUPPORTED;
+  }
+  if (ls->RI.mItr < 1 || ls->GM.mItr < 1 || ls->CG.mItr < 1 || ls->GM.sD < 1 || 2 * ls->RI.mItr > 255 ||
+      ls->GM.sD > 255) {
+    crimson::set_error("device-driven NS solve: iteration limits out of range (RI %d, GM %d x %d, CG %d)",
+                       ls->RI.mItr, ls->GM.mItr, ls->GM.sD, ls->CG.mItr);
+    return CRIMSON_EARG;
+  }
+  return work_setup(w, l, ls, 4, incL, res, s);
+}
+template <class T>
+int ns_graph_enqueue(SolveWork<T> &w, double *d_Ri) {
+  CR_TRY(precond(w.c));
+  return ns_run(w, d_Ri);
+}
+
 // The signature of what a device-driven solve baked in: the matrix and
 // face buffers it reads and the solver's settings.
 std::vector<unsigned long long> ns_signature(const crimson_lhs *l, const crimson_ls *ls) {
@@ -2883,7 +2784,8 @@ std::vector<unsigned long long> ns_signature(const crimson_lhs *l, const crimson
                                        (unsigned long long)l->vdof, (unsigned long long)l->prec,
                                        (unsigned long long)l->gt_is_d, (unsigned long long)ls->RI.mItr,
                                        (unsigned long long)ls->GM.mItr, (unsigned long long)ls->GM.sD,
-                                       (unsigned long long)ls->CG.mItr};
+                                       (unsigned long long)ls->CG.mItr, l->d_S.serial, l->d_S32.serial,
+                                       l->d_sptr.serial, l->d_fent.serial, l->d_ftptr.serial};
   for (const auto &fa : l->face) {
     v.push_back(fa.d_glob.serial);
     v.push_back(fa.d_val.serial);
@@ -2899,18 +2801,17 @@ std::vector<unsigned long long> ns_signature(const crimson_lhs *l, const crimson
 // each captured solve's statistics (the last one's into ls).
 template <class T>
 struct NsGraphExtra : crimson::GraphExtra {
-  NsGraphWork<T> w;
+  SolveWork<T> w;
   crimson_lhs *lhs = nullptr;
   crimson_ls *ls = nullptr;
   int nsolve = 0;
   crimson::DBuf<double> stat;  // G_ARR doubles per captured solve
   std::vector<double> hstat;
-  std::vector<unsigned long long> form_sig_unused;
   int after_launch() override {
     hstat.resize((size_t)G_ARR * nsolve);
     CR_HIP(hipMemcpy(hstat.data(), stat.p, hstat.size() * sizeof(double), hipMemcpyDeviceToHost));
     int rc = CRIMSON_OK;
-    for (int k = 0; k < nsolve && rc == CRIMSON_OK; ++k) rc = ns_graph_stats(hstat.data() + (size_t)G_ARR * k, ls);
+    for (int k = 0; k < nsolve && rc == CRIMSON_OK; ++k) rc = ns_stats(hstat.data() + (size_t)G_ARR * k, ls);
     return rc;
   }
   std::vector<unsigned long long> signature() const override { return ns_signature(lhs, ls); }
@@ -3104,6 +3005,7 @@ extern "C" int crimson_lhs_free(crimson_lhs *l) {
   if (l->ev0) (void)hipEventDestroy(l->ev0);
   if (l->ev1) (void)hipEventDestroy(l->ev1);
   hipStream_t s = l->stream;
+  crimson::work_forget(l);
   delete l;
   if (s) (void)hipStreamDestroy(s);
   return CRIMSON_OK;
@@ -3302,7 +3204,7 @@ namespace {
 template <class T>
 int spmv_timed(crimson_lhs *l, int dof, const T *x, T *y, int reps, double *ms) {
   Ctx<T> c;
-  CR_TRY(c.init(l, 4));
+  CR_TRY(c.init(l, 4, l->stream));
   const unsigned gN = crimson::grid_for(l->nNo, 256);
   const T *V = planes(l, T(0));
   precond_diag_kernel<T><<<gN, 256, 0, c.s>>>(l->nNo, 4, 4, V, l->nnz, l->d_diag.p, c.W.p, c.fix.p);
@@ -3417,16 +3319,13 @@ int check_segment_budget(int mGM, int sD, int mCG, int nfc_launch) {
   return CRIMSON_OK;
 }
 
-template <class T>
-int NsGraphWork<T>::cut() {
-  return cap ? cap->cut() : CRIMSON_OK;
-}
+int seg_cut(SegCapture *cap) { return cap ? cap->cut() : CRIMSON_OK; }
 
 template <class T>
-int capture_into(crimson_graph *g, hipStream_t s, NsGraphWork<T> &w, const std::function<int()> &body) {
+int capture_into(crimson_graph *g, hipStream_t s, SolveWork<T> &w, const std::function<int()> &body) {
   SegCapture cap{g, s};
-  const int nfc = (int)w.c.hfdev.size();
-  CR_TRY(check_segment_budget(w.mGM, w.sD, w.mCG, (w.disjoint && nfc > 1) ? 1 : nfc));
+  const int nfc = w.c.nfc();
+  CR_TRY(check_segment_budget(w.mGM, w.sD, w.mCG, (w.c.disjoint && nfc > 1) ? 1 : nfc));
   CR_TRY(cap.begin());
   w.cap = &cap;
   int rc = body();
