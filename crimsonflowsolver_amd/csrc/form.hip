@@ -5,16 +5,16 @@
 //   node_pack   node-parallel: x and u packed as 6 doubles per node
 //   flux_node   node-parallel gather over the node's elements in element
 //               order, each incidence evaluating its element's metric and
-//               viscous flux q_dI (e3q.f90:100-145) from the packed nodes:
-//               qres, rmass, q = qres * (1/rmass)  (asiq.f90 + qpbc.f90);
-//               writes one 128-byte node record (x, u, p, ac, q)
+//               viscous flux q_dI (e3q.f90:100-145) from the row's packed
+//               nodes, staged once per row in LDS: qres, rmass, q = qres *
+//               (1/rmass)  (asiq.f90 + qpbc.f90); writes one 128-byte node
+//               record (x, u, p, ac, q)
 //   e3_elem     element-parallel e3 (e3.f90 .. e3lhs.f90) on the four node
-//               records: all four quadrature points in registers; writes a
-//               12-double record per element incidence (e, a) at the
-//               incidence's place in the node-major incidence list: node
-//               a's row S_a. of the scalar part of the 3x3 velocity blocks,
-//               its residual row rl_a, and the element scalars Tc, Mu, Cm,
-//               tlW from which every tangent entry is rebuilt
+//               records: all four quadrature points in registers; writes per
+//               element and node a the row S_a. of the scalar part of the 3x3
+//               velocity blocks and the residual row rl_a, and the element
+//               scalars Tc, Mu, Cm, tlW from which every tangent entry is
+//               rebuilt (the residual rows alone without the tangent)
 //   asm_row     row-parallel, 16 lanes per CSR row, one lane per block: the
 //               row's incidence records read as one contiguous run, the
 //               shape gradients rebuilt from the packed nodes, the blocks of
@@ -51,6 +51,14 @@
 
 namespace {
 
+// Orders LDS accesses of the lanes of one wavefront (the lanes of a node or
+// CSR row always share a wavefront).
+__device__ inline void wave_lds_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 // ---------------------------------------------------------------- flux pass
 // x and u of every node packed as kXU doubles: the flux pass gathers a
 // node's x and u in three 16-byte loads, the assembly its x in two loads.
@@ -65,37 +73,47 @@ __global__ void __launch_bounds__(256) node_pack(int nshg, const double *__restr
   o[2] = make_double2(y[i + N], y[i + 2 * N]);
 }
 
-// The coordinates of an element's four nodes (local order) from the packed
-// nodes.
-__device__ inline void gather_x(const double *__restrict__ xu, int4 n4, double (&xl)[4][3]) {
-  const int nd[4] = {n4.x, n4.y, n4.z, n4.w};
+// The x and u of a row's neighbours staged in LDS: kFluxCap of the row's
+// blocks per node, kXU doubles each; later blocks are read from memory.  A row's
+// 24 incidences name its 14 neighbours 72 times; gathered per incidence, the
+// address units were busy 96 % of flux_node's time.  1.3 M nodes (64 x 64 x 320
+// Kuhn cells), node_pack included: 353 us gathered, 295 staged.  (The assembly
+// gathers: it is bound by its sums, and its rows staged this way took 1,600 us
+// instead of 1,535.)
+constexpr int kFluxLanes = 8, kFluxCap = 20;
+// LANES lanes load the row's first CAP blocks' x and u, three 16-byte pieces each.
+template <int LANES, int CAP>
+__device__ inline void stage_row_xu(int lane, int k0, int n, const int *__restrict__ col,
+                                    const double *__restrict__ xu, double *sh) {
+  constexpr int kU = (CAP * 3 + LANES - 1) / LANES;
+  const int m = min(n, CAP) * 3;
+  double2 v[kU];
 #pragma unroll
-  for (int a = 0; a < 4; ++a) {
-    const double *r = xu + (size_t)nd[a] * kXU;
-    const double2 v = *reinterpret_cast<const double2 *>(r);
-    xl[a][0] = v.x;
-    xl[a][1] = v.y;
-    xl[a][2] = r[2];
+  for (int u = 0; u < kU; ++u) {
+    const int i = min(lane + LANES * u, m - 1);  // a row has its diagonal block at least
+    v[u] = reinterpret_cast<const double2 *>(xu + (size_t)col[k0 + i / 3] * kXU)[i % 3];
   }
+#pragma unroll
+  for (int u = 0; u < kU; ++u) {
+    const int i = lane + LANES * u;
+    if (i < m) reinterpret_cast<double2 *>(sh)[i] = v[u];
+  }
+}
+
+__device__ inline void load_xu(const double *p, double (&x)[3], double (&u)[3]) {
+  const double2 *r = reinterpret_cast<const double2 *>(p);
+  x[0] = r[0].x;
+  x[1] = r[0].y;
+  x[2] = r[1].x;
+  u[0] = r[1].y;
+  u[1] = r[2].x;
+  u[2] = r[2].y;
 }
 
 // e3q for one element (e3q.f90:66-145): qdi = mu (grad u + grad u^T) is the
 // same at every quadrature point of a P1 element.  Returns WdetJ; qd holds
 // the 6 distinct components in slots (11,12,13,22,23,33).
-__device__ inline double elem_flux(const double *__restrict__ xu, int4 n4, double mu, double (&qd)[6]) {
-  const int nd[4] = {n4.x, n4.y, n4.z, n4.w};
-  double xl[4][3], ul[4][3];
-#pragma unroll
-  for (int a = 0; a < 4; ++a) {
-    const double2 *r = reinterpret_cast<const double2 *>(xu + (size_t)nd[a] * kXU);
-    const double2 v0 = r[0], v1 = r[1], v2 = r[2];
-    xl[a][0] = v0.x;
-    xl[a][1] = v0.y;
-    xl[a][2] = v1.x;
-    ul[a][0] = v1.y;
-    ul[a][1] = v2.x;
-    ul[a][2] = v2.y;
-  }
+__device__ inline double elem_flux(const double (&xl)[4][3], const double (&ul)[4][3], double mu, double (&qd)[6]) {
   double dx[3][3], W, g[4][3];
   p1_metric(xl, dx, W, g);
   double gu[3][3];  // gu[j][i] = d u_i / d x_j
@@ -114,69 +132,83 @@ __device__ inline double elem_flux(const double *__restrict__ xu, int4 n4, doubl
 }
 
 // qres/rmass gather and qpbc inversion (asiq.f90, qpbc.f90): each of the
-// node's incidences (in element order, kNodeLanes lanes) evaluates its
-// element's flux from the packed nodes; nothing per element is stored.
+// node's incidences (in element order, kFluxLanes lanes) evaluates its
+// element's flux from the neighbours' x and u; nothing per element is stored.
 // q(nshg,9) column-major in the reference's component order: (1,4,7) =
 // (q11,q12,q13), ... so component k = i + 3 (j-1) holds mu(du_i/dx_j +
 // du_j/dx_i).  Writes the node record (with the node's x, y, ac) and, when q
 // is not null, q(nshg,9).
-__global__ void __launch_bounds__(256) flux_node(int nshg, const int *__restrict__ inc_ptr,
-                                                 const int *__restrict__ inc, const int4 *__restrict__ ienp,
-                                                 const double *__restrict__ xu, double mu0, Ens en,
-                                                 const double *__restrict__ x, int numnp,
-                                                 const double *__restrict__ y, const double *__restrict__ ac,
-                                                 double *__restrict__ node, double *__restrict__ q,
-                                                 double *__restrict__ invm) {
+template <class IL>
+__global__ void __launch_bounds__(256) flux_node(int nshg, const int *__restrict__ rowptr,
+                                                 const int *__restrict__ diagk, const int *__restrict__ col,
+                                                 const int *__restrict__ inc_ptr, const int *__restrict__ inc,
+                                                 const IL *__restrict__ iloc, const double *__restrict__ xu,
+                                                 double mu0, Ens en, const double *__restrict__ y,
+                                                 const double *__restrict__ ac, double *__restrict__ node,
+                                                 double *__restrict__ q, double *__restrict__ invm) {
+  __shared__ double xs_all[256 / kFluxLanes][kFluxCap * kXU];
   const int gid = xcd_block() * blockDim.x + threadIdx.x;
-  const int i = gid / kNodeLanes, lane = gid % kNodeLanes;
+  const int i = gid / kFluxLanes, lane = gid % kFluxLanes;
+  const bool live = i < nshg;
+  const int ii = live ? i : nshg - 1;
+  const int k0 = rowptr[ii], ns = rowptr[ii + 1] - k0, d = diagk[ii] - k0;
+  const int p0 = inc_ptr[ii], p1 = live ? inc_ptr[ii + 1] : p0;
+  double *xs = xs_all[threadIdx.x / kFluxLanes];
+  const size_t N = nshg;
+  // the lane's share of the rest of the node's record: p, ac
+  double rest = 0.0;
+  if (lane < 4) rest = lane == 0 ? y[ii + 3 * N] : ac[ii + (lane - 1) * N];
+  IL il = p0 + lane < p1 ? iloc[p0 + lane] : IL(0);
+  stage_row_xu<kFluxLanes, kFluxCap>(lane, k0, ns, col, xu, xs);
+  wave_lds_sync();
+  auto get = [&](int s, double (&x)[3], double (&u)[3]) {
+    // (an either-or would become one flat load of both kinds of memory)
+    load_xu(xs + kXU * min(s, kFluxCap - 1), x, u);
+    if (s >= kFluxCap) load_xu(xu + (size_t)col[k0 + s] * kXU, x, u);
+  };
   double s[6] = {0, 0, 0, 0, 0, 0}, rm = 0.0;
-  if (i < nshg) {
-    for (int p = inc_ptr[i] + lane; p < inc_ptr[i + 1]; p += kNodeLanes) {
-      const int ea = inc[p];
-      double qd[6];
-      const double m = flux_weight(elem_flux(xu, ienp[p], ens_mu(en, ea >> 2, mu0), qd), ea & 3);
+  for (int p = p0 + lane; p < p1; p += kFluxLanes) {
+    const IL iln = p + kFluxLanes < p1 ? iloc[p + kFluxLanes] : IL(0);
+    int sl[4];
+    IncLoc<IL>::places(il, d, sl);
+    double xl[4][3], ul[4][3];
 #pragma unroll
-      for (int k = 0; k < 6; ++k) s[k] += m * qd[k];
-      rm += m;
-    }
+    for (int a = 0; a < 4; ++a) get(sl[a], xl[a], ul[a]);
+    double qd[6];
+    const double mu = en.inst ? ens_mu(en, inc[p] >> 2, mu0) : mu0;
+    const double m = flux_weight(elem_flux(xl, ul, mu, qd), IncLoc<IL>::a(il));
+#pragma unroll
+    for (int k = 0; k < 6; ++k) s[k] += m * qd[k];
+    rm += m;
+    il = iln;
   }
-  // fixed-order reduction over the node's lanes: (0+1)+(2+3)
+  // fixed-order reduction over the node's lanes: ((0+1)+(2+3))+((4+5)+(6+7))
 #pragma unroll
-  for (int off = 1; off < kNodeLanes; off <<= 1) {
+  for (int off = 1; off < kFluxLanes; off <<= 1) {
 #pragma unroll
-    for (int k = 0; k < 6; ++k) s[k] += __shfl_xor(s[k], off, kNodeLanes);
-    rm += __shfl_xor(rm, off, kNodeLanes);
+    for (int k = 0; k < 6; ++k) s[k] += __shfl_xor(s[k], off, kFluxLanes);
+    rm += __shfl_xor(rm, off, kFluxLanes);
   }
-  if (i >= nshg) return;
+  // the record in order: x u | p ac | q, two doubles per lane
+  double xo[3], uo[3];
+  get(d, xo, uo);
+  const double r0 = __shfl(rest, 0, kFluxLanes), r1 = __shfl(rest, 1, kFluxLanes), r2 = __shfl(rest, 2, kFluxLanes),
+               r3 = __shfl(rest, 3, kFluxLanes);
+  if (!live) return;
   const double inv = 1.0 / rm;
-  const size_t N = nshg, NP = numnp;
   if (invm && lane == 0) invm[i] = inv;
-  // the node's record, four doubles per lane
-  double v[4];
-  if (lane == 0) {
-    v[0] = x[i];
-    v[1] = x[i + NP];
-    v[2] = x[i + 2 * NP];
-    v[3] = y[i];
-  } else if (lane == 1) {
-    v[0] = y[i + N];
-    v[1] = y[i + 2 * N];
-    v[2] = y[i + 3 * N];
-    v[3] = ac[i];
-  } else if (lane == 2) {
-    v[0] = ac[i + N];
-    v[1] = ac[i + 2 * N];
-    v[2] = inv * s[0];
-    v[3] = inv * s[1];
-  } else {
-    v[0] = inv * s[2];
-    v[1] = inv * s[3];
-    v[2] = inv * s[4];
-    v[3] = inv * s[5];
+  double2 v;
+  switch (lane) {
+    case 0: v = make_double2(xo[0], xo[1]); break;
+    case 1: v = make_double2(xo[2], uo[0]); break;
+    case 2: v = make_double2(uo[1], uo[2]); break;
+    case 3: v = make_double2(r0, r1); break;
+    case 4: v = make_double2(r2, r3); break;
+    case 5: v = make_double2(inv * s[0], inv * s[1]); break;
+    case 6: v = make_double2(inv * s[2], inv * s[3]); break;
+    default: v = make_double2(inv * s[4], inv * s[5]); break;
   }
-  double2 *nr = reinterpret_cast<double2 *>(node + (size_t)i * kNRec + 4 * lane);
-  nr[0] = make_double2(v[0], v[1]);
-  nr[1] = make_double2(v[2], v[3]);
+  reinterpret_cast<double2 *>(node + (size_t)i * kNRec)[lane] = v;
   if (!q || lane != 0) return;
   q[i + 0 * N] = inv * s[0];
   q[i + 1 * N] = inv * s[1];
@@ -190,221 +222,277 @@ __global__ void __launch_bounds__(256) flux_node(int nshg, const int *__restrict
 }
 
 // ---------------------------------------------------------------- e3
-// With the tangent, the element records of the workgroup's (consecutive)
-// elements are assembled in LDS and stored as one contiguous block with
-// coalesced 16-byte stores (written directly, each thread's 256-byte record
-// reached HBM as partially filled lines); the scalars (32 bytes per element)
-// are stored directly, contiguous across the threads.
-constexpr int kE3Threads = 128;
-// LDS stride of a staged record: one double more than the record, so that
-// the threads' stores at the same offset fall in different banks.
-constexpr int kE3Pad = kRec + 1;
-template <bool LHS>
-__global__ void __launch_bounds__(kE3Threads) __attribute__((amdgpu_waves_per_eu(2))) e3_elem(int nel, const int *__restrict__ ien,
-                                                      const double *__restrict__ node, FormConst c0, Ens en,
-                                                      double *__restrict__ rec, double *__restrict__ esc) {
-  __shared__ double sh_rec[LHS ? kE3Threads * kE3Pad : 1];
-  const int e0 = xcd_block() * kE3Threads;
-  const int e = e0 + threadIdx.x;
-  if (!LHS && e >= nel) return;
-  const int ee = e < nel ? e : nel - 1;  // tail threads evaluate a valid element; nothing of theirs is stored
-  FormConst c = c0;
-  c.mu = ens_mu(en, ee, c0.mu);
-  int nd[4];
-#pragma unroll
-  for (int a = 0; a < 4; ++a) nd[a] = ien[a * (size_t)nel + ee];
-  // the four node records (localx/localy gathers, localy.f90:54-64)
-  double nl[4][kNRec];
-#pragma unroll
-  for (int a = 0; a < 4; ++a) {
-    const double2 *r = reinterpret_cast<const double2 *>(node + (size_t)nd[a] * kNRec);
-#pragma unroll
-    for (int k = 0; k < kNRec / 2; ++k) {
-      const double2 v = r[k];
-      nl[a][2 * k] = v.x;
-      nl[a][2 * k + 1] = v.y;
-    }
-  }
-
-  double g[4][3], W, gg[6];
+// The element sums of e3 (e3.f90 .. e3lhs.f90) over the four quadrature points,
+// from which the residual rows and the tangent's S rows follow.  What does not
+// vary over a P1 element is kept out of the loop: with
+//   A = sum tauM u u^T, B = sum tauBar L L^T, C = sum tauM L u^T
+// the flux sum of the residual is C + (grad u) B + 4 mu (grad u + grad u^T) +
+// (div u sum tauC - sum p) I, the SUPG and tauBar parts of S are rho tlW g_a.(A +
+// B / rho) g_b, and the rule's weights (nq: one at the point's own node, another
+// at the rest) make every nodal sum sum_q N_a(q) f_q = w_other(a) sum f +
+// (w_own(a) - w_other(a)) f_a.  tauM and tauBar take a reciprocal square root each.  Written
+// term by term per point (the form of e3res.f90 and e3lhs.f90) the kernel issued
+// 1,763 vector instructions per wave, this 1,117; it is bound by latency at two
+// waves a SIMD and by the record stores (1.8 GB at 7.9 M elements: 672 us before,
+// 557 now; without the tangent 663 before, 411 now).
+// In: the nodal values.  Out: u -> ubar at the points, a -> (a + ubar . grad u) at
+// the points (RES), g of the first three nodes (g_4 is minus their sum), WdetJ.
+__host__ __device__ constexpr double w_other(int a) { return nq(a == 0 ? 1 : 0, a); }
+__host__ __device__ constexpr double w_diff(int a) { return nq(a, a) - w_other(a); }
+template <class T, bool RES, bool TAN>
+struct E3Sums {
+  T g[3][3], W, gu[3][3], SU[3], SR[3], A[6], B[6], C[3][3], TC, TM, divu;
+};
+constexpr int kSym[3][3] = {{0, 1, 2}, {1, 3, 4}, {2, 4, 5}};  // symmetric 3x3: 00 01 02 11 12 22
+__device__ inline double rsq(double x) { return rsqrt(x); }
+__device__ inline float rsq(float x) { return 1.0f / sqrtf(x); }
+template <class T, bool RES, bool TAN>
+__device__ inline void e3_sums(const FormConst &c, const T (&xl)[4][3], const T (&pl)[4], const T (&ql)[4][6],
+                               T (&ul)[4][3], T (&al)[4][3], E3Sums<T, RES, TAN> &o) {
+  T gg[6], gpd[3];
   {
-    double xl[4][3], dx[3][3];
+    T dx[3][3], g4[4][3];
+    p1_metric(xl, dx, o.W, g4);
+    gijd_tet(dx, gg);
+    // gradients (e3ivar.f90:180-198) and the divergence of the reconstructed
+    // flux (e3ivar.f90:355-367)
+#pragma unroll
+    for (int j = 0; j < 3; ++j) {
+#pragma unroll
+      for (int i = 0; i < 3; ++i)
+        o.gu[j][i] = g4[0][j] * ul[0][i] + g4[1][j] * ul[1][i] + g4[2][j] * ul[2][i] + g4[3][j] * ul[3][i];
+      gpd[j] = g4[0][j] * pl[0] + g4[1][j] * pl[1] + g4[2][j] * pl[2] + g4[3][j] * pl[3];
+    }
 #pragma unroll
     for (int a = 0; a < 4; ++a)
 #pragma unroll
-      for (int i = 0; i < 3; ++i) xl[a][i] = nl[a][N_X + i];
-    p1_metric(xl, dx, W, g);
-    gijd_tet(dx, gg);
+      for (int i = 0; i < 3; ++i)
+        gpd[i] -= g4[a][0] * ql[a][qsym(i)] + g4[a][1] * ql[a][qsym(i + 3)] + g4[a][2] * ql[a][qsym(i + 6)];
+#pragma unroll
+    for (int a = 0; a < 3; ++a)
+#pragma unroll
+      for (int j = 0; j < 3; ++j) o.g[a][j] = g4[a][j];
   }
-  // nodal velocity and pressure; gradients (e3ivar.f90:180-198)
-  double ul[4][3], pl[4];
+  const T rho = T(c.rho), rhoinv = T(1) / rho, rnu = T(c.mu) * rhoinv;
+  const T dts = T(c.Dtgl * c.dtsfct);
+  const T GG = gg[0] * gg[0] + gg[1] * gg[1] + gg[2] * gg[2] + T(2) * (gg[3] * gg[3] + gg[4] * gg[4] + gg[5] * gg[5]);
+  // tau, itau = 0 (e3stab.f90:108-133); fff = 36 for ipord = 1
+  const T tau0 = (T(2) * dts) * (T(2) * dts) + T(36) * (rnu * rnu) * GG;
+  T us[3], as[3];
 #pragma unroll
-  for (int a = 0; a < 4; ++a) {
+  for (int i = 0; i < 3; ++i) {
+    us[i] = T(w_other(0)) * (ul[0][i] + ul[1][i] + ul[2][i]) + T(w_other(3)) * ul[3][i];
+    as[i] = T(w_other(0)) * (al[0][i] + al[1][i] + al[2][i]) + T(w_other(3)) * al[3][i];
+    o.SU[i] = o.SR[i] = T(0);
 #pragma unroll
-    for (int i = 0; i < 3; ++i) ul[a][i] = nl[a][N_U + i];
-    pl[a] = nl[a][N_P];
+    for (int j = 0; j < 3; ++j) o.C[i][j] = T(0);
   }
-  double gu[3][3], gp[3];  // gu[j][i] = du_i/dx_j
 #pragma unroll
-  for (int j = 0; j < 3; ++j) {
+  for (int k = 0; k < 6; ++k) o.A[k] = o.B[k] = T(0);
+  T sf = T(0);
+  o.TM = T(0);
 #pragma unroll
-    for (int i = 0; i < 3; ++i)
-      gu[j][i] = g[0][j] * ul[0][i] + g[1][j] * ul[1][i] + g[2][j] * ul[2][i] + g[3][j] * ul[3][i];
-    gp[j] = g[0][j] * pl[0] + g[1][j] * pl[1] + g[2][j] * pl[2] + g[3][j] * pl[3];
-  }
-  // divergence of the reconstructed flux (e3ivar.f90:355-367)
-  double divq[3] = {0.0, 0.0, 0.0};
-#pragma unroll
-  for (int a = 0; a < 4; ++a) {
-    double qa[9];
-#pragma unroll
-    for (int k = 0; k < 9; ++k) qa[k] = nl[a][N_Q + qsym(k)];
-#pragma unroll
-    for (int i = 0; i < 3; ++i) divq[i] += g[a][0] * qa[i] + g[a][1] * qa[i + 3] + g[a][2] * qa[i + 6];
-  }
-  double al[4][3];
-#pragma unroll
-  for (int a = 0; a < 4; ++a)
-#pragma unroll
-    for (int i = 0; i < 3; ++i) al[a][i] = nl[a][N_A + i];
-
-  const double rho = c.rho, mu = c.mu, rhoinv = 1.0 / rho;
-  const double rnu = mu * rhoinv;
-  const double dts = c.Dtgl * c.dtsfct;
-  const double GG = gg[0] * gg[0] + gg[1] * gg[1] + gg[2] * gg[2] +
-                    2.0 * (gg[3] * gg[3] + gg[4] * gg[4] + gg[5] * gg[5]);
-  const double tau0 = (2.0 * dts) * (2.0 * dts);
-  const double visc = 36.0 * (rnu * rnu) * GG;  // fff = 36 for ipord = 1
-  const double trg = gg[0] + gg[1] + gg[2];
-  const double divu = gu[0][0] + gu[1][1] + gu[2][2];
-  const double ff = c.taucfct / c.dtsfct;
-
-  double RNa[4][3], RGN[3][3], SU[3] = {0, 0, 0}, TC = 0.0, TM = 0.0, SUPG[10], UB[4][3];
-#pragma unroll
-  for (int a = 0; a < 4; ++a)
+  for (int q = 0; q < 4; ++q) {
+    T u[3], aq[3], L[3];
 #pragma unroll
     for (int i = 0; i < 3; ++i) {
-      RNa[a][i] = 0.0;
-      UB[a][i] = 0.0;
+      u[i] = us[i] + T(w_diff(q)) * ul[q][i];
+      aq[i] = as[i] + T(w_diff(q)) * al[q][i];
     }
-#pragma unroll
-  for (int i = 0; i < 3; ++i)
-#pragma unroll
-    for (int j = 0; j < 3; ++j) RGN[i][j] = 0.0;
-#pragma unroll
-  for (int k = 0; k < 10; ++k) SUPG[k] = 0.0;
-
-#pragma unroll
-  for (int qp = 0; qp < 4; ++qp) {
-    const double N0 = nq(qp, 0), N1 = nq(qp, 1), N2 = nq(qp, 2), N3 = nq(qp, 3);
-    double u[3], aq[3];
-#pragma unroll
-    for (int i = 0; i < 3; ++i) {
-      u[i] = N0 * ul[0][i] + N1 * ul[1][i] + N2 * ul[2][i] + N3 * ul[3][i];
-      aq[i] = N0 * al[0][i] + N1 * al[1][i] + N2 * al[2][i] + N3 * al[3][i];
-    }
-    const double pq = N0 * pl[0] + N1 * pl[1] + N2 * pl[2] + N3 * pl[3];
     // strong residual (e3res.f90:775-789)
-    double rL[3];
 #pragma unroll
     for (int i = 0; i < 3; ++i)
-      rL[i] = (aq[i] + u[0] * gu[0][i] + u[1] * gu[1][i] + u[2] * gu[2][i]) * rho + gp[i] - divq[i];
-    // tau, itau = 0 (e3stab.f90:108-133)
-    const double uGu = u[0] * (gg[0] * u[0] + gg[3] * u[1] + gg[5] * u[2]) +
-                       u[1] * (gg[3] * u[0] + gg[1] * u[1] + gg[4] * u[2]) +
-                       u[2] * (gg[5] * u[0] + gg[4] * u[1] + gg[2] * u[2]);
-    const double fact = sqrt((tau0 + uGu) + visc);
-    const double tauC = rho * 0.125 * fact / trg * ff;
-    const double tauM = 1.0 / fact;
-    double tauBar = rL[0] * (gg[0] * rL[0] + gg[3] * rL[1] + gg[5] * rL[2]) +
-                    rL[1] * (gg[3] * rL[0] + gg[1] * rL[1] + gg[4] * rL[2]) +
-                    rL[2] * (gg[5] * rL[0] + gg[4] * rL[1] + gg[2] * rL[2]);
-    tauBar = (tauBar != 0.0) ? tauM / sqrt(tauBar) : 0.0;
-    double ub[3];
-#pragma unroll
-    for (int i = 0; i < 3; ++i) ub[i] = u[i] - tauM * rL[i] * rhoinv;
-    // e3Res, iconvflow = 2 (e3res.f90:99-286)
-    const double tmp = -pq + tauC * divu;
-    double lg[3];  // L . grad u_i
-#pragma unroll
-    for (int i = 0; i < 3; ++i) lg[i] = tauBar * (rL[0] * gu[0][i] + rL[1] * gu[1][i] + rL[2] * gu[2][i]);
+      L[i] = (aq[i] + u[0] * o.gu[0][i] + u[1] * o.gu[1][i] + u[2] * o.gu[2][i]) * rho + gpd[i];
+    const T uGu = u[0] * (gg[0] * u[0] + gg[3] * u[1] + gg[5] * u[2]) +
+                  u[1] * (gg[3] * u[0] + gg[1] * u[1] + gg[4] * u[2]) +
+                  u[2] * (gg[5] * u[0] + gg[4] * u[1] + gg[2] * u[2]);
+    const T s2 = tau0 + uGu;
+    const T tauM = rsq(s2);
+    sf += s2 * tauM;
+    o.TM += tauM;
+    const T LGL = L[0] * (gg[0] * L[0] + gg[3] * L[1] + gg[5] * L[2]) +
+                  L[1] * (gg[3] * L[0] + gg[1] * L[1] + gg[4] * L[2]) +
+                  L[2] * (gg[5] * L[0] + gg[4] * L[1] + gg[2] * L[2]);
+    const T tauB = (LGL != T(0)) ? tauM * rsq(LGL) : T(0);
+    const T tr = tauM * rhoinv;
+    T ub[3], tu[3], tL[3];
 #pragma unroll
     for (int i = 0; i < 3; ++i) {
-      const double rna = (aq[i] + ub[0] * gu[0][i] + ub[1] * gu[1][i] + ub[2] * gu[2][i]) * rho;
-      RNa[0][i] += N0 * rna;
-      RNa[1][i] += N1 * rna;
-      RNa[2][i] += N2 * rna;
-      RNa[3][i] += N3 * rna;
-      const double tl = tauM * rL[i];
-#pragma unroll
-      for (int j = 0; j < 3; ++j) {
-        double v = mu * (gu[i][j] + gu[j][i]) + tl * u[j] + lg[i] * rL[j];
-        if (i == j) v += tmp;
-        RGN[i][j] += v;
-      }
-      SU[i] += ub[i];
+      ub[i] = u[i] - tr * L[i];
+      o.SU[i] += ub[i];
+      tu[i] = tauM * u[i];
+      tL[i] = tauB * L[i];
     }
-    if (LHS) {
-      // e3LHS, iconvflow = 2 (e3lhs.f90:124-129): convection by u-bar, and
-      // the tauBar (L.g_a)(L.g_b) term beside SUPG's tauM rho (u.g_a)(u.g_b)
-      TC += tauC;
-      TM += tauM;
-      const double tb = tauBar * rhoinv;
-      double z[4], zl[4];
-#pragma unroll
-      for (int a = 0; a < 4; ++a) {
-        z[a] = u[0] * g[a][0] + u[1] * g[a][1] + u[2] * g[a][2];
-        zl[a] = rL[0] * g[a][0] + rL[1] * g[a][1] + rL[2] * g[a][2];
-      }
-      int k = 0;
-#pragma unroll
-      for (int a = 0; a < 4; ++a)
-#pragma unroll
-        for (int b = a; b < 4; ++b) SUPG[k++] += tauM * z[a] * z[b] + tb * zl[a] * zl[b];
+    if (RES) {
 #pragma unroll
       for (int i = 0; i < 3; ++i) {
-        UB[0][i] += N0 * ub[i];
-        UB[1][i] += N1 * ub[i];
-        UB[2][i] += N2 * ub[i];
-        UB[3][i] += N3 * ub[i];
+        const T r = aq[i] + ub[0] * o.gu[0][i] + ub[1] * o.gu[1][i] + ub[2] * o.gu[2][i];
+        o.SR[i] += r;
+        al[q][i] = r;
+#pragma unroll
+        for (int j = 0; j < 3; ++j) o.C[i][j] += L[i] * tu[j];
       }
     }
-  }
-
-  double *r = LHS ? sh_rec + threadIdx.x * kE3Pad : rec + (size_t)e * kRec;
-#pragma unroll
-  for (int a = 0; a < 4; ++a) {
-    r[R_A(a) + R_RL + 3] = W * (g[a][0] * SU[0] + g[a][1] * SU[1] + g[a][2] * SU[2]);
 #pragma unroll
     for (int i = 0; i < 3; ++i)
-      r[R_A(a) + R_RL + i] = -W * (RNa[a][i] + g[a][0] * RGN[i][0] + g[a][1] * RGN[i][1] + g[a][2] * RGN[i][2]);
+#pragma unroll
+      for (int j = i; j < 3; ++j) {
+        if (TAN) o.A[kSym[i][j]] += tu[i] * u[j];
+        o.B[kSym[i][j]] += tL[i] * L[j];
+      }
+#pragma unroll
+    for (int i = 0; i < 3; ++i) ul[q][i] = ub[i];
   }
-  if (!LHS) return;
-  const double tlW = c.lhsFct * W;
-  const double tsFct = c.lhmFct * W * rho;
-  const double Mu = 4.0 * (tlW * mu);
-  const double rt = rho * tlW;
+  // tauC = rho fact / (8 tr G) taucfct / dtsfct
+  o.TC = sf * (rho * T(0.125) / (gg[0] + gg[1] + gg[2]) * T(c.taucfct / c.dtsfct));
+  o.divu = o.gu[0][0] + o.gu[1][1] + o.gu[2][2];
+}
+// The S rows: put(a, b, S_ab), and the scalars tlW, Tc, Mu, Cm.
+template <class T, bool RES, bool TAN, class Put>
+__device__ inline void e3_tangent(const FormConst &c, const T (&ub)[4][3], const E3Sums<T, RES, TAN> &o, T &tlW,
+                                  T &Tc, T &Mu, T &Cm, Put put) {
+  const T rho = T(c.rho);
+  tlW = T(c.lhsFct) * o.W;
+  const T ts = T(c.lhmFct) * o.W * rho, rt = rho * tlW;
+  Mu = T(4) * (tlW * T(c.mu));
+  Tc = tlW * o.TC;
+  Cm = tlW * o.TM / rho;
+  // symmetric part g_a . (rho tlW (A + B / rho) + Mu) g_b
+  T M[6], Y[4][4], h[3][3], v[3];
 #pragma unroll
-  for (int a = 0; a < 4; ++a)
+  for (int k = 0; k < 6; ++k) M[k] = rt * o.A[k] + tlW * o.B[k];
+  M[0] += Mu;
+  M[3] += Mu;
+  M[5] += Mu;
 #pragma unroll
-    for (int b = 0; b < 4; ++b) {
-      // convection sum_q N_a (ubar_q . g_b)
-      const double conv = UB[a][0] * g[b][0] + UB[a][1] * g[b][1] + UB[a][2] * g[b][2];
-      const int lo = a < b ? a : b, hi = a < b ? b : a;
-      const int k = lo * 4 - (lo * (lo - 1)) / 2 + (hi - lo);  // index of (lo,hi) in SUPG
-      const double gab = g[a][0] * g[b][0] + g[a][1] * g[b][1] + g[a][2] * g[b][2];
-      r[R_A(a) + b] = tsFct * mm(a, b) + rt * conv + Mu * gab + rt * SUPG[k];
+  for (int a = 0; a < 3; ++a) {
+#pragma unroll
+    for (int i = 0; i < 3; ++i)
+      h[a][i] = M[kSym[i][0]] * o.g[a][0] + M[kSym[i][1]] * o.g[a][1] + M[kSym[i][2]] * o.g[a][2];
+    v[a] = rt * (o.SU[0] * o.g[a][0] + o.SU[1] * o.g[a][1] + o.SU[2] * o.g[a][2]);
+  }
+#pragma unroll
+  for (int a = 0; a < 3; ++a)
+#pragma unroll
+    for (int b = a; b < 3; ++b)
+      Y[a][b] = Y[b][a] = h[a][0] * o.g[b][0] + h[a][1] * o.g[b][1] + h[a][2] * o.g[b][2];
+#pragma unroll
+  for (int a = 0; a < 3; ++a) Y[a][3] = Y[3][a] = -(Y[a][0] + Y[a][1] + Y[a][2]);
+  Y[3][3] = -(Y[0][3] + Y[1][3] + Y[2][3]);
+  // convection sum_q N_a (ubar_q . g_b) (e3lhs.f90:124-129)
+#pragma unroll
+  for (int a = 0; a < 4; ++a) {
+    const T rd = rt * T(w_diff(a));
+    T cv[3];
+#pragma unroll
+    for (int b = 0; b < 3; ++b) {
+      cv[b] = T(w_other(a)) * v[b] + rd * (ub[a][0] * o.g[b][0] + ub[a][1] * o.g[b][1] + ub[a][2] * o.g[b][2]);
+      put(a, b, ts * T(mm(a, b)) + cv[b] + Y[a][b]);
     }
-  if (e < nel) {
-    double2 *d = reinterpret_cast<double2 *>(esc + (size_t)e * kESc);
-    d[0] = make_double2(tlW * TC, Mu);     // Tc, Mu
-    d[1] = make_double2(tlW * TM / rho, tlW);  // Cm, tlW
+    put(a, 3, ts * T(mm(a, 3)) - (cv[0] + cv[1] + cv[2]) + Y[a][3]);
+  }
+}
+
+// The element records of the workgroup's (consecutive) elements are assembled
+// in LDS and stored as one contiguous block with coalesced 16-byte stores
+// (written directly, each thread's record reached HBM as partially filled
+// lines); the scalars (32 bytes per element) are stored directly, contiguous
+// across the threads.  Without the tangent a record holds the residual rows
+// alone: kRecRes doubles, one line per element.
+constexpr int kE3Threads = 128;
+// Workgroups dealt to the XCDs in turns of this many: the records of
+// neighbouring elements are written at the same time (7.9 M elements: 678 us with
+// one range per XCD, 647 in turns).  The nodes are gathered per element: staged
+// in LDS once per workgroup they cost 60 us more than the gathers save.
+constexpr unsigned kE3XcdChunk = 64;
+template <bool LHS>
+struct E3Rec {
+  static constexpr int n = LHS ? kRec : kRecRes;
+  // LDS stride of a staged record: one double more than the record, so that
+  // the threads' stores at the same offset fall in different banks
+  static constexpr int pad = n + 1;
+  __device__ static constexpr int rl(int a) { return LHS ? R_A(a) + R_RL : 4 * a; }
+};
+template <bool LHS>
+__global__ void __launch_bounds__(kE3Threads) __attribute__((amdgpu_waves_per_eu(2)))
+e3_elem(int nel, const int *__restrict__ ien, const double *__restrict__ node, FormConst c0, Ens en,
+        double *__restrict__ rec, double *__restrict__ esc) {
+  using Rec = E3Rec<LHS>;
+  __shared__ double sh_rec[kE3Threads * Rec::pad];
+  const int e0 = xcd_block(kE3XcdChunk) * kE3Threads;
+  const int e = e0 + threadIdx.x;
+  const int ee = e < nel ? e : nel - 1;  // tail threads evaluate a valid element; nothing of theirs is stored
+  FormConst c = c0;
+  c.mu = ens_mu(en, ee, c0.mu);
+  // the four node records (localx/localy gathers, localy.f90:54-64)
+  int nd[4];
+#pragma unroll
+  for (int a = 0; a < 4; ++a) nd[a] = ien[a * (size_t)nel + ee];
+  double xl[4][3], ul[4][3], al[4][3], pl[4], ql[4][6];
+#pragma unroll
+  for (int a = 0; a < 4; ++a) {
+    double nl[kNRec];
+    load_record(node + (size_t)nd[a] * kNRec, nl);
+#pragma unroll
+    for (int i = 0; i < 3; ++i) {
+      xl[a][i] = nl[N_X + i];
+      ul[a][i] = nl[N_U + i];
+      al[a][i] = nl[N_A + i];
+    }
+    pl[a] = nl[N_P];
+#pragma unroll
+    for (int k = 0; k < 6; ++k) ql[a][k] = nl[N_Q + k];
+  }
+  const double psum = sum_n(0) * pl[0] + sum_n(1) * pl[1] + sum_n(2) * pl[2] + sum_n(3) * pl[3];  // sum_q p
+  E3Sums<double, true, LHS> o;
+  e3_sums(c, xl, pl, ql, ul, al, o);
+
+  double *r = sh_rec + threadIdx.x * Rec::pad;
+  {  // e3Res, iconvflow = 2 (e3res.f90:99-286)
+    const double mu4 = 4.0 * c.mu, tp = o.divu * o.TC - psum;
+    double last[3], lastc = 0.0;
+#pragma unroll
+    for (int i = 0; i < 3; ++i) {
+      double f[3];
+#pragma unroll
+      for (int j = 0; j < 3; ++j) {
+        f[j] = o.C[i][j] + mu4 * (o.gu[i][j] + o.gu[j][i]) + o.gu[0][i] * o.B[kSym[0][j]] +
+               o.gu[1][i] * o.B[kSym[1][j]] + o.gu[2][i] * o.B[kSym[2][j]];
+        if (i == j) f[j] += tp;
+      }
+      const double sr = c.rho * o.SR[i];
+      last[i] = 0.0;
+#pragma unroll
+      for (int a = 0; a < 3; ++a) {
+        const double gf = o.g[a][0] * f[0] + o.g[a][1] * f[1] + o.g[a][2] * f[2];
+        r[Rec::rl(a) + i] = -o.W * (w_other(a) * sr + (c.rho * w_diff(a)) * al[a][i] + gf);
+        last[i] -= gf;
+      }
+      r[Rec::rl(3) + i] = -o.W * (w_other(3) * sr + (c.rho * w_diff(3)) * al[3][i] + last[i]);
+    }
+#pragma unroll
+    for (int a = 0; a < 3; ++a) {
+      const double v = o.W * (o.g[a][0] * o.SU[0] + o.g[a][1] * o.SU[1] + o.g[a][2] * o.SU[2]);
+      r[Rec::rl(a) + 3] = v;
+      lastc -= v;
+    }
+    r[Rec::rl(3) + 3] = lastc;
+  }
+  if constexpr (LHS) {
+    double tlW, Tc, Mu, Cm;
+    e3_tangent(c, ul, o, tlW, Tc, Mu, Cm, [&](int a, int b, double v) { r[R_A(a) + b] = v; });
+    if (e < nel) {
+      double2 *d = reinterpret_cast<double2 *>(esc + (size_t)e * kESc);
+      d[0] = make_double2(Tc, Mu);
+      d[1] = make_double2(Cm, tlW);
+    }
   }
   __syncthreads();
   const int cnt = min(kE3Threads, nel - e0);
-  double2 *dst = reinterpret_cast<double2 *>(rec + (size_t)e0 * kRec);
-  for (int i = threadIdx.x; i < cnt * (kRec / 2); i += kE3Threads) {
-    const double *src = sh_rec + (i / (kRec / 2)) * kE3Pad + 2 * (i % (kRec / 2));
+  constexpr int kH = Rec::n / 2;
+  double2 *dst = reinterpret_cast<double2 *>(rec + (size_t)e0 * Rec::n);
+  for (int i = threadIdx.x; i < cnt * kH; i += kE3Threads) {
+    const double *src = sh_rec + (i / kH) * Rec::pad + 2 * (i % kH);
     dst[i] = make_double2(src[0], src[1]);
   }
 }
@@ -478,123 +566,34 @@ __device__ inline void tangent_body(const double (&nl)[4][kNRec], const FormCons
 #pragma unroll
     for (int k = 0; k < 6; ++k) ql[a][k] = (T)nl[a][N_Q + k];
   }
-  T dx[3][3], W, g[4][3], gg[6];
-  p1_metric(xl, dx, W, g);
-  gijd_tet(dx, gg);
-  T gu[3][3], gp[3], divq[3] = {T(0), T(0), T(0)};  // gu[j][i] = du_i/dx_j
+  E3Sums<T, false, true> o;
+  e3_sums(c, xl, pl, ql, ul, al, o);
+  T tlW, Tc, Mu, Cm;
+  e3_tangent(c, ul, o, tlW, Tc, Mu, Cm, [&](int a, int b, T v) { r[R32_S(a) + b] = (float)v; });
 #pragma unroll
   for (int j = 0; j < 3; ++j) {
 #pragma unroll
-    for (int i = 0; i < 3; ++i)
-      gu[j][i] = g[0][j] * ul[0][i] + g[1][j] * ul[1][i] + g[2][j] * ul[2][i] + g[3][j] * ul[3][i];
-    gp[j] = g[0][j] * pl[0] + g[1][j] * pl[1] + g[2][j] * pl[2] + g[3][j] * pl[3];
+    for (int a = 0; a < 3; ++a) r[R_G + a * 3 + j] = (float)o.g[a][j];
+    r[R_G + 9 + j] = (float)(-o.g[0][j] - o.g[1][j] - o.g[2][j]);
   }
-#pragma unroll
-  for (int a = 0; a < 4; ++a)
-#pragma unroll
-    for (int i = 0; i < 3; ++i)
-      divq[i] += g[a][0] * ql[a][qsym(i)] + g[a][1] * ql[a][qsym(i + 3)] + g[a][2] * ql[a][qsym(i + 6)];
-  const T rho = (T)c.rho, mu = (T)c.mu, rhoinv = T(1) / rho;
-  const T rnu = mu * rhoinv;
-  const T dts = (T)(c.Dtgl * c.dtsfct);
-  const T GG = gg[0] * gg[0] + gg[1] * gg[1] + gg[2] * gg[2] + T(2) * (gg[3] * gg[3] + gg[4] * gg[4] + gg[5] * gg[5]);
-  const T tau0 = (T(2) * dts) * (T(2) * dts);
-  const T visc = T(36) * (rnu * rnu) * GG;
-  const T trg = gg[0] + gg[1] + gg[2];
-  const T ff = (T)(c.taucfct / c.dtsfct);
-  T TC = T(0), TM = T(0), SUPG[10], UB[4][3];
-#pragma unroll
-  for (int k = 0; k < 10; ++k) SUPG[k] = T(0);
-#pragma unroll
-  for (int a = 0; a < 4; ++a)
-#pragma unroll
-    for (int i = 0; i < 3; ++i) UB[a][i] = T(0);
-#pragma unroll
-  for (int qp = 0; qp < 4; ++qp) {
-    const T Nq[4] = {(T)nq(qp, 0), (T)nq(qp, 1), (T)nq(qp, 2), (T)nq(qp, 3)};
-    T u[3], aq[3], rL[3];
-#pragma unroll
-    for (int i = 0; i < 3; ++i) {
-      u[i] = Nq[0] * ul[0][i] + Nq[1] * ul[1][i] + Nq[2] * ul[2][i] + Nq[3] * ul[3][i];
-      aq[i] = Nq[0] * al[0][i] + Nq[1] * al[1][i] + Nq[2] * al[2][i] + Nq[3] * al[3][i];
-    }
-    // strong residual (e3res.f90:775-789)
-#pragma unroll
-    for (int i = 0; i < 3; ++i)
-      rL[i] = (aq[i] + u[0] * gu[0][i] + u[1] * gu[1][i] + u[2] * gu[2][i]) * rho + gp[i] - divq[i];
-    const T uGu = u[0] * (gg[0] * u[0] + gg[3] * u[1] + gg[5] * u[2]) +
-                  u[1] * (gg[3] * u[0] + gg[1] * u[1] + gg[4] * u[2]) +
-                  u[2] * (gg[5] * u[0] + gg[4] * u[1] + gg[2] * u[2]);
-    const T fact = sqrt((tau0 + uGu) + visc);
-    const T tauC = rho * T(0.125) * fact / trg * ff;
-    const T tauM = T(1) / fact;
-    T tauBar = rL[0] * (gg[0] * rL[0] + gg[3] * rL[1] + gg[5] * rL[2]) +
-               rL[1] * (gg[3] * rL[0] + gg[1] * rL[1] + gg[4] * rL[2]) +
-               rL[2] * (gg[5] * rL[0] + gg[4] * rL[1] + gg[2] * rL[2]);
-    tauBar = (tauBar != T(0)) ? tauM / sqrt(tauBar) : T(0);
-    TC += tauC;
-    TM += tauM;
-    const T tb = tauBar * rhoinv;
-    T z[4], zl[4];
-#pragma unroll
-    for (int a = 0; a < 4; ++a) {
-      z[a] = u[0] * g[a][0] + u[1] * g[a][1] + u[2] * g[a][2];
-      zl[a] = rL[0] * g[a][0] + rL[1] * g[a][1] + rL[2] * g[a][2];
-    }
-    int k = 0;
-#pragma unroll
-    for (int a = 0; a < 4; ++a)
-#pragma unroll
-      for (int b = a; b < 4; ++b) SUPG[k++] += tauM * z[a] * z[b] + tb * zl[a] * zl[b];
-#pragma unroll
-    for (int i = 0; i < 3; ++i) {
-      const T ub = u[i] - tauM * rL[i] * rhoinv;
-#pragma unroll
-      for (int a = 0; a < 4; ++a) UB[a][i] += Nq[a] * ub;
-    }
-  }
-  const T tlW = (T)c.lhsFct * W;
-  const T tsFct = (T)c.lhmFct * W * rho;
-  const T Mu = T(4) * (tlW * mu);
-  const T rt = rho * tlW;
-#pragma unroll
-  for (int a = 0; a < 4; ++a)
-#pragma unroll
-    for (int b = 0; b < 4; ++b) {
-      const T conv = UB[a][0] * g[b][0] + UB[a][1] * g[b][1] + UB[a][2] * g[b][2];
-      const int lo = a < b ? a : b, hi = a < b ? b : a;
-      const int k = lo * 4 - (lo * (lo - 1)) / 2 + (hi - lo);
-      const T gab = g[a][0] * g[b][0] + g[a][1] * g[b][1] + g[a][2] * g[b][2];
-      r[R32_S(a) + b] = (float)(tsFct * (T)mm(a, b) + rt * conv + Mu * gab + rt * SUPG[k]);
-    }
-#pragma unroll
-  for (int a = 0; a < 4; ++a)
-#pragma unroll
-    for (int j = 0; j < 3; ++j) r[R_G + a * 3 + j] = (float)g[a][j];
   r[R_TLW] = (float)tlW;
-  r[R_TC] = (float)(tlW * TC);
+  r[R_TC] = (float)Tc;
   r[R_MU] = (float)Mu;
-  r[R_CM] = (float)(tlW * TM / rho);
+  r[R_CM] = (float)Cm;
 }
 
-__global__ void __launch_bounds__(256) e3_tangent32(int nel, const int *__restrict__ ien,
-                                                    const double *__restrict__ node, FormConst c0, Ens en,
-                                                    float aspect_fp64, float *__restrict__ rec) {
-  const int e = xcd_block() * blockDim.x + threadIdx.x;
-  if (e >= nel) return;
+__global__ void __launch_bounds__(kE3Threads) e3_tangent32(int nel, const int *__restrict__ ien,
+                                                           const double *__restrict__ node, FormConst c0, Ens en,
+                                                           float aspect_fp64, float *__restrict__ rec) {
+  constexpr int kPad = kRec32 + 1;
+  __shared__ float sh[kE3Threads * kPad];  // the records, stored as one block (as e3_elem's)
+  const int e0 = xcd_block(kE3XcdChunk) * kE3Threads, e = e0 + threadIdx.x;
+  const int ee = e < nel ? e : nel - 1;
   FormConst c = c0;
-  c.mu = ens_mu(en, e, c0.mu);
+  c.mu = ens_mu(en, ee, c0.mu);
   double nl[4][kNRec];
 #pragma unroll
-  for (int a = 0; a < 4; ++a) {
-    const double2 *rr = reinterpret_cast<const double2 *>(node + (size_t)ien[a * (size_t)nel + e] * kNRec);
-#pragma unroll
-    for (int k = 0; k < kNRec / 2; ++k) {
-      const double2 v = rr[k];
-      nl[a][2 * k] = v.x;
-      nl[a][2 * k + 1] = v.y;
-    }
-  }
+  for (int a = 0; a < 4; ++a) load_record(node + (size_t)ien[a * (size_t)nel + ee] * kNRec, nl[a]);
   double xl[4][3];
 #pragma unroll
   for (int a = 0; a < 4; ++a)
@@ -605,9 +604,15 @@ __global__ void __launch_bounds__(256) e3_tangent32(int nel, const int *__restri
     tangent_body<double>(nl, c, r);
   else
     tangent_body<float>(nl, c, r);
-  float4 *o = reinterpret_cast<float4 *>(rec + (size_t)e * kRec32);
 #pragma unroll
-  for (int k = 0; k < kRec32 / 4; ++k) o[k] = make_float4(r[4 * k], r[4 * k + 1], r[4 * k + 2], r[4 * k + 3]);
+  for (int k = 0; k < kRec32; ++k) sh[threadIdx.x * kPad + k] = r[k];
+  __syncthreads();
+  const int cnt = min(kE3Threads, nel - e0);
+  float4 *dst = reinterpret_cast<float4 *>(rec + (size_t)e0 * kRec32);
+  for (int i = threadIdx.x; i < cnt * (kRec32 / 4); i += kE3Threads) {
+    const float *q = sh + (i / (kRec32 / 4)) * kPad + 4 * (i % (kRec32 / 4));
+    dst[i] = make_float4(q[0], q[1], q[2], q[3]);
+  }
 }
 
 // ---------------------------------------------------------------- assembly
@@ -689,27 +694,42 @@ __device__ inline void put_res(double *res, int i, int nshg, const double (&rs)[
   }
 }
 
+// kResLanes lanes per node, each with its incidences' records all in flight
+// (three per lane on a Kuhn mesh's 24).  1.3 M nodes: 430 us with four lanes, one
+// record at a time out of the 256-byte records of the tangent's layout, 248 so.
+constexpr int kResLanes = 8, kResUnroll = 3;
 template <int MODE>
 __global__ void __launch_bounds__(256) res_node(int nshg, const int *__restrict__ inc_ptr,
                                                 const int *__restrict__ inc, const double *__restrict__ rec,
                                                 double *__restrict__ res) {
   const int gid = xcd_block() * blockDim.x + threadIdx.x;
-  const int i = gid / kNodeLanes, lane = gid % kNodeLanes;
+  const int i = gid / kResLanes, lane = gid % kResLanes;
   double rs[4] = {0, 0, 0, 0};
-  if (i < nshg)
-    for (int p = inc_ptr[i] + lane; p < inc_ptr[i + 1]; p += kNodeLanes) {
-      const int ea = inc[p];
-      const double2 *r = reinterpret_cast<const double2 *>(rec + (size_t)(ea >> 2) * kRec + R_A(ea & 3) + R_RL);
-      const double2 r01 = r[0], r23 = r[1];
-      rs[0] += r01.x;
-      rs[1] += r01.y;
-      rs[2] += r23.x;
-      rs[3] += r23.y;
+  const int p1 = inc_ptr[min(i + 1, nshg)];
+  for (int p = inc_ptr[min(i, nshg)] + lane; p < p1; p += kResLanes * kResUnroll) {
+    int ea[kResUnroll];
+#pragma unroll
+    for (int u = 0; u < kResUnroll; ++u) ea[u] = inc[min(p + kResLanes * u, p1 - 1)];
+    double2 r[kResUnroll][2];
+#pragma unroll
+    for (int u = 0; u < kResUnroll; ++u) {
+      const double2 *q = reinterpret_cast<const double2 *>(rec + (size_t)ea[u] * (kRecRes / 4));
+      r[u][0] = q[0];
+      r[u][1] = q[1];
     }
 #pragma unroll
-  for (int off = 1; off < kNodeLanes; off <<= 1)
+    for (int u = 0; u < kResUnroll; ++u)
+      if (p + kResLanes * u < p1) {
+        rs[0] += r[u][0].x;
+        rs[1] += r[u][0].y;
+        rs[2] += r[u][1].x;
+        rs[3] += r[u][1].y;
+      }
+  }
 #pragma unroll
-    for (int k = 0; k < 4; ++k) rs[k] += __shfl_xor(rs[k], off, kNodeLanes);
+  for (int off = 1; off < kResLanes; off <<= 1)
+#pragma unroll
+    for (int k = 0; k < 4; ++k) rs[k] += __shfl_xor(rs[k], off, kResLanes);
   if (i < nshg && lane == 0) put_res<MODE>(res, i, nshg, rs);
 }
 
@@ -809,14 +829,6 @@ __device__ inline void diag_full(const DiagAcc<T> &D, T (&K)[9]) {
     for (int ii = 0; ii < 3; ++ii) K[ii + 3 * jj] = D.K[sym3(ii, jj)];
 }
 
-// Orders LDS accesses of the lanes of one wavefront (the lanes of a CSR row
-// always share a wavefront).
-__device__ inline void wave_lds_sync() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
 // A lane's contribution-list entries (16 bits each), eight at a time: two
 // 64-bit words filled by four independent dword loads, consumed from the low
 // end.  The list of one block is contiguous in lst and sorted by incidence,
@@ -867,6 +879,20 @@ __global__ void slot_table_kernel(int n, const int *__restrict__ order, const in
   const int k0 = rowptr[row], p0 = inc_ptr[row];
   tab[2 * i] = make_int4(row, k0, rowptr[row + 1] - k0, diagk[row] - k0);
   tab[2 * i + 1] = make_int4(p0, inc_ptr[row + 1] - p0, 0, 0);
+}
+
+// The coordinates of an element's four nodes (local order) from the packed
+// nodes.
+__device__ inline void gather_x(const double *__restrict__ xu, int4 n4, double (&xl)[4][3]) {
+  const int nd[4] = {n4.x, n4.y, n4.z, n4.w};
+#pragma unroll
+  for (int a = 0; a < 4; ++a) {
+    const double *r = xu + (size_t)nd[a] * kXU;
+    const double2 v = *reinterpret_cast<const double2 *>(r);
+    xl[a][0] = v.x;
+    xl[a][1] = v.y;
+    xl[a][2] = r[2];
+  }
 }
 
 // Row-parallel assembly, kRowLanes lanes per CSR row; rows are taken in the
@@ -1459,12 +1485,12 @@ int run_formation(crimson_form *f, const double *d_y, const double *d_ac, const 
       e3_elem<false><<<crimson::grid_for(f->nel, kE3Threads), kE3Threads, 0, s>>>(
           f->nel, f->d_ien.p, f->d_node.p, c, f->ens(), f->d_rec.p, f->d_esc.p);
     if (t32)
-      e3_tangent32<<<crimson::grid_for(f->nel, T), T, 0, s>>>(f->nel, f->d_ien.p, f->d_node.p, c, f->ens(),
-                                                              (float)f->prm.aspect_fp64, f->d_rec32.p);
+      e3_tangent32<<<crimson::grid_for(f->nel, kE3Threads), kE3Threads, 0, s>>>(
+          f->nel, f->d_ien.p, f->d_node.p, c, f->ens(), (float)f->prm.aspect_fp64, f->d_rec32.p);
   }
   CR_HIP(hipGetLastError());
   if (timed) CR_HIP(hipEventRecord(f->ev[2], s));
-  const unsigned gn = crimson::grid_for((size_t)f->nshg * kNodeLanes, T);
+  const unsigned gn = crimson::grid_for((size_t)f->nshg * kResLanes, T);
   const unsigned gr = crimson::grid_for((size_t)f->nshg * kRowLanes, T);
   const int runs = f->sched == kSchedNumbering;  // slot i is row i: a wave's rows are consecutive
   if (t32) {
@@ -1534,9 +1560,15 @@ int form_flux_pass(crimson_form *f, const double *d_y, const double *d_ac, const
   const unsigned T = 256;
   hipStream_t s = f->stream;
   node_pack<<<crimson::grid_for(f->nshg, T), T, 0, s>>>(f->nshg, d_x, f->numnp, d_y, f->d_xu.p);
-  flux_node<<<crimson::grid_for((size_t)f->nshg * kNodeLanes, T), T, 0, s>>>(
-      f->nshg, f->d_inc_ptr.p, f->d_inc.p, f->d_ienp.p, f->d_xu.p, f->prm.mu, f->ens(), d_x, f->numnp, d_y, d_ac,
-      f->d_node.p, d_q, d_invm);
+  const unsigned G = crimson::grid_for((size_t)f->nshg * kFluxLanes, T);
+  if (f->wide)
+    flux_node<<<G, T, 0, s>>>(f->nshg, f->d_rowptr.p, f->d_diagk.p, f->d_col.p, f->d_inc_ptr.p, f->d_inc.p,
+                              reinterpret_cast<const unsigned long long *>(f->d_iloc.p), f->d_xu.p, f->prm.mu,
+                              f->ens(), d_y, d_ac, f->d_node.p, d_q, d_invm);
+  else
+    flux_node<<<G, T, 0, s>>>(f->nshg, f->d_rowptr.p, f->d_diagk.p, f->d_col.p, f->d_inc_ptr.p, f->d_inc.p,
+                              (const unsigned *)f->d_iloc.p, f->d_xu.p, f->prm.mu, f->ens(), d_y, d_ac, f->d_node.p,
+                              d_q, d_invm);
   CR_HIP(hipGetLastError());
   return CRIMSON_OK;
 }
@@ -1655,8 +1687,18 @@ extern "C" int crimson_form_setup(int nshg, int numnp, int nel, const int *ien, 
   // Contribution lists of the off-diagonal blocks: for block k of row i, the
   // entries (t << 4 | a << 2 | b) of the row's incidences t = (e,a) whose node
   // ien(e,b) is the block's column, in element order (sparseloc,
-  // fillsparse.f90:41, resolved once).
+  // fillsparse.f90:41, resolved once); the places of each incidence's other
+  // nodes among the row's blocks (IncLoc) on the way.
   std::vector<int> lst_ptr(nnz + 1, 0);
+  int most = 0;
+  for (int i = 0; i < nshg; ++i) most = std::max(most, rp[i + 1] - rp[i]);
+  const bool wide = most > (1 << IncLoc<unsigned>::bits);
+  std::vector<unsigned> iloc;
+  std::vector<unsigned long long> iloc64;
+  if (wide)
+    iloc64.resize(inc.size());
+  else
+    iloc.resize(inc.size());
   for (int i = 0; i < nshg; ++i) {
     if (inc_ptr[i + 1] - inc_ptr[i] >= (1 << 12)) {
       crimson::set_error("node %d belongs to %d elements; at most 4095 supported", i + 1, inc_ptr[i + 1] - inc_ptr[i]);
@@ -1664,6 +1706,7 @@ extern "C" int crimson_form_setup(int nshg, int numnp, int nel, const int *ien, 
     }
     for (int p = inc_ptr[i]; p < inc_ptr[i + 1]; ++p) {
       const int e = inc[p] >> 2, a = inc[p] & 3;
+      int o[3], n = 0;
       for (int b = 0; b < 4; ++b) {
         if (b == a) continue;
         const int j = ien[(size_t)b * nel + e] - 1;
@@ -1673,7 +1716,12 @@ extern "C" int crimson_form_setup(int nshg, int numnp, int nel, const int *ien, 
           return CRIMSON_EGRAPH;
         }
         lst_ptr[k + 1]++;
+        o[n++] = k - rp[i];
       }
+      if (wide)
+        iloc64[p] = IncLoc<unsigned long long>::pack(o, a);
+      else
+        iloc[p] = IncLoc<unsigned>::pack(o, a);
     }
   }
   for (int k = 0; k < nnz; ++k) lst_ptr[k + 1] += lst_ptr[k];
@@ -1683,10 +1731,12 @@ extern "C" int crimson_form_setup(int nshg, int numnp, int nel, const int *ien, 
     std::vector<int> fill(lst_ptr.begin(), lst_ptr.end() - 1);
     for (int i = 0; i < nshg; ++i)
       for (int p = inc_ptr[i]; p < inc_ptr[i + 1]; ++p) {
-        const int e = inc[p] >> 2, a = inc[p] & 3;
-        for (int b = 0; b < 4; ++b) {
+        const int a = inc[p] & 3;
+        const unsigned long long v = wide ? iloc64[p] : iloc[p];
+        const int bits = wide ? IncLoc<unsigned long long>::bits : IncLoc<unsigned>::bits;
+        for (int b = 0, n = 0; b < 4; ++b) {
           if (b == a) continue;
-          const int k = find_col(rp, cols, i, ien[(size_t)b * nel + e] - 1);
+          const int k = rp[i] + (int)(v >> (bits * n++) & ((1u << bits) - 1));
           lst[fill[k]++] = (unsigned short)(((p - inc_ptr[i]) << 4) | (a << 2) | b);
         }
       }
@@ -1706,6 +1756,7 @@ extern "C" int crimson_form_setup(int nshg, int numnp, int nel, const int *ien, 
   f->nel = nel;
   f->nnz = nnz;
   f->prm = *prm;
+  f->wide = wide;
   int rc = CRIMSON_OK;
   auto fail = [&](int code) {
     crimson_form_free(f);
@@ -1724,16 +1775,23 @@ extern "C" int crimson_form_setup(int nshg, int numnp, int nel, const int *ien, 
     }
   std::vector<int> ien0((size_t)nel * 4);
   for (size_t k = 0; k < ien0.size(); ++k) ien0[k] = ien[k] - 1;
-  // per incidence, its element's nodes (the gathers of the flux pass and of
-  // the assembly's shape gradients, read per row as one contiguous run).  One
-  // spare entry (node 0) when there are no elements, so that every read of
-  // entry 0 is in bounds.
+  // per incidence, its element's nodes (the gathers of the assembly's shape
+  // gradients, read per row as one contiguous run).  One spare entry (node 0)
+  // when there are no elements, so that every read of entry 0 is in bounds.
   std::vector<int4> ienp(std::max<size_t>(inc.size(), 1), make_int4(0, 0, 0, 0));
   for (size_t p = 0; p < inc.size(); ++p) {
-    const int e = inc[p] >> 2;
+    const size_t e = inc[p] >> 2;
     ienp[p] = make_int4(ien0[e], ien0[(size_t)nel + e], ien0[2 * (size_t)nel + e], ien0[3 * (size_t)nel + e]);
   }
-  if (inc.empty()) inc.push_back(0);  // the same spare entry (element 0's records are always allocated)
+  // one spare incidence when there are none, so that every read of entry 0 is
+  // in bounds (element 0's records are always allocated)
+  if (inc.empty()) {
+    inc.push_back(0);
+    if (wide)
+      iloc64.push_back(0);
+    else
+      iloc.push_back(0);
+  }
   hipStream_t s = f->stream;
   if ((rc = f->d_ien.upload(ien0.data(), ien0.size(), s)) ||
       (rc = f->d_inc_ptr.upload(inc_ptr.data(), inc_ptr.size(), s)) ||
@@ -1742,6 +1800,9 @@ extern "C" int crimson_form_setup(int nshg, int numnp, int nel, const int *ien, 
       (rc = f->d_rowptr.upload(rp.data(), rp.size(), s)) ||
       (rc = f->d_lst_ptr.upload(lst_ptr.data(), lst_ptr.size(), s)) ||
       (rc = f->d_lst.upload(lst.data(), lst.size(), s)) ||
+      (rc = wide ? f->d_iloc.upload(reinterpret_cast<const unsigned *>(iloc64.data()), 2 * iloc64.size(), s)
+                 : f->d_iloc.upload(iloc.data(), iloc.size(), s)) ||
+      (rc = f->d_col.upload(cols.data(), cols.size(), s)) ||
       (rc = f->d_ienp.upload(ienp.data(), ienp.size(), s)) || (rc = f->d_xu.alloc((size_t)nshg * kXU)) ||
       (rc = f->d_node.alloc((size_t)nshg * kNRec)) || (rc = f->d_q.alloc((size_t)nshg * 9)) ||
       (rc = f->d_rec.alloc((size_t)std::max(nel, 1) * kRec)) ||
@@ -1938,7 +1999,7 @@ std::vector<unsigned long long> graph_signature(const crimson_form *f, const cri
   std::vector<unsigned long long> v = {
       f->d_ien.serial, f->d_inc_ptr.serial, f->d_inc.serial, f->d_diagk.serial, f->d_rowptr.serial,
       f->d_ibc.serial, f->d_lst_ptr.serial, f->d_order.serial, f->d_slot.serial, f->d_lst.serial,
-      f->d_ienp.serial, f->d_xu.serial, f->d_node.serial, f->d_rec.serial, f->d_esc.serial,
+      f->d_ienp.serial, f->d_iloc.serial, f->d_col.serial, f->d_xu.serial, f->d_node.serial, f->d_rec.serial, f->d_esc.serial,
       f->d_rec32.serial, f->d_bc.serial,
       f->d_bcl.serial, f->d_bcn.serial, f->d_inst.serial, f->d_mu_inst.serial, f->d_binst.serial,
       f->d_ienb.serial, f->d_bcode.serial, f->d_bcb.serial, f->d_permit.serial, f->d_brec.serial,

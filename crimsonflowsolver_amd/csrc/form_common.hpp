@@ -32,6 +32,8 @@ __host__ __device__ constexpr double mm(int a, int b) {
 constexpr int kRec = 32;
 __host__ __device__ constexpr int R_A(int a) { return 8 * a; }  // S[a][0..3], rl[a][0..3]
 constexpr int R_RL = 4;
+// Without the tangent: the residual rows alone, node a's at 4 a.
+constexpr int kRecRes = 16;
 // Element scalars: 4 doubles per element (Tc, Mu, Cm, tlW), from which with
 // the shape gradients every tangent entry is rebuilt.
 constexpr int kESc = 4;
@@ -43,6 +45,27 @@ constexpr int R_TLW = 12, R_TC = 13, R_MU = 14, R_CM = 15;
 // Packed node coordinates and velocity, 6 doubles per node (node_pack), the
 // gathers of the flux pass and of the assembly's shape gradients.
 constexpr int kXU = 6;
+// An incidence's element as its node's CSR row sees it: the other three nodes'
+// places among the row's blocks, in local order, and the node's own local
+// number a.  32 bits (10 per place) when no row has more than 1024 blocks, 64
+// bits (20 per place) otherwise.
+template <class IL>
+struct IncLoc {
+  static constexpr int bits = sizeof(IL) == 4 ? 10 : 20;
+  static constexpr IL mask = (IL(1) << bits) - 1;
+  __host__ static IL pack(const int (&o)[3], int a) {
+    return IL(o[0]) | IL(o[1]) << bits | IL(o[2]) << (2 * bits) | IL(a) << (3 * bits);
+  }
+  __device__ static int a(IL v) { return (int)(v >> (3 * bits) & 3); }
+  // the four nodes' places in local order, d the row's diagonal place
+  __device__ static void places(IL v, int d, int (&s)[4]) {
+    const int o0 = (int)(v & mask), o1 = (int)(v >> bits & mask), o2 = (int)(v >> (2 * bits) & mask), n = a(v);
+    s[0] = n == 0 ? d : o0;
+    s[1] = n == 0 ? o0 : n == 1 ? d : o1;
+    s[2] = n <= 1 ? o1 : n == 2 ? d : o2;
+    s[3] = n == 3 ? d : o2;
+  }
+};
 // lumped-mass weight of local node a, m_a = sum_q N_a(q) WdetJ (e3q.f90:120-145)
 __host__ __device__ inline double flux_weight(double W, int a) {
   return a == 0   ? nq(0, 0) * W + nq(1, 0) * W + nq(2, 0) * W + nq(3, 0) * W
@@ -51,7 +74,7 @@ __host__ __device__ inline double flux_weight(double W, int a) {
                   : nq(0, 3) * W + nq(1, 3) * W + nq(2, 3) * W + nq(3, 3) * W;
 }
 constexpr int kRowLanes = 16;   // lanes per CSR row in the assembly
-constexpr int kNodeLanes = 4;   // lanes per node in the flux/residual gathers
+constexpr int kNodeLanes = 4;   // lanes per node in the adjoint's gathers
 
 // Ensemble instances: per-element instance index and per-instance viscosity
 // (both null for a single instance, which uses FormConst::mu).
@@ -132,6 +155,16 @@ __host__ __device__ constexpr int qsym(int k) {
   return k == 0 ? 0 : k == 1 ? 1 : k == 2 ? 2 : k == 3 ? 1 : k == 4 ? 3 : k == 5 ? 4 : k == 6 ? 2 : k == 7 ? 4 : 5;
 }
 
+// A node's record.
+__device__ inline void load_record(const double *r, double (&nl)[kNRec]) {
+#pragma unroll
+  for (int k = 0; k < kNRec / 2; ++k) {
+    const double2 v = reinterpret_cast<const double2 *>(r)[k];
+    nl[2 * k] = v.x;
+    nl[2 * k + 1] = v.y;
+  }
+}
+
 inline FormConst make_const(const crimson_form_params &p) {
   FormConst c;
   c.rho = p.rho;
@@ -188,6 +221,9 @@ struct crimson_form {
   unsigned asm_xcd = 0;                     // assembly workgroups dealt per XCD turn (0: one range each)
   crimson::DBuf<unsigned short> d_lst;
   crimson::DBuf<int4> d_ienp;    // per incidence (node-major): the element's four nodes in local order
+  bool wide = false;                        // a row has more than 1024 blocks: IncLoc in 64 bits
+  crimson::DBuf<unsigned> d_iloc;            // IncLoc per incidence (node-major), two words each when wide
+  crimson::DBuf<int> d_col;                  // CSR columns
   crimson::DBuf<double> d_xu;    // (kXU, nshg): x and u of each node (node_pack)
   crimson::DBuf<double> d_node, d_q, d_rec, d_esc;  // node records; q; element records and scalars
   crimson::DBuf<float> d_rec32;  // FP32 tangent records (precision 32)
