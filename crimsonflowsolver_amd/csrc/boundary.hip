@@ -37,7 +37,7 @@ namespace {
 constexpr double kTriA = 0.3333333333333330000000000000000000;  // symtri.c:20
 constexpr double kTriB = 0.666666666666667;                     // symtri.c:21
 constexpr double kTriC = 0.166666666666667;                     // symtri.c:22
-constexpr int kBV = 17;  // boundary VJP record: (u1,u2,u3,p) cotangents of the 4 nodes, mu cotangent
+constexpr int kBV = 16;  // boundary VJP record: (u1,u2,u3,p) cotangents of the 4 nodes
 
 __device__ inline double tri_pt(int nqb, int q, int a) {
   if (nqb == 1) return kTriA;
@@ -228,9 +228,11 @@ __global__ void __launch_bounds__(256) bnd_vjp_elem(int nelb, int nshg, const in
                                                     const int *__restrict__ bcode, const int *__restrict__ permit,
                                                     int nsrf, int nqb, double influx, double rho, double mu0, Ens en,
                                                     const double *__restrict__ node, const double *__restrict__ w,
-                                                    double *__restrict__ vrec) {
-  const int e = xcd_block() * blockDim.x + threadIdx.x;
-  if (e >= nelb) return;
+                                                    double *__restrict__ vrec, double *__restrict__ part) {
+  __shared__ double sh_mu[256 / 64];
+  const unsigned blk = xcd_block();
+  const int er = blk * blockDim.x + threadIdx.x;
+  const int e = er < nelb ? er : nelb - 1;  // tail threads evaluate a valid element; nothing of theirs is stored
   const double mu = ens_mu(en, e, mu0);
   double xl[4][3], yl[4][4], wl[3][4];
   int g[4];
@@ -371,14 +373,17 @@ __global__ void __launch_bounds__(256) bnd_vjp_elem(int nelb, int nshg, const in
 #pragma unroll
       for (int a = 0; a < 4; ++a) ub[a][kp] += db * Gn[a][j];
     }
-  double *o = vrec + (size_t)e * kBV;
+  if (er < nelb) {
+    double *o = vrec + (size_t)e * kBV;
 #pragma unroll
-  for (int a = 0; a < 4; ++a) {
+    for (int a = 0; a < 4; ++a) {
 #pragma unroll
-    for (int i = 0; i < 3; ++i) o[4 * a + i] = ub[a][i];
-    o[4 * a + 3] = a < 3 ? pb[a] : 0.0;
+      for (int i = 0; i < 3; ++i) o[4 * a + i] = ub[a][i];
+      o[4 * a + 3] = a < 3 ? pb[a] : 0.0;
+    }
   }
-  o[16] = mub;
+  const double ms = block_sum<256>(er < nelb ? mub : 0.0, sh_mu);
+  if (threadIdx.x == 0) part[blk] = ms;
 }
 
 // ybar(node, :) += the boundary records of its incidences (all four tet
@@ -400,21 +405,6 @@ __global__ void __launch_bounds__(256) bnd_vjp_node(int nvn, int nshg, const int
   }
 #pragma unroll
   for (int k = 0; k < 4; ++k) ybar[i + (size_t)nshg * k] = r[k];
-}
-
-// sum of the boundary elements' mu cotangents, one workgroup, fixed order
-__global__ void __launch_bounds__(256) bnd_vjp_mu(int nelb, const double *__restrict__ vrec,
-                                                  double *__restrict__ out) {
-  __shared__ double sh[256];
-  double s = 0.0;
-  for (int e = threadIdx.x; e < nelb; e += 256) s += vrec[(size_t)e * kBV + 16];
-  sh[threadIdx.x] = s;
-  __syncthreads();
-  for (int w = 128; w > 0; w >>= 1) {
-    if ((int)threadIdx.x < w) sh[threadIdx.x] += sh[threadIdx.x + w];
-    __syncthreads();
-  }
-  if (threadIdx.x == 0) *out = sh[0];
 }
 
 }  // namespace
@@ -483,9 +473,9 @@ int form_boundary_pass(crimson_form *f, double *d_res, int mode) {
   CR_HIP(hipGetLastError());
   return CRIMSON_OK;
 }
-size_t form_boundary_vjp_doubles(const crimson_form *f) { return f->nelb ? (size_t)kBV * f->nelb + 1 : 0; }
-int form_boundary_vjp(crimson_form *f, const double *d_w, double *d_ybar, double *mubar, double *d_bvrec) {
-  *mubar = 0.0;
+size_t form_boundary_vjp_doubles(const crimson_form *f) { return (size_t)kBV * f->nelb; }
+int form_boundary_vjp_parts(const crimson_form *f) { return f->nelb ? (int)grid_for(f->nelb, 256) : 0; }
+int form_boundary_vjp(crimson_form *f, const double *d_w, double *d_ybar, double *d_part, double *d_bvrec) {
   if (f->nelb == 0) return CRIMSON_OK;
   hipStream_t s = f->stream;
   if (!d_bvrec) {
@@ -495,14 +485,10 @@ int form_boundary_vjp(crimson_form *f, const double *d_w, double *d_ybar, double
   bnd_vjp_elem<<<grid_for(f->nelb, 256), 256, 0, s>>>(f->nelb, f->nshg, f->d_ienb.p, f->d_bcode.p,
                                                       f->nsrf >= 0 ? f->d_permit.p : nullptr, f->nsrf, f->nqb,
                                                       f->influx, f->prm.rho, f->prm.mu, f->bens(), f->d_node.p, d_w,
-                                                      d_bvrec);
+                                                      d_bvrec, d_part);
   bnd_vjp_node<<<grid_for(f->nvnode, 256), 256, 0, s>>>(f->nvnode, f->nshg, f->d_vnode.p, f->d_vptr.p,
                                                         f->d_vinc.p, d_bvrec, d_ybar);
-  double *d_mu = d_bvrec + (size_t)kBV * f->nelb;
-  bnd_vjp_mu<<<1, 256, 0, s>>>(f->nelb, d_bvrec, d_mu);
   CR_HIP(hipGetLastError());
-  CR_HIP(hipMemcpyAsync(mubar, d_mu, sizeof(double), hipMemcpyDeviceToHost, s));
-  CR_HIP(hipStreamSynchronize(s));
   return CRIMSON_OK;
 }
 }  // namespace crimson

@@ -51,14 +51,6 @@
 
 namespace {
 
-// Orders LDS accesses of the lanes of one wavefront (the lanes of a node or
-// CSR row always share a wavefront).
-__device__ inline void wave_lds_sync() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
 // ---------------------------------------------------------------- flux pass
 // x and u of every node packed as kXU doubles: the flux pass gathers a
 // node's x and u in three 16-byte loads, the assembly its x in two loads.
@@ -81,25 +73,6 @@ __global__ void __launch_bounds__(256) node_pack(int nshg, const double *__restr
 // gathers: it is bound by its sums, and its rows staged this way took 1,600 us
 // instead of 1,535.)
 constexpr int kFluxLanes = 8, kFluxCap = 20;
-// LANES lanes load the row's first CAP blocks' x and u, three 16-byte pieces each.
-template <int LANES, int CAP>
-__device__ inline void stage_row_xu(int lane, int k0, int n, const int *__restrict__ col,
-                                    const double *__restrict__ xu, double *sh) {
-  constexpr int kU = (CAP * 3 + LANES - 1) / LANES;
-  const int m = min(n, CAP) * 3;
-  double2 v[kU];
-#pragma unroll
-  for (int u = 0; u < kU; ++u) {
-    const int i = min(lane + LANES * u, m - 1);  // a row has its diagonal block at least
-    v[u] = reinterpret_cast<const double2 *>(xu + (size_t)col[k0 + i / 3] * kXU)[i % 3];
-  }
-#pragma unroll
-  for (int u = 0; u < kU; ++u) {
-    const int i = lane + LANES * u;
-    if (i < m) reinterpret_cast<double2 *>(sh)[i] = v[u];
-  }
-}
-
 __device__ inline void load_xu(const double *p, double (&x)[3], double (&u)[3]) {
   const double2 *r = reinterpret_cast<const double2 *>(p);
   x[0] = r[0].x;
@@ -159,7 +132,7 @@ __global__ void __launch_bounds__(256) flux_node(int nshg, const int *__restrict
   double rest = 0.0;
   if (lane < 4) rest = lane == 0 ? y[ii + 3 * N] : ac[ii + (lane - 1) * N];
   IL il = p0 + lane < p1 ? iloc[p0 + lane] : IL(0);
-  stage_row_xu<kFluxLanes, kFluxCap>(lane, k0, ns, col, xu, xs);
+  stage_row<kFluxLanes, kFluxCap, 3, kXU>(lane, k0, ns, col, xu, xs);
   wave_lds_sync();
   auto get = [&](int s, double (&x)[3], double (&u)[3]) {
     // (an either-or would become one flat load of both kinds of memory)
@@ -237,8 +210,6 @@ __global__ void __launch_bounds__(256) flux_node(int nshg, const int *__restrict
 // 557 now; without the tangent 663 before, 411 now).
 // In: the nodal values.  Out: u -> ubar at the points, a -> (a + ubar . grad u) at
 // the points (RES), g of the first three nodes (g_4 is minus their sum), WdetJ.
-__host__ __device__ constexpr double w_other(int a) { return nq(a == 0 ? 1 : 0, a); }
-__host__ __device__ constexpr double w_diff(int a) { return nq(a, a) - w_other(a); }
 template <class T, bool RES, bool TAN>
 struct E3Sums {
   T g[3][3], W, gu[3][3], SU[3], SR[3], A[6], B[6], C[3][3], TC, TM, divu;

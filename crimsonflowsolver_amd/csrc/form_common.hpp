@@ -57,6 +57,11 @@ struct IncLoc {
     return IL(o[0]) | IL(o[1]) << bits | IL(o[2]) << (2 * bits) | IL(a) << (3 * bits);
   }
   __device__ static int a(IL v) { return (int)(v >> (3 * bits) & 3); }
+  __device__ static void others(IL v, int (&o)[3]) {
+    o[0] = (int)(v & mask);
+    o[1] = (int)(v >> bits & mask);
+    o[2] = (int)(v >> (2 * bits) & mask);
+  }
   // the four nodes' places in local order, d the row's diagonal place
   __device__ static void places(IL v, int d, int (&s)[4]) {
     const int o0 = (int)(v & mask), o1 = (int)(v >> bits & mask), o2 = (int)(v >> (2 * bits) & mask), n = a(v);
@@ -74,7 +79,11 @@ __host__ __device__ inline double flux_weight(double W, int a) {
                   : nq(0, 3) * W + nq(1, 3) * W + nq(2, 3) * W + nq(3, 3) * W;
 }
 constexpr int kRowLanes = 16;   // lanes per CSR row in the assembly
-constexpr int kNodeLanes = 4;   // lanes per node in the adjoint's gathers
+
+// The rule's weights, N_a at another node's point and how much more at its own: sum_q
+// N_a(q) f_q = w_other(a) sum_q f_q + w_diff(a) f_a.
+__host__ __device__ constexpr double w_other(int a) { return nq(a == 0 ? 1 : 0, a); }
+__host__ __device__ constexpr double w_diff(int a) { return nq(a, a) - w_other(a); }
 
 // Ensemble instances: per-element instance index and per-instance viscosity
 // (both null for a single instance, which uses FormConst::mu).
@@ -162,6 +171,47 @@ __device__ inline void load_record(const double *r, double (&nl)[kNRec]) {
     const double2 v = reinterpret_cast<const double2 *>(r)[k];
     nl[2 * k] = v.x;
     nl[2 * k + 1] = v.y;
+  }
+}
+
+// Orders LDS accesses of the lanes of one wavefront (the lanes of a node or
+// CSR row always share a wavefront).
+__device__ inline void wave_lds_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// Sum over the workgroup, in a fixed order, on thread 0.
+template <int THREADS>
+__device__ inline double block_sum(double v, double (&sh)[THREADS / 64]) {
+#pragma unroll
+  for (int off = 1; off < 64; off <<= 1) v += __shfl_xor(v, off, 64);
+  if (threadIdx.x % 64 == 0) sh[threadIdx.x / 64] = v;
+  __syncthreads();
+  double s = 0.0;
+#pragma unroll
+  for (int k = 0; k < THREADS / 64; ++k) s += sh[k];
+  return s;
+}
+
+// LANES lanes load the first 2 PIECES doubles (16-byte pieces) of the records (of
+// STRIDE doubles) of the row's first CAP blocks into LDS, packed.
+template <int LANES, int CAP, int PIECES, int STRIDE>
+__device__ inline void stage_row(int lane, int k0, int n, const int *__restrict__ col, const double *__restrict__ src,
+                                 double *sh) {
+  constexpr int kU = (CAP * PIECES + LANES - 1) / LANES;
+  const int m = min(n, CAP) * PIECES;
+  double2 v[kU];
+#pragma unroll
+  for (int u = 0; u < kU; ++u) {
+    const int i = min(lane + LANES * u, m - 1);  // a row has its diagonal block at least
+    v[u] = reinterpret_cast<const double2 *>(src + (size_t)col[k0 + i / PIECES] * STRIDE)[i % PIECES];
+  }
+#pragma unroll
+  for (int u = 0; u < kU; ++u) {
+    const int i = lane + LANES * u;
+    if (i < m) reinterpret_cast<double2 *>(sh)[i] = v[u];
   }
 }
 
@@ -302,11 +352,13 @@ int form_wall_rows(crimson_form *f);
 // The ensemble instance of each boundary element (after either of
 // crimson_form_set_boundary / crimson_form_set_instances changes).
 int form_boundary_instances(crimson_form *f);
-// Adjoint of the boundary rows: ybar(nshg,4) += w^T d rl_bnd/d y from the
-// node records of the last flux pass; *mubar = w^T d rl_bnd/d mu.  d_bvrec:
-// a workspace of form_boundary_vjp_doubles(f) doubles, or null for the
-// handle's own (allocated on first use).
-int form_boundary_vjp(crimson_form *f, const double *d_w, double *d_ybar, double *mubar, double *d_bvrec);
+// Adjoint of the boundary rows, enqueued: ybar(nshg,4) += w^T d rl_bnd/d y from
+// the node records of the last flux pass; d_part: the
+// form_boundary_vjp_parts(f) workgroups' parts of w^T d rl_bnd/d mu.  d_bvrec: a
+// workspace of form_boundary_vjp_doubles(f) doubles, or null for the handle's own
+// (allocated on first use).
+int form_boundary_vjp(crimson_form *f, const double *d_w, double *d_ybar, double *d_part, double *d_bvrec);
+int form_boundary_vjp_parts(const crimson_form *f);
 size_t form_boundary_vjp_doubles(const crimson_form *f);
 // Device workspaces of one VJP (crimson_form_vjp_dev): the element records,
 // qbar, 1/rmass, the mu partial sums and the boundary records (null without
