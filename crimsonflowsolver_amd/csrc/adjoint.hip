@@ -55,7 +55,7 @@ constexpr int kVjpCap2 = 16;   // by vjp_node: 40 KB a workgroup, four workgroup
 // The rule's weights (one at the point's own node, another at the rest) give
 // sum_q N_a(q) f_q = w_other(a) sum f + w_diff(a) f_a.  The records are staged in
 // LDS and stored as one block per workgroup, coalesced.  Bound by latency at two
-// waves a SIMD, as e3_elem.  2.2 M elements: 470 us with every point's terms written
+// waves a SIMD, as e3_elem.  1.7 M elements: 470 us with every point's terms written
 // out and 448-byte records stored per thread, 186 so.
 // What a point does not need is parked in LDS (a thread's own slots, bank-conflict
 // free): a and w of the nodes (a's place takes its cotangent) and g.  Kept in
@@ -322,7 +322,7 @@ __device__ inline double own_gradient(const double (&xa)[3], const double (&x0)[
 // summed over the node's incidences (fixed lanes and shuffle tree), times
 // 1/rmass; written with the node's x as its packed record.  The gradient is rebuilt
 // from the row's coordinates (staged in LDS) rather than read: an element then
-// passes 32 bytes on instead of 192.  386 k nodes: 167 us from the records, 65 so.
+// passes 32 bytes on instead of 192.  306 k nodes: 167 us from the records, 65 so.
 template <class IL>
 __global__ void __launch_bounds__(256) vjp_q_node(int nshg, const int *__restrict__ rowptr,
                                                   const int *__restrict__ diagk, const int *__restrict__ col,
@@ -411,7 +411,7 @@ __global__ void __launch_bounds__(256) vjp_q_node(int nshg, const int *__restric
 // viscous flux qdi = mu (grad u + grad u^T) (elem_flux's slots
 // 11,12,13,22,23,33) enters q at its nodes with weight m_a / rmass, so with Q =
 // sum_a m_a qbar_a as a symmetric form (Q_ij twice on the diagonal) ybar_a gets
-// mu t, t = Q g_a, and mubar gets sum_a u_a . t.  386 k nodes: 289 us and 147 us for
+// mu t, t = Q g_a, and mubar gets sum_a u_a . t.  306 k nodes: 289 us and 147 us for
 // an element pass that wrote 128-byte records for it, 159 so (122 are the records).
 template <class IL, bool AC>
 __global__ void __launch_bounds__(256) vjp_node(int nshg, const int *__restrict__ rowptr,

@@ -68,7 +68,7 @@ __global__ void __launch_bounds__(256) node_pack(int nshg, const double *__restr
 // The x and u of a row's neighbours staged in LDS: kFluxCap of the row's
 // blocks per node, kXU doubles each; later blocks are read from memory.  A row's
 // 24 incidences name its 14 neighbours 72 times; gathered per incidence, the
-// address units were busy 96 % of flux_node's time.  1.3 M nodes (64 x 64 x 320
+// address units were busy 96 % of flux_node's time.  1.08 M nodes (64 x 64 x 320
 // Kuhn cells), node_pack included: 353 us gathered, 295 staged.  (The assembly
 // gathers: it is bound by its sums, and its rows staged this way took 1,600 us
 // instead of 1,535.)
@@ -206,7 +206,7 @@ __global__ void __launch_bounds__(256) flux_node(int nshg, const int *__restrict
 // (w_own(a) - w_other(a)) f_a.  tauM and tauBar take a reciprocal square root each.  Written
 // term by term per point (the form of e3res.f90 and e3lhs.f90) the kernel issued
 // 1,763 vector instructions per wave, this 1,117; it is bound by latency at two
-// waves a SIMD and by the record stores (1.8 GB at 7.9 M elements: 672 us before,
+// waves a SIMD and by the record stores (1.8 GB at 6.2 M elements: 672 us before,
 // 557 now; without the tangent 663 before, 411 now).
 // In: the nodal values.  Out: u -> ubar at the points, a -> (a + ubar . grad u) at
 // the points (RES), g of the first three nodes (g_4 is minus their sum), WdetJ.
@@ -372,7 +372,7 @@ __device__ inline void e3_tangent(const FormConst &c, const T (&ub)[4][3], const
 // alone: kRecRes doubles, one line per element.
 constexpr int kE3Threads = 128;
 // Workgroups dealt to the XCDs in turns of this many: the records of
-// neighbouring elements are written at the same time (7.9 M elements: 678 us with
+// neighbouring elements are written at the same time (6.2 M elements: 678 us with
 // one range per XCD, 647 in turns).  The nodes are gathered per element: staged
 // in LDS once per workgroup they cost 60 us more than the gathers save.
 constexpr unsigned kE3XcdChunk = 64;
@@ -666,7 +666,7 @@ __device__ inline void put_res(double *res, int i, int nshg, const double (&rs)[
 }
 
 // kResLanes lanes per node, each with its incidences' records all in flight
-// (three per lane on a Kuhn mesh's 24).  1.3 M nodes: 430 us with four lanes, one
+// (three per lane on a Kuhn mesh's 24).  1.08 M nodes: 430 us with four lanes, one
 // record at a time out of the 256-byte records of the tangent's layout, 248 so.
 constexpr int kResLanes = 8, kResUnroll = 3;
 template <int MODE>

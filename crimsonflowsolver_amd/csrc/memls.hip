@@ -1061,7 +1061,8 @@ __global__ void gt_kernel(size_t nnz, const T *__restrict__ V, const int *__rest
 }
 
 // ----- CG (device-resident iterations with a convergence flag) -----
-// Three launches per iteration on the Schur complement: SP = S P with the
+// Three launches per iteration (two on a formed Schur complement of up to kCgPaired
+// rows, below): SP = S P with the
 // parts of P . SP (s_product_kernel), the residual update with the parts of
 // R . R, and the direction update, which also advances the state.  Every
 // workgroup sums the parts it needs itself, in one fixed order, so that no
@@ -1070,7 +1071,7 @@ __global__ void gt_kernel(size_t nnz, const T *__restrict__ V, const int *__rest
 // launches (28.3 us of kernels per iteration at 36,000 nodes, 120 us at
 // 458,000).
 // The state is kept twice (kCgState doubles each): iteration k reads copy k & 1 and
-// the direction update writes the other, so that no workgroup reads what
+// the direction update (paired: the product) writes the other, so that no workgroup reads what
 // another is writing.
 // State: 0 err, 1 errO, 2 eps2, 3 alpha, 5 done, 6 itr, 7 mItr, 8 suc.
 constexpr int kCgState = 16;
@@ -1160,20 +1161,41 @@ __global__ void __launch_bounds__(256) cg_den_kernel(size_t L, const T *__restri
 }
 // R -= alpha SP (with the faces' rank-one terms), alpha = errO / (P . SP);
 // the workgroup's part of R . R.  E entries per thread and turn (cg_grid).
-template <class T, int E>
+// PAIR (the formed Schur complement): R sits in Q, which takes P too, and X +=
+// alpha P is done here.
+template <class T>
+struct Pair;
+template <>
+struct Pair<double> {
+  using type = double2;
+};
+template <>
+struct Pair<float> {
+  using type = float2;
+};
+template <class T>
+using PairT = typename Pair<T>::type;
+template <class T, int E, bool PAIR>
 __global__ void __launch_bounds__(256) cg_r_kernel(size_t L, double *__restrict__ scal,
                                                    const double *__restrict__ dpart, int nd, FaceList fl,
                                                    T *__restrict__ R, const T *__restrict__ SP,
-                                                   double *__restrict__ rpart) {
+                                                   double *__restrict__ rpart, PairT<T> *__restrict__ Q,
+                                                   T *__restrict__ X, const T *__restrict__ P) {
   __shared__ double sh[4];
   __shared__ T corr[E * 256];
   const double stop = scal[5], errO = scal[1];
-  T r[E], sp[E];
+  T r[E], sp[E], x[E], p[E];
   auto load = [&](size_t base) {
 #pragma unroll
     for (int t = 0; t < E; ++t) {
       const size_t e = base + threadIdx.x + 256 * t;
-      r[t] = e < L ? R[e] : T(0);
+      if constexpr (PAIR) {
+        r[t] = e < L ? Q[e].x : T(0);
+        x[t] = e < L ? X[e] : T(0);
+        p[t] = e < L ? P[e] : T(0);
+      } else {
+        r[t] = e < L ? R[e] : T(0);
+      }
       sp[t] = e < L ? SP[e] : T(0);
     }
   };
@@ -1224,7 +1246,12 @@ __global__ void __launch_bounds__(256) cg_r_kernel(size_t L, double *__restrict_
       const size_t e = base + threadIdx.x + 256 * t;
       if (e < L) {
         const T v = r[t] - alpha * sp[t];
-        R[e] = v;
+        if constexpr (PAIR) {
+          Q[e] = PairT<T>{v, p[t]};
+          X[e] = x[t] + alpha * p[t];
+        } else {
+          R[e] = v;
+        }
         s += (double)v * (double)v;
       }
     }
@@ -1295,6 +1322,152 @@ __global__ void __launch_bounds__(256) cg_p_kernel(size_t L, const double *__res
     base += (size_t)(gridDim.x - nf) * (E * 256);
     if (base < L) load(base);
   }
+}
+
+// ----- the CG on the formed Schur complement: two launches per iteration -----
+// The residual and the direction sit together, Q(j) = (R, P), one 16-byte entry
+// (8 in FP32): the product gathers Q and takes the new direction R + beta P of
+// every column as it goes, so that no sweep stands between the residual update
+// and the product.  Taken up to kCgPaired rows, where a launch costs more than the
+// wider gather.  Whole NS solves of the workloads' iteration counts, three launches
+// and two: 21,800 rows 9.6 and 8.6 ms, 36,000 15.9 and 15.1, 50,000 15.6 and 14.9,
+// 68,000 17.1 and 17.2, 141,000 28.0 and 28.9 (FP32: 4.2 and 3.7, 4.7 and 4.5, 4.9
+// and 4.7, 6.5 and 6.4, 10.2 and 10.4).
+constexpr int kCgPaired = 1 << 16;
+// Q = (X, 0), X = 0
+template <class T>
+__global__ void __launch_bounds__(256) cg_pair_kernel(size_t L, T *__restrict__ X, PairT<T> *__restrict__ Q,
+                                                      const double *__restrict__ skip) {
+  if (skip && *skip != 0.0) return;
+  const size_t e = (size_t)blockIdx.x * 256 + threadIdx.x;
+  if (e >= L) return;
+  Q[e] = PairT<T>{X[e], T(0)};
+  X[e] = T(0);
+}
+// The state after the iteration whose residual's parts are rpart[0, nr): err = R .
+// R and the next test; returns beta = err / errO.
+__device__ inline double cg_advance(const double *__restrict__ scal, const double *__restrict__ rpart, int nr,
+                                    double (&st)[kCgState], double *sh) {
+  const double n = sqrt(sum_parts(rpart, nr, 0.0, sh));  // NORMS(R)
+  const double err = n * n, beta = err / scal[1];
+#pragma unroll
+  for (int k = 0; k < kCgState; ++k) st[k] = scal[k];
+  st[0] = err;
+  check_next(st);
+  return beta;
+}
+// The state after the last iteration (a captured loop's end).
+__global__ void __launch_bounds__(256) cg_close_kernel(const double *__restrict__ scal, double *__restrict__ next,
+                                                       const double *__restrict__ rpart, int nr) {
+  __shared__ double sh[4];
+  double st[kCgState];
+  if (scal[5] != 0.0) {
+    if (threadIdx.x < kCgState) next[threadIdx.x] = scal[threadIdx.x];
+    return;
+  }
+  (void)cg_advance(scal, rpart, nr, st, sh);
+  if (threadIdx.x == 0)
+    for (int k = 0; k < kCgState; ++k) next[k] = st[k];
+}
+// The new direction P = R + beta P of every row, SP = S P and the workgroup's part
+// of P . SP, 16 lanes per row; the first workgroups take the faces' dots with P.
+// next null: the first iteration (beta 0, no state to advance).  The first rows'
+// entries are in flight while the residual's parts are summed.
+template <class T, class OX>
+__global__ void __launch_bounds__(256) s_dir_product_kernel(int nNo, int ntile, const int *__restrict__ sptr,
+                                                        const OX *__restrict__ scol, const T *__restrict__ S,
+                                                        const PairT<T> *__restrict__ Q, T *__restrict__ P,
+                                                        T *__restrict__ SP, double *__restrict__ dpart,
+                                                        const double *__restrict__ scal, double *__restrict__ next,
+                                                        const double *__restrict__ rpart, int nr, FaceList fl,
+                                                        HostFlag hf) {
+  __shared__ double sh[4];
+  const double stop = scal[5];
+  const int nf = fl.nfc * kFaceDotBlocks, blk = (int)blockIdx.x - nf, nwg = (int)gridDim.x - nf;
+  const int lane = threadIdx.x % kSLanes;
+  auto row_of = [&](int vb) {
+    return (int)crimson::xcd_block(kRowXcdChunk, vb, ntile) * (256 / kSLanes) + (int)threadIdx.x / kSLanes;
+  };
+  int row = 0, kb = 0, ke = 0;
+  T v[kSUnroll];
+  PairT<T> x[kSUnroll], own;
+  auto load = [&](int k) {
+    int j[kSUnroll];
+#pragma unroll
+    for (int u = 0; u < kSUnroll; ++u) {
+      const int kc = max(min(k + kSLanes * u, ke - 1), 0);
+      j[u] = col_at(scol, kc, row);
+      v[u] = S[kc];
+    }
+#pragma unroll
+    for (int u = 0; u < kSUnroll; ++u) x[u] = Q[min((unsigned)j[u], (unsigned)nNo - 1u)];  // (a row past the end or empty)
+  };
+  if (blk >= 0) {
+    row = row_of(blk);
+    kb = sptr[min(row, nNo)];
+    ke = sptr[min(row + 1, nNo)];  // rows past the last one: kb = ke
+    own = Q[min(row, nNo - 1)];
+    load(kb + lane);
+  }
+  double beta = 0.0;
+  if (next) {
+    if (stop != 0.0) {
+      if (blockIdx.x == 0 && threadIdx.x < kCgState) next[threadIdx.x] = scal[threadIdx.x];
+      if (blockIdx.x == 0 && threadIdx.x == 0) hf.tell(true);
+      return;
+    }
+    double st[kCgState];
+    beta = cg_advance(scal, rpart, nr, st, sh);
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+      for (int k = 0; k < kCgState; ++k) next[k] = st[k];
+      hf.tell(st[5] != 0.0);
+    }
+    if (st[5] != 0.0) return;
+  } else if (stop != 0.0) {
+    return;
+  }
+  const T bt = (T)beta;
+  if (blk < 0) {
+    face_part(fl, blockIdx.x, sh, [&](int j) {
+      const PairT<T> q = Q[j];
+      return q.x + bt * q.y;
+    });
+    return;
+  }
+  double den = 0.0;
+  for (int vb = blk;;) {
+    const int vn = vb + nwg;
+    int rown = 0, kbn = 0, ken = 0;
+    if (vn < ntile) {
+      rown = row_of(vn);
+      kbn = sptr[min(rown, nNo)];
+      ken = sptr[min(rown + 1, nNo)];
+    }
+    T acc = T(0);
+    for (int k = kb + lane; k < ke; k += kSLanes * kSUnroll) {
+      if (k != kb + lane) load(k);
+#pragma unroll
+      for (int u = 0; u < kSUnroll; ++u)
+        if (k + kSLanes * u < ke) acc += v[u] * (x[u].x + bt * x[u].y);
+    }
+#pragma unroll
+    for (int off = kSLanes / 2; off > 0; off >>= 1) acc += __shfl_xor(acc, off, kSLanes);
+    if (row < nNo && lane == 0) {
+      const T pr = own.x + bt * own.y;
+      P[row] = pr;
+      SP[row] = acc;
+      den += (double)pr * (double)acc;
+    }
+    if (vn >= ntile) break;
+    vb = vn;
+    row = rown;
+    kb = kbn;
+    ke = ken;
+    own = Q[min(row, nNo - 1)];
+    load(kb + lane);
+  }
+  den = block_sum(den, sh);
+  if (threadIdx.x == 0) dpart[blk] = den;
 }
 }  // namespace
 
@@ -1479,11 +1652,13 @@ int cg_sweeps(Ctx<T> &c, size_t L, int it, int nd, const CgAux<T> &ax, T *X, T *
   const CgGrid g = cg_grid(L);
   const int gp = g.blocks + ax.fl.nfc * kFaceDotBlocks;
   if (g.entries == 1) {
-    cg_r_kernel<T, 1><<<g.blocks, 256, 0, c.s>>>(L, scal, dpart, nd, ax.fl, R, SP, rpart);
+    cg_r_kernel<T, 1, false><<<g.blocks, 256, 0, c.s>>>(L, scal, dpart, nd, ax.fl, R, SP, rpart, nullptr, nullptr,
+                                                        nullptr);
     cg_p_kernel<T, 1><<<gp, 256, 0, c.s>>>(L, scal, next, rpart, g.blocks, ax.fl, X, R, P, Pn, ax.W, ax.wdof, ax.off,
                                            ax.Ps, hf);
   } else {
-    cg_r_kernel<T, 4><<<g.blocks, 256, 0, c.s>>>(L, scal, dpart, nd, ax.fl, R, SP, rpart);
+    cg_r_kernel<T, 4, false><<<g.blocks, 256, 0, c.s>>>(L, scal, dpart, nd, ax.fl, R, SP, rpart, nullptr, nullptr,
+                                                        nullptr);
     cg_p_kernel<T, 4><<<gp, 256, 0, c.s>>>(L, scal, next, rpart, g.blocks, ax.fl, X, R, P, Pn, ax.W, ax.wdof, ax.off,
                                            ax.Ps, hf);
   }
@@ -1614,6 +1789,25 @@ int schur_form(Ctx<T> &c, const SchurOp<T> &o) {
   else
     CR_SV(int, l->d_col.p, int, l->d_scol.p);
 #undef CR_SV
+  CR_HIP(hipGetLastError());
+  return CRIMSON_OK;
+}
+// SP = S P of the formed complement with the new direction and the parts of P . SP.
+template <class T>
+int schur_dir_product(Ctx<T> &c, const PairT<T> *Q, T *P, T *SP, const double *scal, double *next, int nr,
+                  const FaceList &fl, HostFlag hf, int &nd) {
+  crimson_lhs *l = c.lhs;
+  const int N = l->nNo, ntile = (int)crimson::grid_for((size_t)N, 256 / kSLanes);
+  nd = std::min(ntile, kCgGrid);
+  const int G = nd + fl.nfc * kFaceDotBlocks;
+  const T *S = schur_buf(l, T(0)).p;
+  double *dpart = c.part.p, *rpart = c.part.p + kCgGrid;
+  if (l->d_scol16.p)
+    s_dir_product_kernel<T, short><<<G, 256, 0, c.s>>>(N, ntile, l->d_sptr.p, l->d_scol16.p, S, Q, P, SP, dpart, scal,
+                                                   next, rpart, nr, fl, hf);
+  else
+    s_dir_product_kernel<T, int><<<G, 256, 0, c.s>>>(N, ntile, l->d_sptr.p, l->d_scol.p, S, Q, P, SP, dpart, scal, next,
+                                                 rpart, nr, fl, hf);
   CR_HIP(hipGetLastError());
   return CRIMSON_OK;
 }
@@ -2121,12 +2315,13 @@ template <class T>
 struct SolveWork : crimson::SolveWorkBase {
   Ctx<T> c;
   crimson::DBuf<T> r0, r, X, MX;          // NS: (3,N)|(N) vectors; X: U_i|P_i, MX: their images
-  crimson::DBuf<T> t3, t4, t5, ps, z;     // CG: R, the two directions; two-pass operator: Ps, Z
+  crimson::DBuf<T> t3, t4, t5, ps, z;     // CG: R (paired: Q), the directions; two-pass operator: Ps, Z
   crimson::DBuf<T> wa, wb, ws, gmU;       // GMRES: the two working vectors, W o w, the basis
   crimson::DBuf<double> gst, npart, h;    // state and small systems; norm parts (2 kSubGrid); h1, h2
   int sD = 0, nB = 0, mRI = 0, mGM = 0, mCG = 0;
   double riAbs = 0, riRel = 0, gmAbs = 0, gmRel = 0, cgAbs = 0, cgRel = 0;
   bool formed = false;    // the Schur complement is formed (schur_ready)
+  bool paired = false;    // its CG keeps R and P together (kCgPaired)
   SegCapture *cap = nullptr;  // the capture in progress, cut between the solve's phases
   size_t oH = 0, ocs = 0, osn = 0, oerr = 0, oy = 0, oA = 0, oBv = 0, oxB = 0, oC = 0, ocu = 0, ocp = 0;
   // a plain solve's flag word (pinned) and the number of its last teller
@@ -2337,6 +2532,43 @@ int cg_run(SolveWork<T> &w, size_t L, T *X, Op op, T *R, T *P, T *P2, T *SP, con
   return CRIMSON_OK;
 }
 
+// cg_run on the formed Schur complement in two launches (s_dir_product_kernel, cg_r_kernel<PAIR>).
+template <class T>
+int cg_run_paired(SolveWork<T> &w, size_t L, T *X, PairT<T> *Q, T *P, T *SP, const FaceList &fl, double absTol,
+                  double relTol, int mItr, double *g, const double *skip, double **state) {
+  Ctx<T> &c = w.c;
+  CR_TRY(dots(c, L, X, static_cast<const T *>(nullptr), 0, 0, true, c.part.p, skip));
+  cg_begin_kernel<<<1, kDotThreads, 0, c.s>>>(c.cgst.p, g, skip, c.part.p, dot_blocks(L), absTol, relTol, mItr);
+  cg_pair_kernel<T><<<crimson::grid_for(L, 256), 256, 0, c.s>>>(L, X, Q, skip);
+  const CgGrid cg = cg_grid(L);
+  double *dpart = c.part.p, *rpart = c.part.p + kCgGrid;
+  auto st = [&](int it) { return c.cgst.p + (it & 1) * kCgState; };
+  const unsigned long long s0 = w.seq;
+  int it = 0;
+  // the product of iteration it tells whether the solve ended with iteration it - 1,
+  // so a plain solve runs past mItr by its lag at most
+  for (; w.polled || it < mItr; ++it) {
+    int nd = 0;
+    CR_TRY(schur_dir_product(c, Q, P, SP, it ? st(it - 1) : st(0), it ? st(it) : nullptr, cg.blocks, fl,
+                         it ? w.flag() : HostFlag{nullptr, 0}, nd));
+    if (cg.entries == 1)
+      cg_r_kernel<T, 1, true><<<cg.blocks, 256, 0, c.s>>>(L, st(it), dpart, nd, fl, nullptr, SP, rpart, Q, X, P);
+    else
+      cg_r_kernel<T, 4, true><<<cg.blocks, 256, 0, c.s>>>(L, st(it), dpart, nd, fl, nullptr, SP, rpart, Q, X, P);
+    CR_HIP(hipGetLastError());
+    bool stop = false;
+    if (w.polled && it > kCgLag) CR_TRY(w.wait(s0 + it - kCgLag, &stop));
+    if (stop) {
+      *state = st(it);
+      return CRIMSON_OK;
+    }
+  }
+  if (it > 0) cg_close_kernel<<<1, 256, 0, c.s>>>(st(it - 1), st(it), rpart, cg.blocks);
+  CR_HIP(hipGetLastError());
+  *state = st(it);
+  return CRIMSON_OK;
+}
+
 // NSSOLVER (memLS.f90:1460-1759) on d_Ri (4, N), PRECOND's W applied on the
 // way in and out.
 template <class T>
@@ -2405,8 +2637,12 @@ int ns_run(SolveWork<T> &w, double *d_Ri) {
     CR_TRY(w.cut());
     CR_TRY(spmv(c, mD, 1, 3, Ui, Pi, -1.0, w.r.p + mn, 1.0, ri));  // P = Rc - D U
     double *state = nullptr;
-    CR_TRY(cg_run(w, (size_t)N, Pi, schur_op, w.t3.p, w.t4.p, w.t5.p, MPb, ax, w.cgAbs, w.cgRel, w.mCG, g, ri,
-                  &state));
+    if (w.paired)
+      CR_TRY(cg_run_paired(w, (size_t)N, Pi, reinterpret_cast<PairT<T> *>(w.t3.p), w.t4.p, MPb, ax.fl, w.cgAbs,
+                           w.cgRel, w.mCG, g, ri, &state));
+    else
+      CR_TRY(cg_run(w, (size_t)N, Pi, schur_op, w.t3.p, w.t4.p, w.t5.p, MPb, ax, w.cgAbs, w.cgRel, w.mCG, g, ri,
+                    &state));
     cg_end_kernel<<<1, 1, 0, c.s>>>(state, g, ri);
     t0 = now_s();
     w.tCG += t0 - t1;
@@ -2553,6 +2789,7 @@ int work_setup(SolveWork<T> &w, crimson_lhs *l, crimson_ls *ls, int dof, const i
     SchurOp<T> so;
     CR_TRY(schur_ready(l, so));
     w.formed = so.formed;
+    w.paired = w.formed && N <= kCgPaired;
     if (!w.formed) {
       CR_TRY(w.ps.alloc(N));
       CR_TRY(w.z.alloc((size_t)4 * N));
@@ -2562,9 +2799,9 @@ int work_setup(SolveWork<T> &w, crimson_lhs *l, crimson_ls *ls, int dof, const i
   }
   if (ls->LS_type != CRIMSON_LS_GMRES) {
     const size_t n = ns ? N : st;
-    CR_TRY(w.t3.alloc(n));
+    CR_TRY(w.t3.alloc(ns && w.paired ? 2 * n : n));
     CR_TRY(w.t4.alloc(n));
-    CR_TRY(w.t5.alloc(n));
+    if (!(ns && w.paired)) CR_TRY(w.t5.alloc(n));
   }
   const unsigned long long before = w.gst.serial;
   CR_TRY(w.gst.alloc(o));
