@@ -583,6 +583,46 @@ __device__ inline double sum_parts(const double *__restrict__ part, int n, doubl
   return block_sum_all(more, sh);
 }
 
+// gst (double, device): the state of the solve and of its last GMRES and
+// CG calls, then the GMRES Hessenberg system, the Gram system and the
+// solution coefficients.
+enum GstIdx : int {
+  G_RI_SKIP = 0,  // the outer loop has stopped (converged or failed)
+  G_RI_ITR,
+  G_RI_SUC,
+  G_RI_INORM,
+  G_RI_FNORM,
+  G_RI_EPS,
+  G_RI_DBPRE,
+  G_ERR,  // 1: singular GE
+  G_GM_CYC = 8,  // this GMRES call does nothing more (done, or not running)
+  G_GM_ARN,      // no further Arnoldi step in this cycle
+  G_GM_EPS,
+  G_GM_I,
+  G_GM_ITR,
+  G_GM_SUC,
+  G_GM_INORM,
+  G_GM_FNORM,
+  G_GM_DBPRE,
+  G_GM_SCALE,
+  G_GM_APPLY,
+  G_GM_RAN,
+  G_GM_EARLY,
+  G_GM_LASTF,  // fNorm and dB of the last GMRES call that ran to the end
+  G_GM_LASTD,
+  G_CG_ITR = 24,
+  G_CG_SUC,
+  G_CG_INORM,
+  G_CG_ERR,
+  G_CG_ERRO,
+  G_RC_N2 = 30,
+  G_NS_CNT,
+  G_GM_E0,  // the first residual norm of the GMRES call
+  G_GM_N1,  // ||y'||^2 after an Arnoldi step's first pass, and whether it took the second
+  G_GM_TWICE,
+  G_ARR = 64
+};
+
 // ----- dots and the Arnoldi step -----
 // v (1024 threads) summed over the workgroup, in every thread, always in the
 // same order.
@@ -658,17 +698,83 @@ __device__ inline double wave_parts(const double *__restrict__ part, int n) {
   return wave_sum(t);
 }
 
-// One Arnoldi step (classical Gram-Schmidt with one DGKS pass) in six
-// launches without a host decision:
-//   arnoldi_spmv   u = scale w (the new basis vector) and y = A u
+// One Arnoldi step (classical Gram-Schmidt with one DGKS pass) without a host
+// decision:
+//   arnoldi_spmv   u = w / ||w|| (the new basis vector) and y = A u; a workgroup of
+//                  its own does gm_givens of the step before (small systems)
 //   face_apply     the coupled faces' terms on y (when there are any)
 //   dots           y against the basis, and y . y
+//   then, up to kOrthMost entries, where a launch costs more than its work:
+//   arnoldi_orth   y -= U h, parts of y . y, and y against the basis again
+//   arnoldi_orth   the second pass, where ||y'||^2 < ||y||^2 / 2 (every workgroup
+//                  takes that decision itself from the same parts), and W o y
+// or, for longer vectors, whose second pass over the basis should not be made before
+// it is known to be needed:
 //   arnoldi_sub    y -= U h, W o y for the next product, parts of y . y
-//   dots, sub      the second pass, where ||y'||^2 < ||y||^2 / 2 (every workgroup
-//                  takes that decision itself from the same parts)
+//   dots, sub      the second pass
 //   gm_givens      the Hessenberg column, rotations, test and 1 / ||y||
-// scale is 1 / ||w||; U_j is stored normalised.  The product gathers W o w, one
-// aligned entry of 2 or 4 components per column, in place of W and w.
+// Every U_j is stored normalised.  The product gathers W o w, one aligned entry of 2
+// or 4 components per column, in place of W and w.
+// Arnoldi step i's Hessenberg column, rotations and test; H (sD+1, sD)
+// column-major; s2: ||y||^2 after the second pass, where it was taken.  One
+// workgroup.  The column and the rotations pass through LDS, where the
+// chain of rotations takes an LDS read a step instead of a memory round trip.
+struct Givens {
+  double *g;
+  int i, sD;
+  const double *h1, *h2, *n2;
+  int nb;
+  double *H, *cs, *sn, *err;
+  HostFlag hf;
+};
+__device__ inline void gm_givens(const Givens &G, double s2, double (&w3)[3][256]) {
+#pragma clang fp contract(off)
+  double *g = G.g;
+  if (g[G_GM_ARN] != 0.0) {
+    if (threadIdx.x == 0) G.hf.tell(true);
+    return;
+  }
+  __syncthreads();  // (w3 may have been read)
+  double(&hc)[256] = w3[0], (&c)[256] = w3[1], (&s)[256] = w3[2];
+  const int t = threadIdx.x, i = G.i, ld = G.sD + 1;
+  const bool gt = g[G_GM_TWICE] != 0.0;
+  if (t < i) {
+    hc[t] = G.h1[t] + (gt ? G.h2[t] : 0.0);
+    if (t < i - 1) {
+      c[t] = G.cs[t];
+      s[t] = G.sn[t];
+    }
+  }
+  __syncthreads();
+  if (t == 0) {
+    const double hl = sqrt(gt ? s2 : g[G_GM_N1]);
+    g[G_GM_ITR] = g[G_GM_ITR] + 1.0;
+    g[G_GM_SCALE] = 1.0 / hl;
+    double a = hc[0];
+    for (int j = 1; j <= i - 1; ++j) {
+      const double b = hc[j];
+      hc[j - 1] = c[j - 1] * a + s[j - 1] * b;
+      a = -s[j - 1] * a + c[j - 1] * b;
+    }
+    const double tmp = sqrt(a * a + hl * hl);
+    const double ci = a / tmp, si = hl / tmp;
+    G.cs[i - 1] = ci;
+    G.sn[i - 1] = si;
+    hc[i - 1] = tmp;
+    const double e = G.err[i - 1];
+    G.err[i] = -si * e;
+    G.err[i - 1] = ci * e;
+    g[G_GM_I] = (double)i;
+    const bool done = fabs(-si * e) < g[G_GM_EPS];
+    if (done) {
+      g[G_GM_SUC] = 1.0;
+      g[G_GM_ARN] = 1.0;
+    }
+    G.hf.tell(done);
+  }
+  __syncthreads();
+  if (t < i) G.H[t + (size_t)ld * (i - 1)] = hc[t];
+}
 template <int NC>
 struct ArnoldiPad {
   static constexpr int n = NC == 3 ? 4 : NC;  // components of a gathered entry
@@ -689,11 +795,27 @@ template <int NC, class T, class IX>
 __global__ void __launch_bounds__(256) arnoldi_spmv_kernel(int nNo, const int *__restrict__ rowptr,
                                                            const IX *__restrict__ col, MatView<T> A,
                                                            const T *__restrict__ w, const T *__restrict__ ws,
-                                                           const double *__restrict__ scale, T *__restrict__ u,
-                                                           T *__restrict__ y, const double *__restrict__ skip) {
+                                                           T *__restrict__ u, T *__restrict__ y, Givens G) {
   constexpr int LANES = NC >= 3 ? kRowLanes : kNarrowLanes, PAD = ArnoldiPad<NC>::n;
-  const double stop = *skip;
-  const int gid = crimson::xcd_block(kRowXcdChunk) * blockDim.x + threadIdx.x;
+  __shared__ double sh[4], w3[3][256];
+  // G.i > 0: the step before ends here, workgroup 0 with its gm_givens, the others
+  // with 1 / ||w||.  (A step launched past the last one, while workgroup 0 tells so,
+  // writes vectors that nothing reads.)
+  double stop = G.g[G_GM_ARN], scale = G.g[G_GM_SCALE];
+  if (G.i > 0) {
+    // workgroup 0 may set the flag during this launch: one thread's read counts
+    if (threadIdx.x == 0) w3[0][0] = stop;
+    const double n1 = G.g[G_GM_N1], twice = G.g[G_GM_TWICE];
+    const double s2 = block_sum_all((int)threadIdx.x < G.nb ? G.n2[threadIdx.x] : 0.0, sh);
+    if (blockIdx.x == 0) {
+      gm_givens(G, s2, w3);
+      return;
+    }
+    stop = w3[0][0];
+    scale = 1.0 / sqrt(twice != 0.0 ? s2 : n1);
+  }
+  const int own = G.i > 0 ? 1 : 0;
+  const int gid = crimson::xcd_block(kRowXcdChunk, blockIdx.x - own, gridDim.x - own) * blockDim.x + threadIdx.x;
   const int row = gid / LANES, lane = threadIdx.x % LANES;
   const int kb = rowptr[min(row, nNo)], ke = rowptr[min(row + 1, nNo)];
   if (stop != 0.0) return;
@@ -718,7 +840,7 @@ __global__ void __launch_bounds__(256) arnoldi_spmv_kernel(int nNo, const int *_
 #pragma unroll
     for (int r = 0; r < NC; ++r) acc[r] += __shfl_xor(acc[r], off, LANES);
   if (row < nNo && lane == 0) {
-    const T s = (T)*scale;
+    const T s = (T)scale;
 #pragma unroll
     for (int r = 0; r < NC; ++r) {
       const size_t e = r + (size_t)NC * row, f = A.r0 + r + (size_t)A.wdof * row;
@@ -747,23 +869,12 @@ __global__ void __launch_bounds__(kDotThreads) dots2_kernel(size_t L, const T *_
   dots_body(L, v, U0, ustride, m, 0, part, sh);
 }
 // h = the dots' sums (np parts each; self: the m-th is ||y||^2), y -= U h and
-// its scaled copy, parts of y . y.  JS threads share an entry's sum over the
-// basis: one for long vectors, four for short ones, which leave a
-// thread alone with a chain of m loads.  n1 (the second pass): taken or left
-// as dgks_pass says.
+// its scaled copy, parts of y . y.  n1 (the second pass): taken or left
+// as dgks_pass says, which is noted in g.
 constexpr int kSubGrid = 1024;
-template <class T, int JS>
-__global__ void __launch_bounds__(kDotThreads) arnoldi_sub_kernel(
-    size_t L, int nc, int pad, const T *__restrict__ W, int wdof, int w0, T *__restrict__ y, T *__restrict__ ys,
-    const T *__restrict__ U0, size_t ustride, int m, int self, const double *__restrict__ part, int np,
-    double *__restrict__ h, double *__restrict__ npart, const double *__restrict__ n0, const double *__restrict__ n1,
-    const double *__restrict__ skip) {
-  if (*skip != 0.0) return;
-  constexpr int kE = kDotThreads / JS;  // entries a turn
-  __shared__ double sh[16];
-  __shared__ T cs[256];
-  __shared__ T comb[JS > 1 ? kDotThreads : 1];
-  if (n1 && !dgks_pass(n0, n1, gridDim.x, sh)) return;
+template <class T>
+__device__ inline void sub_coefs(int m, int self, const double *__restrict__ part, int np, double *__restrict__ h,
+                                 T (&cs)[256]) {
   for (int j = threadIdx.x / 64; j < m + self; j += kDotThreads / 64) {
     const double t = wave_parts(part + (size_t)j * np, np);
     if (threadIdx.x % 64 == 0) {
@@ -771,41 +882,134 @@ __global__ void __launch_bounds__(kDotThreads) arnoldi_sub_kernel(
       if (blockIdx.x == 0) h[j] = t;
     }
   }
+}
+// sum over j = js, js + JS, ... of cs_j U_j(e)
+template <class T, int JS>
+__device__ inline T sub_sum(const T (&cs)[256], const T *__restrict__ U0, size_t ustride, int m, int js, size_t e) {
+  T t = T(0);
+  int j = js;
+  for (; j + 7 * JS < m; j += 8 * JS) {
+    T u[8];
+#pragma unroll
+    for (int q = 0; q < 8; ++q) u[q] = U0[ustride * (j + q * JS) + e];
+#pragma unroll
+    for (int q = 0; q < 8; ++q) t += cs[j + q * JS] * u[q];
+  }
+  for (; j < m; j += JS) t += cs[j] * U0[ustride * j + e];
+  return t;
+}
+template <class T>
+__global__ void __launch_bounds__(kDotThreads) arnoldi_sub_kernel(
+    size_t L, int nc, int pad, const T *__restrict__ W, int wdof, int w0, T *__restrict__ y, T *__restrict__ ys,
+    const T *__restrict__ U0, size_t ustride, int m, int self, const double *__restrict__ part, int np,
+    double *__restrict__ h, double *__restrict__ npart, const double *__restrict__ n0, const double *__restrict__ n1,
+    double *__restrict__ g) {
+  if (g[G_GM_ARN] != 0.0) return;
+  __shared__ double sh[16];
+  __shared__ T cs[256];
+  if (n1) {
+    const double s1 = block_sum_1024((int)threadIdx.x < (int)gridDim.x ? n1[threadIdx.x] : 0.0, sh);
+    const bool take = s1 < 0.5 * *n0;  // dgks_pass
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+      g[G_GM_N1] = s1;
+      g[G_GM_TWICE] = take ? 1.0 : 0.0;
+    }
+    if (!take) return;
+  }
+  sub_coefs(m, self, part, np, h, cs);
   __syncthreads();
-  const int js = threadIdx.x / kE;
   double s = 0.0;
-  for (size_t b = (size_t)blockIdx.x * kE; b < L; b += (size_t)gridDim.x * kE) {
-    const size_t e = b + threadIdx.x % kE;
-    T t = T(0);
-    if (e < L) {
-      int j = js;
-      for (; j + 7 * JS < m; j += 8 * JS) {
-        T u[8];
-#pragma unroll
-        for (int q = 0; q < 8; ++q) u[q] = U0[ustride * (j + q * JS) + e];
-#pragma unroll
-        for (int q = 0; q < 8; ++q) t += cs[j + q * JS] * u[q];
-      }
-      for (; j < m; j += JS) t += cs[j] * U0[ustride * j + e];
-    }
-    if (JS > 1) {
-      __syncthreads();  // the previous turn's sums are read
-      comb[threadIdx.x] = t;
-      __syncthreads();
-      if (js == 0)
-#pragma unroll
-        for (int q = 1; q < JS; ++q) t += comb[threadIdx.x + q * kE];
-    }
-    if (js == 0 && e < L) {
-      const T v = y[e] - t;
-      y[e] = v;
-      const size_t i = e / nc, c = e % nc;
-      ys[pad * i + c] = W[w0 + c + wdof * i] * v;
-      s += (double)v * (double)v;
-    }
+  for (size_t e = (size_t)blockIdx.x * kDotThreads + threadIdx.x; e < L; e += (size_t)gridDim.x * kDotThreads) {
+    const T v = y[e] - sub_sum<T, 1>(cs, U0, ustride, m, 0, e);
+    y[e] = v;
+    const size_t i = e / nc, c = e % nc;
+    ys[pad * i + c] = W[w0 + c + wdof * i] * v;
+    s += (double)v * (double)v;
   }
   s = block_sum_1024(s, sh);
   if (threadIdx.x == 0) npart[blockIdx.x] = s;
+}
+// The same for at most kOrthMost entries, 1024 / JS of them in a workgroup (JS
+// threads share an entry's sum over the basis, so that a short vector does not leave a
+// thread alone with a chain of m loads).  FIRST: also the workgroup's parts of the
+// dots of the new y with the basis, whose entries it has just read; otherwise the
+// second pass and the scaled copy.  22,500 entries, up to 100 vectors: a step of
+// seven launches took 51 us, one of five takes 40.
+constexpr size_t kOrthMost = (size_t)kDotGrid * kDotThreads;
+template <class T, int JS, bool FIRST>
+__global__ void __launch_bounds__(kDotThreads) arnoldi_orth_kernel(
+    size_t L, int nc, int pad, const T *__restrict__ W, int wdof, int w0, T *__restrict__ y, T *__restrict__ ys,
+    const T *__restrict__ U0, size_t ustride, int m, const double *__restrict__ part, int np, double *__restrict__ h,
+    double *__restrict__ npart, double *__restrict__ part2, const double *__restrict__ n0,
+    const double *__restrict__ n1, double *__restrict__ g) {
+  constexpr int kE = kDotThreads / JS;
+  __shared__ double sh[16];
+  __shared__ T cs[256];
+  __shared__ T comb[kDotThreads];
+  const int js = threadIdx.x / kE, te = threadIdx.x % kE;
+  const size_t base = (size_t)blockIdx.x * kE, e = base + te;
+  const bool own = js == 0 && e < L;
+  const T yo = own ? y[e] : T(0);
+  if (g[G_GM_ARN] != 0.0) return;
+  bool take = true;
+  if (!FIRST) {
+    const double s1 = block_sum_1024((int)threadIdx.x < (int)gridDim.x ? n1[threadIdx.x] : 0.0, sh);
+    take = s1 < 0.5 * *n0;  // dgks_pass
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+      g[G_GM_N1] = s1;
+      g[G_GM_TWICE] = take ? 1.0 : 0.0;
+    }
+  }
+  T t = T(0);
+  if (take) {  // the workgroup's
+    sub_coefs(m, FIRST ? 1 : 0, part, np, h, cs);
+    __syncthreads();
+    if (e < L) t = sub_sum<T, JS>(cs, U0, ustride, m, js, e);
+  }
+  if (JS > 1) {
+    comb[threadIdx.x] = t;
+    __syncthreads();
+    if (js == 0)
+#pragma unroll
+      for (int q = 1; q < JS; ++q) t += comb[te + q * kE];
+  }
+  const T v = yo - t;
+  if (own) {
+    if (take) y[e] = v;
+    if (!FIRST) {
+      const size_t i = e / nc, c = e % nc;
+      ys[pad * i + c] = W[w0 + c + wdof * i] * v;
+    }
+  }
+  if (!take) return;
+  const double s = block_sum_1024(own ? (double)v * (double)v : 0.0, sh);  // (its barriers: comb is read)
+  if (threadIdx.x == 0) npart[blockIdx.x] = s;
+  if (!FIRST) return;
+  if (js == 0) comb[te] = own ? v : T(0);
+  __syncthreads();
+  constexpr int kQ = 4;  // vectors of a wave in flight
+  for (int j0 = threadIdx.x / 64; j0 < m; j0 += kQ * (kDotThreads / 64)) {
+    double acc[kQ];
+#pragma unroll
+    for (int q = 0; q < kQ; ++q) acc[q] = 0.0;
+#pragma unroll 4
+    for (int k = 0; k < kE; k += 64) {
+      const int x = k + threadIdx.x % 64;
+      const size_t ec = base + x < L ? base + x : L - 1;  // (its y is zero)
+      const double yv = (double)comb[x];
+#pragma unroll
+      for (int q = 0; q < kQ; ++q) {
+        const int j = j0 + q * (kDotThreads / 64);
+        acc[q] += (double)U0[ustride * (j < m ? j : m - 1) + ec] * yv;
+      }
+    }
+#pragma unroll
+    for (int q = 0; q < kQ; ++q) {
+      const int j = j0 + q * (kDotThreads / 64);
+      acc[q] = wave_sum(acc[q]);
+      if (j < m && threadIdx.x % 64 == 0) part2[(size_t)j * gridDim.x + blockIdx.x] = acc[q];
+    }
+  }
 }
 // The cycle's first vector: w (already R or R - A X with the faces' PRE), its
 // scaled copy and parts of w . w.
@@ -1918,44 +2122,6 @@ int face_functionals(Ctx<T> &c, const MatView<T> &G) {
   return CRIMSON_OK;
 }
 
-// gst (double, device): the state of the solve and of its last GMRES and
-// CG calls, then the GMRES Hessenberg system, the Gram system and the
-// solution coefficients.
-enum GstIdx : int {
-  G_RI_SKIP = 0,  // the outer loop has stopped (converged or failed)
-  G_RI_ITR,
-  G_RI_SUC,
-  G_RI_INORM,
-  G_RI_FNORM,
-  G_RI_EPS,
-  G_RI_DBPRE,
-  G_ERR,  // 1: singular GE
-  G_GM_CYC = 8,  // this GMRES call does nothing more (done, or not running)
-  G_GM_ARN,      // no further Arnoldi step in this cycle
-  G_GM_EPS,
-  G_GM_I,
-  G_GM_ITR,
-  G_GM_SUC,
-  G_GM_INORM,
-  G_GM_FNORM,
-  G_GM_DBPRE,
-  G_GM_SCALE,
-  G_GM_APPLY,
-  G_GM_RAN,
-  G_GM_EARLY,
-  G_GM_LASTF,  // fNorm and dB of the last GMRES call that ran to the end
-  G_GM_LASTD,
-  G_CG_ITR = 24,
-  G_CG_SUC,
-  G_CG_INORM,
-  G_CG_ERR,
-  G_CG_ERRO,
-  G_RC_N2 = 30,
-  G_NS_CNT,
-  G_GM_E0,  // the first residual norm of the GMRES call
-  G_ARR = 64
-};
-
 __device__ inline double dmax(double a, double b) { return a < b ? b : a; }  // std::max's choice
 
 // The deciding kernels: one workgroup of kDotThreads, which sums the dots'
@@ -2027,64 +2193,11 @@ __global__ void __launch_bounds__(kDotThreads) gm_cycle_kernel(double *__restric
   g[G_GM_RAN] = 1.0;
   g[G_GM_I] = 0.0;
 }
-// Arnoldi step i's Hessenberg column, rotations and test; H (sD+1, sD)
-// column-major.  The column and the rotations pass through LDS, where the
-// chain of rotations takes an LDS read a step instead of a memory round trip.
-__global__ void __launch_bounds__(kDotThreads) gm_givens_kernel(double *__restrict__ g, int i, int sD,
-                                                                const double *__restrict__ h1,
-                                                                const double *__restrict__ h2,
-                                                                const double *__restrict__ n1,
-                                                                const double *__restrict__ n2, int nb,
-                                                                double *__restrict__ H, double *__restrict__ cs,
-                                                                double *__restrict__ sn, double *__restrict__ err,
-                                                                HostFlag hf) {
-#pragma clang fp contract(off)
-  if (g[G_GM_ARN] != 0.0) {
-    if (threadIdx.x == 0) hf.tell(true);
-    return;
-  }
-  __shared__ double sh[16], hc[256], c[256], s[256];
-  const int t = threadIdx.x, ld = sD + 1;
-  const double a1 = t < nb ? n1[t] : 0.0, a2 = t < nb ? n2[t] : 0.0;
-  const double s1 = block_sum_1024(a1, sh);
-  const bool gt = s1 < 0.5 * h1[i];  // dgks_pass's decision
-  const double s2 = block_sum_1024(a2, sh);
-  if (t < i) {
-    hc[t] = h1[t] + (gt ? h2[t] : 0.0);
-    if (t < i - 1) {
-      c[t] = cs[t];
-      s[t] = sn[t];
-    }
-  }
-  __syncthreads();
-  if (t == 0) {
-    const double hl = sqrt(gt ? s2 : s1);
-    g[G_GM_ITR] = g[G_GM_ITR] + 1.0;
-    g[G_GM_SCALE] = 1.0 / hl;
-    double a = hc[0];
-    for (int j = 1; j <= i - 1; ++j) {
-      const double b = hc[j];
-      hc[j - 1] = c[j - 1] * a + s[j - 1] * b;
-      a = -s[j - 1] * a + c[j - 1] * b;
-    }
-    const double tmp = sqrt(a * a + hl * hl);
-    const double ci = a / tmp, si = hl / tmp;
-    cs[i - 1] = ci;
-    sn[i - 1] = si;
-    hc[i - 1] = tmp;
-    const double e = err[i - 1];
-    err[i] = -si * e;
-    err[i - 1] = ci * e;
-    g[G_GM_I] = (double)i;
-    const bool done = fabs(-si * e) < g[G_GM_EPS];
-    if (done) {
-      g[G_GM_SUC] = 1.0;
-      g[G_GM_ARN] = 1.0;
-    }
-    hf.tell(done);
-  }
-  __syncthreads();
-  if (t < i) H[t + (size_t)ld * (i - 1)] = hc[t];
+__global__ void __launch_bounds__(kDotThreads) gm_givens_kernel(Givens G) {
+  __shared__ double sh[16], w3[3][256];
+  const double *n2 = G.n2;
+  const double s2 = block_sum_1024((int)threadIdx.x < G.nb ? n2[threadIdx.x] : 0.0, sh);
+  gm_givens(G, s2, w3);
 }
 // the cycle's back substitution, one thread per unknown, a column at a time
 // (its read is in flight during the column before)
@@ -2395,41 +2508,31 @@ int face_apply(Ctx<T> &c, int what, int xdof, const T *X, T *Y, const double *sk
   return CRIMSON_OK;
 }
 
-// Grid of the Arnoldi sweeps over L entries: four threads per entry while
-// that fills the card no more than once (measured at 60 vectors of 20,000 entries: 10
-// -> 6 us), one beyond.
-struct SubGrid {
-  int js, blocks;
-};
-inline SubGrid sub_grid(size_t L) {
-  const int js = L <= (size_t)256 * kSubGrid ? 4 : 1;
-  const size_t e = kDotThreads / js;
-  return SubGrid{js, (int)std::min<size_t>((L + e - 1) / e, kSubGrid)};
-}
 template <class T, class IX>
-void arnoldi_spmv_ix(Ctx<T> &c, const MatView<T> &A, int nd, const IX *col, const T *w, const T *ws,
-                     const double *scale, T *u, T *y, const double *skip) {
+void arnoldi_spmv_ix(Ctx<T> &c, const MatView<T> &A, int nd, const IX *col, const T *w, const T *ws, T *u, T *y,
+                     const Givens &gv) {
   const int *rp = c.lhs->d_rowptr.p;
-  const unsigned G = crimson::grid_for((size_t)c.N * kRowLanes, 256),
-                 Gn = crimson::grid_for((size_t)c.N * kNarrowLanes, 256);
+  const unsigned own = gv.i > 0 ? 1 : 0, G = crimson::grid_for((size_t)c.N * kRowLanes, 256) + own,
+                 Gn = crimson::grid_for((size_t)c.N * kNarrowLanes, 256) + own;
   switch (nd) {
-    case 1: arnoldi_spmv_kernel<1, T, IX><<<Gn, 256, 0, c.s>>>(c.N, rp, col, A, w, ws, scale, u, y, skip); break;
-    case 2: arnoldi_spmv_kernel<2, T, IX><<<Gn, 256, 0, c.s>>>(c.N, rp, col, A, w, ws, scale, u, y, skip); break;
-    case 3: arnoldi_spmv_kernel<3, T, IX><<<G, 256, 0, c.s>>>(c.N, rp, col, A, w, ws, scale, u, y, skip); break;
-    default: arnoldi_spmv_kernel<4, T, IX><<<G, 256, 0, c.s>>>(c.N, rp, col, A, w, ws, scale, u, y, skip); break;
+    case 1: arnoldi_spmv_kernel<1, T, IX><<<Gn, 256, 0, c.s>>>(c.N, rp, col, A, w, ws, u, y, gv); break;
+    case 2: arnoldi_spmv_kernel<2, T, IX><<<Gn, 256, 0, c.s>>>(c.N, rp, col, A, w, ws, u, y, gv); break;
+    case 3: arnoldi_spmv_kernel<3, T, IX><<<G, 256, 0, c.s>>>(c.N, rp, col, A, w, ws, u, y, gv); break;
+    default: arnoldi_spmv_kernel<4, T, IX><<<G, 256, 0, c.s>>>(c.N, rp, col, A, w, ws, u, y, gv); break;
   }
 }
-template <class T>
-void arnoldi_sub(Ctx<T> &c, const SubGrid &sg, size_t L, int nd, const MatView<T> &A, T *y, T *ys, const T *U, int m,
-                 bool self, int np, double *h, double *npart, const double *n0, const double *n1,
-                 const double *skip) {
+// The two passes over vectors of at most kOrthMost entries: a workgroup's
+// entries so few that the vector has as many workgroups as the parts allow.
+template <class T, int JS>
+void arnoldi_orth(Ctx<T> &c, size_t L, int nd, const MatView<T> &A, T *y, T *ys, const T *U, int m, double *h1,
+                  double *h2, double *n1, double *n2, double *g, int &nb) {
   const int pad = nd == 3 ? 4 : nd;
-  if (sg.js == 4)
-    arnoldi_sub_kernel<T, 4><<<sg.blocks, kDotThreads, 0, c.s>>>(L, nd, pad, A.W, A.wdof, A.c0, y, ys, U, L, m,
-                                                                 self ? 1 : 0, c.part.p, np, h, npart, n0, n1, skip);
-  else
-    arnoldi_sub_kernel<T, 1><<<sg.blocks, kDotThreads, 0, c.s>>>(L, nd, pad, A.W, A.wdof, A.c0, y, ys, U, L, m,
-                                                                 self ? 1 : 0, c.part.p, np, h, npart, n0, n1, skip);
+  nb = (int)crimson::grid_for(L, kDotThreads / JS);
+  double *part2 = c.part.p + (size_t)kDotGrid * 264;
+  arnoldi_orth_kernel<T, JS, true><<<nb, kDotThreads, 0, c.s>>>(L, nd, pad, A.W, A.wdof, A.c0, y, ys, U, L, m, c.part.p,
+                                                                dot_blocks(L), h1, n1, part2, nullptr, nullptr, g);
+  arnoldi_orth_kernel<T, JS, false><<<nb, kDotThreads, 0, c.s>>>(L, nd, pad, A.W, A.wdof, A.c0, y, ys, U, L, m, part2,
+                                                                 nb, h2, n2, nullptr, h1 + m, n1, g);
 }
 
 // GMRES (memLS.f90:681-788) for the operator x -> A x + ADD(x), left
@@ -2451,8 +2554,12 @@ int gmres_run(SolveWork<T> &w, const MatView<T> &A, int nd, const T *R, T *X, co
   const double *cyc = g + G_GM_CYC, *arn = g + G_GM_ARN;
   T *U = w.gmU.p, *v = w.wa.p, *y = w.wb.p;
   const unsigned GL = crimson::grid_for(L, 256);
-  const SubGrid sg = sub_grid(L);
+  const bool small = L <= kOrthMost;
   const int nb0 = (int)std::min<size_t>((L + kDotThreads - 1) / kDotThreads, kSubGrid), np = dot_blocks(L);
+  int nb = nb0;  // parts of n1 and n2
+  auto givens = [&](int i, HostFlag hf) {
+    return Givens{g, i, p.sD, h1, h2, n2, nb, w.G(w.oH), w.G(w.ocs), w.G(w.osn), w.G(w.oerr), hf};
+  };
   gm_begin_kernel<<<1, 1, 0, c.s>>>(g, skip);
   fill_kernel<T><<<GL, 256, 0, c.s>>>(L, X, skip);
   for (int l = 1; l <= p.mItr; ++l) {
@@ -2470,23 +2577,37 @@ int gmres_run(SolveWork<T> &w, const MatView<T> &A, int nd, const T *R, T *X, co
     bool stop = false;
     for (int i = 1; i <= p.sD; ++i) {
       T *u = U + L * (size_t)(i - 1);
+      const bool ends = small && i > 1;  // the step before ends in this one's product
+      const Givens gv = givens(ends ? i - 1 : 0, ends ? w.flag() : HostFlag{nullptr, 0});
       if (c.lhs->d_col16.p)
-        arnoldi_spmv_ix(c, A, nd, c.lhs->d_col16.p, v, w.ws.p, g + G_GM_SCALE, u, y, arn);
+        arnoldi_spmv_ix(c, A, nd, c.lhs->d_col16.p, v, w.ws.p, u, y, gv);
       else
-        arnoldi_spmv_ix(c, A, nd, c.lhs->d_col.p, v, w.ws.p, g + G_GM_SCALE, u, y, arn);
+        arnoldi_spmv_ix(c, A, nd, c.lhs->d_col.p, v, w.ws.p, u, y, gv);
       CR_TRY(face_apply(c, kFaceAdd | (p.pre ? kFacePre : 0), nd, u, y, arn));
       CR_TRY(dots(c, L, y, U, L, i, true, c.part.p, arn));
-      arnoldi_sub(c, sg, L, nd, A, y, w.ws.p, U, i, true, np, h1, n1, static_cast<const double *>(nullptr),
-                  static_cast<const double *>(nullptr), arn);
-      dots2_kernel<T><<<dim3(np, (i + kDotGroup - 1) / kDotGroup), kDotThreads, 0, c.s>>>(
-          L, y, U, L, i, c.part.p, h1 + i, n1, sg.blocks, arn);
-      arnoldi_sub(c, sg, L, nd, A, y, w.ws.p, U, i, false, np, h2, n2, h1 + i, n1, arn);
-      gm_givens_kernel<<<1, kDotThreads, 0, c.s>>>(g, i, p.sD, h1, h2, n1, n2, sg.blocks, w.G(w.oH), w.G(w.ocs),
-                                                   w.G(w.osn), w.G(w.oerr), w.flag());
+      if (small) {
+        if (L <= kOrthMost / 4)
+          arnoldi_orth<T, 4>(c, L, nd, A, y, w.ws.p, U, i, h1, h2, n1, n2, g, nb);
+        else if (L <= kOrthMost / 2)
+          arnoldi_orth<T, 2>(c, L, nd, A, y, w.ws.p, U, i, h1, h2, n1, n2, g, nb);
+        else
+          arnoldi_orth<T, 1>(c, L, nd, A, y, w.ws.p, U, i, h1, h2, n1, n2, g, nb);
+        if (i == p.sD) gm_givens_kernel<<<1, kDotThreads, 0, c.s>>>(givens(i, w.flag()));
+      } else {
+        auto sub = [&](int self, double *h, double *n, const double *s0, const double *s1) {
+          arnoldi_sub_kernel<T><<<nb, kDotThreads, 0, c.s>>>(L, nd, pad, A.W, A.wdof, A.c0, y, w.ws.p, U, L, i, self,
+                                                             c.part.p, np, h, n, s0, s1, g);
+        };
+        sub(1, h1, n1, nullptr, nullptr);
+        dots2_kernel<T><<<dim3(np, (i + kDotGroup - 1) / kDotGroup), kDotThreads, 0, c.s>>>(
+            L, y, U, L, i, c.part.p, h1 + i, n1, nb, arn);
+        sub(0, h2, n2, h1 + i, n1);
+        gm_givens_kernel<<<1, kDotThreads, 0, c.s>>>(givens(i, w.flag()));
+      }
       CR_HIP(hipGetLastError());
       std::swap(v, y);
       // a plain solve looks at the step before while this one runs
-      if (w.polled && i > 1) CR_TRY(w.wait(w.seq - 1, &stop));
+      if (w.polled && i > 1) CR_TRY(w.wait(ends && i < p.sD ? w.seq : w.seq - 1, &stop));
       if (stop) break;
     }
     gm_solve_kernel<<<1, 256, 0, c.s>>>(g, p.sD, w.G(w.oH), w.G(w.oerr), w.G(w.oy));
