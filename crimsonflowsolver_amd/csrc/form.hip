@@ -780,16 +780,16 @@ __device__ inline void diag_add(DiagAcc<T> &A, const T *r, int a) {
   A.C += Cm * (ga[0] * ga[0] + ga[1] * ga[1] + ga[2] * ga[2]);
 }
 // The lanes' diagonal partial sums combined by a fixed shuffle tree over
-// the kRowLanes lanes of a row.
-template <class T>
+// the row's lanes.
+template <int LANES, class T>
 __device__ inline void diag_reduce(DiagAcc<T> &D) {
 #pragma unroll
-  for (int off = kRowLanes / 2; off > 0; off >>= 1) {
+  for (int off = LANES / 2; off > 0; off >>= 1) {
 #pragma unroll
-    for (int m = 0; m < 6; ++m) D.K[m] += __shfl_xor(D.K[m], off, kRowLanes);
+    for (int m = 0; m < 6; ++m) D.K[m] += __shfl_xor(D.K[m], off, LANES);
 #pragma unroll
-    for (int m = 0; m < 3; ++m) D.G[m] += __shfl_xor(D.G[m], off, kRowLanes);
-    D.C += __shfl_xor(D.C, off, kRowLanes);
+    for (int m = 0; m < 3; ++m) D.G[m] += __shfl_xor(D.G[m], off, LANES);
+    D.C += __shfl_xor(D.C, off, LANES);
   }
 }
 template <class T>
@@ -866,7 +866,7 @@ __device__ inline void gather_x(const double *__restrict__ xu, int4 n4, double (
   }
 }
 
-// Row-parallel assembly, kRowLanes lanes per CSR row; rows are taken in the
+// Row-parallel assembly, 16 or 32 lanes per CSR row; rows are taken in the
 // handle's schedule order (neighbouring rows together, so that the element
 // records and packed nodes they share are read from L2).  The row's element
 // incidences are taken in chunks of CH, in element order; lane t of a chunk
@@ -874,7 +874,7 @@ __device__ inline void gather_x(const double *__restrict__ xu, int4 n4, double (
 // rebuilds the element's shape gradients from its packed nodes (ienp: the
 // element's four nodes, stored per incidence so that a row reads them as one
 // contiguous run) and stages g, the scalars and the S row in LDS.  Then:
-//  - lane s accumulates off-diagonal block s (and s + 16, ... for long rows)
+//  - lane s accumulates off-diagonal block s (and s + LANES, ... for long rows)
 //    from its contribution list (lst: local incidence << 4 | a << 2 | b, in
 //    element order, built once from the sparseloc positions): fillsparseI's
 //    accumulation (fillsparse.f90:29-63) for that block;
@@ -883,20 +883,19 @@ __device__ inline void gather_x(const double *__restrict__ xu, int4 n4, double (
 //    fixed shuffle tree.
 // Every block of the row is written, so blocks no element touches come out
 // zero (the reference zeroes lhsK/lhsP first, elmgmr.f90:127-130).
-constexpr int kRowsPerBlock = 256 / kRowLanes;
-constexpr int kAsmChunk = 16;  // incidences staged per chunk (even, dividing kRowLanes)
-template <int MODE, int CH = kAsmChunk>
+// LANES is the handle's (row_lanes); CH incidences are staged per chunk.
+template <int MODE, int LANES, int CH = LANES>
 __global__ void __launch_bounds__(256) asm_row(int nshg, const int4 *__restrict__ tab, const int *__restrict__ inc,
                                                const int4 *__restrict__ ienp, const double *__restrict__ xu,
                                                const int *__restrict__ lst_ptr, const unsigned short *__restrict__ lst,
                                                const double *__restrict__ rec, const double *__restrict__ esc,
                                                double *__restrict__ res, AsmOut o, unsigned xc, int runs) {
-  static_assert(CH % 2 == 0 && kRowLanes % CH == 0, "chunk of 2, 4, 8 or 16 incidences");
-  __shared__ double st_all[kRowsPerBlock][CH][kStage];
+  static_assert(CH % 2 == 0 && LANES % CH == 0, "an even chunk that divides the lanes");
+  __shared__ double st_all[256 / LANES][CH][kStage];
   const int gid = xcd_block(xc) * blockDim.x + threadIdx.x;
-  const int slot = gid / kRowLanes, lane = gid % kRowLanes;
+  const int slot = gid / LANES, lane = gid % LANES;
   const bool live = slot < nshg;
-  double(*st)[kStage] = st_all[threadIdx.x / kRowLanes];
+  double(*st)[kStage] = st_all[threadIdx.x / LANES];
   int row = 0, k0 = 0, nslot = 0, sdiag = -1, p0 = 0, ninc = 0;
   if (live) {
     const int4 t0 = tab[2 * slot], t1 = tab[2 * slot + 1];
@@ -908,21 +907,21 @@ __global__ void __launch_bounds__(256) asm_row(int nshg, const int4 *__restrict_
     ninc = t1.y;
   }
   const int nchunk = (ninc + CH - 1) / CH;
-  const int ngroup = (nslot + kRowLanes - 1) / kRowLanes;
-  // Staged plane stores (planes, chunks of 16): when the wave's four rows
+  const int ngroup = (nslot + LANES - 1) / LANES;
+  // Staged plane stores (planes, whole chunks): when the wave's 64 / LANES rows
   // are consecutive rows (runs: the schedule is the numbering) of at most
-  // 16 blocks each, their blocks form one range of every plane; the wave
+  // LANES blocks each, their blocks form one range of every plane; the wave
   // gathers them, the diagonal blocks included, in its staging LDS after
   // the rows are summed and stores each plane's range at once, instead of
   // the off-diagonal blocks and, later, the diagonal ones into the holes
   // they left.
-  const bool wstg = MODE == 1 && CH == kRowLanes && runs && __all(nslot <= kRowLanes);
+  const bool wstg = MODE == 1 && CH == LANES && runs && __all(nslot <= LANES);
   DiagAcc<double> D;
   diag_zero(D);
   double rs[4] = {0, 0, 0, 0};
   BlockAcc<double> A;
   for (int g = 0; g < ngroup; ++g) {
-    const int s = lane + g * kRowLanes;
+    const int s = lane + g * LANES;
     const bool own = s < nslot && s != sdiag;
     block_zero(A);
     // the block's list range and the first chunk's incidences, loaded
@@ -941,11 +940,11 @@ __global__ void __launch_bounds__(256) asm_row(int nshg, const int4 *__restrict_
     lst_fill(lb, lst, q, q1);
     for (int c = 0; c < nchunk; ++c) {
       const int tb = c * CH;
-      // incidence t of the row is held by lane t % 16 whatever the chunk
+      // incidence t of the row is held by lane t % LANES whatever the chunk
       // size, so that every chunk size sums the diagonal block and the
       // residual row in the same order: chunk c occupies lanes lo..lo+CH-1
-      const int lo = CH == kRowLanes ? 0 : tb % kRowLanes;
-      const int lon = CH == kRowLanes ? 0 : (tb + CH) % kRowLanes;
+      const int lo = CH == LANES ? 0 : tb % LANES;
+      const int lon = CH == LANES ? 0 : (tb + CH) % LANES;
       const bool mine = lane >= lo && lane < lo + CH;  // the lane holds a staging slot of this chunk
       const int t = lane - lo;
       // the next chunk's incidences, in flight while this chunk is staged
@@ -1012,12 +1011,12 @@ __global__ void __launch_bounds__(256) asm_row(int nshg, const int4 *__restrict_
     }
     if (own && !wstg) put_block<MODE>(o, k0 + s, A.K, A.Gij, A.C, A.Gji);
   }
-  diag_reduce(D);
+  diag_reduce<LANES>(D);
 #pragma unroll
-  for (int off = kRowLanes / 2; off > 0; off >>= 1)
+  for (int off = LANES / 2; off > 0; off >>= 1)
 #pragma unroll
-    for (int k = 0; k < 4; ++k) rs[k] += __shfl_xor(rs[k], off, kRowLanes);
-  if constexpr (MODE == 1 && CH == kRowLanes) {
+    for (int k = 0; k < 4; ++k) rs[k] += __shfl_xor(rs[k], off, LANES);
+  if constexpr (MODE == 1 && CH == LANES) {
     if (wstg) {
       // the wave's range [kA, kB) of every plane (its live rows are
       // consecutive, so their blocks are)
@@ -1027,8 +1026,8 @@ __global__ void __launch_bounds__(256) asm_row(int nshg, const int4 *__restrict_
         kA = min(kA, __shfl_xor(kA, off, 64));
         kB = max(kB, __shfl_xor(kB, off, 64));
       }
-      const int nb = kB - kA;  // at most 4 rows x 16 blocks
-      double *ob = &st_all[threadIdx.x / 64 * (64 / kRowLanes)][0][0];  // the wave's rows' staging: [plane][block - kA]
+      const int nb = kB - kA;  // at most 64 / LANES rows x LANES blocks
+      double *ob = &st_all[threadIdx.x / 64 * (64 / LANES)][0][0];  // the wave's rows' staging: [plane][block - kA]
       wave_lds_sync();  // the last chunk's readers are done
       double v[16];
       if (lane < nslot && lane != sdiag) {
@@ -1063,16 +1062,16 @@ __global__ void __launch_bounds__(256) asm_row(int nshg, const int4 *__restrict_
 // FP32 tangent assembly (no residual rows): the structure of asm_row with
 // FP32 records (one line per element: g, scalars, S), FP32 accumulation and
 // FP32 planes (MODE 1) or FP64 lhsK/lhsP (MODE 0).
-template <int MODE>
+template <int MODE, int LANES>
 __global__ void __launch_bounds__(256) asm_row32(int nshg, const int4 *__restrict__ tab,
                                                  const int *__restrict__ inc, const int *__restrict__ lst_ptr,
                                                  const unsigned short *__restrict__ lst,
                                                  const float *__restrict__ rec, AsmOut o, unsigned xc) {
-  __shared__ float st_all[kRowsPerBlock][kRowLanes][kStage];
+  __shared__ float st_all[256 / LANES][LANES][kStage];
   const int gid = xcd_block(xc) * blockDim.x + threadIdx.x;
-  const int slot = gid / kRowLanes, lane = gid % kRowLanes;
+  const int slot = gid / LANES, lane = gid % LANES;
   const bool live = slot < nshg;
-  float(*st)[kStage] = st_all[threadIdx.x / kRowLanes];
+  float(*st)[kStage] = st_all[threadIdx.x / LANES];
   int k0 = 0, nslot = 0, sdiag = -1, p0 = 0, ninc = 0;
   if (live) {
     const int4 t0 = tab[2 * slot], t1 = tab[2 * slot + 1];
@@ -1082,41 +1081,41 @@ __global__ void __launch_bounds__(256) asm_row32(int nshg, const int4 *__restric
     p0 = t1.x;
     ninc = t1.y;
   }
-  const int nchunk = (ninc + kRowLanes - 1) / kRowLanes;
-  const int ngroup = (nslot + kRowLanes - 1) / kRowLanes;
+  const int nchunk = (ninc + LANES - 1) / LANES;
+  const int ngroup = (nslot + LANES - 1) / LANES;
   DiagAcc<float> D;
   diag_zero(D);
   for (int g = 0; g < ngroup; ++g) {
-    const int s = lane + g * kRowLanes;
+    const int s = lane + g * LANES;
     const bool own = s < nslot && s != sdiag;
     BlockAcc<float> A;
     block_zero(A);
     const int kq = own ? k0 + s : 0;
     int q = lst_ptr[kq];
     const int q1r = lst_ptr[kq + 1];
-    int nt = min(kRowLanes, ninc);
+    int nt = min(LANES, ninc);
     int ea = lane < nt ? inc[p0 + lane] : 0;
     const int q1 = own ? q1r : q;
     LstBuf lb;
     lst_fill(lb, lst, q, q1);
     for (int c = 0; c < nchunk; ++c) {
-      const int tb = c * kRowLanes;
-      const int ntn = min(kRowLanes, ninc - tb - kRowLanes);
-      const int ean = lane < ntn ? inc[p0 + tb + kRowLanes + lane] : 0;
+      const int tb = c * LANES;
+      const int ntn = min(LANES, ninc - tb - LANES);
+      const int ean = lane < ntn ? inc[p0 + tb + LANES + lane] : 0;
       wave_lds_sync();
       // line 0 of the record (4 pieces of 16 bytes) and node a's S row,
       // unguarded as in asm_row (past the chunk's end: incidence 0)
       float4 pc[4];
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
-        const int t = (j * kRowLanes + lane) >> 2, part = lane & 3;
-        const int et = __shfl(ea, t, kRowLanes);
+        const int t = (j * LANES + lane) >> 2, part = lane & 3;
+        const int et = __shfl(ea, t, LANES);
         pc[j] = *reinterpret_cast<const float4 *>(rec + (size_t)(et >> 2) * kRec32 + 4 * part);
       }
       const float4 sv = *reinterpret_cast<const float4 *>(rec + (size_t)(ea >> 2) * kRec32 + R32_S(ea & 3));
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
-        const int t = (j * kRowLanes + lane) >> 2, part = lane & 3;
+        const int t = (j * LANES + lane) >> 2, part = lane & 3;
         st[t][4 * part + 0] = pc[j].x;
         st[t][4 * part + 1] = pc[j].y;
         st[t][4 * part + 2] = pc[j].z;
@@ -1132,7 +1131,7 @@ __global__ void __launch_bounds__(256) asm_row32(int nshg, const int4 *__restric
         if (lb.n == 0) lst_fill(lb, lst, q, q1);
         const unsigned v = lst_front(lb);
         const int t = (int)(v >> 4) - tb;
-        if (t >= kRowLanes) break;
+        if (t >= LANES) break;
         block_add(A, st[t], (int)((v >> 2) & 3u), (int)(v & 3u));
         lst_pop(lb);
         ++q;
@@ -1142,7 +1141,7 @@ __global__ void __launch_bounds__(256) asm_row32(int nshg, const int4 *__restric
     }
     if (own) put_block<MODE>(o, k0 + s, A.K, A.Gij, A.C, A.Gji);
   }
-  diag_reduce(D);
+  diag_reduce<LANES>(D);
   if (live && lane == 0) {
     float K[9];
     diag_full(D, K);
@@ -1428,6 +1427,42 @@ int ensure_order(crimson_form *f, const double *d_x) {
   return CRIMSON_OK;
 }
 
+// Lanes per row of the assembly: 16 fit a Kuhn row (15 blocks); 32 where a share of
+// the rows is longer (a wave then walks its rows' elements once instead of
+// once per 16 blocks) or where so few rows leave the card idle.  16 and 32 lanes, us
+// into the planes: Delaunay meshes (a third or more of the rows longer) 441 nodes 24
+// and 14, 2,160 40 and 23, 14,007 69 and 51, 40,960 121 and 109; Kuhn meshes 1,144
+// nodes 14 and 11, 5,617 18 and 18, 12,291 24 and 31, 141,197 227 and 281 (FP32 alike).
+constexpr int kLongShare = 4, kFewRows = 6144;
+template <int LANES>
+void assemble(crimson_form *f, int mode, bool t32, double *d_res, const AsmOut &o) {
+  hipStream_t s = f->stream;
+  const unsigned G = crimson::grid_for((size_t)f->nshg * LANES, 256);
+  const int runs = f->sched == kSchedNumbering;  // slot i is row i: a wave's rows are consecutive
+#define CR_ASM(...)                                                                                              \
+  asm_row<__VA_ARGS__><<<G, 256, 0, s>>>(f->nshg, f->d_slot.p, f->d_inc.p, f->d_ienp.p, f->d_xu.p, f->d_lst_ptr.p, \
+                                         f->d_lst.p, f->d_rec.p, f->d_esc.p, d_res, o, f->asm_xcd, runs)
+  if (t32) {
+    if (mode == 0)
+      asm_row32<0, LANES><<<G, 256, 0, s>>>(f->nshg, f->d_slot.p, f->d_inc.p, f->d_lst_ptr.p, f->d_lst.p,
+                                            f->d_rec32.p, o, f->asm_xcd);
+    else
+      asm_row32<1, LANES><<<G, 256, 0, s>>>(f->nshg, f->d_slot.p, f->d_inc.p, f->d_lst_ptr.p, f->d_lst.p,
+                                            f->d_rec32.p, o, f->asm_xcd);
+  } else if (mode == 0) {
+    if (f->asm_chunk == 8)
+      CR_ASM(0, LANES, 8);
+    else
+      CR_ASM(0, LANES);
+  } else {
+    if (f->asm_chunk == 8)
+      CR_ASM(1, LANES, 8);
+    else
+      CR_ASM(1, LANES);
+  }
+#undef CR_ASM
+}
+
 int run_formation(crimson_form *f, const double *d_y, const double *d_ac, const double *d_x,
                   double *d_res, int lhs, int mode, const AsmOut &o, double *d_qout, bool timed = true) {
   const unsigned T = 256;
@@ -1462,37 +1497,17 @@ int run_formation(crimson_form *f, const double *d_y, const double *d_ac, const 
   CR_HIP(hipGetLastError());
   if (timed) CR_HIP(hipEventRecord(f->ev[2], s));
   const unsigned gn = crimson::grid_for((size_t)f->nshg * kResLanes, T);
-  const unsigned gr = crimson::grid_for((size_t)f->nshg * kRowLanes, T);
-  const int runs = f->sched == kSchedNumbering;  // slot i is row i: a wave's rows are consecutive
-  if (t32) {
-    if (mode == 0) {
-      res_node<0><<<gn, T, 0, s>>>(f->nshg, f->d_inc_ptr.p, f->d_inc.p, f->d_rec.p, d_res);
-      asm_row32<0><<<gr, T, 0, s>>>(f->nshg, f->d_slot.p, f->d_inc.p, f->d_lst_ptr.p, f->d_lst.p,
-                                    f->d_rec32.p, o, f->asm_xcd);
-    } else {
-      res_node<1><<<gn, T, 0, s>>>(f->nshg, f->d_inc_ptr.p, f->d_inc.p, f->d_rec.p, d_res);
-      asm_row32<1><<<gr, T, 0, s>>>(f->nshg, f->d_slot.p, f->d_inc.p, f->d_lst_ptr.p, f->d_lst.p,
-                                    f->d_rec32.p, o, f->asm_xcd);
-    }
-  } else if (!lhs) {
+  if (t32 || !lhs) {
     if (mode == 0)
       res_node<0><<<gn, T, 0, s>>>(f->nshg, f->d_inc_ptr.p, f->d_inc.p, f->d_rec.p, d_res);
     else
       res_node<1><<<gn, T, 0, s>>>(f->nshg, f->d_inc_ptr.p, f->d_inc.p, f->d_rec.p, d_res);
-  } else if (mode == 0) {
-    if (f->asm_chunk == 8)
-      asm_row<0, 8><<<gr, T, 0, s>>>(f->nshg, f->d_slot.p, f->d_inc.p, f->d_ienp.p, f->d_xu.p, f->d_lst_ptr.p,
-                                     f->d_lst.p, f->d_rec.p, f->d_esc.p, d_res, o, f->asm_xcd, runs);
+  }
+  if (lhs) {
+    if (f->row_lanes == 32)
+      assemble<32>(f, mode, t32, d_res, o);
     else
-      asm_row<0><<<gr, T, 0, s>>>(f->nshg, f->d_slot.p, f->d_inc.p, f->d_ienp.p, f->d_xu.p, f->d_lst_ptr.p,
-                                  f->d_lst.p, f->d_rec.p, f->d_esc.p, d_res, o, f->asm_xcd, runs);
-  } else {
-    if (f->asm_chunk == 8)
-      asm_row<1, 8><<<gr, T, 0, s>>>(f->nshg, f->d_slot.p, f->d_inc.p, f->d_ienp.p, f->d_xu.p, f->d_lst_ptr.p,
-                                     f->d_lst.p, f->d_rec.p, f->d_esc.p, d_res, o, f->asm_xcd, runs);
-    else
-      asm_row<1><<<gr, T, 0, s>>>(f->nshg, f->d_slot.p, f->d_inc.p, f->d_ienp.p, f->d_xu.p, f->d_lst_ptr.p,
-                                  f->d_lst.p, f->d_rec.p, f->d_esc.p, d_res, o, f->asm_xcd, runs);
+      assemble<16>(f, mode, t32, d_res, o);
   }
   // the wall's rows and tangent (AsBMFG's xKebe goes through bc3lhs too)
   CR_TRY(crimson::form_wall_pass(f, lhs, mode, o.lhsK, o.V, mode == 1 && t32 ? o.V32 : nullptr, o.nnz));
@@ -1662,7 +1677,11 @@ extern "C" int crimson_form_setup(int nshg, int numnp, int nel, const int *ien, 
   // nodes among the row's blocks (IncLoc) on the way.
   std::vector<int> lst_ptr(nnz + 1, 0);
   int most = 0;
-  for (int i = 0; i < nshg; ++i) most = std::max(most, rp[i + 1] - rp[i]);
+  int longer = 0;
+  for (int i = 0; i < nshg; ++i) {
+    most = std::max(most, rp[i + 1] - rp[i]);
+    longer += rp[i + 1] - rp[i] > 16;
+  }
   const bool wide = most > (1 << IncLoc<unsigned>::bits);
   std::vector<unsigned> iloc;
   std::vector<unsigned long long> iloc64;
@@ -1728,6 +1747,7 @@ extern "C" int crimson_form_setup(int nshg, int numnp, int nel, const int *ien, 
   f->nnz = nnz;
   f->prm = *prm;
   f->wide = wide;
+  f->row_lanes = (long long)longer * kLongShare >= nshg || nshg <= kFewRows ? 32 : 16;
   int rc = CRIMSON_OK;
   auto fail = [&](int code) {
     crimson_form_free(f);

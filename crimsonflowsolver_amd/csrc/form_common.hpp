@@ -78,7 +78,6 @@ __host__ __device__ inline double flux_weight(double W, int a) {
          : a == 2 ? nq(0, 2) * W + nq(1, 2) * W + nq(2, 2) * W + nq(3, 2) * W
                   : nq(0, 3) * W + nq(1, 3) * W + nq(2, 3) * W + nq(3, 3) * W;
 }
-constexpr int kRowLanes = 16;   // lanes per CSR row in the assembly
 
 // The rule's weights, N_a at another node's point and how much more at its own: sum_q
 // N_a(q) f_q = w_other(a) sum_q f_q + w_diff(a) f_a.
@@ -267,7 +266,8 @@ struct crimson_form {
   crimson::DBuf<int> d_lst_ptr, d_order;  // d_order: assembly row schedule
   crimson::DBuf<int4> d_slot;              // per schedule slot: the row's offsets (slot_table_kernel)
   int sched = 1;                            // assembly row schedule (kSched*; set at setup)
-  int asm_chunk = 16;                       // incidences per staged chunk of the FP64 assembly
+  int row_lanes = 16;                       // lanes per row of the assembly, 16 or 32 (set at setup)
+  int asm_chunk = 16;                       // incidences per staged chunk of the FP64 assembly: 8, or the row's lanes
   unsigned asm_xcd = 0;                     // assembly workgroups dealt per XCD turn (0: one range each)
   crimson::DBuf<unsigned short> d_lst;
   crimson::DBuf<int4> d_ienp;    // per incidence (node-major): the element's four nodes in local order
