@@ -51,12 +51,13 @@ def build_problem(grid, cfa, M):
 FLOPS_PER_ELEMENT = 8996.0
 FLOPS_PER_NODE = 10.0
 # the formation's kernels as rocprofv3 names them (profiles/*_pmc_traffic.md)
-FORMATION_KERNELS = ("node_pack", "flux_node", "e3_elem<true>", "asm_row<1,16>", "bnd_elem", "bnd_node<1>")
+FORMATION_KERNELS = ("node_pack", "flux_node<unsigned int>", "e3_elem<true>", "asm_row<1,16,16>", "bnd_elem",
+                     "bnd_node<1>")
 
 
 def pmc_kernel_name(name):
     """A rocprofv3 kernel name without its return type, namespace and
-    arguments, spaces removed (``asm_row<1,16>``)."""
+    arguments, spaces removed (``asm_row<1,16,16>``)."""
     n = name[5:] if name.startswith("void ") else name
     n = n.replace("(anonymous namespace)::", "")
     depth = 0
@@ -1056,7 +1057,7 @@ def main():
     # (4 doubles/node) and the contribution lists (2 B per off-diagonal
     # contribution, 12 per element)
     byt = nel * 4 * (12 * 8 + 16) + N * 6 * 8 + nnz * 16 * 8 + N * 4 * 8 + nel * 12 * 2
-    kname = "asm_row<1,8>" if tuned is not None and tuned["fp64"][0].split("/")[1] == "8" else "asm_row<1,16>"
+    kname = "asm_row<1,16,8>" if tuned is not None and tuned["fp64"][0].split("/")[1] == "8" else "asm_row<1,16,16>"
     roof["dominant_kernel"] = {"kernel": kname, "bound": "hbm", "achieved": byt / (tm[2] * 1e-3) / 1e9,
                                "peak": HBM_PEAK_GBS, "unit": "GB/s",
                                "frac": byt / (tm[2] * 1e-3) / 1e9 / HBM_PEAK_GBS, "algorithmic_bytes": byt,

@@ -205,7 +205,7 @@ __global__ void __launch_bounds__(256) flux_node(int nshg, const int *__restrict
 // at the rest) make every nodal sum sum_q N_a(q) f_q = w_other(a) sum f +
 // (w_own(a) - w_other(a)) f_a.  tauM and tauBar take a reciprocal square root each.  Written
 // term by term per point (the form of e3res.f90 and e3lhs.f90) the kernel issued
-// 1,763 vector instructions per wave, this 1,117; it is bound by latency at two
+// 1,763 vector instructions per wave, this 1,185; it is bound by latency at two
 // waves a SIMD and by the record stores (1.8 GB at 6.2 M elements: 672 us before,
 // 557 now; without the tangent 663 before, 411 now).
 // In: the nodal values.  Out: u -> ubar at the points, a -> (a + ubar . grad u) at
