@@ -331,8 +331,8 @@ __global__ void __launch_bounds__(256) vjp_q_node(int nshg, const int *__restric
                                                   const double *__restrict__ vdq, const double *__restrict__ invm,
                                                   double *__restrict__ xq) {
   __shared__ double xs_all[256 / kVjpLanes][kVjpCap * 4];
-  const int gid = xcd_block() * blockDim.x + threadIdx.x;
-  const int i = gid / kVjpLanes, lane = gid % kVjpLanes;
+  const unsigned gid = xcd_block() * blockDim.x + threadIdx.x;
+  const int i = (int)(gid / kVjpLanes), lane = (int)(gid % kVjpLanes);
   const bool live = i < nshg;
   const int ii = live ? i : nshg - 1;
   const int k0 = rowptr[ii], ns = rowptr[ii + 1] - k0, d = diagk[ii] - k0;
@@ -425,8 +425,8 @@ __global__ void __launch_bounds__(256) vjp_node(int nshg, const int *__restrict_
   constexpr int kP = 4;           // lanes per record (without AC two pairs read the same, so that both sum in one order)
   __shared__ double xs_all[256 / kVjpLanes][kVjpCap2 * kXQ];
   const unsigned blk = xcd_block();
-  const int gid = blk * blockDim.x + threadIdx.x;
-  const int i = gid / kVjpLanes, lane = gid % kVjpLanes;
+  const unsigned gid = blk * blockDim.x + threadIdx.x;
+  const int i = (int)(gid / kVjpLanes), lane = (int)(gid % kVjpLanes);
   const bool live = i < nshg;
   const int ii = live ? i : nshg - 1;
   const int k0 = rowptr[ii], ns = rowptr[ii + 1] - k0, d = diagk[ii] - k0;
@@ -548,14 +548,14 @@ void vjp_nodes(crimson_form *f, double *d_ybar, double *d_acbar, const crimson::
   hipStream_t s = f->stream;
   const unsigned gn = crimson::grid_for((size_t)f->nshg * kVjpLanes, 256);
   const IL *il = reinterpret_cast<const IL *>(f->d_iloc.p);
-  vjp_q_node<IL><<<gn, 256, 0, s>>>(f->nshg, f->d_rowptr.p, f->d_diagk.p, f->d_col.p, f->d_inc_ptr.p, f->d_inc.p, il,
+  vjp_q_node<IL><<<gn, 256, 0, s>>>(f->nshg, f->near_ptr(), f->near_diag(), f->d_col.p, f->d_inc_ptr.p, f->d_inc.p, il,
                                     f->d_xu.p, w.vrec2, w.invm, w.qbar);
   if (d_acbar)
-    vjp_node<IL, true><<<gn, 256, 0, s>>>(f->nshg, f->d_rowptr.p, f->d_diagk.p, f->d_col.p, f->d_inc_ptr.p,
+    vjp_node<IL, true><<<gn, 256, 0, s>>>(f->nshg, f->near_ptr(), f->near_diag(), f->d_col.p, f->d_inc_ptr.p,
                                           f->d_inc.p, il, f->d_xu.p, w.qbar, w.vrec, f->prm.mu, f->ens(), d_ybar,
                                           d_acbar, part);
   else
-    vjp_node<IL, false><<<gn, 256, 0, s>>>(f->nshg, f->d_rowptr.p, f->d_diagk.p, f->d_col.p, f->d_inc_ptr.p,
+    vjp_node<IL, false><<<gn, 256, 0, s>>>(f->nshg, f->near_ptr(), f->near_diag(), f->d_col.p, f->d_inc_ptr.p,
                                            f->d_inc.p, il, f->d_xu.p, w.qbar, w.vrec, f->prm.mu, f->ens(), d_ybar,
                                            nullptr, part);
 }

@@ -120,8 +120,8 @@ __global__ void __launch_bounds__(256) flux_node(int nshg, const int *__restrict
                                                  const double *__restrict__ ac, double *__restrict__ node,
                                                  double *__restrict__ q, double *__restrict__ invm) {
   __shared__ double xs_all[256 / kFluxLanes][kFluxCap * kXU];
-  const int gid = xcd_block() * blockDim.x + threadIdx.x;
-  const int i = gid / kFluxLanes, lane = gid % kFluxLanes;
+  const unsigned gid = xcd_block() * blockDim.x + threadIdx.x;
+  const int i = (int)(gid / kFluxLanes), lane = (int)(gid % kFluxLanes);
   const bool live = i < nshg;
   const int ii = live ? i : nshg - 1;
   const int k0 = rowptr[ii], ns = rowptr[ii + 1] - k0, d = diagk[ii] - k0;
@@ -673,8 +673,8 @@ template <int MODE>
 __global__ void __launch_bounds__(256) res_node(int nshg, const int *__restrict__ inc_ptr,
                                                 const int *__restrict__ inc, const double *__restrict__ rec,
                                                 double *__restrict__ res) {
-  const int gid = xcd_block() * blockDim.x + threadIdx.x;
-  const int i = gid / kResLanes, lane = gid % kResLanes;
+  const unsigned gid = xcd_block() * blockDim.x + threadIdx.x;
+  const int i = (int)(gid / kResLanes), lane = (int)(gid % kResLanes);
   double rs[4] = {0, 0, 0, 0};
   const int p1 = inc_ptr[min(i + 1, nshg)];
   for (int p = inc_ptr[min(i, nshg)] + lane; p < p1; p += kResLanes * kResUnroll) {
@@ -892,8 +892,8 @@ __global__ void __launch_bounds__(256) asm_row(int nshg, const int4 *__restrict_
                                                double *__restrict__ res, AsmOut o, unsigned xc, int runs) {
   static_assert(CH % 2 == 0 && LANES % CH == 0, "an even chunk that divides the lanes");
   __shared__ double st_all[256 / LANES][CH][kStage];
-  const int gid = xcd_block(xc) * blockDim.x + threadIdx.x;
-  const int slot = gid / LANES, lane = gid % LANES;
+  const unsigned gid = xcd_block(xc) * blockDim.x + threadIdx.x;
+  const int slot = (int)(gid / LANES), lane = (int)(gid % LANES);
   const bool live = slot < nshg;
   double(*st)[kStage] = st_all[threadIdx.x / LANES];
   int row = 0, k0 = 0, nslot = 0, sdiag = -1, p0 = 0, ninc = 0;
@@ -1068,8 +1068,8 @@ __global__ void __launch_bounds__(256) asm_row32(int nshg, const int4 *__restric
                                                  const unsigned short *__restrict__ lst,
                                                  const float *__restrict__ rec, AsmOut o, unsigned xc) {
   __shared__ float st_all[256 / LANES][LANES][kStage];
-  const int gid = xcd_block(xc) * blockDim.x + threadIdx.x;
-  const int slot = gid / LANES, lane = gid % LANES;
+  const unsigned gid = xcd_block(xc) * blockDim.x + threadIdx.x;
+  const int slot = (int)(gid / LANES), lane = (int)(gid % LANES);
   const bool live = slot < nshg;
   float(*st)[kStage] = st_all[threadIdx.x / LANES];
   int k0 = 0, nslot = 0, sdiag = -1, p0 = 0, ninc = 0;
@@ -1548,11 +1548,11 @@ int form_flux_pass(crimson_form *f, const double *d_y, const double *d_ac, const
   node_pack<<<crimson::grid_for(f->nshg, T), T, 0, s>>>(f->nshg, d_x, f->numnp, d_y, f->d_xu.p);
   const unsigned G = crimson::grid_for((size_t)f->nshg * kFluxLanes, T);
   if (f->wide)
-    flux_node<<<G, T, 0, s>>>(f->nshg, f->d_rowptr.p, f->d_diagk.p, f->d_col.p, f->d_inc_ptr.p, f->d_inc.p,
+    flux_node<<<G, T, 0, s>>>(f->nshg, f->near_ptr(), f->near_diag(), f->d_col.p, f->d_inc_ptr.p, f->d_inc.p,
                               reinterpret_cast<const unsigned long long *>(f->d_iloc.p), f->d_xu.p, f->prm.mu,
                               f->ens(), d_y, d_ac, f->d_node.p, d_q, d_invm);
   else
-    flux_node<<<G, T, 0, s>>>(f->nshg, f->d_rowptr.p, f->d_diagk.p, f->d_col.p, f->d_inc_ptr.p, f->d_inc.p,
+    flux_node<<<G, T, 0, s>>>(f->nshg, f->near_ptr(), f->near_diag(), f->d_col.p, f->d_inc_ptr.p, f->d_inc.p,
                               (const unsigned *)f->d_iloc.p, f->d_xu.p, f->prm.mu, f->ens(), d_y, d_ac, f->d_node.p,
                               d_q, d_invm);
   CR_HIP(hipGetLastError());
@@ -1683,6 +1683,9 @@ extern "C" int crimson_form_setup(int nshg, int numnp, int nel, const int *ien, 
     longer += rp[i + 1] - rp[i] > 16;
   }
   const bool wide = most > (1 << IncLoc<unsigned>::bits);
+  // rows too long even for the wide places: they count the blocks that elements
+  // touch, and the diagonal, alone (at most 3 x 4095 + 1)
+  const bool compact = most > (1 << IncLoc<unsigned long long>::bits);
   std::vector<unsigned> iloc;
   std::vector<unsigned long long> iloc64;
   if (wide)
@@ -1708,11 +1711,33 @@ extern "C" int crimson_form_setup(int nshg, int numnp, int nel, const int *ien, 
         lst_ptr[k + 1]++;
         o[n++] = k - rp[i];
       }
+      if (compact) continue;
       if (wide)
         iloc64[p] = IncLoc<unsigned long long>::pack(o, a);
       else
         iloc[p] = IncLoc<unsigned>::pack(o, a);
     }
+  }
+  std::vector<int> nrp, ncol, ndiag;  // compact: the touched blocks' rows
+  if (compact) {
+    std::vector<int> rank(nnz, 0);
+    nrp.push_back(0);
+    for (int i = 0; i < nshg; ++i) {
+      for (int k = rp[i]; k < rp[i + 1]; ++k) {
+        if (lst_ptr[k + 1] == 0 && k != diagk[i]) continue;
+        rank[k] = (int)ncol.size() - nrp[i];
+        if (k == diagk[i]) ndiag.push_back((int)ncol.size());
+        ncol.push_back(cols[k]);
+      }
+      nrp.push_back((int)ncol.size());
+    }
+    for (int i = 0; i < nshg; ++i)
+      for (int p = inc_ptr[i]; p < inc_ptr[i + 1]; ++p) {
+        int o[3], n = 0;
+        for (int b = 0; b < 4; ++b)
+          if (b != (inc[p] & 3)) o[n++] = rank[find_col(rp, cols, i, ien[(size_t)b * nel + (inc[p] >> 2)] - 1)];
+        iloc64[p] = IncLoc<unsigned long long>::pack(o, inc[p] & 3);
+      }
   }
   for (int k = 0; k < nnz; ++k) lst_ptr[k + 1] += lst_ptr[k];
   // two spare entries: the assembly reads the list in whole dwords
@@ -1726,7 +1751,8 @@ extern "C" int crimson_form_setup(int nshg, int numnp, int nel, const int *ien, 
         const int bits = wide ? IncLoc<unsigned long long>::bits : IncLoc<unsigned>::bits;
         for (int b = 0, n = 0; b < 4; ++b) {
           if (b == a) continue;
-          const int k = rp[i] + (int)(v >> (bits * n++) & ((1u << bits) - 1));
+          const int k = compact ? find_col(rp, cols, i, ien[(size_t)b * nel + (inc[p] >> 2)] - 1)
+                                : rp[i] + (int)(v >> (bits * n++) & ((1u << bits) - 1));
           lst[fill[k]++] = (unsigned short)(((p - inc_ptr[i]) << 4) | (a << 2) | b);
         }
       }
@@ -1793,7 +1819,8 @@ extern "C" int crimson_form_setup(int nshg, int numnp, int nel, const int *ien, 
       (rc = f->d_lst.upload(lst.data(), lst.size(), s)) ||
       (rc = wide ? f->d_iloc.upload(reinterpret_cast<const unsigned *>(iloc64.data()), 2 * iloc64.size(), s)
                  : f->d_iloc.upload(iloc.data(), iloc.size(), s)) ||
-      (rc = f->d_col.upload(cols.data(), cols.size(), s)) ||
+      (rc = compact ? f->d_col.upload(ncol.data(), ncol.size(), s) : f->d_col.upload(cols.data(), cols.size(), s)) ||
+      (rc = f->d_nrp.upload(nrp.data(), nrp.size(), s)) || (rc = f->d_ndiag.upload(ndiag.data(), ndiag.size(), s)) ||
       (rc = f->d_ienp.upload(ienp.data(), ienp.size(), s)) || (rc = f->d_xu.alloc((size_t)nshg * kXU)) ||
       (rc = f->d_node.alloc((size_t)nshg * kNRec)) || (rc = f->d_q.alloc((size_t)nshg * 9)) ||
       (rc = f->d_rec.alloc((size_t)std::max(nel, 1) * kRec)) ||
@@ -1990,7 +2017,7 @@ std::vector<unsigned long long> graph_signature(const crimson_form *f, const cri
   std::vector<unsigned long long> v = {
       f->d_ien.serial, f->d_inc_ptr.serial, f->d_inc.serial, f->d_diagk.serial, f->d_rowptr.serial,
       f->d_ibc.serial, f->d_lst_ptr.serial, f->d_order.serial, f->d_slot.serial, f->d_lst.serial,
-      f->d_ienp.serial, f->d_iloc.serial, f->d_col.serial, f->d_xu.serial, f->d_node.serial, f->d_rec.serial, f->d_esc.serial,
+      f->d_ienp.serial, f->d_iloc.serial, f->d_col.serial, f->d_nrp.serial, f->d_ndiag.serial, f->d_xu.serial, f->d_node.serial, f->d_rec.serial, f->d_esc.serial,
       f->d_rec32.serial, f->d_bc.serial,
       f->d_bcl.serial, f->d_bcn.serial, f->d_inst.serial, f->d_mu_inst.serial, f->d_binst.serial,
       f->d_ienb.serial, f->d_bcode.serial, f->d_bcb.serial, f->d_permit.serial, f->d_brec.serial,

@@ -273,7 +273,11 @@ struct crimson_form {
   crimson::DBuf<int4> d_ienp;    // per incidence (node-major): the element's four nodes in local order
   bool wide = false;                        // a row has more than 1024 blocks: IncLoc in 64 bits
   crimson::DBuf<unsigned> d_iloc;            // IncLoc per incidence (node-major), two words each when wide
-  crimson::DBuf<int> d_col;                  // CSR columns
+  // the columns of the rows that IncLoc's places count in: the CSR's, or, where a row
+  // has more than 2^20 blocks, those of the touched blocks (d_nrp, d_ndiag then)
+  crimson::DBuf<int> d_col, d_nrp, d_ndiag;
+  const int *near_ptr() const { return d_nrp.p ? d_nrp.p : d_rowptr.p; }
+  const int *near_diag() const { return d_ndiag.p ? d_ndiag.p : d_diagk.p; }
   crimson::DBuf<double> d_xu;    // (kXU, nshg): x and u of each node (node_pack)
   crimson::DBuf<double> d_node, d_q, d_rec, d_esc;  // node records; q; element records and scalars
   crimson::DBuf<float> d_rec32;  // FP32 tangent records (precision 32)

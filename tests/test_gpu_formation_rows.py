@@ -59,3 +59,34 @@ def test_formation_long_row(oracle_lib, n):
         err = float(np.abs(a - b).max() / np.abs(b).max())
         print(n, name, err, flush=True)
         assert err <= TOL, (name, err)
+
+
+def test_formation_row_past_the_places(oracle_lib):
+    """A hub whose row holds more than 2^20 blocks, nearly all of them touched by no
+    element (zero in the result): the flux pass then counts its places among the touched
+    blocks alone."""
+    import crimsonflowsolver_amd as cfa
+    ien, x = _ball(20)
+    n, N = 21, (1 << 20) + 64
+    # the hub's nodes keep their numbers, the surface's are spread over the hub's row
+    num = np.concatenate([[1], 2 + np.arange(n - 1) * ((N - 2) // (n - 1))])
+    ien = np.asfortranarray(num[ien - 1].astype(np.int32))
+    X = np.zeros((N, 3), order="F")
+    X[num - 1] = x
+    rng = np.random.default_rng(20)
+    y = np.asfortranarray(rng.normal(size=(N, 4)) * np.array([10.0, 1.0, 1.0, 1.0]))
+    ac = np.asfortranarray(rng.uniform(-20, 20, size=(N, 4)))
+    pairs = np.concatenate([np.arange(N), np.arange(N) * (N + 1)] +
+                           [(N * (ien[:, [a]].astype(np.int64) - 1) + ien - 1).ravel() for a in range(4)])
+    pairs = np.unique(pairs)
+    colm = (np.searchsorted(pairs, N * np.arange(N + 1, dtype=np.int64)) + 1).astype(np.int32)
+    rowp = (pairs % N + 1).astype(np.int32)
+    assert colm[1] - colm[0] == N
+    form = cfa.ElmGMRInterior(ien, colm, rowp, N)
+    res, K, P, q = form(y, ac, X, want_q=True)
+    rres, rK, rP, rq = oracle_lib.elmgmr_interior(ien, y, ac, X, colm, rowp, oracle_lib.make_params(), want_q=True)
+    m = num - 1
+    for name, a, b in (("res", res, rres), ("lhsK", K, rK), ("lhsP", P, rP), ("q", q[m], rq[m])):
+        err = float(np.abs(a - b).max() / np.abs(b).max())
+        print(name, err, flush=True)
+        assert err <= TOL, (name, err)
