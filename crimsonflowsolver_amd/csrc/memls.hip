@@ -2954,24 +2954,27 @@ int precond(Ctx<T> &c) {
 }
 
 // The solve's statistics from a copy of the first G_ARR entries of gst
-// into ls's fields (as nssolver_dev leaves them); CRIMSON_ESINGULAR when GE
-// met a singular pivot.
-int ns_stats(const double *h, crimson_ls *ls) {
-  if (h[G_ERR] != 0.0) {
-    crimson::set_error("memLS GE: singular matrix");
-    return CRIMSON_ESINGULAR;
-  }
+// into ls's fields, as NSSOLVER leaves them; CRIMSON_ESINGULAR when GE met a
+// singular pivot (a plain solve's statistics then reach up to GE, a captured one's are
+// untouched).  A GMRES call whose residual is below absTol at once leaves iNorm and
+// fNorm as they were (GMRES, memLS.f90:681-788): with no other call in the solve ls
+// keeps its own.
+int ns_stats(const double *h, crimson_ls *ls, bool plain) {
+  const bool singular = h[G_ERR] != 0.0;
+  if (singular) crimson::set_error("memLS GE: singular matrix");
+  if (singular && !plain) return CRIMSON_ESINGULAR;
   ls->RI.iNorm = h[G_RI_INORM];
   ls->RI.fNorm = h[G_RI_FNORM];
-  ls->RI.itr = (int)h[G_RI_ITR];
   ls->RI.suc = h[G_RI_SUC] != 0.0;
-  ls->RI.dB = 10.0 * std::log(h[G_RI_FNORM] / h[G_RI_DBPRE]);
   ls->RI.callD = 0.0;
-  ls->GM.iNorm = h[G_GM_INORM];
-  ls->GM.fNorm = h[G_GM_FNORM];
+  const bool ran = h[G_GM_LASTD] != 0.0;
+  if (ran) {
+    ls->GM.iNorm = h[G_GM_INORM];
+    ls->GM.fNorm = h[G_GM_FNORM];
+  }
   ls->GM.itr = (int)h[G_GM_ITR];
   ls->GM.suc = h[G_GM_SUC] != 0.0;
-  ls->GM.dB = h[G_GM_LASTD] != 0.0 ? 10.0 * std::log(h[G_GM_LASTF] / h[G_GM_LASTD]) : 0.0;
+  ls->GM.dB = ran && !(plain && h[G_GM_EARLY] != 0.0) ? 10.0 * std::log(h[G_GM_LASTF] / h[G_GM_LASTD]) : 0.0;
   ls->GM.callD = 0.0;
   ls->CG.iNorm = h[G_CG_INORM];
   ls->CG.fNorm = std::sqrt(h[G_CG_ERR]);
@@ -2979,6 +2982,12 @@ int ns_stats(const double *h, crimson_ls *ls) {
   ls->CG.suc = h[G_CG_SUC] != 0.0;
   ls->CG.dB = 5.0 * std::log(h[G_CG_ERR] / h[G_CG_ERRO]);
   ls->CG.callD = 0.0;
+  if (singular) {
+    ls->RI.dB = h[G_RI_DBPRE];
+    return CRIMSON_ESINGULAR;
+  }
+  ls->RI.itr = (int)h[G_RI_ITR];
+  ls->RI.dB = 10.0 * std::log(h[G_RI_FNORM] / h[G_RI_DBPRE]);
   const double rcn = std::sqrt(h[G_RC_N2]) / ls->RI.fNorm;
   ls->Resc = (int)std::lround(100.0 * rcn * rcn);
   ls->Resm = 100 - ls->Resc;
@@ -3068,7 +3077,7 @@ int solve_run(SolveWork<T> &w, crimson_lhs *l, crimson_ls *ls, int dof, double *
     double h[G_ARR];
     CR_HIP(hipMemcpyAsync(h, w.gst.p, sizeof(h), hipMemcpyDeviceToHost, c.s));
     CR_HIP(hipStreamSynchronize(c.s));
-    CR_TRY(ns_stats(h, ls));
+    CR_TRY(ns_stats(h, ls, true));
     ls->RI.callD = now_s() - t0;
     ls->GM.callD = w.tGM;
     ls->CG.callD = w.tCG;
@@ -3169,7 +3178,7 @@ struct NsGraphExtra : crimson::GraphExtra {
     hstat.resize((size_t)G_ARR * nsolve);
     CR_HIP(hipMemcpy(hstat.data(), stat.p, hstat.size() * sizeof(double), hipMemcpyDeviceToHost));
     int rc = CRIMSON_OK;
-    for (int k = 0; k < nsolve && rc == CRIMSON_OK; ++k) rc = ns_stats(hstat.data() + (size_t)G_ARR * k, ls);
+    for (int k = 0; k < nsolve && rc == CRIMSON_OK; ++k) rc = ns_stats(hstat.data() + (size_t)G_ARR * k, ls, false);
     return rc;
   }
   std::vector<unsigned long long> signature() const override { return ns_signature(lhs, ls); }

@@ -1,0 +1,82 @@
+"""What a memLS solve leaves behind and takes over: the statistics of a solver
+object after solves of another one on the same matrix handle.
+
+The systems are test_gpu_schur's (4x4 blocks on small graphs, D = -G^T
+blockwise, K near twice the identity).
+"""
+import numpy as np
+import pytest
+
+from test_gpu_schur import _system
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def cfa():
+    import crimsonflowsolver_amd as cfa
+    if cfa.device_count() < 1:
+        pytest.fail("no GPU visible: the HIP path must run here")
+    return cfa
+
+
+def _handle(cfa, rowptr, colptr, faces=0):
+    n = rowptr.size - 1
+    return cfa.memLS_LHS_CREATE(n, n, colptr.size, None, rowptr, colptr, faces)
+
+
+def _ns(cfa, absTolGM, maxItr=1, relTolGM=0.1):
+    return cfa.memLS_LS_CREATE(cfa.LS_TYPE_NS, relTol=1e-12, dimKry=20, maxItr=maxItr, relTolIn=[relTolGM, 0.1],
+                               absTolIn=[absTolGM, 1e-10], maxItrIn=[1, 50])
+
+
+def test_gmres_statistics_are_the_solvers_own(cfa):
+    """A solve whose GMRES calls all end at once (residual below absTol) leaves
+    the solver's GM norms as they were: zero in a new one, its last solve's in a
+    used one.  With the momentum solution zero, the second outer iteration's
+    Gram matrix has a zero column: singular, the statistics up to there set."""
+    rowptr, colptr, val, A = _system(60, [(i, (i + k) % 60) for i in range(60) for k in (1, 2, 3)], 5)
+    lhs = _handle(cfa, rowptr, colptr)
+    R = np.asfortranarray(np.random.default_rng(1).standard_normal((4, 60)))
+    used = _ns(cfa, 1e-10)
+    cfa.memLS_SOLVE(lhs, used, 4, R.copy(order="F"), val)
+    before = used.stats("GM")
+    assert before["iNorm"] > 0 and before["itr"] > 0
+    fresh = _ns(cfa, 1e30)
+    cfa.memLS_SOLVE(lhs, fresh, 4, R.copy(order="F"), val)
+    got = fresh.stats("GM")
+    assert (got["iNorm"], got["fNorm"], got["itr"], got["suc"], got["dB"]) == (0, 0, 0, 0, 0)
+    assert fresh.stats("RI")["iNorm"] == used.stats("RI")["iNorm"]
+    two = _ns(cfa, 1e30, maxItr=2)
+    with pytest.raises(cfa.CrimsonError) as e:
+        cfa.memLS_SOLVE(lhs, two, 4, R.copy(order="F"), val)
+    assert e.value.code == 7
+    assert two.stats("RI")["iNorm"] == used.stats("RI")["iNorm"] and two.stats("CG")["itr"] > 0
+
+
+def test_gmres_db_of_a_last_call_that_ends_at_once(cfa):
+    """The second momentum solve of an outer iteration starts from Rm - G P, smaller
+    than Rm; an absTol between the two ends it at once, and GM's dB is then 0."""
+    n = 60
+    rowptr, colptr, val, A = _system(n, [(i, (i + k) % n) for i in range(n) for k in (1, 2, 3)], 5)
+    lhs = _handle(cfa, rowptr, colptr)
+    d = np.abs(np.diag(A)).reshape(n, 4).T
+    # a momentum residual in the range of G, which the pressure removes for the most part
+    p = np.random.default_rng(2).standard_normal(n)
+    G = A.reshape(n, 4, n, 4)[:, :3, :, 3]
+    R = np.zeros((4, n), order="F")
+    R[:3] = np.einsum("aib,b->ia", G, p)
+    L = A.reshape(n, 4, n, 4)[:, 3, :, 3]
+    R[3] = 0.6 * (L @ p)
+    n1 = np.linalg.norm((R / np.sqrt(d))[:3])
+    ls = _ns(cfa, 1e-10, relTolGM=0.9)
+    cfa.memLS_SOLVE(lhs, ls, 4, R.copy(order="F"), val)
+    n2 = ls.stats("GM")["iNorm"]
+    print("norms", n1, n2)
+    assert n2 < 0.85 * n1 and ls.stats("GM")["dB"] != 0
+    # below 0.9 n1 the first call's target is relTol's either way, so that P is the same
+    ls = _ns(cfa, 0.5 * (0.9 * n1 + n2), relTolGM=0.9)
+    cfa.memLS_SOLVE(lhs, ls, 4, R.copy(order="F"), val)
+    got = ls.stats("GM")
+    assert abs(got["iNorm"] - n1) <= 1e-12 * n1
+    assert got["suc"] == 0 and got["dB"] == 0
