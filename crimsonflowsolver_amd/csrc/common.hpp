@@ -150,11 +150,13 @@ int form_wall_enqueue_alpha(crimson_form *f);
 int form_wall_enqueue_correct(crimson_form *f, const double *d_Res4);
 int form_wall_enqueue_update(crimson_form *f);
 
-// What a graph of the solver side adds to a replay: the state it holds on
-// the device, read back after each launch, and the buffers and settings it
-// baked in (a replay is refused once they change).
+// What a graph of the solver side adds to a replay: what it brings up to date
+// before one, the state it holds on the device, read back after each launch,
+// and the buffers and settings it baked in (a replay is refused once they
+// change).
 struct GraphExtra {
   virtual ~GraphExtra() = default;
+  virtual int before_launch() { return CRIMSON_OK; }
   virtual int after_launch() { return CRIMSON_OK; }
   virtual std::vector<unsigned long long> signature() const { return {}; }
 };
@@ -219,12 +221,6 @@ struct SolveWorkBase {
 };
 }  // namespace crimson
 
-// One entry of the coupled faces' merged supports: a node, the face (its place among
-// the coupled ones) and the node's place in that face's support.
-struct CrFaceEnt {
-  int node, f, s;
-};
-
 // memLS matrix handle.  The matrix of block size vdof (1..4) is held as
 // vdof*vdof planes of nnz doubles, plane m = row-major entry (m / vdof,
 // m % vdof) of every block, i.e. Val(m+1, :) of the reference layout.
@@ -245,11 +241,6 @@ struct crimson_lhs {
   crimson::DBuf<double> d_Gt;     // [3][nnz] when !gt_is_d
   crimson::DBuf<float> d_Gt32;    // the same for an FP32 matrix
   std::vector<CrFace> face;
-  // the coupled faces' merged supports and their first entries per 256 nodes,
-  // for the faces whose supports fent_sig lists
-  std::vector<unsigned long long> fent_sig;
-  crimson::DBuf<CrFaceEnt> d_fent;
-  crimson::DBuf<int> d_ftptr;
   // the Schur complement of the NS solver's CG on the graph's two-ring: 0 not
   // looked at yet, 1 its pattern is here (schur_nnz entries, schur_row at most in
   // a row; columns as offsets from the row in d_scol16 where they fit), 2 this

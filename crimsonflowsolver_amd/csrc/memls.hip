@@ -186,7 +186,9 @@ constexpr int kFaceDotBlocks = 4;
 // The faces' supports merged for the residual update: the entries (node,
 // face, place in the face's support) sorted by node, then face; tptr[t] is
 // the first entry of nodes 256 t and above.
-using FaceEnt = CrFaceEnt;
+struct FaceEnt {
+  int node, f, s;
+};
 struct FaceList {
   int nfc;               // coupled faces
   const FaceDev *fd;
@@ -1753,7 +1755,12 @@ struct Ctx {
   std::vector<FaceDev> hfdev;    // fdev on the host
   bool disjoint = true;          // no two coupled faces share a node
   int nfc() const { return (int)hfdev.size(); }
-  FaceList face_list() const { return FaceList{nfc(), fdev.p, lhs->d_fent.p, lhs->d_ftptr.p, fpart.p}; }
+  // their merged supports and the first entries per 256 nodes, for the faces whose
+  // supports fent_sig lists
+  std::vector<unsigned long long> fent_sig;
+  crimson::DBuf<FaceEnt> fent;
+  crimson::DBuf<int> ftptr;
+  FaceList face_list() const { return FaceList{nfc(), fdev.p, fent.p, ftptr.p, fpart.p}; }
 
   int init(crimson_lhs *l, int d, hipStream_t st) {
     lhs = l;
@@ -2079,7 +2086,7 @@ int face_support(crimson_lhs *l, CrFace &fa) {
   return CRIMSON_OK;
 }
 
-// The merged supports of the coupled faces (FaceList), which the handle keeps
+// The merged supports of the coupled faces (FaceList), kept with the workspace
 // while the same faces are coupled.
 template <class T>
 int face_list(Ctx<T> &c) {
@@ -2088,7 +2095,7 @@ int face_list(Ctx<T> &c) {
   std::vector<unsigned long long> sig;
   for (const auto &fa : l->face)
     if (fa.coupled) sig.push_back(fa.support);
-  if (sig == l->fent_sig && l->d_ftptr.p) return CRIMSON_OK;
+  if (sig == c.fent_sig && c.ftptr.p) return CRIMSON_OK;
   std::vector<FaceEnt> ent;
   int f = 0;
   for (const auto &fa : l->face) {
@@ -2105,10 +2112,11 @@ int face_list(Ctx<T> &c) {
     ptr[t] = (int)e;
   }
   ptr.back() = (int)ent.size();
-  CR_TRY(l->d_fent.upload(ent.data(), ent.size(), c.s));
-  CR_TRY(l->d_ftptr.upload(ptr.data(), ptr.size(), c.s));
+  c.fent_sig.clear();
+  CR_TRY(c.fent.upload(ent.data(), ent.size(), c.s));
+  CR_TRY(c.ftptr.upload(ptr.data(), ptr.size(), c.s));
   CR_HIP(hipStreamSynchronize(c.s));
-  l->fent_sig = sig;
+  c.fent_sig = sig;
   return CRIMSON_OK;
 }
 // The faces' functionals q for this solve's matrix and scaling.
@@ -2801,13 +2809,21 @@ int ns_run(SolveWork<T> &w, double *d_Ri) {
   return CRIMSON_OK;
 }
 
+// Whether no two coupled faces share a node.
+bool faces_disjoint(const crimson_lhs *l) {
+  std::vector<int> nodes;
+  for (const auto &fa : l->face)
+    if (fa.coupled) nodes.insert(nodes.end(), fa.glob.begin(), fa.glob.end());
+  std::sort(nodes.begin(), nodes.end());
+  return std::adjacent_find(nodes.begin(), nodes.end()) == nodes.end();
+}
+
 // The coupled faces of this solve (memLS.f90:1965-1986; res[f] != 0 couples Neumann face
 // f) on the device.
 template <class T>
 int face_setup(Ctx<T> &c, const int *incL, const double *res, bool ns) {
   crimson_lhs *l = c.lhs;
   std::vector<FaceDev> fd;
-  std::vector<int> nodes;
   int n = 0;
   for (int f = 0; f < l->nFaces; ++f) {
     CrFace &fa = l->face[f];
@@ -2838,10 +2854,8 @@ int face_setup(Ctx<T> &c, const int *incL, const double *res, bool ns) {
     d.q = ns ? fa.d_q.p : nullptr;
     d.nsup = ns ? fa.nsup : 0;
     fd.push_back(d);
-    nodes.insert(nodes.end(), fa.glob.begin(), fa.glob.end());
   }
-  std::sort(nodes.begin(), nodes.end());
-  c.disjoint = std::adjacent_find(nodes.begin(), nodes.end()) == nodes.end();
+  c.disjoint = faces_disjoint(l);
   const bool same = fd.size() == c.hfdev.size() && c.fdev.p &&
                     std::equal(fd.begin(), fd.end(), c.hfdev.begin(), [](const FaceDev &a, const FaceDev &b) {
                       return a.glob == b.glob && a.valM == b.valM && a.coefp == b.coefp && a.res == b.res &&
@@ -3152,7 +3166,7 @@ std::vector<unsigned long long> ns_signature(const crimson_lhs *l, const crimson
                                        (unsigned long long)l->gt_is_d, (unsigned long long)ls->RI.mItr,
                                        (unsigned long long)ls->GM.mItr, (unsigned long long)ls->GM.sD,
                                        (unsigned long long)ls->CG.mItr, l->d_S.serial, l->d_S32.serial,
-                                       l->d_sptr.serial, l->d_fent.serial, l->d_ftptr.serial};
+                                       l->d_sptr.serial};
   for (const auto &fa : l->face) {
     v.push_back(fa.d_glob.serial);
     v.push_back(fa.d_val.serial);
@@ -3174,6 +3188,24 @@ struct NsGraphExtra : crimson::GraphExtra {
   int nsolve = 0;
   crimson::DBuf<double> stat;  // G_ARR doubles per captured solve
   std::vector<double> hstat;
+  // Faces that crimson_bc_create gave other nodes since the capture, in buffers of the
+  // same sizes: their supports and the merged list follow, in place (buffers of other
+  // sizes change the signature, and the replay is refused).
+  int before_launch() override {
+    Ctx<T> &c = w.c;
+    std::vector<unsigned long long> sig;
+    for (auto &fa : lhs->face)
+      if (fa.coupled) {
+        CR_TRY(face_support(lhs, fa));
+        sig.push_back(fa.support);
+      }
+    if (sig == c.fent_sig || (int)sig.size() != c.nfc()) return CRIMSON_OK;
+    if (c.disjoint && !faces_disjoint(lhs)) {
+      crimson::set_error("crimson_graph_launch: coupled faces share nodes since the capture; capture it again");
+      return CRIMSON_ESTATE;
+    }
+    return face_list(c);
+  }
   int after_launch() override {
     hstat.resize((size_t)G_ARR * nsolve);
     CR_HIP(hipMemcpy(hstat.data(), stat.p, hstat.size() * sizeof(double), hipMemcpyDeviceToHost));

@@ -80,3 +80,58 @@ def test_gmres_db_of_a_last_call_that_ends_at_once(cfa):
     got = ls.stats("GM")
     assert abs(got["iNorm"] - n1) <= 1e-12 * n1
     assert got["suc"] == 0 and got["dB"] == 0
+
+
+def _coupled(cfa, n=60, seed=5):
+    """A ring of 60 nodes with two coupled faces of 10 and 15 nodes."""
+    rowptr, colptr, val, _ = _system(n, [(i, (i + k) % n) for i in range(n) for k in (1, 2, 3)], seed)
+    lhs = _handle(cfa, rowptr, colptr, 2)
+    rng = np.random.default_rng(6)
+    v = [rng.uniform(0.2, 1.0, (3, k)) for k in (10, 15)]
+    for f, start in enumerate((4, 30)):
+        cfa.memLS_BC_CREATE(lhs, f + 1, v[f].shape[1], 3, cfa.BC_TYPE_Neu, np.arange(start, start + v[f].shape[1]) + 1,
+                            np.asfortranarray(v[f]))
+    lhs.set_val(4, val)
+    return lhs, v
+
+
+def _solver(cfa):
+    return cfa.memLS_LS_CREATE(cfa.LS_TYPE_NS, relTol=1e-5, dimKry=40, maxItr=6, relTolIn=[0.1, 0.1], maxItrIn=[2, 200])
+
+
+def test_graph_after_solves_with_other_faces(cfa):
+    """A captured solve with two coupled faces, replayed after plain solves with one of
+    them and with both: accepted, and the plain solve's bits.  Replayed after a
+    face moved to other nodes (as many of them): the plain solve's bits there."""
+    import torch
+    lhs, v = _coupled(cfa)
+    rhs = torch.from_numpy(1e3 * np.random.default_rng(8).standard_normal((60, 4))).cuda()
+    both, one = np.array([7.0, 4.0]), np.array([7.0, 0.0])
+
+    def plain(res):
+        x = rhs.clone()
+        cfa.memLS_SOLVE_dev(lhs, _solver(cfa), 4, x, res=res)
+        return x
+
+    buf = torch.empty_like(rhs)
+    graph = cfa.memLS_SOLVE_graph(lhs, _solver(cfa), 4, buf, res=both)
+
+    def replay():
+        buf.copy_(rhs)
+        torch.cuda.synchronize()
+        graph.launch()
+        return buf.clone()
+
+    want = plain(both)
+    assert torch.equal(replay(), want)
+    assert not torch.equal(plain(one), want)
+    with pytest.raises(cfa.CrimsonError) as e:  # another set is coupled
+        replay()
+    assert e.value.code == 8
+    assert torch.equal(plain(both), want)
+    for _ in range(2):
+        assert torch.equal(replay(), want)
+    cfa.memLS_BC_CREATE(lhs, 2, 15, 3, cfa.BC_TYPE_Neu, np.arange(35, 50) + 1, np.asfortranarray(v[1]))
+    moved = replay()
+    assert torch.equal(moved, plain(both)) and not torch.equal(moved, want)
+    assert torch.equal(replay(), moved)
