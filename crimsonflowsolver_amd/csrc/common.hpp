@@ -214,6 +214,15 @@ struct CrFace {
 };
 
 namespace crimson {
+// The pattern of the Schur complement on the graph's two-ring: a property of the
+// graph, shared by the handle and the workspaces that hold values on it.
+struct SchurPattern {
+  int row = 0;        // entries of the longest row
+  long long nnz = 0;
+  DBuf<int> ptr, col;
+  DBuf<short> col16;  // the columns as offsets from the row, where they fit (col empty)
+};
+
 // A solve's workspaces, as a matrix handle keeps them (memls.hip).
 struct SolveWorkBase {
   virtual ~SolveWorkBase() = default;
@@ -241,17 +250,11 @@ struct crimson_lhs {
   crimson::DBuf<double> d_Gt;     // [3][nnz] when !gt_is_d
   crimson::DBuf<float> d_Gt32;    // the same for an FP32 matrix
   std::vector<CrFace> face;
-  // the Schur complement of the NS solver's CG on the graph's two-ring: 0 not
-  // looked at yet, 1 its pattern is here (schur_nnz entries, schur_row at most in
-  // a row; columns as offsets from the row in d_scol16 where they fit), 2 this
-  // graph keeps the two-pass operator
-  int schur = 0, schur_row = 0;
-  long long schur_nnz = 0;
+  // the Schur complement of the NS solver's CG: 0 not looked at yet, 1 its pattern
+  // is in spat, 2 this graph keeps the two-pass operator
+  int schur = 0;
+  std::shared_ptr<crimson::SchurPattern> spat;
   int band = 0;  // largest |column - row| (with d_col16)
-  crimson::DBuf<int> d_sptr, d_scol;
-  crimson::DBuf<short> d_scol16;
-  crimson::DBuf<double> d_S;
-  crimson::DBuf<float> d_S32;
   // the workspaces of the last plain solve in FP64 and in FP32 (work_take, work_keep)
   std::unique_ptr<crimson::SolveWorkBase> work[2];
   hipEvent_t ev0 = nullptr, ev1 = nullptr;

@@ -1895,9 +1895,6 @@ int cg_den(Ctx<T> &c, size_t L, const T *P, const T *SP, const double *done, int
 }
 
 // ----- the Schur operator: formed (schur_pattern) or in two passes -----
-inline crimson::DBuf<double> &schur_buf(crimson_lhs *l, double) { return l->d_S; }
-inline crimson::DBuf<float> &schur_buf(crimson_lhs *l, float) { return l->d_S32; }
-
 // An allocation that may fail without failing the solve: the error state is
 // cleared and the caller takes the path that needs no such buffer.
 template <class B>
@@ -1914,13 +1911,13 @@ bool try_alloc(B &b, size_t n) {
 // work of one more launch.
 constexpr int kSchurFill = 6;
 template <class IX, class OX>
-int schur_pattern_fill(crimson_lhs *l, const IX *col, crimson::DBuf<OX> &scol, long long n) {
-  if (!try_alloc(scol, (size_t)n)) {
+int schur_pattern_fill(crimson_lhs *l, const IX *col, crimson::SchurPattern &p, crimson::DBuf<OX> &scol) {
+  if (!try_alloc(scol, (size_t)p.nnz)) {
     l->schur = 2;
     return CRIMSON_OK;
   }
   schur_pattern_kernel<IX, OX, true><<<crimson::grid_for(l->nNo, 4), 256, 0, l->stream>>>(l->nNo, l->d_rowptr.p, col,
-                                                                                         nullptr, l->d_sptr.p, scol.p);
+                                                                                         nullptr, p.ptr.p, scol.p);
   CR_HIP(hipGetLastError());
   CR_HIP(hipStreamSynchronize(l->stream));
   l->schur = 1;
@@ -1929,8 +1926,9 @@ int schur_pattern_fill(crimson_lhs *l, const IX *col, crimson::DBuf<OX> &scol, l
 int schur_pattern(crimson_lhs *l) {
   if (l->schur) return CRIMSON_OK;
   const int N = l->nNo;
+  auto p = std::make_shared<crimson::SchurPattern>();
   crimson::DBuf<int> cnt;
-  if (!try_alloc(cnt, (size_t)N) || !try_alloc(l->d_sptr, (size_t)N + 1)) {
+  if (!try_alloc(cnt, (size_t)N) || !try_alloc(p->ptr, (size_t)N + 1)) {
     l->schur = 2;
     return CRIMSON_OK;
   }
@@ -1945,80 +1943,71 @@ int schur_pattern(crimson_lhs *l) {
   std::vector<int> ptr((size_t)N + 1);
   CR_HIP(hipMemcpyAsync(ptr.data() + 1, cnt.p, (size_t)N * sizeof(int), hipMemcpyDeviceToHost, l->stream));
   CR_HIP(hipStreamSynchronize(l->stream));
-  long long n = 0;
-  int most = 0;
   ptr[0] = 0;
   for (int i = 1; i <= N; ++i) {
-    most = std::max(most, ptr[i]);
-    n += ptr[i];
-    ptr[i] = (int)n;
-    if (most > kSchurRow || n > (long long)kSchurFill * l->nnz || n > 0x7fffff00LL) {
+    p->row = std::max(p->row, ptr[i]);
+    p->nnz += ptr[i];
+    ptr[i] = (int)p->nnz;
+    if (p->row > kSchurRow || p->nnz > (long long)kSchurFill * l->nnz || p->nnz > 0x7fffff00LL) {
       l->schur = 2;
-      l->d_sptr.release();
       return CRIMSON_OK;
     }
   }
-  l->schur_row = most;
-  l->schur_nnz = n;
-  CR_TRY(l->d_sptr.upload(ptr.data(), ptr.size(), l->stream));
-  if (l->d_col16.p) {
-    if (2 * l->band <= 32767) return schur_pattern_fill(l, l->d_col16.p, l->d_scol16, n);
-    return schur_pattern_fill(l, l->d_col16.p, l->d_scol, n);
-  }
-  return schur_pattern_fill(l, l->d_col.p, l->d_scol, n);
+  CR_TRY(p->ptr.upload(ptr.data(), ptr.size(), l->stream));
+  CR_HIP(hipStreamSynchronize(l->stream));
+  if (l->d_col16.p && 2 * l->band <= 32767)
+    CR_TRY(schur_pattern_fill(l, l->d_col16.p, *p, p->col16));
+  else if (l->d_col16.p)
+    CR_TRY(schur_pattern_fill(l, l->d_col16.p, *p, p->col));
+  else
+    CR_TRY(schur_pattern_fill(l, l->d_col.p, *p, p->col));
+  if (l->schur == 1) l->spat = p;
+  return CRIMSON_OK;
 }
 
 template <class T>
 struct SchurOp {
-  bool formed = false;
+  const crimson::SchurPattern *pat = nullptr;  // formed: S's pattern and values
+  T *S = nullptr;
   MatView<T> L, Gt, G;
   T *Z = nullptr, *Ps = nullptr;  // two passes: Z(4, N) and the scaled direction
 };
-// S's pattern and storage (before a capture); formed = false when the two
-// passes are taken.
-template <class T>
-int schur_ready(crimson_lhs *l, SchurOp<T> &o) {
-  CR_TRY(schur_pattern(l));
-  o.formed = l->schur == 1 && try_alloc(schur_buf(l, T(0)), (size_t)l->schur_nnz);
-  return CRIMSON_OK;
-}
 // S's values from the matrix and the scaling of this solve.
 template <class T>
 int schur_form(Ctx<T> &c, const SchurOp<T> &o) {
-  if (!o.formed) return CRIMSON_OK;
+  if (!o.pat) return CRIMSON_OK;
   crimson_lhs *l = c.lhs;
+  const crimson::SchurPattern &p = *o.pat;
   const unsigned G = crimson::grid_for(l->nNo, 16);
-  const size_t sh = (size_t)16 * l->schur_row * (sizeof(double) + sizeof(int));
-  T *S = schur_buf(l, T(0)).p;
-#define CR_SV(IX_, CP_, OX_, SP_)                                                                                  \
-  schur_values_kernel<T, IX_, OX_><<<G, 256, sh, c.s>>>(l->nNo, l->d_rowptr.p, CP_, o.L, o.Gt, o.G, l->d_sptr.p, SP_, \
-                                                        S, l->schur_row)
-  if (l->d_scol16.p)
-    CR_SV(short, l->d_col16.p, short, l->d_scol16.p);
+  const size_t sh = (size_t)16 * p.row * (sizeof(double) + sizeof(int));
+#define CR_SV(IX_, CP_, OX_, SP_)                                                                               \
+  schur_values_kernel<T, IX_, OX_><<<G, 256, sh, c.s>>>(l->nNo, l->d_rowptr.p, CP_, o.L, o.Gt, o.G, p.ptr.p, SP_, \
+                                                        o.S, p.row)
+  if (p.col16.p)
+    CR_SV(short, l->d_col16.p, short, p.col16.p);
   else if (l->d_col16.p)
-    CR_SV(short, l->d_col16.p, int, l->d_scol.p);
+    CR_SV(short, l->d_col16.p, int, p.col.p);
   else
-    CR_SV(int, l->d_col.p, int, l->d_scol.p);
+    CR_SV(int, l->d_col.p, int, p.col.p);
 #undef CR_SV
   CR_HIP(hipGetLastError());
   return CRIMSON_OK;
 }
 // SP = S P of the formed complement with the new direction and the parts of P . SP.
 template <class T>
-int schur_dir_product(Ctx<T> &c, const PairT<T> *Q, T *P, T *SP, const double *scal, double *next, int nr,
-                  const FaceList &fl, HostFlag hf, int &nd) {
-  crimson_lhs *l = c.lhs;
-  const int N = l->nNo, ntile = (int)crimson::grid_for((size_t)N, 256 / kSLanes);
+int schur_dir_product(Ctx<T> &c, const SchurOp<T> &o, const PairT<T> *Q, T *P, T *SP, const double *scal, double *next,
+                      int nr, const FaceList &fl, HostFlag hf, int &nd) {
+  const int N = c.N, ntile = (int)crimson::grid_for((size_t)N, 256 / kSLanes);
   nd = std::min(ntile, kCgGrid);
   const int G = nd + fl.nfc * kFaceDotBlocks;
-  const T *S = schur_buf(l, T(0)).p;
+  const crimson::SchurPattern &p = *o.pat;
   double *dpart = c.part.p, *rpart = c.part.p + kCgGrid;
-  if (l->d_scol16.p)
-    s_dir_product_kernel<T, short><<<G, 256, 0, c.s>>>(N, ntile, l->d_sptr.p, l->d_scol16.p, S, Q, P, SP, dpart, scal,
-                                                   next, rpart, nr, fl, hf);
+  if (p.col16.p)
+    s_dir_product_kernel<T, short><<<G, 256, 0, c.s>>>(N, ntile, p.ptr.p, p.col16.p, o.S, Q, P, SP, dpart, scal, next,
+                                                       rpart, nr, fl, hf);
   else
-    s_dir_product_kernel<T, int><<<G, 256, 0, c.s>>>(N, ntile, l->d_sptr.p, l->d_scol.p, S, Q, P, SP, dpart, scal, next,
-                                                 rpart, nr, fl, hf);
+    s_dir_product_kernel<T, int><<<G, 256, 0, c.s>>>(N, ntile, p.ptr.p, p.col.p, o.S, Q, P, SP, dpart, scal, next,
+                                                     rpart, nr, fl, hf);
   CR_HIP(hipGetLastError());
   return CRIMSON_OK;
 }
@@ -2028,14 +2017,14 @@ int schur_apply(Ctx<T> &c, const SchurOp<T> &o, const T *P, T *SP, const double 
   crimson_lhs *l = c.lhs;
   const int N = l->nNo;
   double *dpart = c.part.p;
-  if (o.formed) {
+  if (o.pat) {
     const int ntile = (int)crimson::grid_for((size_t)N, 256 / kSLanes);
     nd = std::min(ntile, kCgGrid);
-    const T *S = schur_buf(l, T(0)).p;
-    if (l->d_scol16.p)
-      s_product_kernel<T, short><<<nd, 256, 0, c.s>>>(N, ntile, l->d_sptr.p, l->d_scol16.p, S, P, SP, dpart, done);
+    const crimson::SchurPattern &p = *o.pat;
+    if (p.col16.p)
+      s_product_kernel<T, short><<<nd, 256, 0, c.s>>>(N, ntile, p.ptr.p, p.col16.p, o.S, P, SP, dpart, done);
     else
-      s_product_kernel<T, int><<<nd, 256, 0, c.s>>>(N, ntile, l->d_sptr.p, l->d_scol.p, S, P, SP, dpart, done);
+      s_product_kernel<T, int><<<nd, 256, 0, c.s>>>(N, ntile, p.ptr.p, p.col.p, o.S, P, SP, dpart, done);
     CR_HIP(hipGetLastError());
     return CRIMSON_OK;
   }
@@ -2441,7 +2430,9 @@ struct SolveWork : crimson::SolveWorkBase {
   crimson::DBuf<double> gst, npart, h;    // state and small systems; norm parts (2 kSubGrid); h1, h2
   int sD = 0, nB = 0, mRI = 0, mGM = 0, mCG = 0;
   double riAbs = 0, riRel = 0, gmAbs = 0, gmRel = 0, cgAbs = 0, cgRel = 0;
-  bool formed = false;    // the Schur complement is formed (schur_ready)
+  // the Schur complement where it is formed (schur_ready): its pattern and values
+  std::shared_ptr<const crimson::SchurPattern> spat;
+  crimson::DBuf<T> S;
   bool paired = false;    // its CG keeps R and P together (kCgPaired)
   SegCapture *cap = nullptr;  // the capture in progress, cut between the solve's phases
   size_t oH = 0, ocs = 0, osn = 0, oerr = 0, oy = 0, oA = 0, oBv = 0, oxB = 0, oC = 0, ocu = 0, ocp = 0;
@@ -2455,7 +2446,7 @@ struct SolveWork : crimson::SolveWorkBase {
   }
   size_t bytes() const override {
     return sizeof(T) * (c.W.n + c.fix.n + r0.n + r.n + X.n + MX.n + t3.n + t4.n + t5.n + ps.n + z.n + wa.n + wb.n +
-                        ws.n + gmU.n) +
+                        ws.n + gmU.n + S.n) +
            sizeof(double) * (c.part.n + gst.n + npart.n + h.n);
   }
   double *G(size_t off) { return gst.p + off; }
@@ -2663,8 +2654,8 @@ int cg_run(SolveWork<T> &w, size_t L, T *X, Op op, T *R, T *P, T *P2, T *SP, con
 
 // cg_run on the formed Schur complement in two launches (s_dir_product_kernel, cg_r_kernel<PAIR>).
 template <class T>
-int cg_run_paired(SolveWork<T> &w, size_t L, T *X, PairT<T> *Q, T *P, T *SP, const FaceList &fl, double absTol,
-                  double relTol, int mItr, double *g, const double *skip, double **state) {
+int cg_run_paired(SolveWork<T> &w, const SchurOp<T> &o, size_t L, T *X, PairT<T> *Q, T *P, T *SP, const FaceList &fl,
+                  double absTol, double relTol, int mItr, double *g, const double *skip, double **state) {
   Ctx<T> &c = w.c;
   CR_TRY(dots(c, L, X, static_cast<const T *>(nullptr), 0, 0, true, c.part.p, skip));
   cg_begin_kernel<<<1, kDotThreads, 0, c.s>>>(c.cgst.p, g, skip, c.part.p, dot_blocks(L), absTol, relTol, mItr);
@@ -2678,7 +2669,7 @@ int cg_run_paired(SolveWork<T> &w, size_t L, T *X, PairT<T> *Q, T *P, T *SP, con
   // so a plain solve runs past mItr by its lag at most
   for (; w.polled || it < mItr; ++it) {
     int nd = 0;
-    CR_TRY(schur_dir_product(c, Q, P, SP, it ? st(it - 1) : st(0), it ? st(it) : nullptr, cg.blocks, fl,
+    CR_TRY(schur_dir_product(c, o, Q, P, SP, it ? st(it - 1) : st(0), it ? st(it) : nullptr, cg.blocks, fl,
                          it ? w.flag() : HostFlag{nullptr, 0}, nd));
     if (cg.entries == 1)
       cg_r_kernel<T, 1, true><<<cg.blocks, 256, 0, c.s>>>(L, st(it), dpart, nd, fl, nullptr, SP, rpart, Q, X, P);
@@ -2733,7 +2724,8 @@ int ns_run(SolveWork<T> &w, double *d_Ri) {
   if (c.nfc() > 0) face_coef_kernel<<<c.nfc(), 1024, 0, c.s>>>(c.fdev.p, 3, c.fcoef.p);
   CR_TRY(face_functionals(c, mG));
   SchurOp<T> so;
-  so.formed = w.formed;
+  so.pat = w.spat.get();
+  so.S = w.S.p;
   so.L = mL;
   so.Gt = Gt;
   so.G = mG;
@@ -2741,7 +2733,7 @@ int ns_run(SolveWork<T> &w, double *d_Ri) {
   CR_TRY(schur_form(c, so));
   CgAux<T> ax;
   ax.fl = c.face_list();
-  if (!so.formed) {
+  if (!so.pat) {
     ax.W = c.W.p;
     ax.wdof = 4;
     ax.off = mG.c0;
@@ -2767,7 +2759,7 @@ int ns_run(SolveWork<T> &w, double *d_Ri) {
     CR_TRY(spmv(c, mD, 1, 3, Ui, Pi, -1.0, w.r.p + mn, 1.0, ri));  // P = Rc - D U
     double *state = nullptr;
     if (w.paired)
-      CR_TRY(cg_run_paired(w, (size_t)N, Pi, reinterpret_cast<PairT<T> *>(w.t3.p), w.t4.p, MPb, ax.fl, w.cgAbs,
+      CR_TRY(cg_run_paired(w, so, (size_t)N, Pi, reinterpret_cast<PairT<T> *>(w.t3.p), w.t4.p, MPb, ax.fl, w.cgAbs,
                            w.cgRel, w.mCG, g, ri, &state));
     else
       CR_TRY(cg_run(w, (size_t)N, Pi, schur_op, w.t3.p, w.t4.p, w.t5.p, MPb, ax, w.cgAbs, w.cgRel, w.mCG, g, ri,
@@ -2870,6 +2862,16 @@ int face_setup(Ctx<T> &c, const int *incL, const double *res, bool ns) {
   return CRIMSON_OK;
 }
 
+// The Schur complement's pattern and storage; spat stays empty when the two
+// passes are taken.
+template <class T>
+int schur_ready(SolveWork<T> &w, crimson_lhs *l) {
+  w.spat.reset();
+  CR_TRY(schur_pattern(l));
+  if (l->schur == 1 && try_alloc(w.S, (size_t)l->spat->nnz)) w.spat = l->spat;
+  return CRIMSON_OK;
+}
+
 // Workspaces and face set-up of one solve (allocations and uploads: all
 // before any capture).
 template <class T>
@@ -2921,11 +2923,9 @@ int work_setup(SolveWork<T> &w, crimson_lhs *l, crimson_ls *ls, int dof, const i
     CR_TRY(w.X.alloc(st * w.mRI));
     CR_TRY(w.MX.alloc(st * w.nB));
     if (!l->gt_is_d) CR_TRY(gt_buf(l, T(0)).alloc((size_t)3 * l->nnz));
-    SchurOp<T> so;
-    CR_TRY(schur_ready(l, so));
-    w.formed = so.formed;
-    w.paired = w.formed && N <= kCgPaired;
-    if (!w.formed) {
+    CR_TRY(schur_ready(w, l));
+    w.paired = w.spat && N <= kCgPaired;
+    if (!w.spat) {
       CR_TRY(w.ps.alloc(N));
       CR_TRY(w.z.alloc((size_t)4 * N));
     }
@@ -3165,8 +3165,7 @@ std::vector<unsigned long long> ns_signature(const crimson_lhs *l, const crimson
                                        (unsigned long long)l->vdof, (unsigned long long)l->prec,
                                        (unsigned long long)l->gt_is_d, (unsigned long long)ls->RI.mItr,
                                        (unsigned long long)ls->GM.mItr, (unsigned long long)ls->GM.sD,
-                                       (unsigned long long)ls->CG.mItr, l->d_S.serial, l->d_S32.serial,
-                                       l->d_sptr.serial};
+                                       (unsigned long long)ls->CG.mItr};
   for (const auto &fa : l->face) {
     v.push_back(fa.d_glob.serial);
     v.push_back(fa.d_val.serial);

@@ -135,3 +135,33 @@ def test_graph_after_solves_with_other_faces(cfa):
     moved = replay()
     assert torch.equal(moved, plain(both)) and not torch.equal(moved, want)
     assert torch.equal(replay(), moved)
+
+
+def test_graph_after_solves_in_the_other_precision(cfa):
+    """A captured FP64 solve, replayed after plain FP32 solves of the same handle."""
+    import torch
+    from crimsonflowsolver_amd import mesh as M
+    from crimsonflowsolver_amd.timestep import ResistanceCylinder
+    c = ResistanceCylinder(M.cylinder_mesh(5, 5, 8), params=cfa.form_params(), ls=_solver(cfa))
+    y, ac = c.state()
+    c.residual(y, ac, y, ac)
+    rhs = c.res4.clone()
+    c.lhs.set_precision(32)  # both precisions' planes are there from here on
+    c.lhs.set_precision(64)
+
+    def plain():
+        x = rhs.clone()
+        cfa.memLS_SOLVE_dev(c.lhs, _solver(cfa), 4, x, res=c.faceres)
+        return x
+
+    buf = rhs.clone()
+    graph = cfa.memLS_SOLVE_graph(c.lhs, _solver(cfa), 4, buf, res=c.faceres)
+    want = plain()
+    for _ in range(2):
+        c.lhs.set_precision(32)
+        plain()
+        c.lhs.set_precision(64)
+        buf.copy_(rhs)
+        torch.cuda.synchronize()
+        graph.launch()
+        assert torch.equal(buf, want)
