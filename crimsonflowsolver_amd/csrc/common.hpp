@@ -9,6 +9,7 @@
 #include <cstdio>
 #include <cstdint>
 #include <memory>
+#include <mutex>
 #include <string>
 #include <vector>
 
@@ -255,6 +256,7 @@ struct crimson_lhs {
   int schur = 0;
   std::shared_ptr<crimson::SchurPattern> spat;
   int band = 0;  // largest |column - row| (with d_col16)
+  mutable std::mutex busy;  // held by a solve, a capture and a replay
   // the workspaces of the last plain solve in FP64 and in FP32 (work_take, work_keep)
   std::unique_ptr<crimson::SolveWorkBase> work[2];
   hipEvent_t ev0 = nullptr, ev1 = nullptr;

@@ -2117,6 +2117,8 @@ extern "C" int crimson_graph_launch(crimson_graph *g) {
     crimson::set_error("crimson_graph_launch: null graph");
     return CRIMSON_EARG;
   }
+  std::unique_lock<std::mutex> hold;
+  if (g->lhs) hold = std::unique_lock<std::mutex>(g->lhs->busy);
   if (g->extra) CR_TRY(g->extra->before_launch());
   std::vector<unsigned long long> sig;
   if (g->f) sig = crimson::graph_signature(g->f, g->lhs);

@@ -3064,9 +3064,10 @@ int cgradv(SolveWork<T> &w, crimson_ls *ls) {
 // The workspace of a plain solve stays with the matrix handle: allocating and
 // freeing it took 5 to 7 ms a solve, a third of the reference case's.  Kept
 // while the process keeps at most kKeepBytes of them (a larger one is freed after its
-// solve, where the solve is long); a solve takes it out, so that a second
-// solve of the handle at the same time has one of its own; given back with the
-// handle, or when an allocation fails (release_idle_work).
+// solve, where the solve is long); a solve takes it out, so that no other thread's
+// release_idle_work frees it meanwhile; given back with the handle, or when an
+// allocation fails (release_idle_work).  Solves of one handle run one at a time
+// (crimson_lhs::busy): they share its faces' buffers and the complement's pattern.
 constexpr size_t kKeepBytes = (size_t)8 << 30;
 template <class T>
 std::unique_ptr<SolveWork<T>> take_work(crimson_lhs *l) {
@@ -3562,6 +3563,7 @@ extern "C" int crimson_ls_solve_dev(crimson_lhs *l, crimson_ls *ls, int dof, dou
     crimson::set_error("crimson_ls_solve_dev: null argument");
     return CRIMSON_EARG;
   }
+  std::lock_guard<std::mutex> hold(l->busy);
   return solve_dev(l, ls, dof, d_Ri, incL, res);
 }
 
@@ -3571,6 +3573,7 @@ extern "C" int crimson_ls_solve(crimson_lhs *l, crimson_ls *ls, int dof, double 
     crimson::set_error("crimson_ls_solve: null argument");
     return CRIMSON_EARG;
   }
+  std::lock_guard<std::mutex> hold(l->busy);
   CR_TRY(crimson_lhs_set_val(l, dof, Val));
   crimson::DBuf<double> dR;
   const size_t L = (size_t)dof * l->nNo;
@@ -3832,6 +3835,7 @@ extern "C" int crimson_ls_graph_create(crimson_lhs *lhs, crimson_ls *ls, int dof
     crimson::set_error("crimson_ls_graph_create: invalid arguments (the NS solver, dof 4)");
     return CRIMSON_EARG;
   }
+  std::lock_guard<std::mutex> hold(lhs->busy);
   if (lhs->vdof != 4 || !(lhs->prec == 32 ? (const void *)lhs->d_V32.p : (const void *)lhs->d_V.p)) {
     crimson::set_error("crimson_ls_graph_create: lhs holds no 4x4 matrix");
     return CRIMSON_ESTATE;
@@ -3860,6 +3864,7 @@ extern "C" int crimson_step_graph_create(crimson_form *f, crimson_lhs *lhs, crim
       crimson::set_error("crimson_step_graph_create: surf_ptr not monotone");
       return CRIMSON_EARG;
     }
+  std::lock_guard<std::mutex> hold(lhs->busy);
   if (crimson::form_params_of(f).precision == 32)
     return step_graph_create_t<float>(f, lhs, ls, d_yold, d_acold, d_y, d_ac, d_yAlpha, d_acAlpha, d_x, d_Res4,
                                       d_iBC, d_BC, ndofBC, nsurf, surf_ptr, d_glob, d_nabi, c1, c2, d_q, faceRes,

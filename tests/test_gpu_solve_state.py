@@ -165,3 +165,76 @@ def test_graph_after_solves_in_the_other_precision(cfa):
         torch.cuda.synchronize()
         graph.launch()
         assert torch.equal(buf, want)
+
+
+def test_solves_of_one_handle_from_threads(cfa):
+    """Three threads at once on one handle that has not solved before: with its
+    Dirichlet face, without it, and replays of a captured solve with it.  Each
+    result has the bits of the same call alone on a handle of its own."""
+    import threading
+
+    import torch
+    n = 3000
+    i = np.arange(n)
+    rp = np.concatenate([[0], np.cumsum(np.full(n, 5))]).astype(np.int32) + 1
+    cols = np.sort((i[:, None] + np.arange(-2, 3)) % n, axis=1)
+    rng = np.random.default_rng(3)
+    val = np.zeros((16, 5 * n), order="F")
+    diag = (cols == i[:, None]).ravel()
+    val[[0, 5, 10, 15]] = np.where(diag, 2.0, -0.1)
+    key = {(a, b): a * 5 + k for a in range(n) for k, b in enumerate(cols[a])}
+    tr = np.array([key[(b, a)] for a in range(n) for b in cols[a]])
+    g = 0.2 * rng.uniform(-1, 1, (3, 5 * n))
+    val[[3, 7, 11]] = g
+    val[12:15] = -g[:, tr]
+    rhs = torch.from_numpy(1e3 * rng.standard_normal((n, 4))).cuda()
+    fixed = np.arange(0, n, 7)
+    neu = np.arange(1, 400, 7)
+    v = rng.uniform(0.2, 1.0, (3, neu.size))
+    res = np.array([0.0, 3.0])
+
+    def handle():
+        lhs = _handle(cfa, rp, (cols.ravel() + 1).astype(np.int32), 2)
+        cfa.memLS_BC_CREATE(lhs, 1, fixed.size, 3, cfa.BC_TYPE_Dir, fixed + 1, np.zeros((3, fixed.size), order="F"))
+        cfa.memLS_BC_CREATE(lhs, 2, neu.size, 3, cfa.BC_TYPE_Neu, neu + 1, np.asfortranarray(v))
+        lhs.set_val(4, val)
+        return lhs
+
+    def solve(lhs, incL):
+        x = rhs.clone()
+        torch.cuda.synchronize()
+        cfa.memLS_SOLVE_dev(lhs, _solver(cfa), 4, x, incL=np.array(incL, np.int32), res=res)
+        return x
+
+    want = [solve(handle(), inc) for inc in ((1, 1), (0, 1), (1, 1))]
+    assert not torch.equal(want[0], want[1])
+    lhs = handle()
+    buf = rhs.clone()
+    graph = cfa.memLS_SOLVE_graph(lhs, _solver(cfa), 4, buf, incL=np.array([1, 1], np.int32), res=res)
+
+    def replay():
+        buf.copy_(rhs)
+        torch.cuda.synchronize()
+        graph.launch()
+        return buf.clone()
+
+    calls = [lambda: solve(lhs, (1, 1)), lambda: solve(lhs, (0, 1)), replay]
+    got, failed = [[], [], []], []
+    start = threading.Barrier(3)
+
+    def work(k):
+        try:
+            start.wait()
+            for _ in range(8):
+                got[k].append(calls[k]())
+        except Exception as e:  # reported below
+            failed.append((k, e))
+
+    threads = [threading.Thread(target=work, args=(k,)) for k in range(3)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not failed, failed
+    for k in range(3):
+        assert len(got[k]) == 8 and all(torch.equal(x, want[k]) for x in got[k]), k
