@@ -47,7 +47,7 @@ EXPORTS = (
     "crimson_measure_peaks", "crimson_form_vjp_ac_dev", "crimson_elmpvsq_vjp_dev", "crimson_lhs_transpose_dev",
     "crimson_ls_graph_create", "crimson_step_graph_create", "crimson_form_set_wall",
     "crimson_form_set_displacement_dev", "crimson_wall_predict_dev", "crimson_wall_correct_dev",
-    "crimson_wall_alpha_dev", "crimson_form_set_wall_state_dev",
+    "crimson_wall_alpha_dev", "crimson_form_set_wall_state_dev", "crimson_release_workspaces",
 )
 
 
@@ -155,6 +155,7 @@ def lib():
         L.crimson_wall_predict_dev.argtypes = [vp, vp, vp, vp, vp]
         L.crimson_wall_correct_dev.argtypes = [vp, vp, vp]
         L.crimson_wall_alpha_dev.argtypes = [vp, vp, vp, vp]
+        L.crimson_release_workspaces.argtypes = []
         L.crimson_graph_launch.argtypes = [vp]
         L.crimson_graph_free.argtypes = [vp]
         L.crimson_form_autotune.argtypes = [vp, vp, vp, vp, vp, vp, C.c_int, C.c_int, C.POINTER(C.c_int), dp]
@@ -610,6 +611,12 @@ def memLS_SOLVE(lhs, ls, dof, Ri, Val, incL=None, res=None):
     il = None if incL is None else _f(incL, np.int32)
     rs = None if res is None else _f(res)
     check(lib().crimson_ls_solve(lhs.h, ls.h, dof, _p(Ri), _p(Val), _p(il), _p(rs)), "memLS_SOLVE")
+
+
+def release_workspaces():
+    """Give the device memory that matrix handles keep for their next solve back
+    (crimson_release_workspaces), for instance before another allocator needs it."""
+    check(lib().crimson_release_workspaces(), "crimson_release_workspaces")
 
 
 def memLS_SOLVE_graph(lhs, ls, dof, Ri_dev, incL=None, res=None):

@@ -44,8 +44,8 @@ inline unsigned long long next_alloc_serial() {
   return ++counter;
 }
 
-// Frees the solver workspaces that matrix handles keep for their next solve
-// (memls.hip); false when there was none.  Called when an allocation fails.
+// Frees what matrix handles keep for their next solve, workspaces and complements'
+// patterns (memls.hip); false when there was none.  Called when an allocation fails.
 bool release_idle_work();
 
 // Owning device allocation.
@@ -251,10 +251,10 @@ struct crimson_lhs {
   crimson::DBuf<double> d_Gt;     // [3][nnz] when !gt_is_d
   crimson::DBuf<float> d_Gt32;    // the same for an FP32 matrix
   std::vector<CrFace> face;
-  // the Schur complement of the NS solver's CG: 0 not looked at yet, 1 its pattern
-  // is in spat, 2 this graph keeps the two-pass operator
-  int schur = 0;
-  std::shared_ptr<crimson::SchurPattern> spat;
+  // the Schur complement of the NS solver's CG: its pattern once it is built, and
+  // whether this graph keeps the two-pass operator
+  std::shared_ptr<const crimson::SchurPattern> spat;
+  bool two_pass = false;
   int band = 0;  // largest |column - row| (with d_col16)
   mutable std::mutex busy;  // held by a solve, a capture and a replay
   // the workspaces of the last plain solve in FP64 and in FP32 (work_take, work_keep)

@@ -1677,18 +1677,25 @@ __global__ void __launch_bounds__(256) s_dir_product_kernel(int nNo, int ntile, 
 }
 }  // namespace
 
-// The solver workspaces that handles keep, process-wide: every handle that holds
-// one, under one lock.
+// What handles keep between solves, process-wide: every handle that holds a workspace
+// or a complement's pattern, under one lock.  Never destroyed: handles may be freed
+// after this library's static objects.
 namespace crimson {
 namespace {
-std::mutex g_work_lock;
-std::vector<crimson_lhs *> g_work_lhs;
+std::mutex &g_work_lock = *new std::mutex;
+std::vector<crimson_lhs *> &g_work_lhs = *new std::vector<crimson_lhs *>;
 size_t g_work_bytes = 0;
+// under the lock: l among the holders or not
+void work_note(crimson_lhs *l) {
+  auto at = std::find(g_work_lhs.begin(), g_work_lhs.end(), l);
+  const bool holds = l->work[0] || l->work[1] || l->spat;
+  if (holds && at == g_work_lhs.end()) g_work_lhs.push_back(l);
+  if (!holds && at != g_work_lhs.end()) g_work_lhs.erase(at);
+}
 std::unique_ptr<SolveWorkBase> work_drop(crimson_lhs *l, int k) {  // under the lock
   std::unique_ptr<SolveWorkBase> w = std::move(l->work[k]);
   if (w) g_work_bytes -= w->bytes();
-  if (!l->work[0] && !l->work[1])
-    g_work_lhs.erase(std::remove(g_work_lhs.begin(), g_work_lhs.end(), l), g_work_lhs.end());
+  work_note(l);
   return w;
 }
 std::unique_ptr<SolveWorkBase> work_take(crimson_lhs *l, bool fp32) {
@@ -1701,25 +1708,36 @@ void work_keep(crimson_lhs *l, bool fp32, std::unique_ptr<SolveWorkBase> w, size
   if (g_work_bytes + w->bytes() > most) return;
   g_work_bytes += w->bytes();
   l->work[fp32 ? 1 : 0] = std::move(w);
-  if (std::find(g_work_lhs.begin(), g_work_lhs.end(), l) == g_work_lhs.end()) g_work_lhs.push_back(l);
+  work_note(l);
 }
-void work_forget(crimson_lhs *l) {
+std::shared_ptr<const SchurPattern> pattern_of(crimson_lhs *l) {
   std::lock_guard<std::mutex> hold(g_work_lock);
+  return l->spat;
+}
+void pattern_keep(crimson_lhs *l, std::shared_ptr<const SchurPattern> p) {
+  std::lock_guard<std::mutex> hold(g_work_lock);
+  l->spat = std::move(p);
+  work_note(l);
+}
+void work_forget(crimson_lhs *l) {  // under the lock
   (void)work_drop(l, 0);
   (void)work_drop(l, 1);
+  l->spat.reset();
+  work_note(l);
 }
 }  // namespace
 bool release_idle_work() {
   std::lock_guard<std::mutex> hold(g_work_lock);
   const bool any = !g_work_lhs.empty();
-  while (!g_work_lhs.empty()) {
-    crimson_lhs *l = g_work_lhs.back();
-    (void)work_drop(l, 0);
-    (void)work_drop(l, 1);
-  }
+  while (!g_work_lhs.empty()) work_forget(g_work_lhs.back());
   return any;
 }
 }  // namespace crimson
+
+extern "C" int crimson_release_workspaces(void) {
+  (void)crimson::release_idle_work();
+  return CRIMSON_OK;
+}
 
 struct crimson_ls {
   SubLs GM, CG, RI;
@@ -1904,32 +1922,29 @@ bool try_alloc(B &b, size_t n) {
   return false;
 }
 
-// The pattern of S, once per handle: schur = 1 when it is there, 2 when this
-// graph keeps the two passes.  S is formed when its rows fit the value kernel's staging
+// The pattern of S, built once per handle and kept with it until it is released
+// (release_idle_work); out stays empty where the graph keeps the two passes
+// (two_pass).  S is formed when its rows fit the value kernel's staging
 // (kSchurRow) and it has at most kSchurFill entries per block: the two passes
 // read 60 bytes per block (32 in FP32), S 10 (6) per entry plus the vector
 // work of one more launch.
 constexpr int kSchurFill = 6;
 template <class IX, class OX>
-int schur_pattern_fill(crimson_lhs *l, const IX *col, crimson::SchurPattern &p, crimson::DBuf<OX> &scol) {
-  if (!try_alloc(scol, (size_t)p.nnz)) {
-    l->schur = 2;
-    return CRIMSON_OK;
-  }
-  schur_pattern_kernel<IX, OX, true><<<crimson::grid_for(l->nNo, 4), 256, 0, l->stream>>>(l->nNo, l->d_rowptr.p, col,
-                                                                                         nullptr, p.ptr.p, scol.p);
+int schur_pattern_fill(crimson_lhs *l, const IX *col, const crimson::SchurPattern &p, const OX *scol) {
+  schur_pattern_kernel<IX, OX, true><<<crimson::grid_for(l->nNo, 4), 256, 0, l->stream>>>(
+      l->nNo, l->d_rowptr.p, col, nullptr, p.ptr.p, const_cast<OX *>(scol));
   CR_HIP(hipGetLastError());
   CR_HIP(hipStreamSynchronize(l->stream));
-  l->schur = 1;
   return CRIMSON_OK;
 }
-int schur_pattern(crimson_lhs *l) {
-  if (l->schur) return CRIMSON_OK;
+int schur_pattern(crimson_lhs *l, std::shared_ptr<const crimson::SchurPattern> &out) {
+  out = crimson::pattern_of(l);
+  if (out || l->two_pass) return CRIMSON_OK;
   const int N = l->nNo;
   auto p = std::make_shared<crimson::SchurPattern>();
   crimson::DBuf<int> cnt;
   if (!try_alloc(cnt, (size_t)N) || !try_alloc(p->ptr, (size_t)N + 1)) {
-    l->schur = 2;
+    l->two_pass = true;
     return CRIMSON_OK;
   }
   const unsigned G = crimson::grid_for(N, 4);
@@ -1949,19 +1964,25 @@ int schur_pattern(crimson_lhs *l) {
     p->nnz += ptr[i];
     ptr[i] = (int)p->nnz;
     if (p->row > kSchurRow || p->nnz > (long long)kSchurFill * l->nnz || p->nnz > 0x7fffff00LL) {
-      l->schur = 2;
+      l->two_pass = true;
       return CRIMSON_OK;
     }
   }
   CR_TRY(p->ptr.upload(ptr.data(), ptr.size(), l->stream));
   CR_HIP(hipStreamSynchronize(l->stream));
-  if (l->d_col16.p && 2 * l->band <= 32767)
-    CR_TRY(schur_pattern_fill(l, l->d_col16.p, *p, p->col16));
+  const bool narrow = l->d_col16.p && 2 * l->band <= 32767;
+  if (!(narrow ? try_alloc(p->col16, (size_t)p->nnz) : try_alloc(p->col, (size_t)p->nnz))) {
+    l->two_pass = true;
+    return CRIMSON_OK;
+  }
+  if (narrow)
+    CR_TRY(schur_pattern_fill(l, l->d_col16.p, *p, p->col16.p));
   else if (l->d_col16.p)
-    CR_TRY(schur_pattern_fill(l, l->d_col16.p, *p, p->col));
+    CR_TRY(schur_pattern_fill(l, l->d_col16.p, *p, p->col.p));
   else
-    CR_TRY(schur_pattern_fill(l, l->d_col.p, *p, p->col));
-  if (l->schur == 1) l->spat = p;
+    CR_TRY(schur_pattern_fill(l, l->d_col.p, *p, p->col.p));
+  out = p;
+  crimson::pattern_keep(l, out);
   return CRIMSON_OK;
 }
 
@@ -2866,9 +2887,8 @@ int face_setup(Ctx<T> &c, const int *incL, const double *res, bool ns) {
 // passes are taken.
 template <class T>
 int schur_ready(SolveWork<T> &w, crimson_lhs *l) {
-  w.spat.reset();
-  CR_TRY(schur_pattern(l));
-  if (l->schur == 1 && try_alloc(w.S, (size_t)l->spat->nnz)) w.spat = l->spat;
+  CR_TRY(schur_pattern(l, w.spat));
+  if (w.spat && !try_alloc(w.S, (size_t)w.spat->nnz)) w.spat.reset();
   return CRIMSON_OK;
 }
 
@@ -3404,7 +3424,10 @@ extern "C" int crimson_lhs_free(crimson_lhs *l) {
   if (l->ev0) (void)hipEventDestroy(l->ev0);
   if (l->ev1) (void)hipEventDestroy(l->ev1);
   hipStream_t s = l->stream;
-  crimson::work_forget(l);
+  {
+    std::lock_guard<std::mutex> kept(crimson::g_work_lock);
+    crimson::work_forget(l);
+  }
   delete l;
   if (s) (void)hipStreamDestroy(s);
   return CRIMSON_OK;

@@ -455,6 +455,15 @@ int crimson_ls_solve(crimson_lhs *lhs, crimson_ls *ls, int dof, double *Ri,
 int crimson_ls_solve_dev(crimson_lhs *lhs, crimson_ls *ls, int dof,
                          double *d_Ri, const int *incL, const double *res);
 
+/* Between solves a matrix handle keeps its last solve's device workspaces (at
+ * most 8 GiB over the process; larger ones are freed after their solve) and the
+ * pattern of the NS solver's Schur complement.  This call gives all of them
+ * back, for instance before another allocator of the process needs the memory;
+ * the next solve allocates again.  The library does so itself when one of its own
+ * allocations fails.  No counterpart in the reference.  Any thread may call it
+ * at any time; running solves and captured graphs keep what they use. */
+int crimson_release_workspaces(void);
+
 /* Uploads Val(dof*dof,nnz) (host, row-major blocks) into the lhs. */
 int crimson_lhs_set_val(crimson_lhs *lhs, int dof, const double *Val);
 

@@ -238,3 +238,35 @@ def test_solves_of_one_handle_from_threads(cfa):
     assert not failed, failed
     for k in range(3):
         assert len(got[k]) == 8 and all(torch.equal(x, want[k]) for x in got[k]), k
+
+
+def test_release_workspaces(cfa):
+    """release_workspaces gives the kept memory back; solves and a captured
+    solve give the same bits before and after."""
+    import torch
+    from crimsonflowsolver_amd import mesh as M
+    from crimsonflowsolver_amd.timestep import ResistanceCylinder
+    c = ResistanceCylinder(M.cylinder_mesh(20, 20, 60), params=cfa.form_params(), ls=_solver(cfa))
+    y, ac = c.state()
+    c.residual(y, ac, y, ac)
+    rhs = c.res4.clone()
+
+    def plain():
+        x = rhs.clone()
+        cfa.memLS_SOLVE_dev(c.lhs, _solver(cfa), 4, x, res=c.faceres)
+        return x
+
+    want = plain()
+    buf = rhs.clone()
+    graph = cfa.memLS_SOLVE_graph(c.lhs, _solver(cfa), 4, buf, res=c.faceres)
+    free = torch.cuda.mem_get_info()[0]
+    cfa.release_workspaces()
+    # at least the basis, 3 N doubles a vector, 40 vectors
+    assert torch.cuda.mem_get_info()[0] - free >= 40 * 3 * c.N * 8
+    torch.cuda.synchronize()
+    graph.launch()
+    assert torch.equal(buf, want)
+    for _ in range(2):
+        assert torch.equal(plain(), want)
+        cfa.release_workspaces()
+        cfa.release_workspaces()
