@@ -1923,8 +1923,8 @@ bool try_alloc(B &b, size_t n) {
 }
 
 // The pattern of S, built once per handle and kept with it until it is released
-// (release_idle_work); out stays empty where the graph keeps the two passes
-// (two_pass).  S is formed when its rows fit the value kernel's staging
+// (release_idle_work); out stays empty where the graph keeps the two passes (two_pass)
+// or an allocation failed (the next solve tries again).  S is formed when its rows fit the value kernel's staging
 // (kSchurRow) and it has at most kSchurFill entries per block: the two passes
 // read 60 bytes per block (32 in FP32), S 10 (6) per entry plus the vector
 // work of one more launch.
@@ -1943,10 +1943,7 @@ int schur_pattern(crimson_lhs *l, std::shared_ptr<const crimson::SchurPattern> &
   const int N = l->nNo;
   auto p = std::make_shared<crimson::SchurPattern>();
   crimson::DBuf<int> cnt;
-  if (!try_alloc(cnt, (size_t)N) || !try_alloc(p->ptr, (size_t)N + 1)) {
-    l->two_pass = true;
-    return CRIMSON_OK;
-  }
+  if (!try_alloc(cnt, (size_t)N) || !try_alloc(p->ptr, (size_t)N + 1)) return CRIMSON_OK;
   const unsigned G = crimson::grid_for(N, 4);
   if (l->d_col16.p)
     schur_pattern_kernel<short, int, false><<<G, 256, 0, l->stream>>>(N, l->d_rowptr.p, l->d_col16.p, cnt.p, nullptr,
@@ -1971,10 +1968,7 @@ int schur_pattern(crimson_lhs *l, std::shared_ptr<const crimson::SchurPattern> &
   CR_TRY(p->ptr.upload(ptr.data(), ptr.size(), l->stream));
   CR_HIP(hipStreamSynchronize(l->stream));
   const bool narrow = l->d_col16.p && 2 * l->band <= 32767;
-  if (!(narrow ? try_alloc(p->col16, (size_t)p->nnz) : try_alloc(p->col, (size_t)p->nnz))) {
-    l->two_pass = true;
-    return CRIMSON_OK;
-  }
+  if (!(narrow ? try_alloc(p->col16, (size_t)p->nnz) : try_alloc(p->col, (size_t)p->nnz))) return CRIMSON_OK;
   if (narrow)
     CR_TRY(schur_pattern_fill(l, l->d_col16.p, *p, p->col16.p));
   else if (l->d_col16.p)

@@ -270,3 +270,103 @@ def test_release_workspaces(cfa):
         assert torch.equal(plain(), want)
         cfa.release_workspaces()
         cfa.release_workspaces()
+
+
+_FAIL_MALLOC = r"""
+#include <dlfcn.h>
+#include <stddef.h>
+/* hipMalloc that fails for one size: the next `fail_times` calls with it */
+size_t fail_size = 0;
+int fail_times = 0, failed = 0;
+int hipMalloc(void **p, size_t n) {
+  static int (*real)(void **, size_t);
+  if (!real) real = (int (*)(void **, size_t))dlsym(dlopen("libamdhip64.so.7", RTLD_NOLOAD | RTLD_LAZY), "hipMalloc");
+  if (n == fail_size && fail_times > 0) {
+    --fail_times;
+    ++failed;
+    return 2; /* hipErrorOutOfMemory */
+  }
+  return real(p, n);
+}
+"""
+
+_FAIL_CHILD = r"""
+import ctypes, sys
+sys.modules["torch"] = None  # the library's own HIP runtime, behind the stand-in
+fake = ctypes.CDLL(sys.argv[1], mode=ctypes.RTLD_GLOBAL)
+import numpy as np
+import crimsonflowsolver_amd as cfa
+size, times, failed = (t.in_dll(fake, k) for t, k in ((ctypes.c_size_t, "fail_size"), (ctypes.c_int, "fail_times"),
+                                                      (ctypes.c_int, "failed")))
+n = 3000
+i = np.arange(n)
+cols = np.sort((i[:, None] + np.arange(-2, 3)) % n, axis=1)
+rng = np.random.default_rng(3)
+val = np.zeros((16, 5 * n), order="F")
+val[[0, 5, 10, 15]] = np.where((cols == i[:, None]).ravel(), 2.0, -0.1)
+key = {(a, b): a * 5 + k for a in range(n) for k, b in enumerate(cols[a])}
+g = 0.2 * rng.uniform(-1, 1, (3, 5 * n))
+val[[3, 7, 11]] = g
+val[12:15] = -g[:, [key[(b, a)] for a in range(n) for b in cols[a]]]
+R = np.asfortranarray(1e3 * rng.standard_normal((4, n)))
+rp = (5 * np.arange(n + 1) + 1).astype(np.int32)
+
+
+def handle():
+    return cfa.memLS_LHS_CREATE(n, n, 5 * n, None, rp, (cols.ravel() + 1).astype(np.int32), 0)
+
+
+def solve(lhs):
+    ls = cfa.memLS_LS_CREATE(cfa.LS_TYPE_NS, relTol=1e-6, dimKry=30, maxItr=5, relTolIn=[0.01, 0.01], maxItrIn=[2, 200])
+    x = R.copy(order="F")
+    cfa.memLS_SOLVE(lhs, ls, 4, x, val)
+    return x
+
+
+def armed(lhs, nbytes, count):
+    before = failed.value
+    size.value, times.value = nbytes, count
+    x = solve(lhs)
+    times.value = 0
+    assert failed.value == before + count, (failed.value, before, count)
+    return x
+
+
+columns, values = 9 * n * 2, 9 * n * 8  # the two-ring has 9 entries a row, within 2-byte offsets
+A = handle()
+want = solve(A)
+cfa.release_workspaces()
+scale = np.abs(want).max()
+# the pattern's buffer, with nothing to give back, and the values', tried again after
+# the new pattern's share of the handle has been given back
+for nbytes, count in ((columns, 1), (values, 2)):
+    B = handle()
+    two = armed(B, nbytes, count)
+    assert not np.array_equal(two, want) and np.abs(two - want).max() <= 1e-3 * scale, nbytes
+    assert np.array_equal(solve(B), want), ("formed again", nbytes)
+    cfa.release_workspaces()
+solve(A)  # idle now
+C = handle()
+assert np.array_equal(armed(C, values, 1), want)  # A's workspace given back, the allocation made
+assert np.array_equal(solve(A), want)
+print("CHILD_OK", flush=True)
+"""
+
+
+def test_failed_allocations_of_the_complement(cfa, tmp_path):
+    """hipMalloc failing for the Schur complement's buffers, in a process of its own with
+    a stand-in in front of the runtime's: that solve takes the two passes, the next
+    one forms the complement; with another handle's workspace idle, that is given
+    back and the allocation made again.  Tolerance: both operators' solutions have
+    residuals under 1e-6 of the right-hand side's (condition numbers under 1e2)."""
+    import os
+    import subprocess
+    import sys
+    src, lib, child = tmp_path / "fail.c", tmp_path / "fail.so", tmp_path / "child.py"
+    src.write_text(_FAIL_MALLOC)
+    child.write_text(_FAIL_CHILD)
+    subprocess.run(["gcc", "-shared", "-fPIC", "-o", str(lib), str(src), "-ldl"], check=True)
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    env = dict(os.environ, PYTHONPATH=root)
+    out = subprocess.run([sys.executable, "-u", str(child), str(lib)], env=env, capture_output=True, text=True, timeout=100)
+    assert out.returncode == 0 and "CHILD_OK" in out.stdout, out.stdout[-2000:] + out.stderr[-2000:]
