@@ -183,19 +183,26 @@ struct FaceDev {
 };
 // Workgroups per face computing S_f's partial sums beside the direction update.
 constexpr int kFaceDotBlocks = 4;
-// The faces' supports merged for the residual update: the entries (node,
-// face, place in the face's support) sorted by node, then face; tptr[t] is
-// the first entry of nodes 256 t and above.
+// The faces' supports merged for the residual update: the nodes of any of them,
+// ascending, each with its entries (face, place in the face's support) in face
+// order; tptr[t] is the first of the nodes 256 t and above.
 struct FaceEnt {
-  int node, f, s;
+  int f, s;
 };
 struct FaceList {
   int nfc;               // coupled faces
   const FaceDev *fd;
+  const int *node, *eptr;  // the nodes and their first entries
   const FaceEnt *ent;
   const int *tptr;       // (N / 256 rounded up) + 1 entries
   double *part;          // kFaceDotBlocks partial sums of S_f per face
 };
+// Faces whose terms c_f S_f a workgroup of the residual update keeps in LDS; a node's
+// entries then cost it two loads each.  (329,000 rows, 24 faces on the same 12,637
+// nodes: an NS solve took 604 ms with every entry summing its face's parts again
+// and one thread walking a node's entries among its idle neighbours, 75 so; one
+// face 35.)
+constexpr int kFaceLds = 256;
 
 // Wave-level sum (64 lanes) then across the 4 waves of a 256-thread group.
 template <class T>
@@ -1387,7 +1394,7 @@ __global__ void __launch_bounds__(256) cg_r_kernel(size_t L, double *__restrict_
                                                    T *__restrict__ R, const T *__restrict__ SP,
                                                    double *__restrict__ rpart, PairT<T> *__restrict__ Q,
                                                    T *__restrict__ X, const T *__restrict__ P) {
-  __shared__ double sh[4];
+  __shared__ double sh[4], fc[kFaceLds];
   __shared__ T corr[E * 256];
   const double stop = scal[5], errO = scal[1];
   T r[E], sp[E], x[E], p[E];
@@ -1406,7 +1413,7 @@ __global__ void __launch_bounds__(256) cg_r_kernel(size_t L, double *__restrict_
     }
   };
   const int nt = (int)((L + 255) / 256);
-  int e0 = 0, e1 = 0;  // the faces' entries of the turn's nodes
+  int e0 = 0, e1 = 0;  // the faces' nodes of the turn
   auto range = [&](size_t base) {
     if (fl.nfc == 0) return;
     const int t0 = (int)(base / 256);
@@ -1418,8 +1425,9 @@ __global__ void __launch_bounds__(256) cg_r_kernel(size_t L, double *__restrict_
   range(base);
   double d = 0.0;
   for (int f = threadIdx.x; f < fl.nfc; f += 256) {
-    const double S = face_sum(fl, f);
-    d += face_coef(fl.fd[f]) * S * S;
+    const double S = face_sum(fl, f), cS = face_coef(fl.fd[f]) * S;
+    d += cS * S;
+    if (f < kFaceLds) fc[f] = cS;
   }
   if (stop != 0.0) return;
   const double den = sum_parts(dpart, nd, d, sh);
@@ -1433,14 +1441,13 @@ __global__ void __launch_bounds__(256) cg_r_kernel(size_t L, double *__restrict_
       for (int t = 0; t < E; ++t) corr[threadIdx.x + 256 * t] = T(0);
       __syncthreads();
       for (int e = e0 + threadIdx.x; e < e1; e += 256) {
-        const int node = fl.ent[e].node;
-        if (e > e0 && fl.ent[e - 1].node == node) continue;  // the node's first entry sums them all
         double v = 0.0;
-        for (int x = e; x < e1 && fl.ent[x].node == node; ++x) {
-          const FaceDev &F = fl.fd[fl.ent[x].f];
-          v += face_coef(F) * face_sum(fl, fl.ent[x].f) * F.q[fl.ent[x].s];
+        for (int x = fl.eptr[e]; x < fl.eptr[e + 1]; ++x) {
+          const FaceEnt en = fl.ent[x];
+          const FaceDev &F = fl.fd[en.f];
+          v += (en.f < kFaceLds ? fc[en.f] : face_coef(F) * face_sum(fl, en.f)) * F.q[en.s];
         }
-        corr[node - (int)base] = (T)v;
+        corr[fl.node[e] - (int)base] = (T)v;
       }
       __syncthreads();
 #pragma unroll
@@ -1773,12 +1780,11 @@ struct Ctx {
   std::vector<FaceDev> hfdev;    // fdev on the host
   bool disjoint = true;          // no two coupled faces share a node
   int nfc() const { return (int)hfdev.size(); }
-  // their merged supports and the first entries per 256 nodes, for the faces whose
-  // supports fent_sig lists
+  // their merged supports (FaceList), for the faces whose supports fent_sig lists
   std::vector<unsigned long long> fent_sig;
+  crimson::DBuf<int> fnode, feptr, ftptr;
   crimson::DBuf<FaceEnt> fent;
-  crimson::DBuf<int> ftptr;
-  FaceList face_list() const { return FaceList{nfc(), fdev.p, fent.p, ftptr.p, fpart.p}; }
+  FaceList face_list() const { return FaceList{nfc(), fdev.p, fnode.p, feptr.p, fent.p, ftptr.p, fpart.p}; }
 
   int init(crimson_lhs *l, int d, hipStream_t st) {
     lhs = l;
@@ -1858,7 +1864,7 @@ int spmv(Ctx<T> &c, const MatView<T> &A, int nr, int nc, const T *x, T *y, doubl
 // direction update (Ps null: none).
 template <class T>
 struct CgAux {
-  FaceList fl{0, nullptr, nullptr, nullptr, nullptr};
+  FaceList fl{};
   const T *W = nullptr;
   int wdof = 0, off = 0;
   T *Ps = nullptr;
@@ -2100,24 +2106,39 @@ int face_list(Ctx<T> &c) {
   for (const auto &fa : l->face)
     if (fa.coupled) sig.push_back(fa.support);
   if (sig == c.fent_sig && c.ftptr.p) return CRIMSON_OK;
-  std::vector<FaceEnt> ent;
+  const int N = l->nNo;
+  std::vector<int> count((size_t)N, 0);
+  size_t total = 0;
+  for (const auto &fa : l->face)
+    if (fa.coupled)
+      for (int j : fa.h_sup) {
+        ++count[j];
+        ++total;
+      }
+  // sized by the entries, whatever the faces share: a capture's buffers stay in place
+  std::vector<int> node(total, 0), eptr(total + 1, 0), ptr((size_t)(N + 255) / 256 + 1, 0);
+  std::vector<FaceEnt> ent(total);
+  int u = 0, e = 0;
+  for (int j = 0; j < N; ++j) {
+    if (j % 256 == 0) ptr[j / 256] = u;
+    if (count[j] == 0) continue;
+    node[u] = j;
+    eptr[u++] = e;
+    e += count[j];
+    count[j] = e - count[j];  // the node's next entry
+  }
+  ptr.back() = u;
+  for (size_t k = u; k < eptr.size(); ++k) eptr[k] = e;
   int f = 0;
   for (const auto &fa : l->face) {
     if (!fa.coupled) continue;
-    for (size_t k = 0; k < fa.h_sup.size(); ++k) ent.push_back(FaceEnt{fa.h_sup[k], f, (int)k});
+    for (size_t k = 0; k < fa.h_sup.size(); ++k) ent[count[fa.h_sup[k]]++] = FaceEnt{f, (int)k};
     ++f;
   }
-  std::sort(ent.begin(), ent.end(),
-            [](const FaceEnt &a, const FaceEnt &b) { return a.node != b.node ? a.node < b.node : a.f < b.f; });
-  std::vector<int> ptr((size_t)(l->nNo + 255) / 256 + 1);
-  size_t e = 0;
-  for (size_t t = 0; t < ptr.size(); ++t) {
-    while (e < ent.size() && ent[e].node < (long long)t * 256) ++e;
-    ptr[t] = (int)e;
-  }
-  ptr.back() = (int)ent.size();
   c.fent_sig.clear();
   CR_TRY(c.fent.upload(ent.data(), ent.size(), c.s));
+  CR_TRY(c.fnode.upload(node.data(), node.size(), c.s));
+  CR_TRY(c.feptr.upload(eptr.data(), eptr.size(), c.s));
   CR_TRY(c.ftptr.upload(ptr.data(), ptr.size(), c.s));
   CR_HIP(hipStreamSynchronize(c.s));
   c.fent_sig = sig;
