@@ -1184,8 +1184,44 @@ __global__ void face_valm_kernel(int n, int dof, int fdof, const int *__restrict
 // update of its kind (memLS's copy unCondU).  One 1024-thread workgroup per
 // face when no two share a node (then they do not see each other's
 // updates), one for all of them otherwise (each face in turn between
-// barriers).  Replaces a dot and an update launch per face and kind.
+// barriers).  Replaces a dot and an update launch per face and kind.  Faces that
+// share nodes and have more than kFaceSerial of them together take those launches
+// (face_dot, face_add): one workgroup walks them all too slowly.  30 Arnoldi steps of
+// GMRESV in one workgroup and in launches, ms: 8 faces with 1,100 nodes together 2.10
+// and 2.16, 24 with 3,300 3.40 and 3.45, 8 with 6,800 5.14 and 4.69, 24 with 13,700
+// 7.43 and 6.17, 56,000 20.1 and 10.8, 301,000 88 and 22.5.
 constexpr int kFaceAdd = 1, kFacePre = 2;
+constexpr size_t kFaceSerial = 4096;
+// F's valM . x, by 1024 threads
+template <class T>
+__device__ inline double face_dot(const FaceDev &F, int xdof, const T *__restrict__ x, double *sh) {
+  const int nc = F.dof < xdof ? F.dof : xdof;
+  double s = 0.0;
+  for (int a = threadIdx.x; a < F.nNo; a += 1024)
+    for (int i = 0; i < nc; ++i) s += F.valM[i + (size_t)F.dof * a] * (double)x[i + (size_t)xdof * F.glob[a]];
+  return block_sum_1024(s, sh);
+}
+template <class T>
+__global__ void __launch_bounds__(1024) face_dot_kernel(const FaceDev *__restrict__ fd, int xdof,
+                                                        const T *__restrict__ x, double *__restrict__ sum,
+                                                        const double *__restrict__ skip) {
+  if (skip && *skip != 0.0) return;
+  __shared__ double sh[16];
+  const double d = face_dot(fd[blockIdx.x], xdof, x, sh);
+  if (threadIdx.x == 0) sum[blockIdx.x] = d;
+}
+template <class T>
+__global__ void __launch_bounds__(256) face_add_kernel(const FaceDev *__restrict__ fd, int f, int kind, int xdof,
+                                                       const double *__restrict__ sum, T *__restrict__ Y,
+                                                       const double *__restrict__ skip) {
+  if (skip && *skip != 0.0) return;
+  const int a = blockIdx.x * 256 + threadIdx.x;
+  const FaceDev F = fd[f];
+  if (a >= F.nNo) return;
+  const double c = (kind == kFaceAdd ? F.res : *F.coefp) * sum[f];
+  const int nc = F.dof < xdof ? F.dof : xdof;
+  for (int i = 0; i < nc; ++i) Y[i + (size_t)xdof * F.glob[a]] += (T)(F.valM[i + (size_t)F.dof * a] * c);
+}
 template <class T>
 __global__ void __launch_bounds__(1024) face_apply_kernel(const FaceDev *__restrict__ fd, int nfc, int what, int xdof,
                                                           const T *__restrict__ X, T *__restrict__ Y,
@@ -1193,13 +1229,7 @@ __global__ void __launch_bounds__(1024) face_apply_kernel(const FaceDev *__restr
   if (skip && *skip != 0.0) return;
   __shared__ double sh[16];
   const int f0 = gridDim.x > 1 ? blockIdx.x : 0, f1 = gridDim.x > 1 ? f0 + 1 : nfc;
-  auto dot = [&](const FaceDev &F, const T *x) {
-    const int nc = F.dof < xdof ? F.dof : xdof;
-    double s = 0.0;
-    for (int a = threadIdx.x; a < F.nNo; a += 1024)
-      for (int i = 0; i < nc; ++i) s += F.valM[i + (size_t)F.dof * a] * (double)x[i + (size_t)xdof * F.glob[a]];
-    return block_sum_1024(s, sh);
-  };
+  auto dot = [&](const FaceDev &F, const T *x) { return face_dot(F, xdof, x, sh); };
   auto add = [&](const FaceDev &F, double c) {
     const int nc = F.dof < xdof ? F.dof : xdof;
     for (int a = threadIdx.x; a < F.nNo; a += 1024)
@@ -1779,6 +1809,7 @@ struct Ctx {
   crimson::DBuf<double> fpart;   // the Schur CG's face dot parts (kFaceDotBlocks per face)
   std::vector<FaceDev> hfdev;    // fdev on the host
   bool disjoint = true;          // no two coupled faces share a node
+  size_t fnodes = 0;             // the coupled faces' nodes together
   int nfc() const { return (int)hfdev.size(); }
   // their merged supports (FaceList), for the faces whose supports fent_sig lists
   std::vector<unsigned long long> fent_sig;
@@ -2537,8 +2568,19 @@ int dots(Ctx<T> &c, size_t L, const T *v, const T *U0, size_t ustride, int m, bo
 template <class T>
 int face_apply(Ctx<T> &c, int what, int xdof, const T *X, T *Y, const double *skip) {
   if (c.nfc() == 0) return CRIMSON_OK;
-  face_apply_kernel<T><<<c.disjoint ? c.nfc() : 1, 1024, 0, c.s>>>(c.fdev.p, c.nfc(), what, xdof, X, Y, c.fsum.p,
-                                                                  skip);
+  if (c.disjoint || c.fnodes <= kFaceSerial) {
+    face_apply_kernel<T><<<c.disjoint ? c.nfc() : 1, 1024, 0, c.s>>>(c.fdev.p, c.nfc(), what, xdof, X, Y, c.fsum.p,
+                                                                    skip);
+  } else {
+    for (int kind = kFaceAdd; kind <= kFacePre; kind <<= 1) {
+      if (!(what & kind)) continue;
+      face_dot_kernel<T><<<c.nfc(), 1024, 0, c.s>>>(c.fdev.p, xdof, kind == kFaceAdd ? X : Y, c.fsum.p, skip);
+      for (int f = 0; f < c.nfc(); ++f)
+        if (c.hfdev[f].nNo > 0)
+          face_add_kernel<T><<<crimson::grid_for(c.hfdev[f].nNo, 256), 256, 0, c.s>>>(c.fdev.p, f, kind, xdof,
+                                                                                     c.fsum.p, Y, skip);
+    }
+  }
   CR_HIP(hipGetLastError());
   return CRIMSON_OK;
 }
@@ -2853,6 +2895,7 @@ int face_setup(Ctx<T> &c, const int *incL, const double *res, bool ns) {
   crimson_lhs *l = c.lhs;
   std::vector<FaceDev> fd;
   int n = 0;
+  c.fnodes = 0;
   for (int f = 0; f < l->nFaces; ++f) {
     CrFace &fa = l->face[f];
     fa.inc = !(incL && incL[f] == 0);
@@ -2882,6 +2925,7 @@ int face_setup(Ctx<T> &c, const int *incL, const double *res, bool ns) {
     d.q = ns ? fa.d_q.p : nullptr;
     d.nsup = ns ? fa.nsup : 0;
     fd.push_back(d);
+    c.fnodes += fa.nNo;
   }
   c.disjoint = faces_disjoint(l);
   const bool same = fd.size() == c.hfdev.size() && c.fdev.p &&

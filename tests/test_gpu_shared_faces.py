@@ -1,8 +1,9 @@
 """Many coupled faces on the same nodes: the NS solver's result against a dense
 direct solve of the system with the faces' rank-one terms, on a graph whose
 Schur complement is formed and on one that keeps the two passes, with fewer and with
-more faces than a workgroup of the residual update keeps in LDS (256); and the time
-of its CG against one face's.
+more faces than a workgroup of the residual update keeps in LDS (256); the time
+of its CG against one face's; and faces with so many shared nodes that ADDBCMUL
+takes its launches per face, against one face of the same term.
 
 Tolerance: test_gpu_schur's (1e-5 of the residual asked, condition numbers
 under 1e4: 1e-2 of the solution's norm).  Without the faces' terms the solution
@@ -43,13 +44,15 @@ def test_shared_faces_against_direct(hub, count):
     assert np.linalg.norm(x - d) <= 1e-2 * np.linalg.norm(d)
 
 
-def test_shared_faces_cost():
-    """100 CG iterations on a cylinder of 115,961 nodes: with 24 coupled faces on the
-    outlet's 1,709 nodes at most four times as long as with one."""
+@pytest.mark.parametrize("kind,grid", [("CG", (48, 48, 60)), ("GMRES", (96, 96, 12))])
+def test_shared_faces_cost(kind, grid):
+    """100 CG iterations on a cylinder of 115,961 nodes, 30 Arnoldi steps on one of 96,525:
+    with 24 coupled faces on the outlet's 1,709 and 7,041 nodes at most four times as
+    long as with one."""
     import torch
     import crimsonflowsolver_amd as cfa
     from crimsonflowsolver_amd import mesh as M
-    m = M.cylinder_mesh(48, 48, 60)
+    m = M.cylinder_mesh(*grid)
     colm, rowp = cfa.genadj(m.ien, m.numnp)
     y, ac = M.poiseuille_state(m, seed=5)
     ibc, _ = M.dirichlet_codes(m)
@@ -67,8 +70,11 @@ def test_shared_faces_cost():
         form.to_lhs(T(y), T(ac), T(m.x), rhs, lhs)
         form.bc3res(rhs, res4_layout=True)
         form.sync()
-        ls = cfa.memLS_LS_CREATE(cfa.LS_TYPE_NS, relTol=1e-12, dimKry=1, maxItr=1, relTolIn=[0.9, 1e-30],
-                                 absTolIn=[1e-30, 1e-30], maxItrIn=[1, 100])
+        if kind == "CG":
+            ls = cfa.memLS_LS_CREATE(cfa.LS_TYPE_NS, relTol=1e-12, dimKry=1, maxItr=1, relTolIn=[0.9, 1e-30],
+                                     absTolIn=[1e-30, 1e-30], maxItrIn=[1, 100])
+        else:
+            ls = cfa.memLS_LS_CREATE(cfa.LS_TYPE_GMRES, relTol=1e-30, absTol=1e-30, dimKry=30, maxItr=1)
         best = 1e9
         for _ in range(4):
             x = rhs.clone()
@@ -76,7 +82,52 @@ def test_shared_faces_cost():
             t = time.perf_counter()
             cfa.memLS_SOLVE_dev(lhs, ls, 4, x, res=np.array([0.0] + [0.3 / count] * count))
             best = min(best, time.perf_counter() - t)
-        assert ls.stats("CG")["itr"] == 100
+        assert (ls.stats("CG")["itr"] == 100) if kind == "CG" else (ls.RI["itr"] == 31)
         ms.append(1e3 * best)
-    print("ms", ms)
-    assert ms[1] <= 4.0 * ms[0]
+    assert ms[1] <= 4.0 * ms[0], ms
+
+
+@pytest.mark.parametrize("bits", [64, 32])
+@pytest.mark.parametrize("kind", ["NS", "GMRES"])
+def test_large_shared_faces_against_one(kind, bits):
+    """Three faces of 2,000 nodes each, all the same with a third of the coefficient,
+    are one face's rank-one term.  Tolerance: both solves to 1e-6 (FP32: 1e-5) of a system
+    with condition number under 1e3.  (NSSOLVER's GE takes pivots under 4.4e-16 as
+    singular, and its Gram matrix holds squares of the residual: 1e-9 is out of its
+    reach.)"""
+    import torch
+    import crimsonflowsolver_amd as cfa
+    n = 6000
+    i = np.arange(n)
+    cols = np.sort((i[:, None] + np.arange(-2, 3)) % n, axis=1)
+    rng = np.random.default_rng(3)
+    val = np.zeros((16, 5 * n), order="F")
+    val[[0, 5, 10, 15]] = np.where((cols == i[:, None]).ravel(), 2.0, -0.1)
+    key = {(a, b): a * 5 + k for a in range(n) for k, b in enumerate(cols[a])}
+    g = 0.2 * rng.uniform(-1, 1, (3, 5 * n))
+    val[[3, 7, 11]] = g
+    val[12:15] = -g[:, [key[(b, a)] for a in range(n) for b in cols[a]]]
+    rhs = torch.from_numpy(1e3 * (rng.standard_normal((n, 4)) + 1.0)).cuda()
+    nodes = np.arange(100, 4100, 2)
+    v = rng.uniform(0.2, 1.0, (3, nodes.size)) / np.sqrt(nodes.size)
+    tol = 1e-6 if bits == 64 else 1e-5
+    out = []
+    for count in (0, 1, 3):
+        lhs = cfa.memLS_LHS_CREATE(n, n, 5 * n, None, (5 * np.arange(n + 1) + 1).astype(np.int32),
+                                   (cols.ravel() + 1).astype(np.int32), max(count, 1))
+        for f in range(count):
+            cfa.memLS_BC_CREATE(lhs, f + 1, nodes.size, 3, cfa.BC_TYPE_Neu, nodes + 1, np.asfortranarray(v))
+        lhs.set_val(4, val)
+        lhs.set_precision(bits)
+        if kind == "NS":
+            ls = cfa.memLS_LS_CREATE(cfa.LS_TYPE_NS, relTol=tol, dimKry=40, maxItr=12, relTolIn=[0.01, 0.01],
+                                     maxItrIn=[2, 200])
+        else:
+            ls = cfa.memLS_LS_CREATE(cfa.LS_TYPE_GMRES, relTol=tol, dimKry=60, maxItr=6)
+        x = rhs.clone()
+        cfa.memLS_SOLVE_dev(lhs, ls, 4, x, res=np.full(count, 30.0 / max(count, 1)) if count else None)
+        assert ls.RI["suc"] == 1
+        out.append(x.cpu().numpy())
+    without, one, three = out
+    assert np.linalg.norm(without - one) > 0.1 * np.linalg.norm(one)
+    assert np.linalg.norm(three - one) <= (1e-3 if bits == 64 else 1e-2) * np.linalg.norm(one)
