@@ -181,21 +181,32 @@ struct FaceDev {
   const double *q;
   int nsup;
 };
-// Workgroups per face computing S_f's partial sums beside the direction update.
-constexpr int kFaceDotBlocks = 4;
+// Workgroups per face computing S_f's partial sums beside the direction update or the
+// product: kFaceDotBlocks for supports of up to kFaceDotShare entries each, twice as
+// many (2^kFaceDotMost at most) until a larger one's shares are so small, so that no
+// face's few workgroups outlast the sweep they stand beside.
+// An outlet of 37,585 nodes (support 77,000), 654,000 rows, FP32: 500 CG iterations took
+// 70.0 ms with four, 62.8 with 32.
+constexpr int kFaceDotLog = 2, kFaceDotBlocks = 1 << kFaceDotLog, kFaceDotMost = 6, kFaceDotShare = 4096;
 // The faces' supports merged for the residual update: the nodes of any of them,
-// ascending, each with its entries (face, place in the face's support) in face
-// order; tptr[t] is the first of the nodes 256 t and above.
+// ascending, each with its first entry (face, place in the face's support) and where
+// the others lie in ent, in face order; tptr[t] is the first of the nodes 256 t and
+// above.
 struct FaceEnt {
   int f, s;
 };
+struct FaceNode {
+  int node, more, end;
+  FaceEnt first;
+};
 struct FaceList {
   int nfc;               // coupled faces
+  int nb, lb;            // workgroups, and partial sums of S_f, per face; nb = 1 << lb
   const FaceDev *fd;
-  const int *node, *eptr;  // the nodes and their first entries
+  const FaceNode *node;
   const FaceEnt *ent;
   const int *tptr;       // (N / 256 rounded up) + 1 entries
-  double *part;          // kFaceDotBlocks partial sums of S_f per face
+  double *part;          // nb partial sums of S_f per face
 };
 // Faces whose terms c_f S_f a workgroup of the residual update keeps in LDS; a node's
 // entries then cost it two loads each.  (329,000 rows, 24 faces on the same 12,637
@@ -580,16 +591,23 @@ __global__ void __launch_bounds__(256) s_product_kernel(int nNo, int ntile, cons
 }
 // The sum of n <= kCgGrid parts, in every thread, always in the same order: every
 // thread's parts are loaded together (one wait instead of eight).
-__device__ inline double sum_parts(const double *__restrict__ part, int n, double more, double *sh) {
-  double v[kCgGrid / 256];
+constexpr int kPartLoads = kCgGrid / 256;
+__device__ inline void load_parts(const double *__restrict__ part, int n, double (&v)[kPartLoads]) {
 #pragma unroll
-  for (int u = 0; u < kCgGrid / 256; ++u) {
+  for (int u = 0; u < kPartLoads; ++u) {
     const int b = threadIdx.x + 256 * u;
     v[u] = b < n ? part[b] : 0.0;
   }
+}
+__device__ inline double sum_loaded(const double (&v)[kPartLoads], double more, double *sh) {
 #pragma unroll
-  for (int u = 0; u < kCgGrid / 256; ++u) more += v[u];
+  for (int u = 0; u < kPartLoads; ++u) more += v[u];
   return block_sum_all(more, sh);
+}
+__device__ inline double sum_parts(const double *__restrict__ part, int n, double more, double *sh) {
+  double v[kPartLoads];
+  load_parts(part, n, v);
+  return sum_loaded(v, more, sh);
 }
 
 // gst (double, device): the state of the solve and of its last GMRES and
@@ -1336,29 +1354,34 @@ __device__ inline void check_next(double *scal) {
 }
 __device__ inline double face_coef(const FaceDev &F) { return *F.coefp; }
 __device__ inline double face_sum(const FaceList &fl, int f) {
+  const double *p = fl.part + (f << fl.lb);
   double S = 0.0;
+  for (int b0 = 0;;) {
 #pragma unroll
-  for (int b = 0; b < kFaceDotBlocks; ++b) S += fl.part[f * kFaceDotBlocks + b];
+    for (int b = 0; b < kFaceDotBlocks; ++b) S += p[b0 + b];
+    b0 += kFaceDotBlocks;
+    if (b0 >= fl.nb) break;
+  }
   return S;
 }
-// Workgroup b of a face's kFaceDotBlocks: its share of q_f . P, entries
-// b * 256 + t + 1024 u; p_at(j) gives the direction at column j.
+// Workgroup b of a face's nb: its share of q_f . P, entries b * 256 + t +
+// 256 nb u; p_at(j) gives the direction at column j.
 template <class P>
 __device__ inline void face_part(const FaceList &fl, int wg, double *sh, P p_at) {
-  const int f = wg / kFaceDotBlocks, b = wg % kFaceDotBlocks;
+  const int f = wg >> fl.lb, b = wg & (fl.nb - 1);
   const int *sup = fl.fd[f].sup;
   const double *q = fl.fd[f].q;
   const int ns = fl.fd[f].nsup;
   double s = 0.0;
-  constexpr int kStep = 256 * kFaceDotBlocks;
-  for (int e0 = b * 256 + threadIdx.x; e0 < ns; e0 += 4 * kStep) {  // four entries' loads together
+  const int step = 256 << fl.lb;
+  for (int e0 = b * 256 + threadIdx.x; e0 < ns; e0 += 4 * step) {  // four entries' loads together
     int j[4];
     double qv[4];
 #pragma unroll
     for (int u = 0; u < 4; ++u) {
-      const int e = min(e0 + kStep * u, ns - 1);
+      const int e = min(e0 + step * u, ns - 1);
       j[u] = sup[e];
-      qv[u] = e0 + kStep * u < ns ? q[e] : 0.0;
+      qv[u] = e0 + step * u < ns ? q[e] : 0.0;
     }
 #pragma unroll
     for (int u = 0; u < 4; ++u) s += qv[u] * (double)p_at(j[u]);
@@ -1453,6 +1476,8 @@ __global__ void __launch_bounds__(256) cg_r_kernel(size_t L, double *__restrict_
   size_t base = (size_t)blockIdx.x * (E * 256);
   load(base);  // all in flight while the parts are summed
   range(base);
+  double pv[kPartLoads];
+  load_parts(dpart, nd, pv);
   double d = 0.0;
   for (int f = threadIdx.x; f < fl.nfc; f += 256) {
     const double S = face_sum(fl, f), cS = face_coef(fl.fd[f]) * S;
@@ -1460,7 +1485,7 @@ __global__ void __launch_bounds__(256) cg_r_kernel(size_t L, double *__restrict_
     if (f < kFaceLds) fc[f] = cS;
   }
   if (stop != 0.0) return;
-  const double den = sum_parts(dpart, nd, d, sh);
+  const double den = sum_loaded(pv, d, sh);
   const double a = errO / den;  // CGRAD's alpha
   if (blockIdx.x == 0 && threadIdx.x == 0) scal[3] = a;
   const T alpha = (T)a;
@@ -1470,14 +1495,15 @@ __global__ void __launch_bounds__(256) cg_r_kernel(size_t L, double *__restrict_
 #pragma unroll
       for (int t = 0; t < E; ++t) corr[threadIdx.x + 256 * t] = T(0);
       __syncthreads();
+      auto term = [&](FaceEnt en) {
+        const FaceDev &F = fl.fd[en.f];
+        return (en.f < kFaceLds ? fc[en.f] : face_coef(F) * face_sum(fl, en.f)) * F.q[en.s];
+      };
       for (int e = e0 + threadIdx.x; e < e1; e += 256) {
-        double v = 0.0;
-        for (int x = fl.eptr[e]; x < fl.eptr[e + 1]; ++x) {
-          const FaceEnt en = fl.ent[x];
-          const FaceDev &F = fl.fd[en.f];
-          v += (en.f < kFaceLds ? fc[en.f] : face_coef(F) * face_sum(fl, en.f)) * F.q[en.s];
-        }
-        corr[fl.node[e] - (int)base] = (T)v;
+        const FaceNode fn = fl.node[e];
+        double v = term(fn.first);
+        for (int x = fn.more; x < fn.end; ++x) v += term(fl.ent[x]);
+        corr[fn.node - (int)base] = (T)v;
       }
       __syncthreads();
 #pragma unroll
@@ -1517,7 +1543,7 @@ __global__ void __launch_bounds__(256) cg_p_kernel(size_t L, const double *__res
                                                    const T *__restrict__ P, T *__restrict__ Pn,
                                                    const T *__restrict__ W, int wdof, int off, T *__restrict__ Ps,
                                                    HostFlag hf) {
-  const int nf = fl.nfc * kFaceDotBlocks, blk = (int)blockIdx.x - nf;
+  const int nf = fl.nfc * fl.nb, blk = (int)blockIdx.x - nf;
   __shared__ double sh[4];
   const double stop = scal[5], errO = scal[1], al = scal[3];
   T r[E], p[E], x[E];
@@ -1626,7 +1652,7 @@ __global__ void __launch_bounds__(256) s_dir_product_kernel(int nNo, int ntile, 
                                                         HostFlag hf) {
   __shared__ double sh[4];
   const double stop = scal[5];
-  const int nf = fl.nfc * kFaceDotBlocks, blk = (int)blockIdx.x - nf, nwg = (int)gridDim.x - nf;
+  const int nf = fl.nfc * fl.nb, blk = (int)blockIdx.x - nf, nwg = (int)gridDim.x - nf;
   const int lane = threadIdx.x % kSLanes;
   auto row_of = [&](int vb) {
     return (int)crimson::xcd_block(kRowXcdChunk, vb, ntile) * (256 / kSLanes) + (int)threadIdx.x / kSLanes;
@@ -1806,16 +1832,18 @@ struct Ctx {
   crimson::DBuf<FaceDev> fdev;   // the coupled faces, in face order
   crimson::DBuf<double> fcoef;   // their PRE coefficients
   crimson::DBuf<double> fsum;    // one dot per coupled face (face_apply_kernel)
-  crimson::DBuf<double> fpart;   // the Schur CG's face dot parts (kFaceDotBlocks per face)
+  crimson::DBuf<double> fpart;   // the Schur CG's face dot parts (1 << flb per face)
+  int flb = 0;
   std::vector<FaceDev> hfdev;    // fdev on the host
   bool disjoint = true;          // no two coupled faces share a node
   size_t fnodes = 0;             // the coupled faces' nodes together
   int nfc() const { return (int)hfdev.size(); }
   // their merged supports (FaceList), for the faces whose supports fent_sig lists
   std::vector<unsigned long long> fent_sig;
-  crimson::DBuf<int> fnode, feptr, ftptr;
+  crimson::DBuf<FaceNode> fnode;
   crimson::DBuf<FaceEnt> fent;
-  FaceList face_list() const { return FaceList{nfc(), fdev.p, fnode.p, feptr.p, fent.p, ftptr.p, fpart.p}; }
+  crimson::DBuf<int> ftptr;
+  FaceList face_list() const { return FaceList{nfc(), 1 << flb, flb, fdev.p, fnode.p, fent.p, ftptr.p, fpart.p}; }
 
   int init(crimson_lhs *l, int d, hipStream_t st) {
     lhs = l;
@@ -1916,7 +1944,7 @@ int cg_sweeps(Ctx<T> &c, size_t L, int it, int nd, const CgAux<T> &ax, T *X, T *
   double *scal = c.cgst.p + (it & 1) * kCgState, *next = c.cgst.p + ((it + 1) & 1) * kCgState;
   double *dpart = c.part.p, *rpart = c.part.p + kCgGrid;
   const CgGrid g = cg_grid(L);
-  const int gp = g.blocks + ax.fl.nfc * kFaceDotBlocks;
+  const int gp = g.blocks + ax.fl.nfc * ax.fl.nb;
   if (g.entries == 1) {
     cg_r_kernel<T, 1, false><<<g.blocks, 256, 0, c.s>>>(L, scal, dpart, nd, ax.fl, R, SP, rpart, nullptr, nullptr,
                                                         nullptr);
@@ -1935,7 +1963,7 @@ int cg_sweeps(Ctx<T> &c, size_t L, int it, int nd, const CgAux<T> &ax, T *X, T *
 template <class T>
 int cg_begin_vec(Ctx<T> &c, size_t L, const CgAux<T> &ax, T *X, T *R, T *P, const double *skip) {
   cg_begin_vec_kernel<T><<<crimson::grid_for(L, 256), 256, 0, c.s>>>(L, X, R, P, ax.W, ax.wdof, ax.off, ax.Ps, skip);
-  if (ax.fl.nfc > 0) cg_begin_face_kernel<T><<<ax.fl.nfc * kFaceDotBlocks, 256, 0, c.s>>>(ax.fl, P, skip);
+  if (ax.fl.nfc > 0) cg_begin_face_kernel<T><<<ax.fl.nfc * ax.fl.nb, 256, 0, c.s>>>(ax.fl, P, skip);
   CR_HIP(hipGetLastError());
   return CRIMSON_OK;
 }
@@ -2051,7 +2079,7 @@ int schur_dir_product(Ctx<T> &c, const SchurOp<T> &o, const PairT<T> *Q, T *P, T
                       int nr, const FaceList &fl, HostFlag hf, int &nd) {
   const int N = c.N, ntile = (int)crimson::grid_for((size_t)N, 256 / kSLanes);
   nd = std::min(ntile, kCgGrid);
-  const int G = nd + fl.nfc * kFaceDotBlocks;
+  const int G = nd + fl.nfc * fl.nb;
   const crimson::SchurPattern &p = *o.pat;
   double *dpart = c.part.p, *rpart = c.part.p + kCgGrid;
   if (p.col16.p)
@@ -2147,29 +2175,28 @@ int face_list(Ctx<T> &c) {
         ++total;
       }
   // sized by the entries, whatever the faces share: a capture's buffers stay in place
-  std::vector<int> node(total, 0), eptr(total + 1, 0), ptr((size_t)(N + 255) / 256 + 1, 0);
+  std::vector<FaceNode> node(total, FaceNode{});
   std::vector<FaceEnt> ent(total);
+  std::vector<int> ptr((size_t)(N + 255) / 256 + 1, 0);
   int u = 0, e = 0;
   for (int j = 0; j < N; ++j) {
     if (j % 256 == 0) ptr[j / 256] = u;
     if (count[j] == 0) continue;
-    node[u] = j;
-    eptr[u++] = e;
+    node[u++] = FaceNode{j, e + 1, e + count[j], FaceEnt{0, 0}};
     e += count[j];
     count[j] = e - count[j];  // the node's next entry
   }
   ptr.back() = u;
-  for (size_t k = u; k < eptr.size(); ++k) eptr[k] = e;
   int f = 0;
   for (const auto &fa : l->face) {
     if (!fa.coupled) continue;
     for (size_t k = 0; k < fa.h_sup.size(); ++k) ent[count[fa.h_sup[k]]++] = FaceEnt{f, (int)k};
     ++f;
   }
+  for (int k = 0; k < u; ++k) node[k].first = ent[node[k].more - 1];
   c.fent_sig.clear();
   CR_TRY(c.fent.upload(ent.data(), ent.size(), c.s));
   CR_TRY(c.fnode.upload(node.data(), node.size(), c.s));
-  CR_TRY(c.feptr.upload(eptr.data(), eptr.size(), c.s));
   CR_TRY(c.ftptr.upload(ptr.data(), ptr.size(), c.s));
   CR_HIP(hipStreamSynchronize(c.s));
   c.fent_sig = sig;
@@ -2909,7 +2936,6 @@ int face_setup(Ctx<T> &c, const int *incL, const double *res, bool ns) {
   }
   CR_TRY(c.fcoef.alloc(std::max(1, n)));
   CR_TRY(c.fsum.alloc(std::max(1, n)));
-  CR_TRY(c.fpart.alloc((size_t)std::max(1, n) * kFaceDotBlocks));
   for (auto &fa : l->face) {
     if (!fa.coupled) continue;
     CR_TRY(fa.d_valM.alloc((size_t)fa.dof * fa.nNo));
@@ -2927,6 +2953,11 @@ int face_setup(Ctx<T> &c, const int *incL, const double *res, bool ns) {
     fd.push_back(d);
     c.fnodes += fa.nNo;
   }
+  int longest = 0;
+  for (const FaceDev &d : fd) longest = std::max(longest, d.nsup);
+  c.flb = kFaceDotLog;
+  while ((kFaceDotShare << c.flb) < longest && c.flb < kFaceDotMost) ++c.flb;
+  CR_TRY(c.fpart.alloc((size_t)std::max(1, n) << c.flb));
   c.disjoint = faces_disjoint(l);
   const bool same = fd.size() == c.hfdev.size() && c.fdev.p &&
                     std::equal(fd.begin(), fd.end(), c.hfdev.begin(), [](const FaceDev &a, const FaceDev &b) {

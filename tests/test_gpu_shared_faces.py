@@ -3,7 +3,8 @@ direct solve of the system with the faces' rank-one terms, on a graph whose
 Schur complement is formed and on one that keeps the two passes, with fewer and with
 more faces than a workgroup of the residual update keeps in LDS (256); the time
 of its CG against one face's; and faces with so many shared nodes that ADDBCMUL
-takes its launches per face, against one face of the same term.
+takes its launches per face, against one face of the same term; and a face with a
+support so large that its dots take more workgroups.
 
 Tolerance: test_gpu_schur's (1e-5 of the residual asked, condition numbers
 under 1e4: 1e-2 of the solution's norm).  Without the faces' terms the solution
@@ -87,6 +88,55 @@ def test_shared_faces_cost(kind, grid):
     assert ms[1] <= 4.0 * ms[0], ms
 
 
+def _ring(n):
+    """A diagonally dominant system with D = -G^T on a ring of five blocks a row."""
+    i = np.arange(n)
+    cols = np.sort((i[:, None] + np.arange(-2, 3)) % n, axis=1)
+    rng = np.random.default_rng(3)
+    val = np.zeros((16, 5 * n), order="F")
+    val[[0, 5, 10, 15]] = np.where((cols == i[:, None]).ravel(), 2.0, -0.1)
+    key = {(a, b): a * 5 + k for a in range(n) for k, b in enumerate(cols[a])}
+    g = 0.2 * rng.uniform(-1, 1, (3, 5 * n))
+    val[[3, 7, 11]] = g
+    val[12:15] = -g[:, [key[(b, a)] for a in range(n) for b in cols[a]]]
+    return (5 * np.arange(n + 1) + 1).astype(np.int32), (cols.ravel() + 1).astype(np.int32), val, rng
+
+
+@pytest.mark.parametrize("bits", [64, 32])
+def test_face_of_many_nodes_against_direct(bits):
+    """A face of 18,000 nodes (a support past 16,384, whose dots take more than four
+    workgroups) and one of 100 against a sparse direct solve with the two rank-one
+    terms (Woodbury).  Tolerances as above."""
+    import scipy.sparse as sp
+    import scipy.sparse.linalg as sla
+    import torch
+    import crimsonflowsolver_amd as cfa
+    n = 20000
+    rowptr, colptr, val, rng = _ring(n)
+    faces = [(np.arange(500, 18500), 30.0), (np.arange(18400, 18500), 10.0)]
+    A = sp.bsr_matrix((val.T.reshape(-1, 4, 4), colptr - 1, rowptr - 1), shape=(4 * n, 4 * n)).tocsc()
+    R = 1e3 * (rng.standard_normal((n, 4)) + 1.0)
+    U = np.zeros((4 * n, 2))
+    lhs = cfa.memLS_LHS_CREATE(n, n, 5 * n, None, rowptr, colptr, 2)
+    for f, (nodes, r) in enumerate(faces):
+        v = rng.uniform(0.2, 1.0, (3, nodes.size)) / np.sqrt(nodes.size)
+        for c in range(3):
+            U[4 * nodes + c, f] = v[c] * np.sqrt(r)
+        cfa.memLS_BC_CREATE(lhs, f + 1, nodes.size, 3, cfa.BC_TYPE_Neu, nodes + 1, np.asfortranarray(v))
+    lu = sla.splu(A)
+    without, Z = lu.solve(R.ravel()), lu.solve(U)
+    d = without - Z @ np.linalg.solve(np.eye(2) + U.T @ Z, U.T @ without)
+    lhs.set_val(4, val)
+    lhs.set_precision(bits)
+    ls = cfa.memLS_LS_CREATE(cfa.LS_TYPE_NS, relTol=1e-6 if bits == 64 else 1e-5, dimKry=40, maxItr=12,
+                             relTolIn=[0.01, 0.01], maxItrIn=[2, 200])
+    x = torch.from_numpy(R).cuda()
+    cfa.memLS_SOLVE_dev(lhs, ls, 4, x, res=np.array([f[1] for f in faces]))
+    assert ls.RI["suc"] == 1
+    assert np.linalg.norm(without - d) > 0.1 * np.linalg.norm(d)
+    assert np.linalg.norm(x.cpu().numpy().ravel() - d) <= (1e-3 if bits == 64 else 1e-2) * np.linalg.norm(d)
+
+
 @pytest.mark.parametrize("bits", [64, 32])
 @pytest.mark.parametrize("kind", ["NS", "GMRES"])
 def test_large_shared_faces_against_one(kind, bits):
@@ -98,23 +148,14 @@ def test_large_shared_faces_against_one(kind, bits):
     import torch
     import crimsonflowsolver_amd as cfa
     n = 6000
-    i = np.arange(n)
-    cols = np.sort((i[:, None] + np.arange(-2, 3)) % n, axis=1)
-    rng = np.random.default_rng(3)
-    val = np.zeros((16, 5 * n), order="F")
-    val[[0, 5, 10, 15]] = np.where((cols == i[:, None]).ravel(), 2.0, -0.1)
-    key = {(a, b): a * 5 + k for a in range(n) for k, b in enumerate(cols[a])}
-    g = 0.2 * rng.uniform(-1, 1, (3, 5 * n))
-    val[[3, 7, 11]] = g
-    val[12:15] = -g[:, [key[(b, a)] for a in range(n) for b in cols[a]]]
+    rowptr, colptr, val, rng = _ring(n)
     rhs = torch.from_numpy(1e3 * (rng.standard_normal((n, 4)) + 1.0)).cuda()
     nodes = np.arange(100, 4100, 2)
     v = rng.uniform(0.2, 1.0, (3, nodes.size)) / np.sqrt(nodes.size)
     tol = 1e-6 if bits == 64 else 1e-5
     out = []
     for count in (0, 1, 3):
-        lhs = cfa.memLS_LHS_CREATE(n, n, 5 * n, None, (5 * np.arange(n + 1) + 1).astype(np.int32),
-                                   (cols.ravel() + 1).astype(np.int32), max(count, 1))
+        lhs = cfa.memLS_LHS_CREATE(n, n, 5 * n, None, rowptr, colptr, max(count, 1))
         for f in range(count):
             cfa.memLS_BC_CREATE(lhs, f + 1, nodes.size, 3, cfa.BC_TYPE_Neu, nodes + 1, np.asfortranarray(v))
         lhs.set_val(4, val)
