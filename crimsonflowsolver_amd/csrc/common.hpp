@@ -255,6 +255,7 @@ struct crimson_lhs {
   // whether this graph keeps the two-pass operator
   std::shared_ptr<const crimson::SchurPattern> spat;
   bool two_pass = false;
+  double lines = -1.0;  // lines_per_row, once it is asked for
   int band = 0;  // largest |column - row| (with d_col16)
   mutable std::mutex busy;  // held by a solve, a capture and a replay
   // the workspaces of the last plain solve in FP64 and in FP32 (work_take, work_keep)

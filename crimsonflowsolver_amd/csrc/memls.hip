@@ -1987,13 +1987,65 @@ bool try_alloc(B &b, size_t n) {
   return false;
 }
 
+// Whether S's columns fit 2-byte offsets (twice the graph's band).
+bool schur_narrow(const crimson_lhs *l) { return l->d_col16.p && 2 * l->band <= 32767; }
+// How scattered the numbering is: the distinct 16-entry lines that the columns of 16
+// consecutive rows name, per row, over a sample of the rows.  1 on a structured
+// numbering, 14 on the same mesh numbered at random.
+double lines_per_row(crimson_lhs *l) {
+  if (l->lines >= 0.0) return l->lines;
+  const int nt = std::max(1, l->nNo / 16), take = std::min(nt, 128);
+  size_t lines = 0, rows = 0;
+  std::vector<int> c;
+  for (int k = 0; k < take; ++k) {
+    const int r0 = 16 * (int)((long long)k * nt / take), r1 = std::min(r0 + 16, l->nNo);
+    c.assign(l->h_col.begin() + l->h_rowptr[r0], l->h_col.begin() + l->h_rowptr[r1]);
+    for (int &v : c) v /= 16;
+    std::sort(c.begin(), c.end());
+    lines += std::unique(c.begin(), c.end()) - c.begin();
+    rows += r1 - r0;
+  }
+  return l->lines = (double)lines / (double)rows;
+}
+// Whether S is formed, as far as the graph's size and numbering tell.  Up to
+// kCgPaired rows always: its two launches an iteration are what counts there.
+// Beyond, S saves bytes (a Kuhn mesh's 65 entries of 10 bytes a row against 14.7
+// blocks of 60; FP32 6 against 32; 2 more with 4-byte columns, of S, and 4 a block, of
+// the matrix) and pays in gathers, 65 a row instead of 29, which leave the L2 once
+// the vector has outgrown it and the numbering is scattered; in FP32, where it saves
+// least, once the mesh is large.  Ms of a loose NS solve, formed and two passes
+// (lines_per_row in brackets):
+//   FP64, 2-byte columns  141 k 6.9, 9.2; 458 k 27.3, 34.6; 1,078 k 75.6, 94.1
+//     4-byte [14]         141 k 12.5, 13.5; 327 k 34.6, 40.1; 390 k 51.3, 50.2;
+//                         458 k 65.8, 62.0; 1,078 k 265, 201
+//     [7.5]               270 k 19.3, 25.8; 458 k 45.2, 48.6; 1,078 k 160, 147
+//     [5.2]               458 k 39.4, 43.7; 1,078 k 124, 126
+//     [1]                 511 k 66.3, 73.7; 1,078 k 75.9, 94.1
+//   FP32, 2-byte columns  141 k 6.0, 6.8; 458 k 17.7, 18.4; 675 k 29.5, 31.5;
+//                         1,078 k 52.9, 50.9
+//     4-byte [14]         72 k 5.8, 5.8; 141 k 11.0, 9.9; 458 k 41.5, 40.5
+//     [7.5]               81 k 5.2, 5.6; 270 k 15.5, 16.3; 1,078 k 109, 100
+//     [1]                 300 k 27.7, 28.9; 378 k 31.1, 31.9; 486 k 38.1, 37.4;
+//                         1,078 k 52.9, 50.3
+bool schur_pays(crimson_lhs *l, bool fp32) {
+  const int N = l->nNo;
+  if (N <= kCgPaired) return true;
+  if (fp32) return schur_narrow(l) ? N <= 3 << 18 : N <= 3 << 17 && (l->d_col16.p || lines_per_row(l) <= 10.0);
+  if (N <= 5 << 16 || l->d_col16.p) return true;  // (2-byte columns: a window of 65,536 entries)
+  return lines_per_row(l) <= (N <= 1 << 19 ? 10.0 : 6.0);
+}
+
 // The pattern of S, built once per handle and kept with it until it is released
 // (release_idle_work); out stays empty where the graph keeps the two passes (two_pass)
-// or an allocation failed (the next solve tries again).  S is formed when its rows fit the value kernel's staging
-// (kSchurRow) and it has at most kSchurFill entries per block: the two passes
-// read 60 bytes per block (32 in FP32), S 10 (6) per entry plus the vector
-// work of one more launch.
-constexpr int kSchurFill = 6;
+// or an allocation failed (the next solve tries again).  A row of more than kSchurRow
+// entries, anywhere, keeps the whole graph on the two passes: so do the Delaunay
+// meshes of point clouds from about 6,500 nodes on, whose convex hull has a few nodes of
+// many neighbours (1 row of 6,480, 10 of 14,007); meshes of bounded degree have none
+// (a Delaunay mesh without its hull's slivers: 110 at most).  At most kSchurFill entries
+// per block, kSchurFillLong past kCgPaired rows (a block and an entry of FP64 and 4-byte
+// columns take as many bytes at 5.3).  At a fill of 4.8, ms formed and in two passes: 39 k
+// rows FP64 2.2, 2.8, FP32 1.8, 2.2; 238 k rows FP64 9.6, 11.5, FP32 7.5, 7.2.
+constexpr int kSchurFill = 6, kSchurFillLong = 5;
 template <class IX, class OX>
 int schur_pattern_fill(crimson_lhs *l, const IX *col, const crimson::SchurPattern &p, const OX *scol) {
   schur_pattern_kernel<IX, OX, true><<<crimson::grid_for(l->nNo, 4), 256, 0, l->stream>>>(
@@ -2021,18 +2073,19 @@ int schur_pattern(crimson_lhs *l, std::shared_ptr<const crimson::SchurPattern> &
   CR_HIP(hipMemcpyAsync(ptr.data() + 1, cnt.p, (size_t)N * sizeof(int), hipMemcpyDeviceToHost, l->stream));
   CR_HIP(hipStreamSynchronize(l->stream));
   ptr[0] = 0;
+  const long long fill = N <= kCgPaired ? kSchurFill : kSchurFillLong;
   for (int i = 1; i <= N; ++i) {
     p->row = std::max(p->row, ptr[i]);
     p->nnz += ptr[i];
     ptr[i] = (int)p->nnz;
-    if (p->row > kSchurRow || p->nnz > (long long)kSchurFill * l->nnz || p->nnz > 0x7fffff00LL) {
+    if (p->row > kSchurRow || p->nnz > fill * l->nnz || p->nnz > 0x7fffff00LL) {
       l->two_pass = true;
       return CRIMSON_OK;
     }
   }
   CR_TRY(p->ptr.upload(ptr.data(), ptr.size(), l->stream));
   CR_HIP(hipStreamSynchronize(l->stream));
-  const bool narrow = l->d_col16.p && 2 * l->band <= 32767;
+  const bool narrow = schur_narrow(l);
   if (!(narrow ? try_alloc(p->col16, (size_t)p->nnz) : try_alloc(p->col, (size_t)p->nnz))) return CRIMSON_OK;
   if (narrow)
     CR_TRY(schur_pattern_fill(l, l->d_col16.p, *p, p->col16.p));
@@ -2977,6 +3030,8 @@ int face_setup(Ctx<T> &c, const int *incL, const double *res, bool ns) {
 // passes are taken.
 template <class T>
 int schur_ready(SolveWork<T> &w, crimson_lhs *l) {
+  w.spat.reset();
+  if (!schur_pays(l, sizeof(T) == 4)) return CRIMSON_OK;
   CR_TRY(schur_pattern(l, w.spat));
   if (w.spat && !try_alloc(w.S, (size_t)w.spat->nnz)) w.spat.reset();
   return CRIMSON_OK;
