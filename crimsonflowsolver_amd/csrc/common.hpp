@@ -128,6 +128,14 @@ __device__ inline unsigned xcd_block(unsigned chunk, unsigned b, unsigned nb) {
 __device__ inline unsigned xcd_block(unsigned chunk) { return xcd_block(chunk, blockIdx.x, gridDim.x); }
 __device__ inline unsigned xcd_block() { return xcd_block(0u); }
 
+// Orders LDS accesses of the lanes of one wavefront (the lanes of a node or CSR row
+// always share a wavefront).
+__device__ inline void wave_lds_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 // Number of workgroups of `threads` covering n items.
 inline unsigned grid_for(size_t n, unsigned threads) {
   return (unsigned)((n + threads - 1) / threads);
@@ -196,7 +204,7 @@ struct crimson_graph {
 struct CrFace {
   int nNo = 0, dof = 0, bGrp = CRIMSON_BC_DIR;
   bool created = false, coupled = false, inc = true;
-  double res = 0.0, nS = 0.0;
+  double res = 0.0;
   std::vector<int> glob;      // 0-based node
   std::vector<double> val;    // (dof, nNo)
   crimson::DBuf<int> d_glob;

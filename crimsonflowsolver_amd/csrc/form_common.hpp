@@ -173,13 +173,7 @@ __device__ inline void load_record(const double *r, double (&nl)[kNRec]) {
   }
 }
 
-// Orders LDS accesses of the lanes of one wavefront (the lanes of a node or
-// CSR row always share a wavefront).
-__device__ inline void wave_lds_sync() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
+using crimson::wave_lds_sync;
 
 // Sum over the workgroup, in a fixed order, on thread 0.
 template <int THREADS>

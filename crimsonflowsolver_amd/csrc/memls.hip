@@ -37,11 +37,11 @@
 
 #include "common.hpp"
 
+using crimson::wave_lds_sync;
+
 namespace {
 
 constexpr int kRowLanes = 16;  // lanes per CSR row in the SpMV kernels
-constexpr int kRedThreads = 256;
-constexpr int kChunk = 1024;   // vector entries per workgroup in the dot sweeps
 // Row kernels deal their workgroups to the XCDs in turns of this many
 // (crimson::xcd_block(chunk)): rows gather the vector at neighbours a mesh
 // layer away, which the shared MALL then holds for all XCDs.  One FP64
@@ -256,13 +256,6 @@ constexpr int kNarrowUnroll = 4;
 // gathers both of its operands of a column as one 4-wide entry (two 16-byte
 // loads in FP64, one in FP32): SP_i = W_i (sum_j L_ij Ps_j - Gt_ij . Z(1:3, j)) + fix_i P_i.
 // `done`: the CG's converged flag; launches after it return at once.
-template <class T>
-__global__ void scale_p_kernel(int n, const T *__restrict__ W, int wdof, int off, const T *__restrict__ x,
-                               T *__restrict__ y, const double *__restrict__ done) {
-  if (done && *done != 0.0) return;
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) y[i] = W[off + (size_t)wdof * i] * x[i];
-}
 template <class T, class IX, int U = kNarrowUnroll>
 __global__ void __launch_bounds__(256) g_product_kernel(int nNo, const int *__restrict__ rowptr,
                                                         const IX *__restrict__ col, MatView<T> G,
@@ -389,12 +382,6 @@ __global__ void __launch_bounds__(256) schur_kernel(int nNo, const int *__restri
 // the passes read: schur_pattern) keeps the two passes.
 constexpr int kSchurRow = 320;   // entries of a row of S at most: 16 rows' staging fits 64 KB of LDS
 constexpr int kSchurHash = 512;  // LDS hash slots per row, a power of two above kSchurRow
-// Orders LDS accesses of the lanes of one wavefront.
-__device__ inline void wave_lds_sync() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
 // FILL false: cnt[row] = the row's entries (kSchurRow + 1 when it has more);
 // FILL true: the row's columns, ascending, at scol[sptr[row]] (as offsets
 // from the row when OX is short).
@@ -633,7 +620,6 @@ enum GstIdx : int {
   G_GM_DBPRE,
   G_GM_SCALE,
   G_GM_APPLY,
-  G_GM_RAN,
   G_GM_EARLY,
   G_GM_LASTF,  // fNorm and dB of the last GMRES call that ran to the end
   G_GM_LASTD,
@@ -1932,8 +1918,9 @@ struct CgAux {
 struct CgGrid {
   int entries, blocks;
 };
+constexpr size_t kCgWide = (size_t)256 * kCgGrid / 2;  // entries past which a thread takes four
 inline CgGrid cg_grid(size_t L) {
-  const int E = L > (size_t)256 * kCgGrid / 2 ? 4 : 1;
+  const int E = L > kCgWide ? 4 : 1;
   return CgGrid{E, (int)std::min<size_t>((L + (size_t)256 * E - 1) / ((size_t)256 * E), kCgGrid)};
 }
 // The iterations' vector work: iteration `it` after its operator left SP and nd
@@ -2295,7 +2282,6 @@ __global__ void __launch_bounds__(kDotThreads) ns_begin_kernel(double *__restric
 }
 // skip (may be null): the outer loop is over, the call does nothing
 __global__ void gm_begin_kernel(double *__restrict__ g, const double *__restrict__ skip) {
-  g[G_GM_RAN] = 0.0;
   g[G_GM_ARN] = 1.0;
   if (skip && *skip != 0.0) {
     g[G_GM_CYC] = 1.0;
@@ -2334,7 +2320,6 @@ __global__ void __launch_bounds__(kDotThreads) gm_cycle_kernel(double *__restric
   g[G_GM_DBPRE] = g[G_GM_FNORM];
   g[G_GM_SCALE] = 1.0 / e0;
   g[G_GM_ARN] = 0.0;
-  g[G_GM_RAN] = 1.0;
   g[G_GM_I] = 0.0;
 }
 __global__ void __launch_bounds__(kDotThreads) gm_givens_kernel(Givens G) {
@@ -2818,6 +2803,7 @@ int cg_run_paired(SolveWork<T> &w, const SchurOp<T> &o, size_t L, T *X, PairT<T>
   CR_TRY(dots(c, L, X, static_cast<const T *>(nullptr), 0, 0, true, c.part.p, skip));
   cg_begin_kernel<<<1, kDotThreads, 0, c.s>>>(c.cgst.p, g, skip, c.part.p, dot_blocks(L), absTol, relTol, mItr);
   cg_pair_kernel<T><<<crimson::grid_for(L, 256), 256, 0, c.s>>>(L, X, Q, skip);
+  static_assert(kCgPaired <= kCgWide, "one entry a thread");
   const CgGrid cg = cg_grid(L);
   double *dpart = c.part.p, *rpart = c.part.p + kCgGrid;
   auto st = [&](int it) { return c.cgst.p + (it & 1) * kCgState; };
@@ -2829,10 +2815,7 @@ int cg_run_paired(SolveWork<T> &w, const SchurOp<T> &o, size_t L, T *X, PairT<T>
     int nd = 0;
     CR_TRY(schur_dir_product(c, o, Q, P, SP, it ? st(it - 1) : st(0), it ? st(it) : nullptr, cg.blocks, fl,
                          it ? w.flag() : HostFlag{nullptr, 0}, nd));
-    if (cg.entries == 1)
-      cg_r_kernel<T, 1, true><<<cg.blocks, 256, 0, c.s>>>(L, st(it), dpart, nd, fl, nullptr, SP, rpart, Q, X, P);
-    else
-      cg_r_kernel<T, 4, true><<<cg.blocks, 256, 0, c.s>>>(L, st(it), dpart, nd, fl, nullptr, SP, rpart, Q, X, P);
+    cg_r_kernel<T, 1, true><<<cg.blocks, 256, 0, c.s>>>(L, st(it), dpart, nd, fl, nullptr, SP, rpart, Q, X, P);
     CR_HIP(hipGetLastError());
     bool stop = false;
     if (w.polled && it > kCgLag) CR_TRY(w.wait(s0 + it - kCgLag, &stop));
