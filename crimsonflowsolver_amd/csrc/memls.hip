@@ -207,13 +207,14 @@ struct FaceList {
   const FaceEnt *ent;
   const int *tptr;       // (N / 256 rounded up) + 1 entries
   double *part;          // nb partial sums of S_f per face
+  const double *coef;    // c_f
 };
 // Faces whose terms c_f S_f a workgroup of the residual update keeps in LDS; a node's
 // entries then cost it two loads each.  (329,000 rows, 24 faces on the same 12,637
 // nodes: an NS solve took 604 ms with every entry summing its face's parts again
 // and one thread walking a node's entries among its idle neighbours, 75 so; one
 // face 35.)
-constexpr int kFaceLds = 256;
+constexpr int kFaceLds = 256;  // one per thread
 
 // Wave-level sum (64 lanes) then across the 4 waves of a 256-thread group.
 template <class T>
@@ -578,23 +579,16 @@ __global__ void __launch_bounds__(256) s_product_kernel(int nNo, int ntile, cons
 }
 // The sum of n <= kCgGrid parts, in every thread, always in the same order: every
 // thread's parts are loaded together (one wait instead of eight).
-constexpr int kPartLoads = kCgGrid / 256;
-__device__ inline void load_parts(const double *__restrict__ part, int n, double (&v)[kPartLoads]) {
+__device__ inline double sum_parts(const double *__restrict__ part, int n, double more, double *sh) {
+  double v[kCgGrid / 256];
 #pragma unroll
-  for (int u = 0; u < kPartLoads; ++u) {
+  for (int u = 0; u < kCgGrid / 256; ++u) {
     const int b = threadIdx.x + 256 * u;
     v[u] = b < n ? part[b] : 0.0;
   }
-}
-__device__ inline double sum_loaded(const double (&v)[kPartLoads], double more, double *sh) {
 #pragma unroll
-  for (int u = 0; u < kPartLoads; ++u) more += v[u];
+  for (int u = 0; u < kCgGrid / 256; ++u) more += v[u];
   return block_sum_all(more, sh);
-}
-__device__ inline double sum_parts(const double *__restrict__ part, int n, double more, double *sh) {
-  double v[kPartLoads];
-  load_parts(part, n, v);
-  return sum_loaded(v, more, sh);
 }
 
 // gst (double, device): the state of the solve and of its last GMRES and
@@ -1338,16 +1332,12 @@ __device__ inline void check_next(double *scal) {
   scal[1] = scal[0];  // errO = err
   scal[6] += 1.0;
 }
-__device__ inline double face_coef(const FaceDev &F) { return *F.coefp; }
 __device__ inline double face_sum(const FaceList &fl, int f) {
   const double *p = fl.part + (f << fl.lb);
   double S = 0.0;
-  for (int b0 = 0;;) {
 #pragma unroll
-    for (int b = 0; b < kFaceDotBlocks; ++b) S += p[b0 + b];
-    b0 += kFaceDotBlocks;
-    if (b0 >= fl.nb) break;
-  }
+  for (int b = 0; b < kFaceDotBlocks; ++b) S += p[b];
+  for (int b = kFaceDotBlocks; b < fl.nb; ++b) S += p[b];
   return S;
 }
 // Workgroup b of a face's nb: its share of q_f . P, entries b * 256 + t +
@@ -1462,16 +1452,27 @@ __global__ void __launch_bounds__(256) cg_r_kernel(size_t L, double *__restrict_
   size_t base = (size_t)blockIdx.x * (E * 256);
   load(base);  // all in flight while the parts are summed
   range(base);
-  double pv[kPartLoads];
-  load_parts(dpart, nd, pv);
-  double d = 0.0;
-  for (int f = threadIdx.x; f < fl.nfc; f += 256) {
-    const double S = face_sum(fl, f), cS = face_coef(fl.fd[f]) * S;
-    d += cS * S;
-    if (f < kFaceLds) fc[f] = cS;
+  // a face's first parts and coefficient are in flight with them; what follows from
+  // these is LDS work that a launch past the end of the solve need not do
+  double d = 0.0, fp[kFaceDotBlocks] = {}, cf = 0.0;
+  if ((int)threadIdx.x < fl.nfc) {
+#pragma unroll
+    for (int b = 0; b < kFaceDotBlocks; ++b) fp[b] = fl.part[(threadIdx.x << fl.lb) + b];
+    cf = fl.coef[threadIdx.x];
   }
   if (stop != 0.0) return;
-  const double den = sum_loaded(pv, d, sh);
+  if ((int)threadIdx.x < fl.nfc) {
+    double S = 0.0;
+#pragma unroll
+    for (int b = 0; b < kFaceDotBlocks; ++b) S += fp[b];
+    for (int b = kFaceDotBlocks; b < fl.nb; ++b) S += fl.part[(threadIdx.x << fl.lb) + b];
+    d = (fc[threadIdx.x] = cf * S) * S;
+  }
+  for (int f = threadIdx.x + kFaceLds; f < fl.nfc; f += kFaceLds) {
+    const double S = face_sum(fl, f);
+    d += fl.coef[f] * S * S;
+  }
+  const double den = sum_parts(dpart, nd, d, sh);
   const double a = errO / den;  // CGRAD's alpha
   if (blockIdx.x == 0 && threadIdx.x == 0) scal[3] = a;
   const T alpha = (T)a;
@@ -1483,7 +1484,7 @@ __global__ void __launch_bounds__(256) cg_r_kernel(size_t L, double *__restrict_
       __syncthreads();
       auto term = [&](FaceEnt en) {
         const FaceDev &F = fl.fd[en.f];
-        return (en.f < kFaceLds ? fc[en.f] : face_coef(F) * face_sum(fl, en.f)) * F.q[en.s];
+        return (en.f < kFaceLds ? fc[en.f] : fl.coef[en.f] * face_sum(fl, en.f)) * F.q[en.s];
       };
       for (int e = e0 + threadIdx.x; e < e1; e += 256) {
         const FaceNode fn = fl.node[e];
@@ -1829,7 +1830,7 @@ struct Ctx {
   crimson::DBuf<FaceNode> fnode;
   crimson::DBuf<FaceEnt> fent;
   crimson::DBuf<int> ftptr;
-  FaceList face_list() const { return FaceList{nfc(), 1 << flb, flb, fdev.p, fnode.p, fent.p, ftptr.p, fpart.p}; }
+  FaceList face_list() const { return FaceList{nfc(), 1 << flb, flb, fdev.p, fnode.p, fent.p, ftptr.p, fpart.p, fcoef.p}; }
 
   int init(crimson_lhs *l, int d, hipStream_t st) {
     lhs = l;
