@@ -366,8 +366,8 @@ class ElmGMRInterior:
     def wall_alpha(self, uold, u, ualpha):
         check(lib().crimson_wall_alpha_dev(self.h, _p(uold), _p(u), _p(ualpha)), "crimson_wall_alpha_dev")
 
-    # row schedule (numbering, Morton, Morton-ordered runs of 64 rows) / FP64 incidence chunk /
-    # XCD dealing (one range per XCD, or turns of 64 workgroups)
+    # row schedule (numbering, Morton, Morton-ordered runs of 64 rows) / FP64 incidence chunk
+    # ("16": as many as the row's lanes, 16 or 32) / XCD dealing (one range per XCD, or turns of 64 workgroups)
     AUTOTUNE_CANDIDATES = tuple(f"{s}/{c}/{d}" for d in ("range", "turns64") for c in (16, 8)
                                 for s in ("natural", "morton", "tiles"))
 

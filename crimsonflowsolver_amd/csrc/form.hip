@@ -15,7 +15,7 @@
 //               velocity blocks and the residual row rl_a, and the element
 //               scalars Tc, Mu, Cm, tlW from which every tangent entry is
 //               rebuilt (the residual rows alone without the tangent)
-//   asm_row     row-parallel, 16 lanes per CSR row, one lane per block: the
+//   asm_row     row-parallel, 16 or 32 lanes per CSR row, one lane per block: the
 //               row's incidence records read as one contiguous run, the
 //               shape gradients rebuilt from the packed nodes, the blocks of
 //               the row from the row's element incidences in element order
@@ -207,7 +207,7 @@ __global__ void __launch_bounds__(256) flux_node(int nshg, const int *__restrict
 // term by term per point (the form of e3res.f90 and e3lhs.f90) the kernel issued
 // 1,763 vector instructions per wave, this 1,185; it is bound by latency at two
 // waves a SIMD and by the record stores (1.8 GB at 6.2 M elements: 672 us before,
-// 557 now; without the tangent 663 before, 411 now).
+// 583 now; without the tangent 663 before, 411 now).
 // In: the nodal values.  Out: u -> ubar at the points, a -> (a + ubar . grad u) at
 // the points (RES), g of the first three nodes (g_4 is minus their sum), WdetJ.
 template <class T, bool RES, bool TAN>
@@ -1928,9 +1928,9 @@ extern "C" int crimson_form_interior_to_lhs(crimson_form *f, const double *d_y, 
 // Morton order of the nodes, or runs of consecutive rows in Morton order of
 // their centroids), its workgroups' dealing to the XCDs (a contiguous range
 // each, or turns of kAsmXcdChunk) and, for the FP64 assembly, its incidence
-// chunk (16 or 8).  No candidate changes a result: schedule and dealing
-// order rows, never sums, and both chunk sizes give incidence t to lane
-// t % 16.
+// chunk (the row's lanes, 16 or 32, or 8; the candidates' "16" is the former).  No
+// candidate changes a result: schedule and dealing order rows, never sums, and both
+// chunk sizes give incidence t to lane t % row_lanes.
 constexpr unsigned kAsmXcdChunk = 64;
 extern "C" int crimson_form_autotune(crimson_form *f, const double *d_y, const double *d_ac, const double *d_x,
                                      double *d_res, crimson_lhs *lhs, int reps, int mask, int *choice,

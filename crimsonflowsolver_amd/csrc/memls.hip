@@ -212,8 +212,8 @@ struct FaceList {
 // Faces whose terms c_f S_f a workgroup of the residual update keeps in LDS; a node's
 // entries then cost it two loads each.  (329,000 rows, 24 faces on the same 12,637
 // nodes: an NS solve took 604 ms with every entry summing its face's parts again
-// and one thread walking a node's entries among its idle neighbours, 75 so; one
-// face 35.)
+// and one thread walking a node's entries among its idle neighbours, 69 so; one
+// face 32.)
 constexpr int kFaceLds = 256;  // one per thread
 
 // Wave-level sum (64 lanes) then across the 4 waves of a 256-thread group.
@@ -379,8 +379,7 @@ __global__ void __launch_bounds__(256) schur_kernel(int nNo, const int *__restri
 // directly (the scaling is in S).
 // The pattern is a property of the graph: built once per handle on the
 // device, one wave per row, the union of the neighbours' rows in an LDS hash
-// set.  A row with more than kSchurRow entries (or an S of more bytes than
-// the passes read: schur_pattern) keeps the two passes.
+// set.  Where S is not formed (schur_pays, schur_pattern) the two passes stay.
 constexpr int kSchurRow = 320;   // entries of a row of S at most: 16 rows' staging fits 64 KB of LDS
 constexpr int kSchurHash = 512;  // LDS hash slots per row, a power of two above kSchurRow
 // FILL false: cnt[row] = the row's entries (kSchurRow + 1 when it has more);
@@ -524,7 +523,8 @@ __global__ void __launch_bounds__(256) schur_values_kernel(int nNo, const int *_
 // most that many parts; the next tile's row pointers are loaded during a tile.
 // Bound by the read of S: 65 entries per row and 458,000 rows (297 MB) take 74 us,
 // 4.0 TB/s of a copy's 4.65; the two passes it replaces took 92 us.  A lane loads kSUnroll
-// entries at once, so that the Kuhn meshes' rows (65 at most) are one turn: 98 us
+// entries at once, so that the Kuhn meshes' rows (65 at most) are one turn (30 to 45 % of
+// a Delaunay mesh's rows have more than 80 entries and take a second): 98 us
 // with four, 90 with 8 lanes of eight, 99 with 32 lanes of two, 95 with a wave
 // per run of four rows summed through LDS; unbounded grid 67 us, but then a dot
 // kernel of its own follows.
@@ -3857,15 +3857,17 @@ struct SegCapture {
   }
 };
 
-// The launches one segment of a device-driven solve holds at most, from the
-// solver's limits (GMRES: per Arnoldi step about 16 launches, every coupled
-// face batched or not; CG: about 8 per iteration), checked before capturing.
+// An upper bound of the launches one segment of a device-driven solve holds, from the
+// solver's limits, checked before capturing: 16 launches an Arnoldi step and 4 more per
+// coupled face that is not batched, 8 a CG iteration and one per such face.  (Five to
+// seven a step, and two to five an iteration, are enqueued, 2 more per face a step where
+// the faces share many nodes; the bound keeps what a capture may ask for where it was.)
 int check_segment_budget(int mGM, int sD, int mCG, int nfc_launch) {
   const size_t gm = (size_t)mGM * ((size_t)sD * (16 + 4 * nfc_launch) + 16);
   const size_t cg = (size_t)mCG * (8 + nfc_launch) + 8;
   if (gm > kMaxSegmentLaunches || cg > kMaxSegmentLaunches) {
-    crimson::set_error("device-driven NS solve: a GMRES call of %d cycles x %d steps (%zu launches) or a CG call of "
-                       "%d iterations (%zu launches) exceeds the %zu launches a captured segment may hold",
+    crimson::set_error("device-driven NS solve: a GMRES call of %d cycles x %d steps (up to %zu launches) or a CG call "
+                       "of %d iterations (up to %zu launches) exceeds the %zu launches a captured segment may hold",
                        mGM, sD, gm, mCG, cg, kMaxSegmentLaunches);
     return CRIMSON_EUNSUPPORTED;
   }

@@ -231,7 +231,7 @@ int crimson_wall_alpha_dev(crimson_form *f, const double *d_uold,
  * candidate c = 0..11: row schedule c % 3 (0 the caller's numbering, 1
  * Morton order of the nodes, 2 runs of 64 consecutive rows in Morton order
  * of their centroids), 8-incidence assembly chunks if (c / 3) % 2 (else
- * 16; FP64 handles only), workgroups dealt to the XCDs in turns of 64 if
+ * as many as the row's lanes, 16 or 32; FP64 handles only), workgroups dealt to the XCDs in turns of 64 if
  * c / 6 (else one contiguous range per XCD).  mask selects the candidates
  * tried (bit c = candidate c; 0 = all valid ones).  *choice receives the
  * winner, ms_out (12 doubles, may be NULL) the mean assembly milliseconds
