@@ -2012,13 +2012,14 @@ double lines_per_row(crimson_lhs *l) {
 //   FP32, 2-byte columns  141 k 6.0, 6.8; 458 k 17.7, 18.4; 675 k 29.5, 31.5;
 //                         1,078 k 52.9, 50.9
 //     4-byte [14]         72 k 5.8, 5.8; 141 k 11.0, 9.9; 458 k 41.5, 40.5
-//     [7.5]               81 k 5.2, 5.6; 270 k 15.5, 16.3; 1,078 k 109, 100
+//     [7.5]               81 k 5.2, 5.6; 270 k 15.5, 16.3; 458 k 26.7, 31.1;
+//                         1,078 k 109, 100
 //     [1]                 300 k 27.7, 28.9; 378 k 31.1, 31.9; 486 k 38.1, 37.4;
-//                         1,078 k 52.9, 50.3
+//                         511 k 42.1, 40.0; 1,078 k 52.9, 50.3
 bool schur_pays(crimson_lhs *l, bool fp32) {
   const int N = l->nNo;
   if (N <= kCgPaired) return true;
-  if (fp32) return schur_narrow(l) ? N <= 3 << 18 : N <= 3 << 17 && (l->d_col16.p || lines_per_row(l) <= 10.0);
+  if (fp32) return schur_narrow(l) ? N <= 3 << 18 : N <= 15 << 15 && (l->d_col16.p || lines_per_row(l) <= 10.0);
   if (N <= 5 << 16 || l->d_col16.p) return true;  // (2-byte columns: a window of 65,536 entries)
   return lines_per_row(l) <= (N <= 1 << 19 ? 10.0 : 6.0);
 }
