@@ -1830,7 +1830,9 @@ struct Ctx {
   crimson::DBuf<FaceNode> fnode;
   crimson::DBuf<FaceEnt> fent;
   crimson::DBuf<int> ftptr;
-  FaceList face_list() const { return FaceList{nfc(), 1 << flb, flb, fdev.p, fnode.p, fent.p, ftptr.p, fpart.p, fcoef.p}; }
+  FaceList face_list() const {
+    return FaceList{nfc(), 1 << flb, flb, fdev.p, fnode.p, fent.p, ftptr.p, fpart.p, fcoef.p};
+  }
 
   int init(crimson_lhs *l, int d, hipStream_t st) {
     lhs = l;

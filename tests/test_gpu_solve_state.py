@@ -368,5 +368,6 @@ def test_failed_allocations_of_the_complement(cfa, tmp_path):
     subprocess.run(["gcc", "-shared", "-fPIC", "-o", str(lib), str(src), "-ldl"], check=True)
     root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
     env = dict(os.environ, PYTHONPATH=root)
-    out = subprocess.run([sys.executable, "-u", str(child), str(lib)], env=env, capture_output=True, text=True, timeout=100)
+    out = subprocess.run([sys.executable, "-u", str(child), str(lib)], env=env, capture_output=True, text=True,
+                         timeout=100)
     assert out.returncode == 0 and "CHILD_OK" in out.stdout, out.stdout[-2000:] + out.stderr[-2000:]
